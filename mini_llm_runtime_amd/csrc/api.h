@@ -81,6 +81,12 @@ int mlr_gemm_simple(const void* x, const void* w, const void* bias, int bias_is_
                     int out_is_f32, int swiglu, int dtype, int m, int n, int k, const void* multiply,
                     const int* multiply_rows, float glu_limit, float glu_alpha, hipStream_t stream);
 
+// The product of the 32-bit path on the matrix cores, in float32 throughout.  Needs k % 4 == 0 and 16-byte aligned
+// operands.  slices > 1 (a value mlr_gemm_f32_slices returned for this shape): as for mlr_gemm_bf16.
+int mlr_gemm_f32_slices(int m, int n, int k, int max_slices);
+int mlr_gemm_f32(const float* x, const float* w, const float* bias, float* y, int swiglu, int slices, int m, int n, int k,
+                 const float* multiply, const int* multiply_rows, float glu_limit, float glu_alpha, hipStream_t stream);
+
 // The same product in bfloat16 on the matrix cores (float32 accumulation).  Needs
 // k % 8 == 0 and 16-byte aligned x and w; any m and n.  With slices > 1 (a value
 // mlr_gemm_bf16_slices returned for this shape) y is float32 [slices, m, n]: partial
@@ -162,6 +168,7 @@ int mlr_gemm_merge_fused_bf16(const float* attn_partial, const int* context_lens
 // pool > 0 (with a window): beside its window a query also sees pooled entries, one key and value for every
 // run of `pool` positions whose last position is <= p - window, read from pages of their own (same layout,
 // `block_size` entries a page, entry b of a request at pooled_table[entry][b / block_size]) in the same softmax.
+// single_of (cu_q, or null): only the tokens of entries with one token; the other rows of `out` are left alone.
 int mlr_paged_attention_simple(const void* q, int64_t q_stride, const void* key_pages,
                                const void* value_pages, const int* block_table, int table_width,
                                const int* token_entry, const int* positions, void* out, int dtype,
@@ -169,7 +176,8 @@ int mlr_paged_attention_simple(const void* q, int64_t q_stride, const void* key_
                                int block_size, int num_pages, float scale, int window, int chunk,
                                const float* sinks, const void* pooled_keys, const void* pooled_values,
                                const int* pooled_table, int pooled_width, int pooled_pages, int pool,
-                               const float* score_bias, float softcap, int keep_first, hipStream_t stream);
+                               const float* score_bias, float softcap, int keep_first, const int* single_of,
+                               hipStream_t stream);
 
 // x (float32 [rows, hidden], in place) += weight * y * rsqrt(mean(y^2) + eps), y [rows, hidden] float32
 // or `dtype`, or `slices` float32 partial sums [slices, rows, hidden].  Then mode 1: out = next_weight * x *

@@ -1,0 +1,235 @@
+// float32 paged attention of prompt portions on the matrix cores, for one head size (MLR_HEAD_DIM, up to 80 and multiples of 32 up to 128): the
+// true 32-bit counterpart of the tiled kernel in attention_mfma.hip, with the same page layouts and the same lane
+// layouts (scores transposed, S^T[key, query], so that probabilities go from one product to the next in registers).
+//
+// v_mfma_f32_16x16x4_f32: D[16x16] += A[16x4] B[4x16].  Lane l holds A[row l % 16][k l / 16], B[k l / 16][col l % 16],
+// D[row (l / 16) * 4 + i][col l % 16].  The order of k is free as long as both sides agree, so a lane reads 4 consecutive k
+// (16 bytes) and product i of four takes element i of every lane.
+//
+// Bound by the matrix cores (256 operations a clock and compute unit in float32): a 64-key tile of 64 queries at head size 64 is
+// 4,096 clocks of them for 32 KB of keys and values, which one LDS buffer with the next tile on its way in registers keeps up
+// with; a workgroup takes 64 queries of one head, four wavefronts 16 each.
+// Measured at 0.5B sizes (14 query and 2 key/value heads of 64), prompts of 391, 268, 145 and 22 tokens in one step: 479 us with the
+// plain kernel (a wavefront per token and head, attention_simple.hip), 44 us here.
+#include "common.h"
+#include "mfma.h"
+
+#ifndef MLR_HEAD_DIM
+#error "compile with -DMLR_HEAD_DIM=<multiple of 16>"
+#endif
+
+#if MLR_HEAD_DIM <= 80 || (MLR_HEAD_DIM <= 128 && MLR_HEAD_DIM % 32 == 0)  // whole pieces for every thread, see below
+namespace mlr {
+namespace f32_attention {
+
+constexpr int D = MLR_HEAD_DIM;
+constexpr int kDimTiles = D / 16;
+constexpr int kTileQ = 64;                 // queries of a workgroup
+constexpr int kTileK = D > 80 ? 32 : 64;   // keys in LDS at a time
+constexpr int kSubTiles = kTileK / 16;
+// rows padded to 32 bytes modulo 64: 16 rows x 4 pieces of 16 bytes are then read without bank conflicts
+constexpr int kKLd = D + 8;
+constexpr int kVLd = kTileK + 8;
+constexpr int kPieces = kTileK * D / 4 / 256;  // 16-byte pieces of a thread, of the key and of the value tile
+static_assert(kTileK * D / 4 % 256 == 0, "whole pieces for every thread");
+
+__global__ __launch_bounds__(256) void attn_prefill_f32_kernel(
+    const float* __restrict__ q, int64_t q_stride, const float* __restrict__ key_pages, const float* __restrict__ value_pages,
+    const int* __restrict__ block_table, int table_width, const int* __restrict__ tiles, const int* __restrict__ cu_q,
+    const int* __restrict__ context_lens, float* __restrict__ out, int heads, int kv_heads, int block_size, int num_pages,
+    float scale, int window, int chunk, const float* __restrict__ sinks) {
+  __shared__ __attribute__((aligned(16))) float ks[kTileK * kKLd];
+  __shared__ __attribute__((aligned(16))) float vs[D * kVLd];
+  __shared__ int sm_bad;
+  const int tile = blockIdx.x / heads;
+  const int head = blockIdx.x - tile * heads;
+  const int kvh = head / (heads / kv_heads);
+  const int entry = tiles[2 * tile];
+  const int q0 = tiles[2 * tile + 1];
+  const int tid = threadIdx.x;
+  const int lane = tid % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int col = lane % 16, quarter = lane / 16;
+  const int t_first = cu_q[entry];
+  const int q_len = cu_q[entry + 1] - t_first;
+  const int pos0 = context_lens[entry] - q_len;
+  const int* table = block_table + static_cast<int64_t>(entry) * table_width;
+  if (tid == 0) sm_bad = 0;
+
+  const int qi = q0 + wave * 16 + col;
+  const bool q_ok = qi < q_len;
+  const int pq = pos0 + qi;
+  const int pq_first = first_visible_key(pq, window, chunk);
+  f32x4_t qo[kDimTiles];
+  const float* qrow = q + static_cast<int64_t>(t_first + (q_ok ? qi : 0)) * q_stride + static_cast<int64_t>(head) * D;
+#pragma unroll
+  for (int g = 0; g < kDimTiles; ++g) {
+    qo[g] = *reinterpret_cast<const f32x4_t*>(qrow + g * 16 + quarter * 4);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) qo[g][j] *= scale;
+  }
+
+  const int k_end = pos0 + min(q0 + kTileQ, q_len);           // one past the last key that a query here sees
+  const int k_first = first_visible_key(pos0 + q0, window, chunk);  // the first one
+  const int w_last = pos0 + min(q0 + wave * 16 + 15, q_len - 1);
+  const int w_first = first_visible_key(pos0 + q0 + wave * 16, window, chunk);
+  const int w_max_first = first_visible_key(pos0 + q0 + wave * 16 + 15, window, chunk);
+  const bool wave_has_queries = q0 + wave * 16 < q_len;
+
+  f32x4_t k_flight[kPieces], v_flight[kPieces];
+  bool bad = false;
+  auto fetch = [&](int kt0) {
+    if (kt0 >= k_end) return;
+#pragma unroll
+    for (int i = 0; i < kPieces; ++i) {
+      const int c = tid + i * 256;
+      const int key = kt0 + c / (D / 4), dim = c % (D / 4) * 4;
+      const int logical = min(key, k_end - 1) / block_size;
+      const int page = table[logical];
+      const bool in = static_cast<unsigned>(page) < static_cast<unsigned>(num_pages);
+      if (!in) bad = bad || (key < k_end && key >= k_first);
+      const int64_t base = static_cast<int64_t>(in ? page : 0) * kv_heads + kvh;
+      k_flight[i] = *reinterpret_cast<const f32x4_t*>(key_pages + (base * block_size + key % block_size) * D + dim);
+    }
+#pragma unroll
+    for (int i = 0; i < kPieces; ++i) {
+      const int c = tid + i * 256;
+      const int key = kt0 + c % (kTileK / 4) * 4, dim = c / (kTileK / 4);  // 4 keys: they lie in one page, whose size is a multiple of 4
+      const int logical = min(key, k_end - 1) / block_size;
+      const int page = table[logical];
+      const bool in = static_cast<unsigned>(page) < static_cast<unsigned>(num_pages);
+      const int64_t base = static_cast<int64_t>(in ? page : 0) * kv_heads + kvh;
+      f32x4_t v = *reinterpret_cast<const f32x4_t*>(value_pages + (base * D + dim) * block_size + key % block_size);
+      // values that no query here may see are cleared: what a page holds there may be anything, and 0 * NaN would come through
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (!in || key + e >= k_end || key + e < k_first) v[e] = 0.f;
+      v_flight[i] = v;
+    }
+  };
+  auto stash = [&]() {
+#pragma unroll
+    for (int i = 0; i < kPieces; ++i) {
+      const int c = tid + i * 256;
+      *reinterpret_cast<f32x4_t*>(ks + c / (D / 4) * kKLd + c % (D / 4) * 4) = k_flight[i];
+      *reinterpret_cast<f32x4_t*>(vs + c / (kTileK / 4) * kVLd + c % (kTileK / 4) * 4) = v_flight[i];
+    }
+  };
+
+  float m_run = -INFINITY, l_run = 0.f;
+  f32x4_t acc[kDimTiles];
+#pragma unroll
+  for (int dt = 0; dt < kDimTiles; ++dt) acc[dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+  const int k_begin = k_first / kTileK * kTileK;
+  fetch(k_begin);
+  for (int kt0 = k_begin; kt0 < k_end; kt0 += kTileK) {
+    __syncthreads();  // everybody has done with the tile before
+    stash();
+    __syncthreads();
+    fetch(kt0 + kTileK);  // on its way while this tile is computed
+    if (!(wave_has_queries && kt0 <= w_last && kt0 + kTileK > w_first)) continue;
+    f32x4_t s[kSubTiles];
+#pragma unroll
+    for (int sub = 0; sub < kSubTiles; ++sub) {
+      s[sub] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int g = 0; g < kDimTiles; ++g) {
+        const f32x4_t k = *reinterpret_cast<const f32x4_t*>(ks + (sub * 16 + col) * kKLd + g * 16 + quarter * 4);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) s[sub] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[j], qo[g][j], s[sub], 0, 0, 0);
+      }
+    }
+    if (!(kt0 + kTileK - 1 <= pos0 + q0 + wave * 16 && kt0 >= w_max_first)) {  // some query here does not see all of it
+#pragma unroll
+      for (int sub = 0; sub < kSubTiles; ++sub)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int key = kt0 + sub * 16 + quarter * 4 + i;
+          if (!(key <= pq && key >= pq_first)) s[sub][i] = -INFINITY;
+        }
+    }
+    float top = -INFINITY;
+#pragma unroll
+    for (int sub = 0; sub < kSubTiles; ++sub)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) top = fmaxf(top, s[sub][i]);
+    top = fmaxf(top, __shfl_xor(top, 16, kWave));
+    top = fmaxf(top, __shfl_xor(top, 32, kWave));
+    const float m_new = fmaxf(m_run, top);
+    const float m_use = m_new == -INFINITY ? 0.f : m_new;  // a query that has seen no key yet
+    const float alpha = m_run == -INFINITY ? 0.f : expf(m_run - m_use);
+    float sum = 0.f;
+#pragma unroll
+    for (int sub = 0; sub < kSubTiles; ++sub)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        s[sub][i] = expf(s[sub][i] - m_use);
+        sum += s[sub][i];
+      }
+    l_run = l_run * alpha + sum;
+    m_run = m_new;
+#pragma unroll
+    for (int dt = 0; dt < kDimTiles; ++dt) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[dt][i] *= alpha;
+#pragma unroll
+      for (int sub = 0; sub < kSubTiles; ++sub) {
+        const f32x4_t v = *reinterpret_cast<const f32x4_t*>(vs + (dt * 16 + col) * kVLd + sub * 16 + quarter * 4);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[i], s[sub][i], acc[dt], 0, 0, 0);
+      }
+    }
+  }
+  if (bad) atomicOr(&sm_bad, 1);
+  __syncthreads();
+  float l = l_run;
+  l += __shfl_xor(l, 16, kWave);
+  l += __shfl_xor(l, 32, kWave);
+  float keep = 1.0f;
+  if (sinks != nullptr) {  // one more term exp(sink) of the denominator, with no key and no value
+    const float sink = sinks[head];
+    const float m_new = fmaxf(m_run, sink);
+    keep = m_run == -INFINITY ? 0.f : expf(m_run - m_new);
+    l = l * keep + expf(sink - m_new);
+  }
+  if (!q_ok) return;
+  const float inv = sm_bad != 0 ? __builtin_nanf("") : keep / l;
+  float* orow = out + (static_cast<int64_t>(t_first + qi) * heads + head) * D;
+#pragma unroll
+  for (int dt = 0; dt < kDimTiles; ++dt) {
+    f32x4_t v = acc[dt];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] *= inv;
+    *reinterpret_cast<f32x4_t*>(orow + dt * 16 + quarter * 4) = v;
+  }
+}
+
+}  // namespace f32_attention
+}  // namespace mlr
+
+using namespace mlr;
+
+// Attention of the query tiles in `tiles` ([num_tiles][2]: entry, first query; 64 queries per tile) in float32, with the arguments
+// of mlr_attention_prefill.  A page id out of range among the keys that a tile sees makes the tile's rows NaN.
+extern "C" int mlr_attention_prefill_f32(const float* q, int64_t q_stride, const float* key_pages, const float* value_pages,
+                                         const int* block_table, int table_width, const int* tiles, int num_tiles, const int* cu_q,
+                                         const int* context_lens, float* out, int heads, int kv_heads, int block_size, int num_pages,
+                                         float scale, int window, int chunk, const float* sinks, hipStream_t stream) {
+  MLR_REQUIRE(q && key_pages && value_pages && block_table && tiles && cu_q && context_lens && out, "null pointer");
+  MLR_REQUIRE(num_tiles > 0 && heads > 0 && kv_heads > 0 && heads % kv_heads == 0, "bad sizes");
+  MLR_REQUIRE(block_size > 0 && block_size % 4 == 0, "block_size must be a multiple of 4");
+  MLR_REQUIRE(num_pages > 0 && table_width > 0, "page sizes must be > 0");
+  MLR_REQUIRE(q_stride >= static_cast<int64_t>(heads) * MLR_HEAD_DIM && q_stride % 4 == 0, "q_stride must cover a row and keep 16-byte alignment");
+  MLR_REQUIRE(reinterpret_cast<uintptr_t>(q) % 16 == 0 && reinterpret_cast<uintptr_t>(key_pages) % 16 == 0 &&
+                  reinterpret_cast<uintptr_t>(value_pages) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0,
+              "operands must be 16-byte aligned");
+  MLR_REQUIRE(scale > 0.f && scale < INFINITY && window >= 0 && chunk >= 0 && !(window > 0 && chunk > 0), "bad scale, window or chunk");
+  MLR_REQUIRE(static_cast<int64_t>(num_tiles) * heads < (1ll << 31), "too many tiles for one launch");
+  f32_attention::attn_prefill_f32_kernel<<<dim3(static_cast<unsigned>(num_tiles) * heads), 256, 0, stream>>>(
+      q, q_stride, key_pages, value_pages, block_table, table_width, tiles, cu_q, context_lens, out, heads, kv_heads, block_size,
+      num_pages, scale, window, chunk, sinks);
+  MLR_LAUNCH_CHECK();
+  return 0;
+}
+#endif

@@ -24,7 +24,7 @@ __global__ __launch_bounds__(64) void paged_attention_simple_kernel(
     int heads, int kv_heads, int head_dim, int block_size, int num_pages, float scale, int window, int chunk,
     const float* __restrict__ sinks, const T* __restrict__ pooled_keys, const T* __restrict__ pooled_values,
     const int* __restrict__ pooled_table, int pooled_width, int pooled_pages, int pool,
-    const float* __restrict__ score_bias, float softcap, int keep_first) {
+    const float* __restrict__ score_bias, float softcap, int keep_first, const int* __restrict__ single_of) {
   __shared__ float qs[MAXD];
   __shared__ float ps[kWave];
   __shared__ int64_t offs[kWave];
@@ -34,6 +34,8 @@ __global__ __launch_bounds__(64) void paged_attention_simple_kernel(
   const int h = blockIdx.y;
   const int lane = threadIdx.x;
   const int entry = token_entry[t];
+  // with `single_of` (the entries' first rows) only entries of one token are taken: another kernel has the others
+  if (single_of != nullptr && entry >= 0 && entry < entries && single_of[entry + 1] - single_of[entry] != 1) return;
   const int p = positions[t];
   const int kvh = h / (heads / kv_heads);
   T* orow = out + (static_cast<int64_t>(t) * heads + h) * head_dim;
@@ -153,7 +155,8 @@ extern "C" int mlr_paged_attention_simple(const void* q, int64_t q_stride, const
                                           int block_size, int num_pages, float scale, int window, int chunk,
                                           const float* sinks, const void* pooled_keys, const void* pooled_values,
                                           const int* pooled_table, int pooled_width, int pooled_pages, int pool,
-                                          const float* score_bias, float softcap, int keep_first, hipStream_t stream) {
+                                          const float* score_bias, float softcap, int keep_first, const int* single_of,
+                                          hipStream_t stream) {
   MLR_REQUIRE(q && key_pages && value_pages && block_table && token_entry && positions && out, "null pointer");
   MLR_REQUIRE(tokens > 0 && entries > 0 && heads > 0 && kv_heads > 0, "sizes must be > 0");
   MLR_REQUIRE(heads % kv_heads == 0, "query heads must be a multiple of KV heads");
@@ -178,7 +181,7 @@ extern "C" int mlr_paged_attention_simple(const void* q, int64_t q_stride, const
       block_table, table_width, token_entry, positions, static_cast<T*>(out), entries, heads, kv_heads, head_dim, \
       block_size, num_pages, scale, window, chunk, sinks, static_cast<const T*>(pooled_keys),                    \
       static_cast<const T*>(pooled_values), pooled_table, pooled_width, pooled_pages, pool, score_bias, softcap,  \
-      keep_first)
+      keep_first, single_of)
   if (head_dim > 256) {
     if (dtype == kF32)
       MLR_SIMPLE(float, kMaxHeadDim);
@@ -193,14 +196,14 @@ extern "C" int mlr_paged_attention_simple(const void* q, int64_t q_stride, const
         static_cast<const float*>(value_pages), block_table, table_width, token_entry, positions,
         static_cast<float*>(out), entries, heads, kv_heads, head_dim, block_size, num_pages, scale, window, chunk,
         sinks, static_cast<const float*>(pooled_keys), static_cast<const float*>(pooled_values), pooled_table,
-        pooled_width, pooled_pages, pool, score_bias, softcap, keep_first);
+        pooled_width, pooled_pages, pool, score_bias, softcap, keep_first, single_of);
   else
     paged_attention_simple_kernel<bf16, 256><<<grid, kWave, 0, stream>>>(
         static_cast<const bf16*>(q), q_stride, static_cast<const bf16*>(key_pages),
         static_cast<const bf16*>(value_pages), block_table, table_width, token_entry, positions,
         static_cast<bf16*>(out), entries, heads, kv_heads, head_dim, block_size, num_pages, scale, window, chunk,
         sinks, static_cast<const bf16*>(pooled_keys), static_cast<const bf16*>(pooled_values), pooled_table,
-        pooled_width, pooled_pages, pool, score_bias, softcap, keep_first);
+        pooled_width, pooled_pages, pool, score_bias, softcap, keep_first, single_of);
   MLR_LAUNCH_CHECK();
   return 0;
 }

@@ -1,6 +1,6 @@
 // y[M, N] = x[M, K] * w[N, K]^T (+ bias), plain float32 FMA arithmetic.
 //
-// This is the matrix product of the true 32-bit path (no matrix-core input
+// A matrix product of the true 32-bit path (no matrix-core input
 // rounding of any kind) and accepts bfloat16 operands as well, which makes it
 // the reference the MFMA kernels are checked against on the GPU.  64x64 output
 // tile per workgroup, 16-wide K slices staged through LDS, 4x4 outputs per lane.

@@ -60,6 +60,7 @@ CORE = Module(
     (
         "elementwise.hip",
         "gemm_simple.hip",
+        "gemm_f32.hip",
         "gemm_mfma.hip",
         "gemm_fused.hip",
         "gemm_stream.hip",
@@ -82,7 +83,7 @@ def attention_module(head_dim: int) -> Module:
     if head_dim % 16 or not 16 <= head_dim <= 256:
         raise ValueError("the MFMA attention kernels take head sizes in steps of 16 up to 256")
     return Module(
-        f"attention_d{head_dim}", ("attention_mfma.hip",), (f"MLR_HEAD_DIM={head_dim}",), ("common.h", "mfma.h")
+        f"attention_d{head_dim}", ("attention_mfma.hip", "attention_f32.hip"), (f"MLR_HEAD_DIM={head_dim}",), ("common.h", "mfma.h")
     )
 
 

@@ -96,6 +96,8 @@ _SIGNATURES = {
     "mlr_rope_kv_write": ([_VP, _I, _VP, _VP, _VP, _VP, _VP, _I, _I, _I, _I, _I, _I, _I, _I, _VP], _I),
     "mlr_qkv_finish": ([_VP, _I, _VP, _VP, _VP, _VP, _VP, _VP, _I, _I, _I, _I, _I, _I, _I, _VP], _I),
     "mlr_gemm_simple": ([_VP, _VP, _VP, _I, _VP, _I, _I, _I, _I, _I, _I, _VP, _VP, _F, _F, _VP], _I),
+    "mlr_gemm_f32": ([_VP, _VP, _VP, _VP, _I, _I, _I, _I, _I, _VP, _VP, _F, _F, _VP], _I),
+    "mlr_gemm_f32_slices": ([_I, _I, _I, _I], _I),
     "mlr_gemm_bf16": ([_VP, _VP, _VP, _I, _VP, _I, _I, _I, _I, _I, _I, _I, _VP, _I, _F, _VP, _VP, _F, _F, _VP], _I),
     "mlr_moe_route": ([_VP, _VP, _VP, _VP, _I, _I, _I, _I, _I, _F, _I, _I, _VP], _I),
     "mlr_moe_tile_rows": ([_I], _I),
@@ -121,8 +123,11 @@ _SIGNATURES = {
     "mlr_gemm_merge_fused_bf16": ([_VP, _VP, _I, _I, _I, _I, _I, _VP, _VP, _I, _VP, _I, _I, _I, _I, _VP], _I),
     "mlr_paged_attention_simple": (
         [_VP, _I64, _VP, _VP, _VP, _I, _VP, _VP, _VP, _I, _I, _I, _I, _I, _I, _I, _I, _F, _I, _I, _VP, _VP, _VP, _VP,
-         _I, _I, _I, _VP, _F, _I, _VP],
+         _I, _I, _I, _VP, _F, _I, _VP, _VP],
         _I,
+    ),
+    "mlr_attention_prefill_f32": (
+        [_VP, _I64, _VP, _VP, _VP, _I, _VP, _I, _VP, _VP, _VP, _I, _I, _I, _I, _F, _I, _I, _VP, _VP], _I,
     ),
     "mlr_sample": ([_VP, _VP, _VP, _VP, _VP, _I, _I, _VP], _I),
     "mlr_sample_scratch": ([_I, _I], _I64),
@@ -146,6 +151,9 @@ _SIGNATURES = {
 
 # what `linear` may do to its sums before it stores them (the entry points' `swiglu` argument)
 _EPILOGUES = {None: 0, "swiglu": 1, "relu2": 2, "sigmoid": 3, "gelu_tanh": 4, "clamped_glu": 5, "geglu": 6}
+
+# head sizes whose kernels every build has and whose tiles fit (attention_f32.hip)
+F32_TILE_HEAD_DIMS = tuple(d for d in build.DEFAULT_HEAD_DIMS if d <= 128)
 
 from .plans import PAGED_ATTENTION, QUERY_TILE, WIDE_QUERY_TILE, attention_plan, query_tiles  # noqa: F401
 
@@ -573,8 +581,8 @@ class HipOps:
         delta (as with partial_sums); it may then come back unrun, as a `PendingLinear` that the norm
         runs together with the addition to the residual stream.
 
-        bfloat16 products run on the matrix cores when k is a multiple of 8; float32
-        products, and everything with kernel="fma", run as plain 32-bit FMA arithmetic.
+        bfloat16 products run on the matrix cores when k is a multiple of 8, float32 products (in float32) when it is
+        a multiple of 4; other products, and everything with kernel="fma", run as plain 32-bit FMA arithmetic.
         swiglu: the rows of `weight` are groups (gate 2j, gate 2j+1, up 2j, up 2j+1) and
         the result is silu(gate) * up, [M, N / 2].
         partial_sums: the caller hands the result to a norm as a not-yet-added delta and
@@ -669,6 +677,16 @@ class HipOps:
                 glu_limit, glu_alpha, self._stream(),
             )
             return y
+        if kernel == "auto" and self.dtype == torch.float32 and k % 4 == 0 and k <= 1 << 22 and self._aligned(x, weight, out):
+            cut = 1
+            if partial_sums and not swiglu and out is None:
+                cut = self.lib.mlr_gemm_f32_slices(m, n, k, self.max_k_slices)
+            y = self._into(out, (cut, m, n) if cut > 1 else (m, n // 2 if swiglu else n), out_dtype)
+            self._call(
+                "mlr_gemm_f32", self._ptr(x), self._ptr(weight), self._ptr(bias), self._ptr(y), epilogue, cut, m, n, k,
+                self._ptr(multiply), self._ptr(multiply_rows), glu_limit, glu_alpha, self._stream(),
+            )
+            return y
         y = self._into(out, (m, n // 2 if swiglu else n), out_dtype)
         self._call(
             "mlr_gemm_simple", self._ptr(x), self._ptr(weight), self._ptr(bias), bias_f32, self._ptr(y),
@@ -676,6 +694,11 @@ class HipOps:
             self._ptr(multiply_rows), glu_limit, glu_alpha, self._stream(),
         )
         return y
+
+    @staticmethod
+    def _aligned(*tensors: Optional[torch.Tensor]) -> bool:
+        """Every tensor starts at a multiple of 16 bytes (a view into a larger one need not)."""
+        return all(t is None or t.data_ptr() % 16 == 0 for t in tensors)
 
     def _into(self, out: Optional[torch.Tensor], shape: Sequence[int], dtype: torch.dtype) -> torch.Tensor:
         return self._empty(shape, dtype) if out is None else self._check(out, "linear output", dtype, shape)
@@ -1087,13 +1110,34 @@ class HipOps:
             if num_tiles and (block_size & (block_size - 1) or not 8 <= block_size <= lib.mlr_attention_key_tile()):
                 use_mfma = False  # the tiled prefill kernel takes power-of-two pages from 8 up to its key tile
         if not use_mfma:
+            # Prompt portions in float32 run in tiles on the matrix cores (in float32) where the mask is a plain one; the plain kernel
+            # then takes the entries of one token only.  (0.5B sizes, prompts of 391, 268, 145 and 22 tokens: 479 us with the plain
+            # kernel, 44 us in tiles.)  Other masks, pages and head sizes keep the plain kernel, which takes them all.
+            singles = None
+            if (
+                kernel == "auto" and self.dtype == torch.float32 and num_tiles and head_dim in F32_TILE_HEAD_DIMS
+                and block_size % 4 == 0 and stride % 4 == 0 and pooled is None and score_bias is None and not cap and not keep_first
+                and self._aligned(qkv, key_pages, value_pages)
+            ):
+                self._check(ctx.cu_q, "cu_q", torch.int32, (entries + 1,))
+                self._check(ctx.context_lens, "context lengths", torch.int32, (entries,))
+                tiles = self._check(plan.query_tiles, "query tiles", torch.int32, (num_tiles, 2))
+                self._call(
+                    "mlr_attention_prefill_f32", self._ptr(qkv), stride, self._ptr(key_pages), self._ptr(value_pages),
+                    self._ptr(block_table), width, self._ptr(tiles), num_tiles, self._ptr(ctx.cu_q), self._ptr(ctx.context_lens),
+                    self._ptr(out), num_heads, num_kv_heads, block_size, num_pages, float(scale), int(window or 0), chunk,
+                    self._ptr(sinks), self._stream(), lib=self.attention_library(head_dim),
+                )
+                if not num_decode:
+                    return out
+                singles = ctx.cu_q
             self._call(
                 "mlr_paged_attention_simple", self._ptr(qkv), stride, self._ptr(key_pages), self._ptr(value_pages),
                 self._ptr(block_table), width, self._ptr(ctx.token_entry), self._ptr(ctx.positions),
                 self._ptr(out), self.code, tokens, entries, num_heads, num_kv_heads, head_dim, block_size,
                 num_pages, float(scale), int(window or 0), chunk, self._ptr(sinks), self._ptr(pooled_keys),
                 self._ptr(pooled_values), self._ptr(pooled_table), pooled_width, pooled_pages, pool,
-                self._ptr(score_bias), cap, keep_first, self._stream(),
+                self._ptr(score_bias), cap, keep_first, self._ptr(singles), self._stream(),
             )
             return out
         self._check(ctx.cu_q, "cu_q", torch.int32, (entries + 1,))

@@ -1,0 +1,95 @@
+"""The float32 kernels of the 32-bit path on the matrix cores, against float64 and against the plain kernels."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from test_gpu_kernels import _attend, _attention_reference, _paged_case, _rand
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from mini_llm_runtime_amd.kernels.ops import HipOps
+
+    return HipOps(dtype=torch.float32, device="cuda:0")
+
+
+def _sum_error(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """What k products and additions in float32 may be off by, in whatever order: k roundings of half a unit in the last place of
+    sums that are at most the sum of the products' sizes."""
+    return x.shape[1] * 2.0**-24 * (x.double().abs() @ w.double().abs().t()) + 1e-30
+
+
+# edges of both kernels: one token, a full slab of 16, one more, the last of the few, the first of the tiled, a tile and one row; features around the
+# 16 of a workgroup and the 64 of a tile; k of one piece, around a step of 32 and around several steps
+@pytest.mark.parametrize("m", [1, 16, 17, 33, 64, 65, 129])
+@pytest.mark.parametrize("n", [1, 16, 66, 130])
+@pytest.mark.parametrize("k", [4, 32, 36, 100, 420])
+def test_product(ops, m, n, k):
+    x, w, b = _rand((m, k), torch.float32, 1), _rand((n, k), torch.float32, 2), _rand((n,), torch.float32, 3)
+    ref, bound = x.double() @ w.double().t(), _sum_error(x, w)
+    got = ops.linear(x.cuda(), w.cuda(), b.cuda()).cpu().double()
+    assert ((got - (ref + b.double())).abs() <= bound + 2.0**-23 * (ref.abs() + b.abs())).all()
+
+
+@pytest.mark.parametrize("m", [5, 40, 70])
+@pytest.mark.parametrize("epilogue", ["swiglu", "clamped", "geglu", "relu2", "sigmoid", "gelu_tanh", "multiply", "rows"])
+def test_epilogues_are_the_plain_kernels(ops, m, epilogue):
+    n, k = 72, 64
+    x, w, b = _rand((m, k), torch.float32, 4).cuda(), _rand((n, k), torch.float32, 5, 0.3).cuda(), _rand((n,), torch.float32, 6).cuda()
+    kw, bias = {
+        "swiglu": (dict(swiglu=True), None), "clamped": (dict(clamped_glu=(1.5, 1.7)), b), "geglu": (dict(geglu=True), b),
+        "multiply": (dict(activation="sigmoid", multiply=_rand((m, n), torch.float32, 7).cuda()), b),
+        "rows": (dict(multiply=_rand((9, n), torch.float32, 8).cuda(), multiply_rows=(torch.arange(m, dtype=torch.int32) % 9).cuda()), None),
+    }.get(epilogue, (dict(activation=epilogue), b))
+    got, plain = ops.linear(x, w, bias, **kw), ops.linear(x, w, bias, kernel="fma", **kw)
+    assert got.shape == plain.shape
+    # the sums differ by their order (64 roundings of values of a few units); the gatings multiply two of them
+    torch.testing.assert_close(got, plain, atol=2e-4, rtol=2e-5)
+
+
+def test_partial_sums_add_up(ops):
+    x, w, b = _rand((100, 4864), torch.float32, 9), _rand((90, 4864), torch.float32, 10), _rand((90,), torch.float32, 11)
+    got = ops.linear(x.cuda(), w.cuda(), b.cuda(), partial_sums=True).cpu().double()
+    assert got.dim() == 3 and got.shape[1:] == (100, 90)
+    ref = x.double() @ w.double().t() + b.double()
+    assert ((got.sum(0) - ref).abs() <= _sum_error(x, w) + 2.0**-23 * ref.abs()).all()
+
+
+def test_operands_off_16_bytes_take_the_plain_kernel(ops):
+    """A view that starts 4 bytes into a tensor is no operand for 16-byte loads: same result, another kernel."""
+    flat = _rand((64 * 70 + 1,), torch.float32, 12).cuda()
+    x, w = flat[1:].view(70, 64), _rand((32, 64), torch.float32, 13).cuda()
+    torch.testing.assert_close(ops.linear(x, w), ops.linear(x, w, kernel="fma"), atol=0, rtol=0)
+    torch.testing.assert_close(ops.linear(x, w), ops.linear(x.clone(), w), atol=1e-4, rtol=1e-5)
+
+
+@pytest.mark.parametrize("heads,kv_heads,head_dim,block", [(14, 2, 64, 16), (4, 4, 16, 4), (3, 1, 80, 8), (6, 2, 96, 32), (4, 1, 128, 16), (2, 1, 48, 12), (2, 2, 32, 128)])
+@pytest.mark.parametrize("mask", [dict(window=None), dict(window=37), dict(window=None, chunk=50)])
+def test_prompt_attention(ops, heads, kv_heads, head_dim, block, mask):
+    """Whole prompts around the tile's 64 queries, portions behind cached tokens, single tokens beside them."""
+    entries = [(64, 64), (65, 65), (2, 2), (200, 1), (131, 131), (150, 33), (1, 1)]
+    q, kp, vp, table, ctx, dense, te, pos = _paged_case(entries, heads, kv_heads, head_dim, block, torch.float32, 14)
+    args = (q.cuda(), kp.cuda(), vp.cuda(), table.cuda(), ctx)
+    sinks = _rand((heads,), torch.float32, 15).cuda()
+    kw = dict(num_heads=heads, num_kv_heads=kv_heads, head_dim=head_dim, block_size=block, scale=head_dim**-0.5, **mask)
+    for sink in (None, sinks):
+        got = _attend(ops, *args, sinks=sink, **kw).cpu()
+        plain = _attend(ops, *args, kernel="fma", sinks=sink, **kw).cpu()
+        # weights add up to one and values are a few units: sums of 64 to 200 products in another order
+        torch.testing.assert_close(got, plain, atol=5e-6, rtol=1e-5)
+    if "chunk" not in mask:
+        ref = _attention_reference(q, dense, te, pos, heads, kv_heads, head_dim, head_dim**-0.5, mask["window"])
+        torch.testing.assert_close(_attend(ops, *args, **kw).cpu().double(), ref, atol=5e-6, rtol=1e-5)
+
+
+def test_prompt_attention_refuses_a_page_that_is_not_there(ops):
+    q, kp, vp, table, ctx, *_ = _paged_case([(100, 100), (70, 70)], 2, 1, 64, 16, torch.float32, 16)
+    table = table.clone()
+    table[1, 2] = kp.shape[0]  # a visible page of the second request
+    kw = dict(num_heads=2, num_kv_heads=1, head_dim=64, block_size=16, scale=0.125, window=None)
+    got = _attend(ops, q.cuda(), kp.cuda(), vp.cuda(), table.cuda(), ctx, **kw).cpu()
+    assert torch.isfinite(got[:100]).all() and torch.isnan(got[100 + 64 :]).all()
