@@ -965,6 +965,354 @@ __global__ __launch_bounds__(256 * kKeyGroups) void attn_prefill_kernel(
   }
 }
 
+// ---- prompts at head sizes 64 and 128 -------------------------------------------------------------------
+// The same work with 32 x 32 products: a wavefront takes 32 queries of one head, so a key or value operand read from LDS serves
+// twice the products of attn_prefill_kernel's 16 (what bounded that kernel), a query's scores of 64 keys lie in two lanes, and their
+// maximum needs one exchange.
+//  * Keys and values go from the pages straight into LDS (no staging registers, no LDS stores).  A page of 16 positions or more
+//    holds 16 consecutive keys, and all their dims of a value head as one block, so 16 keys are the unit that one wavefront
+//    fetches, with one page id, through a buffer resource over the page's rows of this head: a page that is not there, and
+//    positions past the last key, are out of its range and arrive as zeros.
+//  * Key rows in LDS: row r of 32 holds the key that makes a lane's accumulator elements 8 consecutive keys (see key_in_16),
+//    which is the operand of the second product; 16-byte pieces are stored in the order piece ^ key, as sixteen rows side by side
+//    would otherwise lie on the same banks.  Value rows need neither: 32 dims of 16 keys are 1 KB, read in one piece.
+//  * The running maximum only moves when a score exceeds it by 2^8: until then the weights are up to 2^8 instead of 1, which
+//    costs no precision (float32 sums, bfloat16's exponent), and the 64 (D = 128) accumulators are rarely rescaled.
+// KG: groups of wavefronts that take the key tiles in turn.  1: four wavefronts, 128 queries.  2: two and two, 64 queries, for
+// the head size whose few tiles are as many long chains on a part of the compute units.
+// CAP: capped scores.
+// Bound by the softmax's vector instructions beside the products (two wavefronts a SIMD overlap them in part).  Measured against
+// attn_prefill_kernel's best tiles, whole prompts, microseconds (TFLOP/s): 28 heads of 128: 1,024 tokens 35 to 28, 2,048 84 (358) to 52
+// (581), 8,191 902 (533; the wide tiles, which its rule chose, 1,098: 268 registers leave one wavefront a SIMD) to 547 (879), 16,384
+// 3,358 (573) to 2,029 (949); 14 heads of 64: 2,048 29 to 23, 8,191 263 (457) to 156 (770), 16,384 924 (521) to 556 (865).
+#if MLR_HEAD_DIM == 64 || MLR_HEAD_DIM == 128
+#define MLR_HAS_PROMPT 1
+constexpr int kPromptKeys = 64;
+constexpr float kPromptSlack = 8.0f;  // in base 2
+
+// The key, among 16, that LDS row w of 16 holds.
+__host__ __device__ constexpr int key_in_16(int w) { return (w / 4) % 2 * 8 + w / 8 * 4 + w % 4; }
+
+// The larger of a lane's value and that of the lane 32 places away.  (The exchange of the two halves of a wavefront between two
+// registers; a shuffle would go through LDS and wait for every operand on its way from there.)
+__device__ __forceinline__ float max_of_halves(float v) {
+  float a = v, b = v;
+  asm("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+  return fmaxf(a, b);
+}
+
+// Everything that this wavefront asked for has arrived, then the workgroup's barrier.  (The builtin and not inline assembly: the
+// compiler, which counts what is on its way, then knows, and does not wait again for loads that were sent later.)
+__device__ __forceinline__ void wait_and_meet() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+constexpr int prompt_lds_bytes(int groups) { return 2 * groups * kPromptKeys * D * 4; }
+
+template <int KG, bool CAP>
+__global__ __launch_bounds__(256, 2) void attn_prompt_kernel(
+    const bf16* __restrict__ q, int64_t q_stride, const bf16* __restrict__ key_pages, const bf16* __restrict__ value_pages,
+    const int* __restrict__ block_table, int table_width, const int* __restrict__ tiles, const int* __restrict__ cu_q,
+    const int* __restrict__ context_lens, bf16* __restrict__ out, int num_tiles, int heads, int kv_heads, int bs_shift,
+    int num_pages, float scale, int window, int chunk, float* __restrict__ partial, const float* __restrict__ sinks,
+    int keep_partial, float softcap) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char prefill_lds[];
+  __shared__ int sm_bad;
+  constexpr int kQueryWaves = 4 / KG;
+  constexpr int kWgQ = 32 * kQueryWaves;
+  constexpr int kTileBytes = kPromptKeys * D * 2;    // of keys, and of values
+  constexpr int kPieceRow = D / 8;                   // 16-byte pieces of a key row
+  constexpr int kLoads = D / 32;                     // 1 KB loads of 16 keys, and of their values
+  constexpr int kHeadSteps = D / 16;                 // products over the head's dims
+  constexpr int kDims = D / 32;                      // blocks of 32 dims
+  const int block_size = 1 << bs_shift;
+  // workgroup -> (tile, head): as attn_prefill_kernel
+  const int total = num_tiles * heads;
+  const int round = blockIdx.x / 256, in_round = blockIdx.x % 256;
+  const int work = (round & 1) == 0 ? (round / 2) * 256 + in_round : total - 1 - ((round / 2) * 256 + in_round);
+  const int tile = work / heads;
+  const int head = work - tile * heads;
+  const int entry = tiles[2 * tile];
+  const int q0 = tiles[2 * tile + 1];
+  const int kvh = head / (heads / kv_heads);
+  const int tid = threadIdx.x;
+  const int lane = tid % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int group = wave / kQueryWaves;   // key group
+  const int qw = wave % kQueryWaves;      // which 32 queries
+  const int r32 = lane % 32, h = lane / 32;
+
+  const int t_first = cu_q[entry];
+  const int q_len = cu_q[entry + 1] - t_first;
+  const int pos0 = context_lens[entry] - q_len;
+  const int* table = block_table + static_cast<int64_t>(entry) * table_width;
+  if (tid == 0) sm_bad = 0;
+
+  const int qi = q0 + qw * 32 + r32;
+  const bool q_ok = qi < q_len;
+  const int pq = pos0 + qi;
+  const int pq_first = first_visible_key(pq, window, chunk);
+  bf16x8_t qo[kHeadSteps];
+  const bf16* qrow = q + static_cast<int64_t>(t_first + (q_ok ? qi : 0)) * q_stride + static_cast<int64_t>(head) * D;
+#pragma unroll
+  for (int st = 0; st < kHeadSteps; ++st) qo[st] = load_bf16x8(qrow + st * 16 + h * 8);
+
+  // keys of the workgroup, whole tiles of 64 from a multiple of 64 on; this workgroup's run of them (gridDim.y runs)
+  const int k_end = pos0 + min(q0 + kWgQ, q_len);
+  const int k_first = first_visible_key(pos0 + q0, window, chunk);
+  const int k_zero = k_first / kPromptKeys * kPromptKeys;
+  constexpr int kTurn = KG * kPromptKeys;
+  const int turns = (k_end - k_zero + kTurn - 1) / kTurn;
+  const int turns_each = (turns + static_cast<int>(gridDim.y) - 1) / static_cast<int>(gridDim.y);
+  const int k_begin = k_zero + static_cast<int>(blockIdx.y) * turns_each * kTurn;
+  const int k_stop = min(k_end, k_begin + turns_each * kTurn);
+  // the wavefront's own queries
+  const bool wave_has_queries = q0 + qw * 32 < q_len;
+  const int w_min_pos = pos0 + q0 + qw * 32;
+  const int w_last = pos0 + min(q0 + qw * 32 + 31, q_len - 1);
+  const int w_first = first_visible_key(w_min_pos, window, chunk);
+  const int w_max_first = first_visible_key(w_min_pos + 31, window, chunk);
+  const float cap1 = CAP ? 2.0f * 1.44269504088896340736f * scale / softcap : 0.f;  // see cap_scores
+  const float cap2 = softcap * 1.44269504088896340736f;
+  const float scale2 = CAP ? 1.0f : scale * 1.44269504088896340736f;
+
+  float m_run = -INFINITY, l_run = 0.f;  // l: this lane's share of the sum
+  f32x16_t acc[kDims];
+#pragma unroll
+  for (int dt = 0; dt < kDims; ++dt)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[dt][e] = 0.f;
+  bool bad = false;
+
+  // A wavefront brings KG times 16 keys of its group's tile.  Load i of them: LDS rows w = i * (64 / kPieceRow) + lane / kPieceRow,
+  // slot lane % kPieceRow; of the values: dims i * 32 + lane / 2, 8 keys each.
+  unsigned k_off[kLoads];
+#pragma unroll
+  for (int i = 0; i < kLoads; ++i) {
+    const int w = i * (64 / kPieceRow) + lane / kPieceRow;
+    const int key = D == 128 ? w % 16 : w / 2 % 8;
+    k_off[i] = static_cast<unsigned>(key_in_16(w) * D + ((lane % kPieceRow) ^ key) * 8) * 2u;
+  }
+  const unsigned v_off = static_cast<unsigned>(lane / 2 * block_size + lane % 2 * 8) * 2u;
+  const int last_page = (k_end - 1) >> bs_shift;
+  const int my_key = qw * KG * 16;  // first key of this wavefront's share of a tile
+  // The page ids come as vector loads, which are counted with the tiles' own (a scalar load on its way would turn every wait for
+  // LDS into a wait for everything); they are asked for a turn ahead of their use and waited for with that turn's tile.
+  const __amdgpu_buffer_rsrc_t ids_buf = make_buffer(table, static_cast<unsigned>(table_width) * 4u);
+  int ids[KG];
+  auto lookup = [&](int kt0) {
+#pragma unroll
+    for (int u = 0; u < KG; ++u)
+      ids[u] = __builtin_amdgcn_raw_buffer_load_b32(ids_buf, static_cast<unsigned>(min((kt0 + my_key + u * 16) >> bs_shift, last_page)) * 4u, 0, 0);
+  };
+  auto fetch = [&](int kt0, int buf) {  // with the ids that lookup(kt0) left
+#pragma unroll
+    for (int u = 0; u < KG; ++u) {
+      const int key0 = kt0 + my_key + u * 16;
+      const int page = __builtin_amdgcn_readfirstlane(ids[u]);
+      const bool in = static_cast<unsigned>(page) < static_cast<unsigned>(num_pages);
+      if (!in && key0 < k_end && key0 + 15 >= k_first) bad = true;
+      const int64_t base = (static_cast<int64_t>(in ? page : 0) * kv_heads + kvh) * block_size * D;
+      const int in_page = key0 & (block_size - 1);
+      const __amdgpu_buffer_rsrc_t k_buf = make_buffer(key_pages + base + in_page * D, in ? 16u * D * 2u : 0u);
+      const __amdgpu_buffer_rsrc_t v_buf = make_buffer(value_pages + base + in_page, in ? static_cast<unsigned>(D * block_size - in_page) * 2u : 0u);
+      const unsigned past = key0 + lane % 2 * 8 < k_end ? 0u : kOutOfBuffer;
+      unsigned char* const dst = prefill_lds + ((buf * KG + group) * 2) * kTileBytes + (my_key + u * 16) * D * 2;
+#pragma unroll
+      for (int i = 0; i < kLoads; ++i)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(k_buf, (__attribute__((address_space(3))) void*)(dst + i * 1024), 16, k_off[i], 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < kLoads; ++i)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(v_buf, (__attribute__((address_space(3))) void*)(dst + kTileBytes + i * 1024), 16,
+                                                 (v_off + static_cast<unsigned>(i * 64 * block_size)) | past, 0, 0, 0);
+    }
+  };
+
+  const int k_mine = k_begin + group * kPromptKeys;
+  if (k_mine < k_stop) {
+    lookup(k_mine);
+    fetch(k_mine, 0);
+    lookup(k_mine + kTurn);
+  }
+  const int k_row = r32 * D * 2;                                  // this lane's key row, of the first 32
+  const int k_key = D == 128 ? r32 % 16 : r32 / 2 % 8;
+  int buf = 0;
+  for (int kt0 = k_mine; kt0 - group * kPromptKeys < k_stop; kt0 += kTurn, buf ^= 1) {
+    // this wavefront's share of the tile has landed; behind the barrier everybody's has, and the other buffer is free
+    wait_and_meet();
+    if (kt0 + kTurn < k_stop) {
+      fetch(kt0 + kTurn, buf ^ 1);
+      lookup(kt0 + 2 * kTurn);
+    }
+    unsigned char* const ks = prefill_lds + ((buf * KG + group) * 2) * kTileBytes;
+    unsigned char* const vs = ks + kTileBytes;
+    const int turn0 = kt0 - group * kPromptKeys;
+    if (k_end % 8 != 0 && turn0 <= k_end && k_end < turn0 + kTurn) {
+      // the 8 values that the last key is among: those past it are cleared, since 0 * NaN would come through
+      const int at = k_end - kt0, d = tid % (256 / KG);
+      if (at >= 0 && at < kPromptKeys && d < D) {
+        u16x8_t* const piece = reinterpret_cast<u16x8_t*>(vs + (at / 16 * D + d) * 32 + at % 16 / 8 * 16);
+        u16x8_t bits = *piece;
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (e >= k_end % 8) bits[e] = 0;
+        *piece = bits;
+      }
+      __syncthreads();
+    }
+    if (!(wave_has_queries && kt0 < k_stop && kt0 <= w_last && kt0 + kPromptKeys > w_first)) continue;
+
+    // All key operands are asked for before the first product: read one by one, each would be waited for (a trip to LDS is four
+    // products long).
+    bf16x8_t keys[kHeadSteps][2];
+#pragma unroll
+    for (int st = 0; st < kHeadSteps; ++st)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) keys[st][b] = load_bf16x8(ks + b * 32 * D * 2 + k_row + (((st * 2 + h) ^ k_key) * 16));
+    __builtin_amdgcn_sched_barrier(0);
+    f32x16_t s[2];
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) s[b][e] = 0.f;
+#pragma unroll
+    for (int st = 0; st < kHeadSteps; ++st)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) s[b] = mfma_32x32x16(keys[st][b], qo[st], s[b]);
+    // and the first half of the value operands before the softmax, which hides their way
+    auto value_operand = [&](int g, int dt) { return load_bf16x8(vs + (g * D + dt * 32 + r32) * 32 + h * 16); };
+    bf16x8_t values[2][kDims];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int g = 0; g < 2; ++g)
+#pragma unroll
+      for (int dt = 0; dt < kDims; ++dt) values[g][dt] = value_operand(g, dt);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (CAP) {
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) s[b][e] = fmaf(__builtin_amdgcn_rcpf(1.0f + fast_exp2(s[b][e] * cap1)), -2.0f * cap2, cap2);
+    }
+    if (!(kt0 + kPromptKeys - 1 <= w_min_pos && kt0 >= w_max_first)) {  // some query here does not see all of it
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const int key = kt0 + b * 32 + e / 8 * 16 + h * 8 + e % 8;  // see key_in_16
+          if (!(q_ok && key <= pq && key >= pq_first)) s[b][e] = -INFINITY;
+        }
+    }
+    float top = -INFINITY;
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) top = fmaxf(top, s[b][e]);
+    top = max_of_halves(top) * scale2;
+    if (__any(top > m_run + kPromptSlack)) {  // always so with the first key that a query sees
+      const float m_new = fmaxf(m_run, top);
+      const float alpha = m_new == -INFINITY ? 1.0f : fast_exp2(m_run - m_new);
+      l_run *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < kDims; ++dt)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[dt][e] *= alpha;
+      m_run = m_new;
+    }
+    const float m_use = m_run == -INFINITY ? 0.f : m_run;  // a query that has seen no key yet
+    float sum = 0.f;
+    bf16x8_t p[4];  // weights of 16 keys each, this lane's 8
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      float v[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        v[e] = fast_exp2(fmaf(s[g / 2][g % 2 * 8 + e], scale2, -m_use));
+        sum += v[e];
+      }
+      const u32x4_t words = {pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7])};
+      p[g] = __builtin_bit_cast(bf16x8_t, words);
+    }
+    l_run += sum;
+    bf16x8_t later[2][kDims];
+#pragma unroll
+    for (int g = 0; g < 2; ++g)
+#pragma unroll
+      for (int dt = 0; dt < kDims; ++dt) later[g][dt] = value_operand(2 + g, dt);
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+#pragma unroll
+      for (int dt = 0; dt < kDims; ++dt) acc[dt] = mfma_32x32x16(g < 2 ? values[g][dt] : later[g - 2][dt], p[g], acc[dt]);
+  }
+
+  __syncthreads();  // the tiles are done with
+  if constexpr (KG > 1) {
+    float* const handover = reinterpret_cast<float*>(prefill_lds);  // [component][thread of the group]
+    static_assert(KG == 1 || (2 + kDims * 16) * 128 * 4 <= prompt_lds_bytes(KG), "the handover fits the tile buffers");
+    const int at = tid % 128;
+    if (group > 0) {
+      handover[at] = m_run;
+      handover[128 + at] = l_run;
+#pragma unroll
+      for (int dt = 0; dt < kDims; ++dt)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) handover[(2 + dt * 16 + e) * 128 + at] = acc[dt][e];
+    }
+    if (bad) atomicOr(&sm_bad, 1);
+    __syncthreads();
+    if (group > 0) return;
+    const float m_other = handover[at];
+    const float m_new = fmaxf(m_run, m_other);
+    const float w_mine = m_run == -INFINITY ? 0.f : fast_exp2(m_run - m_new);
+    const float w_other = m_other == -INFINITY ? 0.f : fast_exp2(m_other - m_new);
+    l_run = l_run * w_mine + handover[128 + at] * w_other;
+#pragma unroll
+    for (int dt = 0; dt < kDims; ++dt)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[dt][e] = acc[dt][e] * w_mine + handover[(2 + dt * 16 + e) * 128 + at] * w_other;
+    m_run = m_new;
+  } else {
+    if (bad) atomicOr(&sm_bad, 1);
+    __syncthreads();
+  }
+  const bool poisoned = sm_bad != 0;
+  float l = l_run;
+  l += __shfl_xor(l, 32, kWave);
+  if (gridDim.y > 1 || keep_partial) {
+    // this run's share, unnormalised: [tile, head, run, query of the tile, head size + 2]
+    float* dst = partial + (((static_cast<int64_t>(tile) * heads + head) * gridDim.y + blockIdx.y) * kWgQ + (qw * 32 + r32)) * kPartialStride;
+#pragma unroll
+    for (int dt = 0; dt < kDims; ++dt)
+#pragma unroll
+      for (int e = 0; e < 16; e += 2)
+        *reinterpret_cast<f32x2_t*>(dst + dt * 32 + e / 4 * 8 + h * 4 + e % 4) =
+            poisoned ? f32x2_t{__builtin_nanf(""), __builtin_nanf("")} : f32x2_t{acc[dt][e], acc[dt][e + 1]};
+    if (h == 0) {
+      dst[D] = m_run;
+      dst[D + 1] = l;
+    }
+    return;
+  }
+  if (!q_ok) return;
+  const float keep = join_sink(sinks, head, m_run, l);
+  const float inv = poisoned ? __builtin_nanf("") : keep / l;
+  bf16* orow = out + (static_cast<int64_t>(t_first + qi) * heads + head) * D;
+#pragma unroll
+  for (int dt = 0; dt < kDims; ++dt)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      u16x4_t packed;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) packed[e] = f32_to_bf16(acc[dt][g * 4 + e] * inv).bits;
+      *reinterpret_cast<u16x4_t*>(orow + dt * 32 + g * 8 + h * 4) = packed;
+    }
+}
+
+#endif  // MLR_HAS_PROMPT
+
 // Merge of the key runs of a prompt tile (see attn_prefill_kernel): for every query of the tile
 // and every head, m = max m_j, w_j = 2^(m_j - m), O = sum w_j a_j / sum w_j l_j, in the runs'
 // order.  One workgroup per (tile, head).
@@ -1180,6 +1528,18 @@ int mlr_attention_prefill(const void* q, int64_t q_stride, const void* key_pages
                              reinterpret_cast<const void*>(attn_prefill_kernel<D <= 128 ? 2 : 1, true>)};
     for (const void* kernel : kernels)
       if (e == hipSuccess) e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kPrefillLds);
+#ifdef MLR_HAS_PROMPT
+    {
+      const void* wide_kernels[] = {reinterpret_cast<const void*>(attn_prompt_kernel<1, false>),
+                                    reinterpret_cast<const void*>(attn_prompt_kernel<1, true>)};
+      const void* narrow_kernels[] = {reinterpret_cast<const void*>(attn_prompt_kernel<2, false>),
+                                      reinterpret_cast<const void*>(attn_prompt_kernel<2, true>)};
+      for (const void* kernel : wide_kernels)
+        if (e == hipSuccess) e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, prompt_lds_bytes(1));
+      for (const void* kernel : narrow_kernels)
+        if (e == hipSuccess) e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, prompt_lds_bytes(2));
+    }
+#endif
     if (e != hipSuccess) {
       set_error(std::string("mlr_attention_prefill: cannot raise the LDS limit: ") + hipGetErrorString(e));
       return -1;
@@ -1187,6 +1547,24 @@ int mlr_attention_prefill(const void* q, int64_t q_stride, const void* key_pages
     configured = true;
   }
   const dim3 grid(static_cast<unsigned>(num_tiles) * heads, splits);
+  // The 32 x 32 kernel takes pages of whole runs of 16 keys and softmax weights over one range of keys; what else there is
+  // (smaller pages, keys weighed one by one, first tokens kept beside a window) stays with the kernel below.
+  bool launched = false;
+#ifdef MLR_HAS_PROMPT
+  if (block_size >= 16 && score_bias == nullptr && keep_first == 0) {
+#define MLR_PROMPT(groups, cap)                                                                                       \
+  attn_prompt_kernel<groups, cap><<<grid, 256, prompt_lds_bytes(groups), stream>>>(                                   \
+      static_cast<const bf16*>(q), q_stride, static_cast<const bf16*>(key_pages), static_cast<const bf16*>(value_pages), \
+      block_table, table_width, tiles, cu_q, context_lens, static_cast<bf16*>(out), num_tiles, heads, kv_heads, bs_shift, \
+      num_pages, scale, window, chunk, partial, (splits > 1 || keep_partial) ? nullptr : sinks, keep_partial, softcap)
+      if (wide && softcap > 0.f) MLR_PROMPT(1, true);
+      else if (wide) MLR_PROMPT(1, false);
+      else if (softcap > 0.f) MLR_PROMPT(2, true);
+      else MLR_PROMPT(2, false);
+#undef MLR_PROMPT
+      launched = true;
+  }
+#endif
   // a wavefront's 64 pieces of a tile lie in one page: whole key rows (D / 8 pieces each, a power
   // of two) that fit a page, and as many pieces of a value page
   const bool uniform = (D & (D - 1)) == 0 && D * block_size >= 512;
@@ -1205,13 +1583,15 @@ int mlr_attention_prefill(const void* q, int64_t q_stride, const void* key_pages
           static_cast<bf16*>(out), num_tiles, heads, kv_heads, bs_shift, num_pages, scale, window, chunk, partial,  \
           (splits > 1 || keep_partial) ? nullptr : sinks, keep_partial, score_bias, softcap, keep_first);  \
   } while (0)
-  if constexpr (D <= 128) {
-    if (wide)
-      MLR_PREFILL(2);
-    else
+  if (!launched) {
+    if constexpr (D <= 128) {
+      if (wide)
+        MLR_PREFILL(2);
+      else
+        MLR_PREFILL(1);
+    } else {
       MLR_PREFILL(1);
-  } else {
-    MLR_PREFILL(1);
+    }
   }
 #undef MLR_PREFILL
   MLR_LAUNCH_CHECK();

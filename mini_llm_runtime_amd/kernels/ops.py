@@ -1195,6 +1195,10 @@ class HipOps:
             tiles, wide = plan.query_tiles, 0
             num_wide = int(getattr(plan, "num_wide_query_tiles", 0))
             enough = self.tuning.wide_attention_groups
+            if head_dim == 128 and block_size >= 16 and score_bias is None and not keep_first:
+                # the 32 x 32 kernel: at this head size its narrow tiles have a compute unit to themselves (128 KB of LDS), so the
+                # wide ones win from half as many on
+                enough //= 2
             behind = int(getattr(plan, "long_prefix", 0))  # 1: thousands of keys before every tile, 2: twice that
             if behind:
                 enough = enough * 3 // 4  # heavy tiles everywhere: fewer of them keep the compute units busy

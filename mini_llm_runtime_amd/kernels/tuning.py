@@ -26,6 +26,9 @@ class KernelTuning:
     # Prompt attention takes tiles of 128 queries instead of 64 once tiles x heads reach this many
     # workgroups (fewer leave compute units idle behind the heaviest tiles).
     # Behind thousands of cached keys every tile is heavy and three quarters of that are enough.
+    # With the 32 x 32 kernel (head sizes 64 and 128), narrow / wide, microseconds: head size 64, 14 heads: 2,048 tokens (224 wide
+    # workgroups) 23 / 34, 4,096 (448) 60 / 65, 8,191 (896) 190 / 156; head size 128 (where half of this is the line), 28 heads:
+    # 1,024 (224) 29 / 29, 2,048 (448) 70 / 52, 4,096 203 / 148; 16 heads: 1,024 (128) 19 / 27, 2,048 (256) 46 / 47.
     wide_attention_groups: int = 512
     # Behind twice as many keys, fewer workgroups than this have the keys of every tile cut into
     # runs (up to 8) with a workgroup each, until there are this many.

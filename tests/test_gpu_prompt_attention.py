@@ -1,0 +1,65 @@
+"""The 32 x 32 prompt attention (head sizes 64 and 128) at the edges of its tiles, against the plain 32-bit kernel."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from test_gpu_kernels import _attend, _paged_case, _rand, _tol, _wide_ops
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", params=["narrow", "wide"])
+def ops(request):
+    from mini_llm_runtime_amd.kernels.ops import HipOps
+    from mini_llm_runtime_amd.kernels.tuning import KernelTuning
+
+    if request.param == "wide":
+        return _wide_ops()
+    return HipOps(torch.bfloat16, "cuda", tuning=KernelTuning(wide_attention_groups=1 << 30))
+
+
+# queries around 32 (a wavefront), 64 and 128 (a workgroup); last keys at every kind of place among 8, 16 and 64; portions behind
+# cached tokens; what no key was written to holds NaN
+ENTRIES = [(2, 2), (31, 31), (33, 33), (64, 64), (65, 65), (127, 127), (129, 129), (200, 70), (331, 5), (192, 130), (77, 1)]
+
+
+@pytest.mark.parametrize("heads,kv_heads,head_dim,block", [(14, 2, 64, 16), (4, 1, 128, 16), (3, 3, 64, 64), (2, 1, 128, 32)])
+@pytest.mark.parametrize(
+    "mask", [dict(window=None), dict(window=50), dict(window=None, chunk=48), dict(window=None, softcap=3.0)], ids=["causal", "window", "chunk", "cap"]
+)
+@pytest.mark.parametrize("sink", [False, True])
+def test_edges(ops, heads, kv_heads, head_dim, block, mask, sink):
+    q, kp, vp, table, ctx, *_ = _paged_case(ENTRIES, heads, kv_heads, head_dim, block, torch.bfloat16, 51, spike=True)
+    args = (q.cuda(), kp.cuda(), vp.cuda(), table.cuda(), ctx)
+    kw = dict(num_heads=heads, num_kv_heads=kv_heads, head_dim=head_dim, block_size=block, scale=head_dim**-0.5, **mask)
+    if sink:
+        kw["sinks"] = _rand((heads,), torch.float32, 52, 2.0).cuda()
+    got, plain = _attend(ops, *args, **kw).cpu(), _attend(ops, *args, kernel="fma", **kw).cpu()
+    assert torch.isfinite(got).all()
+    torch.testing.assert_close(got.double(), plain.double(), **_tol(torch.bfloat16))
+
+
+@pytest.mark.parametrize("head_dim", [64, 128])
+def test_scores_that_keep_rising(ops, head_dim):
+    """Every tile of keys scores higher than all before it, by less and by more than the running maximum's slack."""
+    for step in (0.5, 4.0, 40.0):
+        n = 300
+        q, kp, vp, table, ctx, *_ = _paged_case([(n, n)], 2, 1, head_dim, 16, torch.bfloat16, 53)
+        q[:, : 2 * head_dim] = 1.0
+        for p in range(n):
+            kp[table[0, p // 16], :, p % 16] = step * (p // 64) / head_dim + 0.01 * (p % 7)
+        kw = dict(num_heads=2, num_kv_heads=1, head_dim=head_dim, block_size=16, scale=1.0, window=None)
+        args = (q.cuda(), kp.cuda(), vp.cuda(), table.cuda(), ctx)
+        got, plain = _attend(ops, *args, **kw).cpu(), _attend(ops, *args, kernel="fma", **kw).cpu()
+        torch.testing.assert_close(got.double(), plain.double(), **_tol(torch.bfloat16))
+
+
+def test_a_page_that_is_not_there(ops):
+    q, kp, vp, table, ctx, *_ = _paged_case([(100, 100), (300, 300)], 2, 1, 64, 16, torch.bfloat16, 54)
+    table = table.clone()
+    table[1, 9] = -1  # positions 144..159 of the second request
+    kw = dict(num_heads=2, num_kv_heads=1, head_dim=64, block_size=16, scale=0.125, window=None)
+    got = _attend(ops, q.cuda(), kp.cuda(), vp.cuda(), table.cuda(), ctx, **kw).cpu()
+    assert torch.isfinite(got[:228]).all() and torch.isnan(got[100 + 256 :]).all()
