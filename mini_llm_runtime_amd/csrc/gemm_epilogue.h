@@ -232,6 +232,66 @@ __device__ __forceinline__ void store4(const GemmEpilogue& ep, int64_t m, int n,
   }
 }
 
+// A whole tile of finished bfloat16 results through LDS.  A lane of the accumulators holds 4 consecutive features of one token, so
+// stores straight from them are 8 bytes (4 after a pairing) every 32 rows: a wavefront's store touches 32 lines and fills a
+// sixteenth of each.  Staged in LDS the rows of the tile leave 16 bytes a lane, whole lines at a time.  For plain sums, with a bias or
+// without, and the pairings, of whole products (no slices of k, no multiplier); see stages_tile.
+__host__ __device__ inline bool stages_tile(const GemmEpilogue& ep, int slices, int N) {
+  const bool paired = ep.swiglu == kEpSwiglu || ep.swiglu == kEpGeglu;
+  return slices == 1 && !ep.out_is_f32 && ep.multiply == nullptr && (paired || ep.swiglu == kEpNone) && N % (paired ? 16 : 8) == 0 &&
+         reinterpret_cast<uintptr_t>(ep.y) % 16 == 0;
+}
+// LDS that staging a tile takes: rows of `features` results, padded by 16 bytes so that neighbouring rows fall on other banks.
+constexpr int staged_tile_bytes(int tokens, int features) { return tokens * (features * 2 + 16); }
+
+// KIND: kEpNone, kEpSwiglu or kEpGeglu.  acc[i][j]: block i of 32 features, block j of 32 tokens of this wavefront, which starts at feature
+// `feature0` and token `token0` of the tile; lane column r32, half h.  All THREADS of the workgroup, behind a barrier.
+template <int KIND, int THREADS, int BM, int BN, int NI, int NJ>
+__device__ __forceinline__ void stage_tile(const GemmEpilogue& ep, const f32x16_t (&acc)[NI][NJ], unsigned char* lds, const float* scales,
+                                           int feature0, int token0, int r32, int h, int m0, int n0, int M, int N) {
+  constexpr bool kPaired = KIND == kEpSwiglu || KIND == kEpGeglu;
+  constexpr int kOut = kPaired ? BN / 2 : BN;
+  constexpr int kRow = kOut * 2 + 16;
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int f = feature0 + i * 32 + g * 8 + h * 4;
+      float b[4] = {0.f, 0.f, 0.f, 0.f};
+      if (KIND != kEpSwiglu && ep.bias != nullptr && n0 + f < N) {  // n0 + f + 3 < N too: both are multiples of 4
+#pragma unroll
+        for (int e = 0; e < 4; ++e) b[e] = load_as_f32(ep.bias, n0 + f + e, ep.bias_is_f32);
+      }
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        const int token = token0 + j * 32 + r32;
+        const float scale = ep.row_sumsq != nullptr ? scales[token] : 1.f;
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = acc[i][j][g * 4 + e] * scale + b[e];
+        if constexpr (KIND == kEpSwiglu) {
+          *reinterpret_cast<uint32_t*>(lds + token * kRow + f) = pack_bf16x2(silu(v[0]) * v[2], silu(v[1]) * v[3]);
+        } else if constexpr (KIND == kEpGeglu) {
+          *reinterpret_cast<uint32_t*>(lds + token * kRow + f) = pack_bf16x2(gelu_tanh(v[0]) * v[2], gelu_tanh(v[1]) * v[3]);
+        } else {
+          typedef uint32_t words_t __attribute__((ext_vector_type(2)));
+          *reinterpret_cast<words_t*>(lds + token * kRow + f * 2) = words_t{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+        }
+      }
+    }
+  __syncthreads();
+  const int n_out = kPaired ? N / 2 : N, first = kPaired ? n0 / 2 : n0;
+  constexpr int kRowPieces = kOut / 8;
+  constexpr int kAll = BM * kRowPieces;
+#pragma unroll 4
+  for (int p = threadIdx.x; p < kAll; p += THREADS) {
+    const int row = p / kRowPieces, col = p - row * kRowPieces;
+    if (m0 + row < M && first + col * 8 < n_out)
+      *reinterpret_cast<u32x4_t*>(static_cast<bf16*>(ep.y) + static_cast<int64_t>(m0 + row) * n_out + first + col * 8) =
+          *reinterpret_cast<const u32x4_t*>(lds + row * kRow + col * 16);
+  }
+}
+
 // Store one accumulator tile (4 consecutive features of one token per lane): the
 // final result, or this K slice's partial sums.
 template <bool ACTIVATIONS = true>
