@@ -930,10 +930,11 @@ class HipOps:
             )
             return q
         if fused is None:
-            # Measured at 2,048 tokens: the fused kernel wins while the product is small (0.5B to 3B
-            # widths, and any width up to some 512 tokens); where the plain product would run in
-            # 256 x 256 tiles (7B, 32B) it is 15 % faster followed by the rotation kernel.
-            large = m > 64 and -(-m // 256) * -(-width // 256) >= 144
+            # The fused kernel has 64 x 64 tiles only; beyond 2^33 multiply-adds the plain product in the planner's tiles with the
+            # rotation kernel behind it is the faster way.  Fused / plain, in a replayed graph, us: 0.5B sizes at 4,096 tokens (4.2e9)
+            # 27 / 29; 1.5B at 1,536 (4.8e9) 25 / 27, at 4,096 (1.3e10) 60 / 43; 7B at 512 (8.5e9) 42 / 44, at 768 (1.3e10) 54 / 46, at
+            # 1,024 69 / 58, at 2,048 129 / 83; 14B at 400 (1.5e10) 75 / 76, at 512 88 / 78.
+            large = m > 64 and m * width * k >= 1 << 33
             fused = can_fuse and not large
         elif fused and not can_fuse:
             raise KernelError("the fused query/key/value kernel takes bfloat16 tokens and a full rotation")
