@@ -345,13 +345,13 @@ int mlr_gate_group_norm(const float* y, const float* projected, int width, int g
                         hipStream_t stream);
 
 // Routed experts (moe.hip).  mlr_moe_route: per token, from the router's float32 logits [tokens,
-// experts]: s = sigmoid(z) (score_kind 0), softmax(z) over all experts (1), or z itself for the choice and the softmax over
+// experts] (or `slices` partial sums of them, [slices, tokens, experts]): s = sigmoid(z) (score_kind 0), softmax(z) over all experts (1), or z itself for the choice and the softmax over
 // the chosen z as weights (2), choice scores c = s + correction (float32 [experts], or null); the
 // expert axis is cut into `groups` contiguous blocks of experts / groups; block score = top-2 sum of
 // c; eligible are the experts of the `keep` highest blocks; ids [tokens, top] = arg-top-`top` of c over
 // the eligible (ties to the lower index), weights [tokens, top] = s[id] * scale, with `normalise` divided by the
 // sum of a token's chosen s (+ 1e-20) first.
-int mlr_moe_route(const float* logits, const float* correction, int* ids, float* weights, int tokens, int experts,
+int mlr_moe_route(const float* logits, int slices, const float* correction, int* ids, float* weights, int tokens, int experts,
                   int top, int groups, int keep, float scale, int score_kind, int normalise, hipStream_t stream);
 // out[j, t, :] = weights[t, j] * h[t, :] where ids[t, j] >= first: experts without matrices that hand their input on.
 int mlr_moe_identity(const void* h, const int* ids, const float* weights, float* out, int dtype, int tokens, int top,

@@ -35,9 +35,9 @@ __device__ __forceinline__ void wave_argmax(float& v, int& i) {
 // consecutive experts scores top-2 sum of its c; c := -inf outside the `keep` highest blocks; then
 // `top` rounds of arg-max over c (ties to the lower index), each winner e leaving ids = e and
 // weights = s[e] * scale.
-__global__ __launch_bounds__(kWave) void moe_route_kernel(const float* __restrict__ logits,
+__global__ __launch_bounds__(kWave) void moe_route_kernel(const float* __restrict__ logits, int slices,
                                                           const float* __restrict__ correction,
-                                                          int* __restrict__ ids, float* __restrict__ weights,
+                                                          int* __restrict__ ids, float* __restrict__ weights, int tokens,
                                                           int experts, int top, int groups, int keep, float scale,
                                                           int score_kind, int normalise) {
   extern __shared__ float route_lds[];
@@ -47,18 +47,23 @@ __global__ __launch_bounds__(kWave) void moe_route_kernel(const float* __restric
   const int t = blockIdx.x;
   const int lane = threadIdx.x;
   const int per = experts / groups;
-  const float* z = logits + static_cast<int64_t>(t) * experts;
+  auto logit = [&](int e) {
+    float z = 0.f;
+    for (int p = 0; p < slices; ++p) z += logits[(static_cast<int64_t>(p) * tokens + t) * experts + e];
+    return z;
+  };
   float z_max = 0.f, z_inv = 1.f;
   if (score_kind == 1) {
     float mx = -INFINITY;
-    for (int e = lane; e < experts; e += kWave) mx = fmaxf(mx, z[e]);
+    for (int e = lane; e < experts; e += kWave) mx = fmaxf(mx, logit(e));
     z_max = wave_max(mx);
     float sum = 0.f;
-    for (int e = lane; e < experts; e += kWave) sum += expf(z[e] - z_max);
+    for (int e = lane; e < experts; e += kWave) sum += expf(logit(e) - z_max);
     z_inv = 1.0f / wave_sum(sum);
   }
   for (int e = lane; e < experts; e += kWave) {
-    const float sv = score_kind == 2 ? z[e] : (score_kind == 1 ? expf(z[e] - z_max) * z_inv : 1.0f / (1.0f + expf(-z[e])));
+    const float z = logit(e);
+    const float sv = score_kind == 2 ? z : (score_kind == 1 ? expf(z - z_max) * z_inv : 1.0f / (1.0f + expf(-z)));
     s[e] = sv;
     c[e] = sv + (correction != nullptr ? correction[e] : 0.f);
   }
@@ -127,6 +132,139 @@ __global__ __launch_bounds__(kWave) void moe_route_kernel(const float* __restric
   }
 }
 
+// The same for up to 64 R experts, 64 groups and 64 choices: a lane keeps R experts in registers (expert r * 64 + lane), a round of
+// arg-max is a maximum over the wavefront by lane moves and a vote for the lowest index, and only the groups' top-2 sums go through
+// LDS.  The logits may come as `slices` partial sums [slices, tokens, experts], added up in order.
+// Bound by latency: the plain kernel's rounds go through LDS six times each.  64 experts in 8 groups, 6 choices: 8 tokens 10.5 to 4.7
+// us, 2,000 tokens 13.3 to 6.9.
+template <int R>
+__global__ __launch_bounds__(kWave) void moe_route_lanes_kernel(const float* __restrict__ logits, int slices,
+                                                                const float* __restrict__ correction, int* __restrict__ ids,
+                                                                float* __restrict__ weights, int tokens, int experts, int top,
+                                                                int groups, int keep, float scale, int score_kind, int normalise) {
+  __shared__ float lds[R * kWave];
+  const int t = blockIdx.x;
+  const int lane = threadIdx.x;
+  float z[R], s[R], c[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int e = r * kWave + lane;
+    z[r] = 0.f;
+    for (int p0 = 0; p0 < slices; p0 += 8) {  // eight on their way at once
+      float part[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        part[u] = logits[(static_cast<int64_t>(min(p0 + u, slices - 1)) * tokens + t) * experts + min(e, experts - 1)];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) z[r] += p0 + u < slices ? part[u] : 0.f;
+    }
+  }
+  float z_max = 0.f, z_inv = 1.f;
+  if (score_kind == 1) {
+    float mx = -INFINITY, sum = 0.f;
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      if (r * kWave + lane < experts) mx = fmaxf(mx, z[r]);
+    z_max = wave_max(mx);
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      if (r * kWave + lane < experts) sum += expf(z[r] - z_max);
+    z_inv = 1.0f / wave_sum(sum);
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int e = r * kWave + lane;
+    s[r] = score_kind == 2 ? z[r] : (score_kind == 1 ? expf(z[r] - z_max) * z_inv : 1.0f / (1.0f + expf(-z[r])));
+    c[r] = s[r] + (correction != nullptr && e < experts ? correction[e] : 0.f);
+  }
+  // the lowest index among the largest of v[r] (index index(r), below `count`); NaN never wins; `count` if there is none
+  auto arg_max = [&](const float(&v)[R], int count, float& best) {
+    float mine = -INFINITY;
+    int index = 0x7fffffff;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int e = r * kWave + lane;
+      if (e < count && (v[r] > mine || (v[r] == mine && e < index))) {
+        mine = v[r];
+        index = e;
+      }
+    }
+    best = wave_max(mine);
+    int found = count;
+#pragma unroll
+    for (int r = R - 1; r >= 0; --r) {
+      const unsigned long long lanes = __ballot(index == r * kWave + lane && mine == best);
+      if (lanes != 0) found = r * kWave + __ffsll(lanes) - 1;
+    }
+    return found;
+  };
+  const int per = experts / groups;
+  if (groups > 1 && keep < groups) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) lds[r * kWave + lane] = c[r];
+    __syncthreads();
+    float gs[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) gs[r] = -INFINITY;
+    if (lane < groups) {
+      float a = -INFINITY, b = -INFINITY;  // running top-2 of the block
+#pragma unroll 8
+      for (int i = 0; i < per; ++i) {
+        const float v = lds[lane * per + i];
+        if (v > a) {
+          b = a;
+          a = v;
+        } else if (v > b) {
+          b = v;
+        }
+      }
+      gs[0] = per > 1 ? a + b : a;
+    }
+    unsigned long long kept = 0;
+    bool mine_kept = lane >= groups;  // groups that are kept already, or do not exist, are out of the choice
+    for (int k = 0; k < keep; ++k) {
+      const float v = mine_kept ? __builtin_nanf("") : gs[0];
+      float one[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) one[r] = r == 0 ? v : __builtin_nanf("");
+      float best;
+      const int g = arg_max(one, groups, best);
+      if (g >= groups) break;  // only NaN left
+      kept |= 1ull << g;
+      mine_kept = mine_kept || lane == g;
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int e = r * kWave + lane;
+      if (e < experts && !((kept >> (e / per)) & 1)) c[r] = -INFINITY;
+    }
+  }
+  float chosen_sum = 0.f, z_top = 0.f, my_weight = 0.f;
+  int my_id = 0;
+  for (int k = 0; k < top; ++k) {
+    float best;
+    int i = arg_max(c, experts, best);
+    if (i >= experts) i = 0;  // only if every score left is NaN: keep the id in range
+    float si = 0.f;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      if (i / kWave == r) si = lane_value(s[r], i % kWave);
+      if (i == r * kWave + lane) c[r] = -INFINITY;
+    }
+    if (k == 0) z_top = si;
+    const float w = score_kind == 2 ? expf(si - z_top) : si;
+    chosen_sum += w;
+    if (lane == k) {
+      my_id = i;
+      my_weight = w * scale;
+    }
+  }
+  if (lane < top) {
+    ids[static_cast<int64_t>(t) * top + lane] = my_id;
+    weights[static_cast<int64_t>(t) * top + lane] = normalise ? my_weight * (1.0f / (chosen_sum + 1e-20f)) : my_weight;
+  }
+}
+
 // Experts that hand their input on: where ids[t, j] >= first (such an expert has no matrices and the grouped
 // products skip its pairs) out[j, t, :] = weights[t, j] * h[t, :].  One workgroup per pair.
 template <typename T>
@@ -156,10 +294,18 @@ __global__ __launch_bounds__(1024) void moe_align_kernel(const int* __restrict__
   const int tid = threadIdx.x;
   for (int e = tid; e < experts; e += blockDim.x) counts[e] = 0;
   __syncthreads();
-  for (int p = tid; p < pairs; p += blockDim.x) {
-    const int e = ids[p];
-    if (e >= 0 && e < experts) atomicAdd(&counts[e], 1);
-  }
+  // eight ids of a thread are asked for at once: one after the other each would be a trip to L2
+  auto for_each_pair = [&](auto&& use) {
+    for (int p0 = tid; p0 < pairs; p0 += 8 * 1024) {
+      int e[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) e[u] = ids[min(p0 + u * 1024, pairs - 1)];
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (p0 + u * 1024 < pairs && e[u] >= 0 && e[u] < experts) use(p0 + u * 1024, e[u]);
+    }
+  };
+  for_each_pair([&](int, int e) { atomicAdd(&counts[e], 1); });
   __syncthreads();
   if (tid < kWave) {  // the first wavefront: where every expert's run and tiles start, 64 experts at a time
     int at = 0, nt = 0;
@@ -201,10 +347,7 @@ __global__ __launch_bounds__(1024) void moe_align_kernel(const int* __restrict__
   }
   for (int e = tid; e < experts; e += blockDim.x) counts[e] = 0;
   __syncthreads();
-  for (int p = tid; p < pairs; p += blockDim.x) {
-    const int e = ids[p];
-    if (e >= 0 && e < experts) sorted[start[e] + atomicAdd(&counts[e], 1)] = p;
-  }
+  for_each_pair([&](int p, int e) { sorted[start[e] + atomicAdd(&counts[e], 1)] = p; });
 }
 
 // ---- the clamped gating in a grouped product's epilogue ------------------------------------------------
@@ -400,15 +543,18 @@ __global__ __launch_bounds__(256) void moe_gemm_mfma_kernel(const bf16* __restri
 }
 
 // Streaming through LDS (tiles of 16 rows, as above): the same work with loads that cover whole lines.
-// A workgroup owns 16 rows of a tile and 64 features; k in slices of 128.  Sixteen neighbouring lanes
-// fetch the 256 contiguous bytes that a slice holds of one weight row (the kernel above reads 64 bytes
-// of 16 different rows per instruction, which streams a large matrix at little more than half the
-// rate), two slices ahead in registers, and stage them through two LDS buffers whose rows of 288 bytes
-// are free of bank conflicts for the operand pattern of the 16 x 16 x 32 block.  Wavefront w multiplies
-// features w * 16 .. + 16.
+// A workgroup owns 16 rows of a tile and 64 features; k in slices of 128, loaded straight into four LDS buffers, three of them
+// on their way (48 KB of weights a workgroup, two workgroups a compute unit: a step through registers had 16 to 32 KB on their way).  Sixteen
+// neighbouring lanes fetch the 256 contiguous bytes that a slice holds of one weight row (the kernel above reads 64 bytes of 16
+// different rows per instruction, which streams a large matrix at little more than half the rate); the 16-byte pieces of a row lie in the
+// order piece ^ row % 16, so that the operand reads of sixteen rows fall on different banks.  Wavefront w multiplies features w * 16 .. + 16.
+// Bound by HBM: 8 tokens, 64 experts with 6 choices, matrices of 768 x 2,048: up 25.5 to 22.3 us, down 23.7 to 23.3 (up to 48 experts'
+// 151 MB for each of the two: 6.5 TB/s).  Tiles start their features at different places, or neighbours would ask the same channels at once.
 constexpr int kStCols = 64;
 constexpr int kStK = 128;
-constexpr int kStLd = kStK + 16;  // bf16 elements per LDS row: 288 bytes
+constexpr int kStBuffers = 4;
+constexpr int kStBufferBytes = (kStCols + kMoeRows) * kStK * 2;
+constexpr int kStLds = kStBuffers * kStBufferBytes;
 
 template <bool UP>
 __global__ __launch_bounds__(256) void moe_gemm_stream_kernel(const bf16* __restrict__ a, const bf16* __restrict__ w,
@@ -418,82 +564,76 @@ __global__ __launch_bounds__(256) void moe_gemm_stream_kernel(const bf16* __rest
                                                               const float* __restrict__ pair_weights,
                                                               void* __restrict__ out, int tokens, int top, int N, int K,
                                                               int act, int a_rows, float glu_limit, float glu_alpha) {
-  const int expert = tiles[2 * blockIdx.x];
+  // Workgroups go to the eight dies in turn and the unused tiles lie at the end of the list: each run of features starts at
+  // another tile, or the same dies would find them every time (35 of 48 tiles used: five on some dies, four on others).
+  const int tile = (blockIdx.x + blockIdx.y) % gridDim.x;
+  const int expert = tiles[2 * tile];
   if (expert < 0) return;
-  const int row0 = tiles[2 * blockIdx.x + 1];
+  const int row0 = tiles[2 * tile + 1];
   const int row_end = offsets[expert + 1];
-  __shared__ __attribute__((aligned(16))) bf16 ws[2][kStCols * kStLd];
-  __shared__ __attribute__((aligned(16))) bf16 xs[2][kMoeRows * kStLd];
-  __shared__ int pair_of[kMoeRows];
-  const int tid = threadIdx.x;
-  const int lane = tid % kWave;
-  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  extern __shared__ __attribute__((aligned(16))) unsigned char moe_lds[];
+  const int lane = threadIdx.x % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int n0 = blockIdx.y * kStCols;
-  if (tid < kMoeRows) pair_of[tid] = row0 + tid < row_end ? sorted[row0 + tid] : -1;
-  __syncthreads();
   const unsigned row_bytes = static_cast<unsigned>(K) * 2u;
   const __amdgpu_buffer_rsrc_t wbuf =
       make_buffer(w + static_cast<int64_t>(expert) * N * K, static_cast<unsigned>(N) * row_bytes);
   const __amdgpu_buffer_rsrc_t abuf = make_buffer(a, static_cast<unsigned>(a_rows) * row_bytes);
-  // per slice a thread moves four 16-byte pieces of the weight tile (rows prow, prow + 16, ...) and one
-  // of the input tile (row prow), all at k piece `piece` of the slice
-  const int piece = tid % 16;
-  const int prow = tid / 16;
+  // A load fills 4 rows of a buffer (1 KB): rows 4 * (4 * i + wave) + lane / 16 of the weights for i = 0..3, then rows 4 * wave +
+  // lane / 16 of the input tile; the row modulo 16 is the same for all five, so is the piece that this lane brings
+  const int my_row = 4 * wave + lane / 16;
+  const int piece = (lane % 16) ^ my_row;
   unsigned w_off[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const int row = n0 + prow + i * 16;
+    const int row = n0 + i * 16 + my_row;
     w_off[i] = row < N ? static_cast<unsigned>(row) * row_bytes + piece * 16u : kOutOfBuffer;
   }
-  const int my_pair = pair_of[prow];
-  const int src = my_pair < 0 ? -1 : (UP ? my_pair / top : row0 + prow);
-  const unsigned x_off = src >= 0 ? static_cast<unsigned>(src) * row_bytes + piece * 16u : kOutOfBuffer;
-  const int lds_at = prow * kStLd + piece * 8;
-  bf16x8_t w_a[4], w_b[4], x_a, x_b;  // two slices on their way
-  auto fetch = [&](bf16x8_t(&wreg)[4], bf16x8_t& xreg, int k0) {
-    const bool k_in = k0 + piece * 8 < K;
-    const unsigned koff = static_cast<unsigned>(k0) * 2u;
+  const int my_pair = sorted[min(row0 + my_row, row_end - 1)];
+  const int slices = (K + kStK - 1) / kStK;
+  unsigned x_off = 0;
+  auto fetch_weights = [&](int slice, int buf) {
+    const unsigned koff = static_cast<unsigned>(slice) * kStK * 2u;
+    const bool in = slice < slices && slice * kStK + piece * 8 < K;
+    unsigned char* const dst = moe_lds + buf * kStBufferBytes + wave * 1024;
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      wreg[i] = buffer_load_bf16x8_once(wbuf, k_in && w_off[i] != kOutOfBuffer ? w_off[i] + koff : kOutOfBuffer);
-    xreg = buffer_load_bf16x8(abuf, k_in && x_off != kOutOfBuffer ? x_off + koff : kOutOfBuffer);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(wbuf, (__attribute__((address_space(3))) void*)(dst + i * 4096), 16,
+                                               in && w_off[i] != kOutOfBuffer ? w_off[i] + koff : kOutOfBuffer, 0, 0, 2);
   };
-  auto stage = [&](const bf16x8_t(&wreg)[4], const bf16x8_t& xreg, int buf) {
+  auto fetch_rows = [&](int slice, int buf) {
+    const bool in = slice < slices && slice * kStK + piece * 8 < K && x_off != kOutOfBuffer;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+        abuf, (__attribute__((address_space(3))) void*)(moe_lds + buf * kStBufferBytes + wave * 1024 + 16384), 16,
+        in ? x_off + static_cast<unsigned>(slice) * kStK * 2u : kOutOfBuffer, 0, 0, 0);
+  };
+  // the weights do not wait for the lookup of the rows
 #pragma unroll
-    for (int i = 0; i < 4; ++i) *reinterpret_cast<bf16x8_t*>(&ws[buf][lds_at + i * 16 * kStLd]) = wreg[i];
-    *reinterpret_cast<bf16x8_t*>(&xs[buf][lds_at]) = xreg;
-  };
+  for (int s = 0; s < kStBuffers - 1; ++s) fetch_weights(s, s);
+  x_off = row0 + my_row < row_end ? static_cast<unsigned>(UP ? my_pair / top : row0 + my_row) * row_bytes + piece * 16u : kOutOfBuffer;
+#pragma unroll
+  for (int s = 0; s < kStBuffers - 1; ++s) fetch_rows(s, s);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // they were sent together and arrive together; from here on slices are waited for one by one
   const int col = lane % 16;
   const int quad = lane / 16;
   f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-  auto multiply = [&](int buf) {
-    const bf16* wt = &ws[buf][(wave * 16 + col) * kStLd + quad * 8];
-    const bf16* xt = &xs[buf][col * kStLd + quad * 8];
+  for (int s = 0; s < slices; ++s) {
+    // this slice has landed (this wavefront's share; the barrier answers for the others), and everybody has multiplied the one before
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((kStBuffers - 2) * 5) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    fetch_weights(s + kStBuffers - 1, (s + kStBuffers - 1) % kStBuffers);
+    fetch_rows(s + kStBuffers - 1, (s + kStBuffers - 1) % kStBuffers);  // into the buffer of the slice before
+    const unsigned char* const base = moe_lds + s % kStBuffers * kStBufferBytes;
 #pragma unroll
-    for (int ks = 0; ks < kStK / 32; ++ks)
-      acc = mfma_16x16x32(*reinterpret_cast<const bf16x8_t*>(wt + ks * 32),
-                          *reinterpret_cast<const bf16x8_t*>(xt + ks * 32), acc);
-  };
-  const int slices = (K + kStK - 1) / kStK;
-  fetch(w_a, x_a, 0);
-  if (slices > 1) fetch(w_b, x_b, kStK);
-  stage(w_a, x_a, 0);
-  __syncthreads();
-  // two slices a turn, so that the register sets and the LDS buffers keep their names; `slices` is the
-  // same for every thread, so are the barriers
-  for (int s = 0; s < slices; s += 2) {
-    if (s + 2 < slices) fetch(w_a, x_a, (s + 2) * kStK);
-    multiply(0);
-    if (s + 1 < slices) stage(w_b, x_b, 1);
-    __syncthreads();
-    if (s + 1 >= slices) break;
-    if (s + 3 < slices) fetch(w_b, x_b, (s + 3) * kStK);
-    multiply(1);
-    if (s + 2 < slices) stage(w_a, x_a, 0);
-    __syncthreads();
+    for (int ks = 0; ks < kStK / 32; ++ks) {
+      const int slot = ((ks * 4 + quad) ^ col) * 16;
+      acc = mfma_16x16x32(load_bf16x8(base + (wave * 16 + col) * 256 + slot), load_bf16x8(base + 16384 + col * 256 + slot), acc);
+    }
   }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing may still be on its way into LDS when the workgroup ends
   // acc[i]: feature n0 + wave * 16 + quad * 4 + i of tile row `col`
-  const int pair = pair_of[col];
+  const int pair = row0 + col < row_end ? sorted[row0 + col] : -1;
   if (pair < 0) return;
   const int token = pair / top;
   const int choice = pair - token * top;
@@ -523,85 +663,92 @@ __global__ __launch_bounds__(256) void moe_gemm_stream_kernel(const bf16* __rest
   }
 }
 
-// Tiled (prompts, where an expert sees hundreds of rows): a workgroup owns a tile of 64 x RB rows and
-// 128 features; k in slices of 64 through two LDS buffers (rows padded to 144 bytes: free of bank
-// conflicts for the operand pattern of the 32 x 32 x 16 block), the next slice on its way into
-// registers while this one is multiplied.  Wavefront (wr, wc) of 2 x 2 owns rows wr * 32 RB .. + 32 RB
-// and features wc * 64 .. + 64: 2 RB blocks of 32 x 32; with RB = 2 every operand read from LDS serves
-// two products.
+// Tiled (prompts, where an expert sees hundreds of rows): a workgroup owns a tile of 64 x RB rows and 128 features; k in slices of
+// 64 loaded straight into two LDS buffers (a lane brings 16 bytes of the row that the tile's order names; pieces in the order
+// piece ^ (row / 2) % 8).  Wavefront (wr, wc) of 2 x 2 owns rows wr * 32 RB .. + 32 RB and features wc * 64 .. + 64; the last
+// quarter of a slice's products is kept for behind the barrier, where the next slice's first operands are on their way.  Finished
+// tiles leave through LDS in whole lines: the down product's rows go to as many places as it has rows, 512 bytes each.
+// Workgroup -> (tile, features): workgroups go to the eight dies in turn; a die gets every eighth pair of neighbouring tiles (mostly one
+// expert's) and takes their features one after the other, both tiles at a time, so that the rows and the expert's weights come from its L2.
+// Bound by the operands' way through L2 and LDS (each 64 x RB + 128 rows of a slice make 64 RB x 128 products of it) and by tiles
+// that are not full: 2,000 tokens, 64 experts with 6 choices (187 rows an expert in tiles of 128), 768 x 2,048: up 94.5 to 91.4 us,
+// down 128 to 93 (400 TFLOP/s of the asked-for products, 550 with the padding).  Four buffers of 32 k instead: up the same, down 102.
 constexpr int kBigCols = 128;
 constexpr int kBigK = 64;
-constexpr int kBigLd = kBigK + 8;  // bf16 elements per LDS row
 constexpr int big_rows(int rb) { return 64 * rb; }
-constexpr int big_lds_bytes(int rb) { return 2 * (kBigCols + big_rows(rb)) * kBigLd * 2 + big_rows(rb) * 4; }
+constexpr int big_buffer_bytes(int rb) { return (kBigCols + big_rows(rb)) * kBigK * 2; }
+constexpr int kBigRowF32 = kBigCols * 4 + 16, kBigRowBf16 = kBigCols * 2 + 16;  // staged rows, padded to other banks
+constexpr int big_lds_bytes(int rb) {
+  return big_rows(rb) * kBigRowF32 > 2 * big_buffer_bytes(rb) ? big_rows(rb) * kBigRowF32 : 2 * big_buffer_bytes(rb);
+}
 
 template <bool UP, int RB>
 __global__ __launch_bounds__(256) void moe_gemm_tiled_kernel(const bf16* __restrict__ a, const bf16* __restrict__ w,
                                                              const int* __restrict__ sorted,
                                                              const int* __restrict__ offsets,
-                                                             const int* __restrict__ tiles,
+                                                             const int* __restrict__ tiles, int max_tiles,
                                                              const float* __restrict__ pair_weights,
                                                              void* __restrict__ out, int tokens, int top, int N, int K,
                                                              int act, int a_rows, float glu_limit, float glu_alpha) {
   constexpr int kRows = big_rows(RB);
-  const int expert = tiles[2 * blockIdx.x];
+  constexpr int kBuffer = big_buffer_bytes(RB);
+  // runs of 8 rows, dealt out to four wavefronts: 4 of weights, then the input's (loops over them go to 8 and break: with a bound that
+  // depends on the template's parameters the host pass left the kernel uninstantiated, without a message)
+  constexpr int kLoads = (kBigCols + kRows) / 8 / 4;
+  const int columns = (N + kBigCols - 1) / kBigCols;
+  const int local = blockIdx.x / 8, in_pair = local % (2 * columns);
+  const int tile = (local / (2 * columns) * 8 + blockIdx.x % 8) * 2 + in_pair % 2;
+  if (tile >= max_tiles) return;
+  const int expert = tiles[2 * tile];
   if (expert < 0) return;
-  const int row0 = tiles[2 * blockIdx.x + 1];
-  const int row_end = offsets[expert + 1];
+  const int n0 = in_pair / 2 * kBigCols;
+  const int row0 = tiles[2 * tile + 1];
+  const int rows = min(kRows, offsets[expert + 1] - row0);
   extern __shared__ __attribute__((aligned(16))) unsigned char moe_lds[];
-  bf16* const ws = reinterpret_cast<bf16*>(moe_lds);   // [2][kBigCols][kBigLd]
-  bf16* const xs = ws + 2 * kBigCols * kBigLd;         // [2][kRows][kBigLd]
-  int* const pair_of = reinterpret_cast<int*>(xs + 2 * kRows * kBigLd);  // [kRows]
+  __shared__ int pair_of[kRows];
   const int tid = threadIdx.x;
   const int lane = tid % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int wr = wave / 2;
   const int wc = wave % 2;
-  const int n0 = blockIdx.y * kBigCols;
-  if (tid < kRows) pair_of[tid] = row0 + tid < row_end ? sorted[row0 + tid] : -1;
-  __syncthreads();
   const unsigned row_bytes = static_cast<unsigned>(K) * 2u;
-  const __amdgpu_buffer_rsrc_t wbuf =
-      make_buffer(w + static_cast<int64_t>(expert) * N * K, static_cast<unsigned>(N) * row_bytes);
+  const __amdgpu_buffer_rsrc_t wbuf = make_buffer(w + (static_cast<int64_t>(expert) * N + n0) * K, static_cast<unsigned>(min(kBigCols, N - n0)) * row_bytes);
   const __amdgpu_buffer_rsrc_t abuf = make_buffer(a, static_cast<unsigned>(a_rows) * row_bytes);
-  // what this thread moves per slice: 16-byte pieces of the weight tile and of the input tile
-  // (piece c: row c / 8, k piece c % 8), the same rows for every slice
-  constexpr int kWPieces = kBigCols * 8 / 256;
-  constexpr int kXPieces = kRows * 8 / 256;
-  unsigned w_off[kWPieces], x_off[kXPieces];
-  const int piece = tid % 8;  // the same for all of a thread's pieces: 256 is a multiple of 8
+  // Which pairs this tile's rows are: all lookups are sent at once and without conditions, then the weights of the first two slices,
+  // which do not depend on them (looked up one by one ahead of the first load, they took longer than a slice of products each).
+  constexpr int kRowLoads = kLoads - 4;
+  int pairs_of_lane[4];
 #pragma unroll
-  for (int i = 0; i < kWPieces; ++i) {
-    const int row = (tid + i * 256) / 8;
-    w_off[i] = n0 + row < N ? static_cast<unsigned>(n0 + row) * row_bytes + piece * 16u : kOutOfBuffer;
-  }
+  for (int p = 0; p < 4; ++p)
+    if (p < kRowLoads) pairs_of_lane[p] = sorted[row0 + min(8 * (4 * p + wave) + lane / 8, rows - 1)];
+  const int pair_of_thread = sorted[row0 + min(tid, rows - 1)];
+  const int piece = (lane % 8) ^ ((4 * (wave % 2) + lane / 16) % 8);
+  const int slices = (K + kBigK - 1) / kBigK;
+  unsigned off[8];
+  auto fetch = [&](int slice, int buf, bool weights) {
+    const unsigned past = slice < slices && slice * kBigK + piece * 8 < K ? 0u : kOutOfBuffer;
+    const unsigned koff = static_cast<unsigned>(slice) * kBigK * 2u;
 #pragma unroll
-  for (int i = 0; i < kXPieces; ++i) {
-    const int row = (tid + i * 256) / 8;
-    const int pair = pair_of[row];
-    const int src = pair < 0 ? -1 : (UP ? pair / top : row0 + row);
-    x_off[i] = src >= 0 ? static_cast<unsigned>(src) * row_bytes + piece * 16u : kOutOfBuffer;
-  }
-  const int lds_at = (tid / 8) * kBigLd + piece * 8;  // piece i of either tile: + i * 32 rows
-  bf16x8_t wreg[kWPieces], xreg[kXPieces];
-  auto fetch = [&](int k0) {
-    const bool k_in = k0 + piece * 8 < K;
-    const unsigned koff = static_cast<unsigned>(k0) * 2u;
-#pragma unroll
-    for (int i = 0; i < kWPieces; ++i)
-      wreg[i] = buffer_load_bf16x8(wbuf, k_in && w_off[i] != kOutOfBuffer ? w_off[i] + koff : kOutOfBuffer);
-#pragma unroll
-    for (int i = 0; i < kXPieces; ++i)
-      xreg[i] = buffer_load_bf16x8(abuf, k_in && x_off[i] != kOutOfBuffer ? x_off[i] + koff : kOutOfBuffer);
+    for (int p = 0; p < 8; ++p) {
+      if (p >= kLoads) break;
+      if ((p < 4) != weights) continue;
+      const unsigned at = p < 4 ? (off[p] + koff) | past : (past != 0u || off[p] == kOutOfBuffer ? kOutOfBuffer : off[p] + koff);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          p < 4 ? wbuf : abuf, (__attribute__((address_space(3))) void*)(moe_lds + buf * kBuffer + (4 * p + wave) * 1024), 16, at, 0, 0, 0);
+    }
   };
-  auto stage = [&](int buf) {
 #pragma unroll
-    for (int i = 0; i < kWPieces; ++i)
-      *reinterpret_cast<bf16x8_t*>(ws + buf * kBigCols * kBigLd + lds_at + i * 32 * kBigLd) = wreg[i];
+  for (int p = 0; p < 4; ++p)  // rows past the last feature: past the resource
+    off[p] = static_cast<unsigned>(8 * (4 * p + wave) + lane / 8) * row_bytes + piece * 16u;
+  fetch(0, 0, true);
+  fetch(1, 1, true);
 #pragma unroll
-    for (int i = 0; i < kXPieces; ++i)
-      *reinterpret_cast<bf16x8_t*>(xs + buf * kRows * kBigLd + lds_at + i * 32 * kBigLd) = xreg[i];
-  };
+  for (int p = 0; p < 4; ++p) {
+    if (p >= kRowLoads) break;
+    const int at = 8 * (4 * p + wave) + lane / 8;
+    off[4 + p] = at < rows ? static_cast<unsigned>(UP ? pairs_of_lane[p] / top : row0 + at) * row_bytes + piece * 16u : kOutOfBuffer;
+  }
+  if (tid < kRows) pair_of[tid] = tid < rows ? pair_of_thread : -1;
   f32x16_t acc[RB][2];
 #pragma unroll
   for (int r = 0; r < RB; ++r)
@@ -611,52 +758,79 @@ __global__ __launch_bounds__(256) void moe_gemm_tiled_kernel(const bf16* __restr
       for (int i = 0; i < 16; ++i) acc[r][b][i] = 0.f;
   const int r32 = lane % 32;
   const int khalf = lane / 32;  // which 8 of a block's 16 k
-  fetch(0);
-  stage(0);
+  const bool idle = __builtin_amdgcn_readfirstlane(static_cast<int>(wr * 32 * RB >= rows)) != 0;  // a tile with rows for the first wavefronts only
+  const int swz = (r32 / 2) % 8;
+  struct Operands {
+    bf16x8_t w[2], x[RB];
+  };
+  auto read = [&](int buf, int ks) {
+    Operands o;
+    const unsigned char* const base = moe_lds + buf * kBuffer + (((ks * 2 + khalf) ^ swz) * 16);
+#pragma unroll
+    for (int b = 0; b < 2; ++b) o.w[b] = load_bf16x8(base + (wc * 64 + b * 32 + r32) * 128);
+#pragma unroll
+    for (int r = 0; r < RB; ++r) o.x[r] = load_bf16x8(base + (kBigCols + (wr * RB + r) * 32 + r32) * 128);
+    return o;
+  };
+  auto multiply = [&](const Operands& o) {
+#pragma unroll
+    for (int r = 0; r < RB; ++r)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) acc[r][b] = mfma_32x32x16(o.w[b], o.x[r], acc[r][b]);
+  };
+  fetch(0, 0, false);
+  fetch(1, 1, false);
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kRowLoads) : "memory");
   __syncthreads();
+  Operands cur = read(0, 0);
   int buf = 0;
-  for (int k0 = 0; k0 < K; k0 += kBigK) {
-    const bool more = k0 + kBigK < K;
-    if (more) fetch(k0 + kBigK);
-    const bf16* wt = ws + buf * kBigCols * kBigLd + (wc * 64 + r32) * kBigLd + khalf * 8;
-    const bf16* xt = xs + buf * kRows * kBigLd + (wr * 32 * RB + r32) * kBigLd + khalf * 8;
+  for (int s = 0; s < slices; ++s) {
+    if (!idle) {
 #pragma unroll
-    for (int ks = 0; ks < kBigK / 16; ++ks) {
-      const bf16x8_t w0 = *reinterpret_cast<const bf16x8_t*>(wt + ks * 16);
-      const bf16x8_t w1 = *reinterpret_cast<const bf16x8_t*>(wt + 32 * kBigLd + ks * 16);
-#pragma unroll
-      for (int r = 0; r < RB; ++r) {
-        const bf16x8_t xb = *reinterpret_cast<const bf16x8_t*>(xt + r * 32 * kBigLd + ks * 16);
-        acc[r][0] = mfma_32x32x16(w0, xb, acc[r][0]);
-        acc[r][1] = mfma_32x32x16(w1, xb, acc[r][1]);
+      for (int ks = 0; ks < kBigK / 16 - 1; ++ks) {
+        const Operands next = read(buf, ks + 1);
+        multiply(cur);
+        cur = next;
       }
     }
-    if (more) stage(buf ^ 1);
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     __syncthreads();
+    fetch(s + 2, buf, true);
+    fetch(s + 2, buf, false);
     buf ^= 1;
+    if (!idle) {
+      const Operands kept = cur;
+      cur = read(buf, 0);
+      multiply(kept);
+    }
   }
-  // acc[r][b][i]: feature n0 + wc * 64 + b * 32 + (i / 4) * 8 + khalf * 4 + i % 4 of tile row
-  // wr * 32 RB + r * 32 + r32
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();  // the slices are done with
+  // acc[r][b][i]: feature n0 + wc * 64 + b * 32 + (i / 4) * 8 + khalf * 4 + i % 4 of tile row wr * 32 RB + r * 32 + r32.
+  // N is a multiple of 8: four features are all inside or all outside.
+  const bool paired = UP && act == 5;
+  const bool staged = !UP || N % (paired ? 16 : 8) == 0;  // rows of results are multiples of 16 bytes
 #pragma unroll
   for (int r = 0; r < RB; ++r) {
-    const int row = wr * 32 * RB + r * 32 + r32;
+    const int row = (wr * RB + r) * 32 + r32;
     const int pair = pair_of[row];
     if (pair < 0) continue;
-    const int token = pair / top;
-    const int choice = pair - token * top;
     const float pw = UP ? 1.f : pair_weights[pair];
 #pragma unroll
     for (int b = 0; b < 2; ++b)
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
-        const int n = n0 + wc * 64 + b * 32 + g * 8 + khalf * 4;
-        if (n >= N) continue;  // N is a multiple of 8 here: four features are all inside or all outside
+        const int f = wc * 64 + b * 32 + g * 8 + khalf * 4;
         float v[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) v[i] = acc[r][b][g * 4 + i];
-        if (UP && act == 5) {
-          store_clamped_glu(static_cast<bf16*>(out) + static_cast<int64_t>(row0 + row) * (N / 2) + n / 2, v, glu_limit, glu_alpha);
-        } else if (UP) {
+        if constexpr (!UP) {
+          *reinterpret_cast<f32x4_t*>(moe_lds + row * kBigRowF32 + f * 4) = f32x4_t{pw * v[0], pw * v[1], pw * v[2], pw * v[3]};
+        } else if (paired) {
+          bf16* const to = staged ? reinterpret_cast<bf16*>(moe_lds + row * kBigRowBf16) + f / 2
+                                  : static_cast<bf16*>(out) + static_cast<int64_t>(row0 + row) * (N / 2) + (n0 + f) / 2;
+          if (staged || n0 + f < N) store_clamped_glu(to, v, glu_limit, glu_alpha);
+        } else {
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             if (act == 2) {
@@ -668,12 +842,25 @@ __global__ __launch_bounds__(256) void moe_gemm_tiled_kernel(const bf16* __restr
           }
           const u16x4_t packed = {f32_to_bf16(v[0]).bits, f32_to_bf16(v[1]).bits, f32_to_bf16(v[2]).bits,
                                   f32_to_bf16(v[3]).bits};
-          *reinterpret_cast<u16x4_t*>(static_cast<bf16*>(out) + static_cast<int64_t>(row0 + row) * N + n) = packed;
-        } else {
-          float* dst = static_cast<float*>(out) + (static_cast<int64_t>(choice) * tokens + token) * N + n;
-          *reinterpret_cast<f32x4_t*>(dst) = f32x4_t{pw * v[0], pw * v[1], pw * v[2], pw * v[3]};
+          *reinterpret_cast<u16x4_t*>(moe_lds + row * kBigRowBf16 + f * 2) = packed;
         }
       }
+  }
+  if (!staged) return;
+  __syncthreads();
+  const int width = (paired ? N / 2 : N) * (UP ? 2 : 4);               // bytes of a row of results
+  const int first = (paired ? n0 / 2 : n0) * (UP ? 2 : 4);             // where this tile's part of it starts
+  const int pieces = (paired ? kBigCols / 2 : kBigCols) * (UP ? 2 : 4) / 16;  // 8, 16 or 32
+  for (int p = tid; p < rows * pieces; p += 256) {
+    const int row = p / pieces, at = (p - row * pieces) * 16;
+    if (first + at >= width) continue;
+    int64_t to = row0 + row;
+    if constexpr (!UP) {
+      const int pair = pair_of[row], token = pair / top;
+      to = static_cast<int64_t>(pair - token * top) * tokens + token;
+    }
+    *reinterpret_cast<u32x4_t*>(static_cast<unsigned char*>(out) + to * width + first + at) =
+        *reinterpret_cast<const u32x4_t*>(moe_lds + row * (UP ? kBigRowBf16 : kBigRowF32) + at);
   }
 }
 
@@ -691,8 +878,13 @@ static int launch_moe_tiled(const bf16* a, const bf16* w, const int* sorted, con
     }
     configured = true;
   }
-  const dim3 grid(max_tiles, (n + kBigCols - 1) / kBigCols);
-  moe_gemm_tiled_kernel<UP, RB><<<grid, 256, big_lds_bytes(RB), stream>>>(a, w, sorted, offsets, tiles, pair_weights, out,
+  const int64_t groups = static_cast<int64_t>((max_tiles + 15) / 16 * 16) * ((n + kBigCols - 1) / kBigCols);
+  if (groups >= (1ll << 31)) {
+    set_error("mlr_moe_gemm: too many tiles for one launch");
+    return -1;
+  }
+  const unsigned grid = static_cast<unsigned>(groups);
+  moe_gemm_tiled_kernel<UP, RB><<<grid, 256, big_lds_bytes(RB), stream>>>(a, w, sorted, offsets, tiles, max_tiles, pair_weights, out,
                                                                         tokens, top, n, k, act, a_rows, glu_limit,
                                                                         glu_alpha);
   return 0;
@@ -704,18 +896,30 @@ using namespace mlr;
 
 extern "C" {
 
-int mlr_moe_route(const float* logits, const float* correction, int* ids, float* weights, int tokens, int experts,
+int mlr_moe_route(const float* logits, int slices, const float* correction, int* ids, float* weights, int tokens, int experts,
                   int top, int groups, int keep, float scale, int score_kind, int normalise, hipStream_t stream) {
   MLR_REQUIRE(logits && ids && weights, "null pointer");
+  MLR_REQUIRE(slices >= 1, "logits come whole or in slices");
   MLR_REQUIRE(score_kind >= 0 && score_kind <= 2, "scores are sigmoids (0), a softmax (1) or the logits themselves (2)");
   MLR_REQUIRE(score_kind != 2 || correction == nullptr, "a softmax over the chosen logits has no correction");
   MLR_REQUIRE(tokens > 0 && experts > 0 && top > 0 && top <= experts, "sizes must be > 0 and top <= experts");
   MLR_REQUIRE(groups > 0 && experts % groups == 0 && keep > 0 && keep <= groups, "bad groups");
   MLR_REQUIRE(top <= keep * (experts / groups), "the kept groups hold fewer experts than a token uses");
   MLR_REQUIRE(experts <= 4096, "at most 4096 experts");
+  const int norm = normalise || score_kind == 2;
+  if (experts <= 4 * kWave && groups <= kWave && top <= kWave) {
+    if (experts <= kWave)
+      moe_route_lanes_kernel<1><<<tokens, kWave, 0, stream>>>(logits, slices, correction, ids, weights, tokens, experts, top, groups,
+                                                              keep, scale, score_kind, norm);
+    else
+      moe_route_lanes_kernel<4><<<tokens, kWave, 0, stream>>>(logits, slices, correction, ids, weights, tokens, experts, top, groups,
+                                                              keep, scale, score_kind, norm);
+    MLR_LAUNCH_CHECK();
+    return 0;
+  }
   const size_t lds = (2 * static_cast<size_t>(experts) + groups) * sizeof(float);
-  moe_route_kernel<<<tokens, kWave, lds, stream>>>(logits, correction, ids, weights, experts, top, groups, keep, scale,
-                                                   score_kind, normalise || score_kind == 2);
+  moe_route_kernel<<<tokens, kWave, lds, stream>>>(logits, slices, correction, ids, weights, tokens, experts, top, groups, keep,
+                                                   scale, score_kind, norm);
   MLR_LAUNCH_CHECK();
   return 0;
 }
@@ -797,11 +1001,19 @@ int mlr_moe_gemm(const void* a, const void* w, const int* sorted, const int* off
       if (status != 0) return -1;
     } else if (static_cast<int64_t>(n) * k * 2 >= (1ll << 20)) {
       // an expert's matrix of a megabyte or more: whole lines through LDS
+      static bool configured = false;
+      if (!configured) {
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(moe_gemm_stream_kernel<true>), hipFuncAttributeMaxDynamicSharedMemorySize, kStLds);
+        if (e == hipSuccess)
+          e = hipFuncSetAttribute(reinterpret_cast<const void*>(moe_gemm_stream_kernel<false>), hipFuncAttributeMaxDynamicSharedMemorySize, kStLds);
+        MLR_REQUIRE(e == hipSuccess, std::string("cannot raise the LDS limit: ") + hipGetErrorString(e));
+        configured = true;
+      }
       const dim3 stream_grid(max_tiles, (n + kStCols - 1) / kStCols);
       if (up)
-        moe_gemm_stream_kernel<true><<<stream_grid, 256, 0, stream>>>(ab, wb, sorted, offsets, tiles, pair_weights, out, tokens, top, n, k, act, rows, glu_limit, glu_alpha);
+        moe_gemm_stream_kernel<true><<<stream_grid, 256, kStLds, stream>>>(ab, wb, sorted, offsets, tiles, pair_weights, out, tokens, top, n, k, act, rows, glu_limit, glu_alpha);
       else
-        moe_gemm_stream_kernel<false><<<stream_grid, 256, 0, stream>>>(ab, wb, sorted, offsets, tiles, pair_weights, out, tokens, top, n, k, act, rows, glu_limit, glu_alpha);
+        moe_gemm_stream_kernel<false><<<stream_grid, 256, kStLds, stream>>>(ab, wb, sorted, offsets, tiles, pair_weights, out, tokens, top, n, k, act, rows, glu_limit, glu_alpha);
     } else {
       // four wavefronts (64 features) a workgroup, or two where that leaves the compute units with too
       // few workgroups to keep their loads in flight

@@ -99,7 +99,7 @@ _SIGNATURES = {
     "mlr_gemm_f32": ([_VP, _VP, _VP, _VP, _I, _I, _I, _I, _I, _VP, _VP, _F, _F, _VP], _I),
     "mlr_gemm_f32_slices": ([_I, _I, _I, _I], _I),
     "mlr_gemm_bf16": ([_VP, _VP, _VP, _I, _VP, _I, _I, _I, _I, _I, _I, _I, _VP, _I, _F, _VP, _VP, _F, _F, _VP], _I),
-    "mlr_moe_route": ([_VP, _VP, _VP, _VP, _I, _I, _I, _I, _I, _F, _I, _I, _VP], _I),
+    "mlr_moe_route": ([_VP, _I, _VP, _VP, _VP, _I, _I, _I, _I, _I, _F, _I, _I, _VP], _I),
     "mlr_moe_tile_rows": ([_I], _I),
     "mlr_moe_max_tiles": ([_I, _I, _I], _I),
     "mlr_moe_align": ([_VP, _I, _I, _I, _I, _VP, _VP, _VP, _VP], _I),
@@ -2124,14 +2124,16 @@ class HipOps:
             raise KernelError(f"router scores are one of {', '.join(kinds)}")
         if scores == "chosen_softmax" and correction is not None:
             raise KernelError("a softmax over the chosen logits has no correction")
-        self._check(logits, "router logits", torch.float32, (None, None))
-        tokens, experts = logits.shape
+        # logits [T, experts], or a stack of partial sums as `linear` may return it
+        slices = logits.shape[0] if logits.dim() == 3 else 1
+        self._check(logits, "router logits", torch.float32, (None,) * max(2, logits.dim()))
+        tokens, experts = logits.shape[-2:]
         if correction is not None:
             self._check(correction, "router correction", torch.float32, (experts,))
         ids = self._empty((tokens, top), torch.int32)
         weights = self._empty((tokens, top), torch.float32)
         self._call(
-            "mlr_moe_route", self._ptr(logits), self._ptr(correction), self._ptr(ids), self._ptr(weights), tokens,
+            "mlr_moe_route", self._ptr(logits), slices, self._ptr(correction), self._ptr(ids), self._ptr(weights), tokens,
             experts, int(top), int(groups), int(keep_groups), float(scale), kinds.index(scores), int(bool(normalise)),
             self._stream(),
         )

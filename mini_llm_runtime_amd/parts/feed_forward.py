@@ -309,7 +309,8 @@ class RoutedExperts(FeedForward):
 
     def forward(self, ctx: StepContext, h: torch.Tensor):
         ops = ctx.ops
-        logits = ops.linear(h, self.router_weight, self.router_bias, out_dtype=torch.float32)
+        # a narrow product (as many features as experts): the routing adds up partial sums over slices of k
+        logits = ops.linear(h, self.router_weight, self.router_bias, out_dtype=torch.float32, partial_sums=True)
         ids, weights = ops.route_experts(
             logits, self.correction, top=self.top, groups=self.groups, keep_groups=self.keep_groups,
             scale=self.router_scale,

@@ -1,0 +1,104 @@
+"""Routing from registers and from partial sums, and the grouped products at the edges of their tiles."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from test_gpu_kernels import _rand
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from mini_llm_runtime_amd.kernels.ops import HipOps
+
+    return HipOps(torch.bfloat16, "cuda")
+
+
+def _route(z, correction, top, groups, keep, scale, scores, normalise):
+    """The rule in 64 bits; logits that are equal stay equal, and of equal choices the lowest index wins."""
+    z = z.double()
+    s = {"sigmoid": torch.sigmoid(z), "softmax": torch.softmax(z, -1), "chosen_softmax": z}[scores]
+    c = s if correction is None else s + correction.double()
+    if keep < groups:
+        blocks = c.view(len(z), groups, -1)
+        best = blocks.topk(min(2, blocks.shape[-1]), dim=-1).values.sum(-1)
+        kept = torch.sort(best, dim=-1, descending=True, stable=True).indices[:, :keep]
+        mask = torch.ones_like(best, dtype=torch.bool).scatter_(1, kept, False)
+        c = blocks.masked_fill(mask[:, :, None], float("-inf")).reshape(z.shape)
+    ids = torch.sort(c, dim=-1, descending=True, stable=True).indices[:, :top]
+    w = s.gather(1, ids)
+    if scores == "chosen_softmax":
+        w = torch.softmax(w, -1)
+    elif normalise:
+        w = w / (w.sum(-1, keepdim=True) + 1e-20)
+    return ids, w * scale
+
+
+# one lane, a full wavefront, one expert more, all four registers of a lane, the most that fit; 257 experts and 80 groups: the plain kernel
+@pytest.mark.parametrize("experts,top,groups,keep", [
+    (1, 1, 1, 1), (5, 5, 1, 1), (64, 6, 8, 3), (64, 64, 1, 1), (65, 4, 5, 2), (192, 8, 64, 7), (256, 64, 16, 9), (257, 6, 1, 1), (160, 3, 80, 5),
+])
+@pytest.mark.parametrize("scores,normalise", [("sigmoid", False), ("softmax", True), ("chosen_softmax", False)])
+@pytest.mark.parametrize("slices", [1, 2, 9])
+def test_routing(ops, experts, top, groups, keep, scores, normalise, slices):
+    tokens = 37
+    # multiples of 1/16: scores are equal or further apart than rounding; one pair of equals in every row, and those cut off at 8
+    g = torch.Generator().manual_seed(experts + top)
+    z = torch.stack([torch.randperm(experts, generator=g) for _ in range(tokens)]).float().sub(experts // 2) / 16
+    z = z.clamp(-8, 8) if scores != "chosen_softmax" else z
+    if experts > 3:
+        z[:, 3] = z[:, 0]
+    parts = torch.stack([z / 2] + [torch.zeros_like(z)] * (slices - 2) + [z / 2]) if slices > 1 else z  # exact in any order
+    want_ids, want = _route(z, None, top, groups, keep, 1.7, scores, normalise)
+    ids, w = ops.route_experts(parts.cuda(), None, top=top, groups=groups, keep_groups=keep, scale=1.7, scores=scores, normalise=normalise)
+    assert torch.equal(ids.cpu().long(), want_ids)
+    # exp, a division and sums of at most 256 terms in float32, each within a few units of 2^-24
+    assert ((w.cpu().double() - want).abs() <= (experts + 16) * 2.0**-24 * want + 1e-12).all()
+
+
+def test_routing_of_infinities_and_nan(ops):
+    inf, nan = float("inf"), float("nan")
+    z = torch.tensor([[nan, 1.0, 0.5, 2.0], [-inf, -inf, -inf, -inf], [nan] * 4, [inf, 1.0, nan, -inf]])
+    ids, w = ops.route_experts(z.cuda(), None, top=2, groups=1, keep_groups=1, scale=1.0)
+    # NaN is never chosen while there is a number; with none left the id stays in range
+    assert ids.tolist() == [[3, 1], [0, 1], [0, 0], [0, 1]]
+    assert torch.equal(w[1].cpu(), torch.zeros(2)) and w[3, 0].item() == 1.0
+
+
+# rows an expert around the tiles of 16, 64 and 128, one expert without rows; features around 64 and 128; slices of 64 and 128 k and tails
+@pytest.mark.parametrize("rows", [(1, 0, 15), (16, 17, 0), (63, 0, 65), (64, 129, 1), (127, 128, 0), (257, 3, 130)])
+@pytest.mark.parametrize("hidden,inner", [(8, 8), (72, 136), (520, 200), (1032, 264)])
+@pytest.mark.parametrize("tiles", [0, 1, 2])
+def test_grouped_products(rows, hidden, inner, tiles):
+    from mini_llm_runtime_amd.kernels.ops import HipOps
+    from mini_llm_runtime_amd.kernels.tuning import KernelTuning
+
+    never = 1 << 20
+    tuning = KernelTuning(moe_tiled_rows=1 if tiles else never, moe_wide_tiled_rows=1 if tiles == 2 else never)
+    ops = HipOps(torch.bfloat16, "cuda", tuning=tuning)
+    experts, tokens = len(rows), sum(rows)
+    h = _rand((tokens, hidden), torch.bfloat16, 81)
+    up = _rand((experts * inner, hidden), torch.bfloat16, 82, hidden**-0.5)
+    down = _rand((experts * hidden, inner), torch.bfloat16, 83, inner**-0.5)
+    chosen = torch.repeat_interleave(torch.arange(experts), torch.tensor(rows))[torch.randperm(tokens, generator=torch.Generator().manual_seed(84))]
+    ids = chosen.to(torch.int32)[:, None].contiguous()
+    weights = torch.rand((tokens, 1), generator=torch.Generator().manual_seed(85)) + 0.5
+    args = (h.cuda(), up.cuda(), down.cuda(), ids.cuda(), weights.cuda())
+    got = ops.expert_products(*args, experts=experts, activation="relu2")[0].cpu().double()
+    want, slack = torch.zeros(tokens, hidden, dtype=torch.double), torch.zeros(tokens, hidden, dtype=torch.double)
+    for e in range(experts):
+        of = (chosen == e).nonzero()[:, 0]
+        u, d = up.double()[e * inner : (e + 1) * inner], down.double()[e * hidden : (e + 1) * hidden]
+        x = h.double()[of]
+        a = (x @ u.t()).clamp(min=0) ** 2
+        # the hidden sums and their squares in float32, one rounding to bfloat16, the sums over inner in float32
+        da = 2 * (x @ u.t()).abs() * hidden * 2.0**-24 * (x.abs() @ u.abs().t()) + 2.0**-8 * a + 1e-7
+        pw = weights.double()[of]
+        want[of] = pw * (a @ d.t())
+        slack[of] = pw * (da @ d.abs().t() + (inner + 2) * 2.0**-24 * ((a + da) @ d.abs().t())) + 1e-7
+    assert ((got - want).abs() <= slack).all()
+    same = ops.expert_products(*args, experts=experts, activation="relu2")[0].cpu().double()
+    assert torch.equal(got, same)
