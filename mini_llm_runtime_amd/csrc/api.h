@@ -358,7 +358,7 @@ int mlr_moe_identity(const void* h, const int* ids, const float* weights, float*
                      int hidden, int first, hipStream_t stream);
 // The (token, choice) pairs p = token * top + choice sorted by expert: sorted [pairs], offsets
 // [experts + 1], tiles [max_tiles, 2] = (expert, first row of `sorted`) with up to
-// mlr_moe_tile_rows(big) rows each (16, or 64 with `big`), unused tiles (-1, 0).  max_tiles >=
+// mlr_moe_tile_rows(big) rows each (16, or with `big` 1 to 3 64, 128 or 256), unused tiles (-1, 0).  max_tiles >=
 // mlr_moe_max_tiles(pairs, experts, big).
 int mlr_moe_tile_rows(int big);
 int mlr_moe_max_tiles(int pairs, int experts, int big);
@@ -369,9 +369,9 @@ int mlr_moe_align(const int* ids, int pairs, int experts, int big, int max_tiles
 // none, 2 squared ReLU, 3 sigmoid, 5 the clamped gating of rows woven in pairs (n gate and up rows give n / 2
 // activations a row: out [pairs, n / 2]; n a multiple of 4; glu_limit, glu_alpha as for the products' epilogue).
 // up 0: a = the rows of the first product [pairs, k]; out float32
-// [top, tokens, n], out[choice, token] = pair_weights[p] * (a[r] w[e]^T).  mfma 1 and 2: on the matrix
-// cores (bfloat16, k % 8 == 0; 1 streams tiles of 16 rows, 2 runs tiles of 64 rows through LDS and
-// needs n % 8 == 0), 0: plain 32-bit FMA arithmetic (tiles of 16 rows).
+// [top, tokens, n], out[choice, token] = pair_weights[p] * (a[r] w[e]^T).  mfma 1 to 4: on the matrix
+// cores (bfloat16, k % 8 == 0; 1 streams tiles of 16 rows, 2 to 4 run tiles of 64, 128 and 256 rows through LDS and
+// need n % 8 == 0), 0: plain 32-bit FMA arithmetic (tiles of 16 rows).
 int mlr_moe_gemm(const void* a, const void* w, const int* sorted, const int* offsets, const int* tiles,
                  const float* pair_weights, void* out, int up, int dtype, int mfma, int max_tiles, int tokens, int top,
                  int n, int k, int act, float glu_limit, float glu_alpha, hipStream_t stream);

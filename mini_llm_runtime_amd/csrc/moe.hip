@@ -682,6 +682,19 @@ constexpr int big_lds_bytes(int rb) {
   return big_rows(rb) * kBigRowF32 > 2 * big_buffer_bytes(rb) ? big_rows(rb) * kBigRowF32 : 2 * big_buffer_bytes(rb);
 }
 
+__device__ __forceinline__ u16x4_t activated4(float (&v)[4], int act) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if (act == 2) {
+      v[i] = fmaxf(v[i], 0.f);
+      v[i] *= v[i];
+    } else if (act == 3) {
+      v[i] = 1.0f / (1.0f + __expf(-v[i]));
+    }
+  }
+  return u16x4_t{f32_to_bf16(v[0]).bits, f32_to_bf16(v[1]).bits, f32_to_bf16(v[2]).bits, f32_to_bf16(v[3]).bits};
+}
+
 template <bool UP, int RB>
 __global__ __launch_bounds__(256) void moe_gemm_tiled_kernel(const bf16* __restrict__ a, const bf16* __restrict__ w,
                                                              const int* __restrict__ sorted,
@@ -831,18 +844,7 @@ __global__ __launch_bounds__(256) void moe_gemm_tiled_kernel(const bf16* __restr
                                   : static_cast<bf16*>(out) + static_cast<int64_t>(row0 + row) * (N / 2) + (n0 + f) / 2;
           if (staged || n0 + f < N) store_clamped_glu(to, v, glu_limit, glu_alpha);
         } else {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            if (act == 2) {
-              v[i] = fmaxf(v[i], 0.f);
-              v[i] *= v[i];
-            } else if (act == 3) {
-              v[i] = 1.0f / (1.0f + __expf(-v[i]));
-            }
-          }
-          const u16x4_t packed = {f32_to_bf16(v[0]).bits, f32_to_bf16(v[1]).bits, f32_to_bf16(v[2]).bits,
-                                  f32_to_bf16(v[3]).bits};
-          *reinterpret_cast<u16x4_t*>(moe_lds + row * kBigRowBf16 + f * 2) = packed;
+          *reinterpret_cast<u16x4_t*>(moe_lds + row * kBigRowBf16 + f * 2) = activated4(v, act);
         }
       }
   }
@@ -864,29 +866,263 @@ __global__ __launch_bounds__(256) void moe_gemm_tiled_kernel(const bf16* __restr
   }
 }
 
-template <bool UP, int RB>
-static int launch_moe_tiled(const bf16* a, const bf16* w, const int* sorted, const int* offsets, const int* tiles,
-                            const float* pair_weights, void* out, int max_tiles, int tokens, int top, int n, int k,
+// Tiles of 256 rows and 256 features by eight wavefronts in two groups that take turns, one multiplying while the other reads its
+// operands: the loop of gemm_phased_kernel (its comment explains the phases and the wait counts) over gathered rows.  What differs:
+//  * quarter X0 holds the tile's rows 0 .. 127 and X1 the others, and a group takes 64 of each, so that the groups share the work of a
+//    tile that is not full; blocks of 32 rows without rows are not multiplied (187 rows: six of eight).
+//  * the first slice's weights are asked for ahead of its rows, whose places have to be looked up first.
+//  * the down product's rows are twice as wide as LDS has room for: they leave in two halves.
+// An expert with up to 256 rows has its weights read once.  The workgroup -> (tile, features) map is the kernel's above.
+// 2,000 tokens, 64 experts with 6 choices (187 rows an expert), 768 x 2,048, against the 128-row tiles: up 91.4 to 69.9 us (201 MB of
+// weights alone take 31), down 93 to 91: its twelve slices are short beside the first loads and the 512 KB of results that a compute unit's
+// two tiles leave, and with one workgroup there nothing runs meanwhile.
+constexpr int kSqRows = 256, kSqCols = 256;
+constexpr int kSqQuarter = 128 * 128;
+constexpr int kSqBuffer = 4 * kSqQuarter;  // W0, W1, X0, X1: 64 k of 128 rows each
+constexpr int kSqRowF32 = kSqCols * 4 + 16, kSqRowBf16 = kSqCols * 2 + 16;
+constexpr int kSqLds = kSqRows * kSqRowBf16;
+static_assert(kSqLds >= 2 * kSqBuffer && kSqLds >= kSqRows / 2 * kSqRowF32, "two slices, and half a tile of 32-bit results, fit");
+constexpr unsigned kNoRow = 0xfffffff0u;  // at or past the end of any input below 4 GB whose rows are whole pieces of 16 bytes
+
+template <bool UP>
+__global__ __launch_bounds__(512, 2) void moe_gemm_phased_kernel(const bf16* __restrict__ a, const bf16* __restrict__ w,
+                                                                const int* __restrict__ sorted, const int* __restrict__ offsets,
+                                                                const int* __restrict__ tiles, int max_tiles,
+                                                                const float* __restrict__ pair_weights, void* __restrict__ out,
+                                                                int tokens, int top, int N, int K, int act, int a_rows,
+                                                                float glu_limit, float glu_alpha) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char moe_lds[];
+  __shared__ int pair_of[kSqRows];
+  const int columns = (N + kSqCols - 1) / kSqCols;
+  const int local = blockIdx.x / 8, in_pair = local % (2 * columns);
+  const int tile = (local / (2 * columns) * 8 + blockIdx.x % 8) * 2 + in_pair % 2;
+  if (tile >= max_tiles) return;
+  const int expert = tiles[2 * tile];
+  if (expert < 0) return;
+  const int n0 = in_pair / 2 * kSqCols;
+  const int row0 = tiles[2 * tile + 1];
+  const int rows = min(kSqRows, offsets[expert + 1] - row0);
+  const int tid = threadIdx.x;
+  const int lane = tid % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int wm = wave / 4, wn = wave % 4;  // wavefronts w and w + 4 share a SIMD: one of each group
+  const int r32 = lane % 32, h = lane / 32;
+  const unsigned row_bytes = static_cast<unsigned>(K) * 2u;
+  const __amdgpu_buffer_rsrc_t w_buf = make_buffer(w + (static_cast<int64_t>(expert) * N + n0) * K, static_cast<unsigned>(min(kSqCols, N - n0)) * row_bytes);
+  const __amdgpu_buffer_rsrc_t x_buf = make_buffer(a, static_cast<unsigned>(a_rows) * row_bytes);
+  const int steps = (K + 63) / 64;
+  // A quarter is 16 runs of 8 rows; this wavefront brings runs `wave` and `wave` + 8.  Row r of Wj: feature r / 32 * 64 + j * 32 + r % 32.
+  const int row = 8 * wave + lane / 8;
+  const int piece = (lane % 8) ^ ((4 * (wave % 2) + lane / 16) % 8);
+  const unsigned w_off = static_cast<unsigned>(row / 32 * 64 + row % 32) * row_bytes + piece * 16u;
+  int looked_up[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int p = 0; p < 2; ++p) looked_up[i][p] = UP ? sorted[row0 + min(i * 128 + p * 64 + row, rows - 1)] : 0;
+  const int pair_of_thread = sorted[row0 + min(tid, rows - 1)];
+  auto fetch_weights = [&](int step, int j) {
+    const unsigned past = step < steps && step * 64 + piece * 8 < K ? 0u : kOutOfBuffer;
+    const unsigned off = w_off + j * 32u * row_bytes + step * 128u;
+    unsigned char* const dst = moe_lds + (step & 1) * kSqBuffer + j * kSqQuarter + wave * 1024;
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(w_buf, (__attribute__((address_space(3))) void*)(dst + p * 8192), 16,
+                                               (off + p * 128u * row_bytes) | past, 0, 0, 0);
+  };
+  fetch_weights(0, 0);
+  fetch_weights(0, 1);
+  unsigned x_off[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      const int at = i * 128 + p * 64 + row;
+      x_off[i][p] = at < rows ? static_cast<unsigned>(UP ? looked_up[i][p] / top : row0 + at) * row_bytes + piece * 16u : kNoRow;
+    }
+  if (tid < kSqRows) pair_of[tid] = tid < rows ? pair_of_thread : -1;
+  auto fetch_rows = [&](int step, int i) {
+    const bool in = step < steps && step * 64 + piece * 8 < K;
+    unsigned char* const dst = moe_lds + (step & 1) * kSqBuffer + (2 + i) * kSqQuarter + wave * 1024;
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(x_buf, (__attribute__((address_space(3))) void*)(dst + p * 8192), 16,
+                                               in && x_off[i][p] != kNoRow ? x_off[i][p] + step * 128u : kNoRow, 0, 0, 0);
+  };
+
+  f32x16_t acc[2][4];  // feature half; row half * 2 + block of 32
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[j][i][e] = 0.f;
+  // whether this group has rows in each half
+  bool any[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) any[i] = __builtin_amdgcn_readfirstlane(static_cast<int>(i * 128 + wm * 64 < rows)) != 0;
+  const int swz = (r32 / 2) % 8;
+  const int w_base = (wn * 32 + r32) * 128;
+  const int x_base = 2 * kSqQuarter + (wm * 64 + r32) * 128;
+  struct Weights {
+    bf16x8_t v[4];
+  };
+  struct Rows {
+    bf16x8_t v[4][2];
+  };
+  auto read_weights = [&](Weights& t, int buf, int j) {
+    if (!any[0]) return;
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk)
+      t.v[kk] = load_bf16x8(moe_lds + buf * kSqBuffer + j * kSqQuarter + w_base + (((kk * 2 + h) ^ swz) * 16));
+  };
+  auto read_rows = [&](Rows& t, int buf, int i) {
+    if (!any[i]) return;
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+        t.v[kk][b] = load_bf16x8(moe_lds + buf * kSqBuffer + i * kSqQuarter + x_base + b * 32 * 128 + (((kk * 2 + h) ^ swz) * 16));
+  };
+#define MLR_READ_DONE(pending)                                                                   \
+  do {                                                                                           \
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(pending) : "memory");                    \
+    __builtin_amdgcn_sched_barrier(0);                                                           \
+    __builtin_amdgcn_s_barrier();                                                                \
+    __builtin_amdgcn_sched_barrier(0);                                                           \
+  } while (0)
+  auto multiply = [&](const Weights& t, const Rows& b, int j, int i) {
+    __builtin_amdgcn_s_setprio(1);
+    if (any[i]) {
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) acc[j][i * 2 + c] = mfma_32x32x16(t.v[kk], b.v[kk][c], acc[j][i * 2 + c]);
+    }
+    __builtin_amdgcn_s_setprio(0);
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  fetch_rows(0, 0);
+  fetch_rows(0, 1);
+  fetch_rows(1, 0);
+  fetch_weights(1, 0);
+  fetch_weights(1, 1);
+  Weights wa, wb;
+  Rows xr;
+  MLR_READ_DONE(8);  // W0, W1 and X0 of the first step (X1 is the next, as in every later step)
+  read_weights(wa, 0, 0);
+  if (wave >= 4) __builtin_amdgcn_s_barrier();  // the second group stays one phase behind
+  __builtin_amdgcn_sched_barrier(0);
+  auto step_of = [&](int step, Weights& w0, Weights& w1) {
+    const int buf = step & 1;
+    fetch_rows(step + 1, 1);
+    read_rows(xr, buf, 0);
+    MLR_READ_DONE(10);
+    multiply(w0, xr, 0, 0);
+    fetch_rows(step + 2, 0);
+    read_weights(w1, buf, 1);
+    MLR_READ_DONE(10);
+    multiply(w1, xr, 1, 0);
+    fetch_weights(step + 2, 0);
+    read_rows(xr, buf, 1);
+    MLR_READ_DONE(8);
+    multiply(w1, xr, 1, 1);
+    fetch_weights(step + 2, 1);
+    read_weights(w1, buf ^ 1, 0);
+    MLR_READ_DONE(12);
+    multiply(w0, xr, 0, 1);
+  };
+  int step = 0;
+  for (; step + 1 < steps; step += 2) {
+    step_of(step, wa, wb);
+    step_of(step + 1, wb, wa);
+  }
+  if (step < steps) step_of(step, wa, wb);
+#undef MLR_READ_DONE
+  if (wave < 4) __builtin_amdgcn_s_barrier();
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing may still be on its way into LDS
+  __syncthreads();
+
+  // acc[j][i * 2 + c][e]: feature n0 + wn * 64 + j * 32 + (e / 4) * 8 + h * 4 + e % 4 of tile row i * 128 + wm * 64 + c * 32 + r32.
+  // N is a multiple of 8: four features are all inside or all outside.
+  const bool paired = UP && act == 5;
+  const bool staged = !UP || N % (paired ? 16 : 8) == 0;  // rows of results are multiples of 16 bytes
+  const int width = (paired ? N / 2 : N) * (UP ? 2 : 4);                         // bytes of a row of results
+  const int first = (paired ? n0 / 2 : n0) * (UP ? 2 : 4);                       // where this tile's part of it starts
+  const int pieces = (paired ? kSqCols / 2 : kSqCols) * (UP ? 2 : 4) / 16;       // 16, 32 or 64
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int half0 = UP ? 0 : i * 128;  // the first tile row that is in LDS
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const int at = i * 128 + wm * 64 + c * 32 + r32;
+      const int pair = pair_of[at];
+      if (pair < 0) continue;
+      const float pw = UP ? 1.f : pair_weights[pair];
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const int f = wn * 64 + j * 32 + g * 8 + h * 4;
+          float v[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = acc[j][i * 2 + c][g * 4 + e];
+          if constexpr (!UP) {
+            *reinterpret_cast<f32x4_t*>(moe_lds + (at - half0) * kSqRowF32 + f * 4) = f32x4_t{pw * v[0], pw * v[1], pw * v[2], pw * v[3]};
+          } else if (paired) {
+            bf16* const to = staged ? reinterpret_cast<bf16*>(moe_lds + at * kSqRowBf16) + f / 2
+                                    : static_cast<bf16*>(out) + static_cast<int64_t>(row0 + at) * (N / 2) + (n0 + f) / 2;
+            if (staged || n0 + f < N) store_clamped_glu(to, v, glu_limit, glu_alpha);
+          } else {
+            *reinterpret_cast<u16x4_t*>(moe_lds + at * kSqRowBf16 + f * 2) = activated4(v, act);
+          }
+        }
+    }
+    if (!staged || (UP && i == 0)) continue;
+    __syncthreads();
+    const int held = UP ? rows : min(128, rows - half0);
+    for (int p = tid; p < held * pieces; p += 512) {
+      const int at = p / pieces, byte = (p - at * pieces) * 16;
+      if (first + byte >= width) continue;
+      int64_t to = row0 + at;
+      if constexpr (!UP) {
+        const int pair = pair_of[half0 + at], token = pair / top;
+        to = static_cast<int64_t>(pair - token * top) * tokens + token;
+      }
+      *reinterpret_cast<u32x4_t*>(static_cast<unsigned char*>(out) + to * width + first + byte) =
+          *reinterpret_cast<const u32x4_t*>(moe_lds + at * (UP ? kSqRowBf16 : kSqRowF32) + byte);
+    }
+    if (!UP && i == 0) __syncthreads();  // the next half takes its place
+  }
+}
+
+using MoeTiledKernel = void (*)(const bf16*, const bf16*, const int*, const int*, const int*, int, const float*, void*, int, int, int, int,
+                                int, int, float, float);
+struct MoeTiles {
+  MoeTiledKernel kernel;
+  int threads, cols, lds;
+};
+static int launch_moe_tiled(const MoeTiles& t, bool& configured, const bf16* a, const bf16* w, const int* sorted, const int* offsets,
+                            const int* tiles, const float* pair_weights, void* out, int max_tiles, int tokens, int top, int n, int k,
                             int act, int a_rows, float glu_limit, float glu_alpha, hipStream_t stream) {
-  static bool configured = false;
   if (!configured) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(moe_gemm_tiled_kernel<UP, RB>),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, big_lds_bytes(RB));
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(t.kernel), hipFuncAttributeMaxDynamicSharedMemorySize, t.lds);
     if (e != hipSuccess) {
       set_error(std::string("mlr_moe_gemm: cannot raise the LDS limit: ") + hipGetErrorString(e));
       return -1;
     }
     configured = true;
   }
-  const int64_t groups = static_cast<int64_t>((max_tiles + 15) / 16 * 16) * ((n + kBigCols - 1) / kBigCols);
+  const int64_t groups = static_cast<int64_t>((max_tiles + 15) / 16 * 16) * ((n + t.cols - 1) / t.cols);
   if (groups >= (1ll << 31)) {
     set_error("mlr_moe_gemm: too many tiles for one launch");
     return -1;
   }
-  const unsigned grid = static_cast<unsigned>(groups);
-  moe_gemm_tiled_kernel<UP, RB><<<grid, 256, big_lds_bytes(RB), stream>>>(a, w, sorted, offsets, tiles, max_tiles, pair_weights, out,
-                                                                        tokens, top, n, k, act, a_rows, glu_limit,
-                                                                        glu_alpha);
+  hipLaunchKernelGGL(t.kernel, dim3(static_cast<unsigned>(groups)), dim3(t.threads), t.lds, stream, a, w, sorted, offsets, tiles, max_tiles,
+                     pair_weights, out, tokens, top, n, k, act, a_rows, glu_limit, glu_alpha);
   return 0;
 }
 
@@ -939,9 +1175,9 @@ int mlr_moe_identity(const void* h, const int* ids, const float* weights, float*
   return 0;
 }
 
-// Rows of one tile of the grouped products: `big` 0 the kernels for few rows an expert (16), 1 and 2
-// the tiled matrix-core kernel for many (64 and 128).
-int mlr_moe_tile_rows(int big) { return big ? big_rows(big) : kMoeRows; }
+// Rows of one tile of the grouped products: `big` 0 the kernels for few rows an expert (16), 1 to 3
+// the tiled matrix-core kernels for many (64, 128 and 256).
+int mlr_moe_tile_rows(int big) { return big == 3 ? kSqRows : (big ? big_rows(big) : kMoeRows); }
 
 // The most tiles `pairs` pairs over `experts` experts can make.
 int mlr_moe_max_tiles(int pairs, int experts, int big) {
@@ -952,7 +1188,7 @@ int mlr_moe_max_tiles(int pairs, int experts, int big) {
 int mlr_moe_align(const int* ids, int pairs, int experts, int big, int max_tiles, int* sorted, int* offsets, int* tiles,
                   hipStream_t stream) {
   MLR_REQUIRE(ids && sorted && offsets && tiles, "null pointer");
-  MLR_REQUIRE(pairs > 0 && experts > 0 && experts <= 4096 && max_tiles > 0 && big >= 0 && big <= 2, "bad sizes");
+  MLR_REQUIRE(pairs > 0 && experts > 0 && experts <= 4096 && max_tiles > 0 && big >= 0 && big <= 3, "bad sizes");
   MLR_REQUIRE(max_tiles >= mlr_moe_max_tiles(pairs, experts, big), "too few tiles for these pairs");
   moe_align_kernel<<<1, 1024, 2 * static_cast<size_t>(experts) * sizeof(int), stream>>>(
       ids, pairs, experts, mlr_moe_tile_rows(big), max_tiles, sorted, offsets, tiles);
@@ -963,8 +1199,8 @@ int mlr_moe_align(const int* ids, int pairs, int experts, int big, int max_tiles
 // One of the two grouped products (`up` 1: act = f(h w_up^T) for the sorted rows, `act` 0 none, 2
 // squared ReLU, 3 sigmoid, 5 the clamped gating over rows woven in pairs, whose rows of `act` are n / 2 wide; `up` 0: out[choice, token] = weight * (act w_down^T), float32).  a and w
 // in `dtype`; w is [experts, n, k].  `mfma` 1: the streaming matrix-core kernel (bfloat16, k % 8 == 0;
-// tiles of 16 rows), 2 and 3: the tiled one (tiles of 64 and of 128 rows, as mlr_moe_align made them
-// with `big` 1 and 2; n % 8 == 0 too); 0: plain arithmetic (tiles of 16 rows).
+// tiles of 16 rows), 2 to 4: the tiled ones (tiles of 64, 128 and 256 rows, as mlr_moe_align made them
+// with `big` 1 to 3; n % 8 == 0 too); 0: plain arithmetic (tiles of 16 rows).
 int mlr_moe_gemm(const void* a, const void* w, const int* sorted, const int* offsets, const int* tiles,
                  const float* pair_weights, void* out, int up, int dtype, int mfma, int max_tiles, int tokens, int top,
                  int n, int k, int act, float glu_limit, float glu_alpha, hipStream_t stream) {
@@ -977,7 +1213,7 @@ int mlr_moe_gemm(const void* a, const void* w, const int* sorted, const int* off
   MLR_REQUIRE((n + kMoeCols - 1) / kMoeCols <= 65535, "too many features for one launch");
   const dim3 grid(max_tiles, (n + kMoeCols - 1) / kMoeCols);
   if (mfma) {
-    MLR_REQUIRE(mfma >= 1 && mfma <= 3, "mfma must be within 0..3");
+    MLR_REQUIRE(mfma >= 1 && mfma <= 4, "mfma must be within 0..4");
     MLR_REQUIRE(dtype == kBF16 && k % 8 == 0, "the matrix-core kernels take bfloat16 and k % 8 == 0");
     MLR_REQUIRE(mfma == 1 || n % 8 == 0, "the tiled kernel needs n % 8 == 0");
     MLR_REQUIRE(reinterpret_cast<uintptr_t>(a) % 16 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0 &&
@@ -991,13 +1227,13 @@ int mlr_moe_gemm(const void* a, const void* w, const int* sorted, const int* off
     const bf16* wb = static_cast<const bf16*>(w);
     const int rows = static_cast<int>(a_rows);
     if (mfma >= 2) {
-      int status;
-      if (mfma == 2)
-        status = up ? launch_moe_tiled<true, 1>(ab, wb, sorted, offsets, tiles, pair_weights, out, max_tiles, tokens, top, n, k, act, rows, glu_limit, glu_alpha, stream)
-                    : launch_moe_tiled<false, 1>(ab, wb, sorted, offsets, tiles, pair_weights, out, max_tiles, tokens, top, n, k, act, rows, glu_limit, glu_alpha, stream);
-      else
-        status = up ? launch_moe_tiled<true, 2>(ab, wb, sorted, offsets, tiles, pair_weights, out, max_tiles, tokens, top, n, k, act, rows, glu_limit, glu_alpha, stream)
-                    : launch_moe_tiled<false, 2>(ab, wb, sorted, offsets, tiles, pair_weights, out, max_tiles, tokens, top, n, k, act, rows, glu_limit, glu_alpha, stream);
+      static const MoeTiles kinds[3][2] = {
+          {{moe_gemm_tiled_kernel<false, 1>, 256, kBigCols, big_lds_bytes(1)}, {moe_gemm_tiled_kernel<true, 1>, 256, kBigCols, big_lds_bytes(1)}},
+          {{moe_gemm_tiled_kernel<false, 2>, 256, kBigCols, big_lds_bytes(2)}, {moe_gemm_tiled_kernel<true, 2>, 256, kBigCols, big_lds_bytes(2)}},
+          {{moe_gemm_phased_kernel<false>, 512, kSqCols, kSqLds}, {moe_gemm_phased_kernel<true>, 512, kSqCols, kSqLds}}};
+      static bool configured[3][2] = {};
+      const int status = launch_moe_tiled(kinds[mfma - 2][up != 0], configured[mfma - 2][up != 0], ab, wb, sorted, offsets, tiles, pair_weights,
+                                          out, max_tiles, tokens, top, n, k, act, rows, glu_limit, glu_alpha, stream);
       if (status != 0) return -1;
     } else if (static_cast<int64_t>(n) * k * 2 >= (1ll << 20)) {
       // an expert's matrix of a megabyte or more: whole lines through LDS

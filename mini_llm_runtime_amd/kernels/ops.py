@@ -2201,6 +2201,9 @@ class HipOps:
         big = int(bool(mfma) and pairs >= self.tuning.moe_tiled_rows * experts)
         if big and pairs >= self.tuning.moe_wide_tiled_rows * experts:
             big = 2  # tiles of 128 rows
+            square_tiles = experts * (1 + (pairs // experts + 16) // 256)  # an expert near 256 rows may have a few more
+            if square_tiles * ((min(wide, hidden) + 255) // 256) >= self.tuning.moe_square_groups:
+                big = 3  # tiles of 256 rows and 256 features
         if big:
             mfma = 1 + big
         max_tiles = self.lib.mlr_moe_max_tiles(pairs, experts, big)

@@ -59,9 +59,15 @@ class KernelTuning:
     # run in tiles of 64 rows through LDS; below, in tiles of 16 rows that stream the weights.
     moe_tiled_rows: int = 32
     moe_wide_tiled_rows: int = 96  # and from this many on in tiles of 128 rows
+    # Beyond that line, tiles of 256 rows and 256 features where the narrower product has this many of them (an expert's pairs on average
+    # give its number of tiles).  Both products together, 128-row / 256-row tiles, microseconds: 64 experts of 768 x 2,048: 128 pairs
+    # an expert (192 tiles) 185 / 142, 187 191 / 159, 600 460 / 387; 128 experts of it: 96 (384) 265 / 259, 187 361 / 325; 16 experts of
+    # it: 187 (48) 65 / 85, 400 (96) 92 / 95, 600 (144) 135 / 125; 32 of 512 x 1,024: 256 (128) 58 / 66, 400 (128) 71 / 72, 600 (192)
+    # 108 / 99; 8 of 14,336 x 4,096: 187 (128) 600 / 708, 256 (256) 1,001 / 751; 32 of 5,760 x 2,880: 96 (384) 516 / 492, 320 1,019 / 917.
+    moe_square_groups: int = 140
 
     def __post_init__(self) -> None:
-        for name in ("moe_tiled_rows", "moe_wide_tiled_rows", "decode_partition", "decode_max_groups", "max_k_slices", "wide_attention_groups", "key_run_groups", "fuse_weight_bytes",
+        for name in ("moe_tiled_rows", "moe_wide_tiled_rows", "moe_square_groups", "decode_partition", "decode_max_groups", "max_k_slices", "wide_attention_groups", "key_run_groups", "fuse_weight_bytes",
                      "finish_weight_bytes", "finish_activation_bytes", "finish_min_tokens",
                      "finish_max_tokens"):
             value = getattr(self, name)

@@ -68,16 +68,18 @@ def test_routing_of_infinities_and_nan(ops):
     assert torch.equal(w[1].cpu(), torch.zeros(2)) and w[3, 0].item() == 1.0
 
 
-# rows an expert around the tiles of 16, 64 and 128, one expert without rows; features around 64 and 128; slices of 64 and 128 k and tails
-@pytest.mark.parametrize("rows", [(1, 0, 15), (16, 17, 0), (63, 0, 65), (64, 129, 1), (127, 128, 0), (257, 3, 130)])
+# rows an expert around the tiles of 16, 64, 128 and 256, one expert without rows; features around 64, 128 and 256; slices of 64 and 128 k
+# and tails, one to seventeen slices of 64
+@pytest.mark.parametrize("rows", [(1, 0, 15), (16, 17, 0), (63, 0, 65), (64, 129, 1), (127, 128, 0), (257, 3, 130), (191, 193, 256)])
 @pytest.mark.parametrize("hidden,inner", [(8, 8), (72, 136), (520, 200), (1032, 264)])
-@pytest.mark.parametrize("tiles", [0, 1, 2])
+@pytest.mark.parametrize("tiles", [0, 1, 2, 3])
 def test_grouped_products(rows, hidden, inner, tiles):
     from mini_llm_runtime_amd.kernels.ops import HipOps
     from mini_llm_runtime_amd.kernels.tuning import KernelTuning
 
     never = 1 << 20
-    tuning = KernelTuning(moe_tiled_rows=1 if tiles else never, moe_wide_tiled_rows=1 if tiles == 2 else never)
+    tuning = KernelTuning(moe_tiled_rows=1 if tiles else never, moe_wide_tiled_rows=1 if tiles > 1 else never,
+                          moe_square_groups=1 if tiles > 2 else never)
     ops = HipOps(torch.bfloat16, "cuda", tuning=tuning)
     experts, tokens = len(rows), sum(rows)
     h = _rand((tokens, hidden), torch.bfloat16, 81)
@@ -102,3 +104,27 @@ def test_grouped_products(rows, hidden, inner, tiles):
     assert ((got - want).abs() <= slack).all()
     same = ops.expert_products(*args, experts=experts, activation="relu2")[0].cpu().double()
     assert torch.equal(got, same)
+
+
+@pytest.mark.parametrize("inner", [4, 12, 72])  # 8, 24 and 144 woven rows: results of 8, 24 and 144 bytes (the second is stored directly)
+@pytest.mark.parametrize("tiles", [1, 2, 3])
+def test_gated_products_of_woven_rows(inner, tiles):
+    """The gating in the epilogue is the plain product's, whatever the tile."""
+    from mini_llm_runtime_amd.kernels.ops import HipOps
+    from mini_llm_runtime_amd.kernels.tuning import KernelTuning
+
+    never = 1 << 20
+    tuning = KernelTuning(moe_tiled_rows=1, moe_wide_tiled_rows=1 if tiles > 1 else never, moe_square_groups=1 if tiles > 2 else never)
+    experts, tokens, hidden = 3, 400, 136
+    h = _rand((tokens, hidden), torch.bfloat16, 86).cuda()
+    up = _rand((experts * 2 * inner, hidden), torch.bfloat16, 87, 0.2).cuda()
+    down = _rand((experts * hidden, inner), torch.bfloat16, 88, 0.2).cuda()
+    ids = torch.randint(0, experts, (tokens, 2), generator=torch.Generator().manual_seed(89)).to(torch.int32).cuda()
+    weights = torch.ones((tokens, 2), device="cuda")
+    kw = dict(experts=experts, activation="clamped_glu", glu=(7.0, 1.7), woven=True)
+    got = HipOps(torch.bfloat16, "cuda", tuning=tuning).expert_products(h, up, down, ids, weights, **kw).double()
+    want = HipOps(torch.bfloat16, "cuda").expert_products(h, up, down, ids, weights, kernel="fma", **kw).double()
+    # an activation may round to the neighbouring bfloat16: 2^-8 of it (and another 2^-8 where the two gatings differ), times |down|
+    act = torch.full((1,), 2.0**-7, dtype=torch.double, device="cuda")
+    bound = act * 8.0 * 7.0 * down.double().abs().sum(-1).max()
+    assert ((got - want).abs() <= bound).all() and ((got - want).norm() <= 2.0**-7 * want.norm())
