@@ -959,6 +959,151 @@ __global__ __launch_bounds__(512, 2) void gemm_phased_kernel(const bf16* __restr
     }
 }
 
+// ---- tiled, 128 x 128, two groups of wavefronts that share the slices of k ---------------------------------
+// Eight wavefronts, four to a group; either group multiplies the whole tile (a wavefront 64 x 64), one the even slices of 64 k
+// and one the odd, and they take turns as in gemm_phased_kernel: while one multiplies a slice from registers the other reads
+// its next one from LDS.  A group has two LDS buffers of its own; a slice is asked for as soon as its buffer has been
+// read, an iteration (two slices of the tile) ahead.  At the end each group hands the sums of half the features to the other.
+// Bound, like the larger tile, by the LDS reads beside the products (64 x 64 a wavefront: as many cycles of one as of the other).
+// Measured against gemm_direct's 128 x 128 tile (two workgroups of four wavefronts a unit where there are as many), weights from
+// memory, microseconds: 2,000 x 2,048 x 2,048 (256 tiles) 27.1 to 24.8, k = 4,096 49.7 to 41.8; 1,048 x 3,584 x 3,584 38.6 to 34.7;
+// 768 x 4,608 x 3,584 41 to 32; in slices 1,024 x 1,536 x 8,960 46 to 42, 160 x 5,120 x 27,648 130 to 86.  See takes_turns for where it is used.
+constexpr int kTurnSlice = 256 * 128;  // bytes: 64 k of 128 features, then of 128 tokens
+constexpr int kTurnLds = 4 * kTurnSlice;
+static_assert(kTurnLds >= 65536 + staged_tile_bytes(128, 128), "the sums that change hands, and the staged tile behind them, fit");
+
+__global__ __launch_bounds__(512, 2) void gemm_turns_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, GemmEpilogue ep,
+                                                           TileOrder order, int M, int N, int K) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  __shared__ float scales[128];
+  const int lane = threadIdx.x % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int group = wave / 4, w4 = wave % 4;  // wavefronts w and w + 4 share a SIMD: one of each group
+  const int wr = w4 / 2, wc = w4 % 2;
+  const int r32 = lane % 32, h = lane / 32;
+  int slice, mt, nt;
+  place_workgroup(order, blockIdx.x, slice, mt, nt);
+  const int n0 = nt * 128, m0 = mt * 128;
+  RowScaleLoads<1, 1> owed;
+  if (ep.row_sumsq != nullptr) row_scales_issue(ep, owed, m0, 128, M);
+  const int chunks = K / 8;
+  const int slices = order.slices;
+  const int k_slices = (K + 63) / 64;
+  const int per = (k_slices + slices - 1) / slices;
+  const int s_begin = slice * per;
+  const int steps = min(k_slices, s_begin + per) - s_begin;
+  const int x_rows = min(128, M - m0);
+  const __amdgpu_buffer_rsrc_t w_buf = make_buffer(w + static_cast<int64_t>(n0) * K, static_cast<unsigned>(min(128, N - n0)) * K * 2u);
+  const __amdgpu_buffer_rsrc_t x_buf = make_buffer(x + static_cast<int64_t>(m0) * K, static_cast<unsigned>(x_rows) * K * 2u);
+  // a slice is 32 runs of 8 rows, 16 of weights and 16 of tokens; this wavefront brings every fourth to its group
+  const int piece = (lane % 8) ^ ((4 * (w4 % 2) + lane / 16) % 8);  // 16-byte pieces in the order piece ^ (row / 2) % 8
+  const unsigned row_off = static_cast<unsigned>(8 * w4 + lane / 8) * K * 2u + piece * 16u;
+  auto fetch = [&](int it) {
+    const int s = s_begin + 2 * it + group;
+    const unsigned past = 2 * it + group < steps && piece < chunks - s * 8 ? 0u : kOutOfBuffer;
+    unsigned char* const dst = smem + (group * 2 + (it & 1)) * kTurnSlice + w4 * 1024;
+#pragma unroll
+    for (int p = 0; p < 8; ++p)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(p < 4 ? w_buf : x_buf, (__attribute__((address_space(3))) void*)(dst + p * 4096), 16,
+                                               (row_off + (p % 4) * 64u * K + s * 128u) | past, 0, 0, 0);
+  };
+  f32x16_t acc[2][2];  // features, tokens
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+  const bool idle = __builtin_amdgcn_readfirstlane(static_cast<int>(wr * 64 >= x_rows)) != 0;  // no tokens: keeps time only
+  const int swz = (r32 / 2) % 8;
+#define MLR_TURN()                        \
+  do {                                    \
+    __builtin_amdgcn_sched_barrier(0);    \
+    __builtin_amdgcn_s_barrier();         \
+    __builtin_amdgcn_sched_barrier(0);    \
+  } while (0)
+  fetch(0);
+  fetch(1);
+  asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+  MLR_TURN();
+  if (group == 1) __builtin_amdgcn_s_barrier();  // the second group stays one phase behind
+  __builtin_amdgcn_sched_barrier(0);
+  const int iterations = (steps + 1) / 2;
+  for (int it = 0; it < iterations; ++it) {
+    bf16x8_t wv[4][2], xv[4][2];
+    if (!idle) {
+      const unsigned char* const base = smem + (group * 2 + (it & 1)) * kTurnSlice;
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+          wv[kk][b] = load_bf16x8(base + (wc * 64 + b * 32 + r32) * 128 + (((kk * 2 + h) ^ swz) * 16));
+          xv[kk][b] = load_bf16x8(base + (128 + wr * 64 + b * 32 + r32) * 128 + (((kk * 2 + h) ^ swz) * 16));
+        }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the group has read its buffer once all of it is past the barrier
+    MLR_TURN();
+    fetch(it + 2);
+    if (!idle) {
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) acc[i][j] = mfma_32x32x16(wv[kk][i], xv[kk][j], acc[i][j]);
+      __builtin_amdgcn_s_setprio(0);
+    }
+    asm volatile("s_waitcnt vmcnt(8)" ::: "memory");  // all but the slice just asked for: the next one has landed
+    MLR_TURN();
+  }
+#undef MLR_TURN
+  if (group == 0) __builtin_amdgcn_s_barrier();
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing may still be on its way into LDS
+  if (ep.row_sumsq != nullptr) row_scales_finish(ep, owed, m0, 128, M, K, scales);
+  __syncthreads();
+  // group g finishes feature block g of its wavefronts
+  f32x16_t sum[1][2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const f32x16_t given = group == 0 ? acc[1][j] : acc[0][j];
+    sum[0][j] = group == 0 ? acc[0][j] : acc[1][j];
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      *reinterpret_cast<f32x4_t*>(smem + ((wave * 2 + j) * 4 + g) * 1024 + lane * 16) = f32x4_t{given[g * 4], given[g * 4 + 1], given[g * 4 + 2], given[g * 4 + 3]};
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const f32x4_t other = *reinterpret_cast<const f32x4_t*>(smem + (((wave ^ 4) * 2 + j) * 4 + g) * 1024 + lane * 16);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sum[0][j][g * 4 + e] += other[e];
+    }
+  const int feature0 = wc * 64 + group * 32, token0 = wr * 64;
+  if (stages_tile(ep, slices, N)) {
+    if (ep.swiglu == kEpSwiglu)
+      stage_tile<kEpSwiglu, 512, 128, 128>(ep, sum, smem + 65536, scales, feature0, token0, r32, h, m0, n0, M, N);
+    else if (ep.swiglu == kEpGeglu)
+      stage_tile<kEpGeglu, 512, 128, 128>(ep, sum, smem + 65536, scales, feature0, token0, r32, h, m0, n0, M, N);
+    else
+      stage_tile<kEpNone, 512, 128, 128>(ep, sum, smem + 65536, scales, feature0, token0, r32, h, m0, n0, M, N);
+    return;
+  }
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int m = m0 + token0 + j * 32 + r32;
+    const float scale = ep.row_sumsq != nullptr ? scales[token0 + j * 32 + r32] : 1.f;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const float v[4] = {sum[0][j][g * 4 + 0] * scale, sum[0][j][g * 4 + 1] * scale, sum[0][j][g * 4 + 2] * scale,
+                          sum[0][j][g * 4 + 3] * scale};
+      finish4(ep, slice, slices, m, n0 + feature0 + g * 8 + h * 4, M, N, v);
+    }
+  }
+}
+
 using DirectKernel = void (*)(const bf16*, const bf16*, GemmEpilogue, TileOrder, int, int, int);
 // `wave_rows`: rows of wavefronts in the tile (a last token tile that fills only the first is light)
 static int launch_direct(DirectKernel kernel, int tile_tokens, int tile_features, int threads, int wave_rows, int lds_bytes,
@@ -1106,11 +1251,21 @@ struct TilingCost {
 // tiles already go round (7B gate-up at 2,048 tokens 533 against 517 on weights from memory).
 constexpr TilingCost kTilingCosts[] = {{11, 64, 64, 8, 0.314f, 0.226f, 4.6f, 0.9f, 1.3f},
                                        {23, 128, 128, 2, 0.634f, 0.535f, 3.3f, 0.9f, 3.7f},
+                                       {23, 128, 128, 1, 0.424f, 0.559f, 4.943f, 0.275f, 3.f},  // where takes_turns
                                        {45, 256, 256, 1, 1.024f, 1.655f, 7.8f, 0.421f, 5.7f},
                                        {46, 256, 192, 1, 0.803f, 1.428f, 5.4f, 0.37f, 4.5f},
                                        {47, 256, 160, 1, 0.804f, 1.3f, 5.4f, 0.305f, 3.6f},
                                        {48, 256, 320, 1, 1.38f, 2.115f, 12.f, 0.289f, 1.2f}};
 constexpr int kComputeUnits = 256;
+// 128 x 128 tiles: gemm_turns where a tile has its compute unit to itself and eight steps of k or more, gemm_direct elsewhere.  650
+// products cut into up to 4 slices, gemm_turns' time over gemm_direct's: up to 256 tiles, 24 steps or more 0.81 (0.58 to 0.91), 12 to 23
+// steps 0.93, 8 to 11 0.95 to 0.98, 4 to 7 1.01; more tiles 1.13 to 1.41: two workgroups of gemm_direct on a unit fill each other's waits
+// also at the tiles' beginnings and ends.
+static bool takes_turns(int m, int n, int k, int slices) {
+  const int64_t groups = static_cast<int64_t>((m + 127) / 128) * ((n + 127) / 128) * slices;
+  const int ksteps = (k + kBK - 1) / kBK;
+  return groups <= kComputeUnits && (ksteps + slices - 1) / slices >= 8;
+}
 static float tiled_time_us(const TilingCost& c, int m, int n, int k, int slices) {
   const int64_t tiles = static_cast<int64_t>((m + c.tile_tokens - 1) / c.tile_tokens) * ((n + c.tile_features - 1) / c.tile_features);
   const int64_t groups = tiles * slices;
@@ -1137,6 +1292,7 @@ static GemmPlan plan_many_tokens(int m, int n, int k, int max_slices) {
     for (int slices = 1; slices <= min(max_slices, 4); ++slices) {
       if (slices > 1 && ksteps / slices < 3) break;  // every slice keeps a few steps (0.5B output
                                                      // projection at 128 tokens, 14 steps: whole 8.0 us, in 4 slices 5.4)
+      if (c.kernel == 23 && (c.resident == 1) != takes_turns(m, n, k, slices)) continue;
       float t = tiled_time_us(c, m, n, k, slices);
       if (slices > 1) t += (4.f * slices - 2.f) * m * n / 5.7e6f;
       if (best_time == 0.f || t < best_time) best = {c.kernel, slices}, best_time = t;
@@ -1145,7 +1301,8 @@ static GemmPlan plan_many_tokens(int m, int n, int k, int max_slices) {
 }
 
 // The kernel for a shape: 16 = gemm_skinny_split, 11 / 22 / 44 = gemm_tiled with 64 x 64,
-// 128 x 128 (four wavefronts each) and 256 x 256 (sixteen wavefronts) tiles, 23 = gemm_direct with 128 x 128,
+// 128 x 128 (four wavefronts each) and 256 x 256 (sixteen wavefronts) tiles, 23 = 128 x 128 by gemm_turns (24) or
+// gemm_direct (25) as takes_turns has it,
 // 45 = gemm_phased with 256 x 256 (eight wavefronts in two groups), 46 / 47 / 48 = gemm_direct with tiles of 256 tokens x 192 features (twelve
 // wavefronts of 64 x 64), x 160 features (ten of 128 x 32) and x 320 features (eight of 64 x 160), 14 = gemm_tiled
 // with tiles of 32 tokens x 64 features (two wavefronts): for up to 32 tokens it stages half the
@@ -1299,12 +1456,17 @@ static int gemm_bf16(const bf16* xb, const bf16* wb, const GemmEpilogue& ep, int
       return launch_direct(gemm_direct_kernel<1, 4, 1, 2, 5>, 256, 160, 640, 2, direct_lds_bytes(256, 160, 10, 64, 2), configured,
                            xb, wb, ep, m, n, k, slices, stream);
     }
-    case 23: {
+    case 23: return gemm_bf16(xb, wb, ep, m, n, k, slices, takes_turns(m, n, k, slices) ? 24 : 25, stream);
+    case 24: {  // 128 x 128, eight wavefronts in two groups that share the slices of k
+      static bool configured = false;
+      return launch_direct(gemm_turns_kernel, 128, 128, 512, 2, kTurnLds, configured, xb, wb, ep, m, n, k, slices, stream);
+    }
+    case 25: {
       static bool configured = false;
       return launch_direct(gemm_direct_kernel<1, 2, 2, 2, 2>, 128, 128, 256, 2, direct_lds_bytes(128, 128, 4, 64, 2), configured,
                            xb, wb, ep, m, n, k, slices, stream);
     }
-    default: set_error("mlr_gemm_bf16: kernel must be 0 (chosen by shape), 16, 14, 11, 22, 23, 44 to 48 or 62 to 68"); return -1;
+    default: set_error("mlr_gemm_bf16: kernel must be 0 (chosen by shape), 16, 14, 11, 22 to 25, 44 to 48 or 62 to 68"); return -1;
   }
 }
 

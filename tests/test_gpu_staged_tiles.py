@@ -19,7 +19,7 @@ def ops():
 
 # one, two, three and seven steps of k (odd and even numbers take the two register sets in another order), tails of k; tokens and
 # features around a tile, a last token tile whose second group of wavefronts has no tokens (257 .. 384)
-@pytest.mark.parametrize("kernel", [23, 45, 46, 47, 48])
+@pytest.mark.parametrize("kernel", [23, 24, 25, 45, 46, 47, 48])
 @pytest.mark.parametrize("m,n,k", [(1, 16, 8), (255, 256, 64), (257, 272, 136), (384, 528, 72), (385, 976, 200), (130, 1328, 424)])
 @pytest.mark.parametrize("epilogue", ["plain", "bias", "swiglu", "geglu"])
 def test_staged_results_are_the_stored_ones(ops, kernel, m, n, k, epilogue):
@@ -36,7 +36,7 @@ def test_staged_results_are_the_stored_ones(ops, kernel, m, n, k, epilogue):
         assert ((stored.double() - ref).abs() <= bound).all()
 
 
-@pytest.mark.parametrize("kernel", [23, 45, 46, 47, 48])
+@pytest.mark.parametrize("kernel", [23, 24, 25, 45, 46, 47, 48])
 @pytest.mark.parametrize("n", [20, 100, 268])
 def test_rows_of_other_widths_are_stored_directly(ops, kernel, n):
     """Rows that are no multiple of 16 bytes, and results that do not start at one."""
@@ -49,12 +49,13 @@ def test_rows_of_other_widths_are_stored_directly(ops, kernel, n):
     assert torch.equal(off, ops.linear(x, w, mfma_kernel=kernel))
 
 
+@pytest.mark.parametrize("kernel", [24, 25, 45])
 @pytest.mark.parametrize("slices", [2, 3, 5])
-def test_square_tiles_cut_along_k(ops, slices):
+def test_tiles_cut_along_k(ops, slices, kernel):
     """Slices of one, two and three steps (five steps of k in 2, 3 and 5)."""
     m, n, k = 300, 300, 264
     x, w = _rand((m, k), torch.bfloat16, 77).cuda(), _rand((n, k), torch.bfloat16, 78, 0.1).cuda()
-    got = ops.linear(x, w, partial_sums=True, slices=slices, mfma_kernel=45)
+    got = ops.linear(x, w, partial_sums=True, slices=slices, mfma_kernel=kernel)
     ref = x.double() @ w.double().t()
     bound = k * 2.0**-24 * (x.double().abs() @ w.double().abs().t()) + 1e-6
     assert got.shape == (slices, m, n) and ((got.double().sum(0) - ref).abs() <= bound).all()
