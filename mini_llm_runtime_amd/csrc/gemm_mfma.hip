@@ -7,13 +7,13 @@
 // which gives 8-byte stores and lets an epilogue see neighbouring features.
 //
 // Kernels:
-//  * gemm_skinny_split: up to 16 tokens (decode at small batch).  Bound by streaming
-//    w once, and a single compute unit can only keep a few dozen cache lines in
-//    flight, so the stream has to be spread over all of them: a workgroup owns 16
-//    output features and one slice of K (grid.y slices); its wavefronts split the
-//    slice between them (interleaved, so the workgroup reads contiguous spans of
-//    every weight row), keep eight 16-byte loads in flight per lane, and add their
-//    partial sums through LDS.  Activations come straight from L2.
+//  * gemm_lines: up to 16 tokens (decode at small batch).  Bound by streaming w once, and a single compute
+//    unit can only keep a few dozen cache lines in flight, so the stream has to be spread over all of
+//    them: a workgroup owns 16 to 64 output features and one slice of K (grid.y slices), and its
+//    wavefronts bring whole lines of the weight rows straight into LDS, each for itself.
+//  * gemm_skinny_split: the fused query/key/value product of 17 to 64 tokens, and small matrices at as
+//    many: 16 output features and a slice of K a workgroup, its wavefronts split the slice between them
+//    (interleaved), keep eight 16-byte loads in flight per lane, and add their partial sums through LDS.
 //  * gemm_tiled: everything else.  An output tile per workgroup (256 x 256 with
 //    sixteen wavefronts for large products, 128 x 128 or 64 x 64 with four, whichever
 //    is the largest that still keeps the compute units busy), K in
@@ -29,7 +29,7 @@
 //    [slice, M, N]; the consumer (the residual-adding norm kernel) sums them in a
 //    fixed order, so results do not depend on which slice finishes first.
 //  * Both also run the query/key/value product with bias, rotation and the cache write as
-//    their epilogue (QkvTarget): the streaming kernel for up to 64 tokens (in slabs of 16),
+//    their epilogue (QkvTarget): the streaming kernels for up to 64 tokens (in slabs of 16 beyond 16),
 //    the tiled one beyond.
 // K must be a multiple of 8 (16-byte rows); other shapes take the FMA kernel.
 //
@@ -44,8 +44,8 @@
 
 namespace mlr {
 
-// ---- skinny, up to 16 tokens: wavefronts split K ------------------------------------------
-// MT: slabs of 16 tokens a workgroup multiplies its weight rows with (1 for the plain product).
+// ---- skinny, wavefronts split K ------------------------------------------
+// MT: slabs of 16 tokens a workgroup multiplies its weight rows with.
 template <int WAVES, bool QKV, int MT>
 __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_split_kernel(const bf16* __restrict__ x,
                                                                        const bf16* __restrict__ w,
@@ -144,6 +144,153 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_split_kernel(const bf1
                  token < M, v);
     }
   }
+}
+
+// ---- up to 16 tokens, whole lines through LDS ------------------------------------------------------------
+// A workgroup owns 16 NB features and a slice of k; its four wavefronts take steps of 64 k in turn, each through LDS buffers of its own, so
+// nothing is waited for but a wavefront's own loads: eight rows' whole lines of 128 bytes an instruction, three or four steps on
+// their way.  At the end the wavefronts' sums meet in LDS.  Bound by what a compute unit takes in: reading 64 bytes of 16 rows an
+// instruction into registers, as gemm_skinny_split does, it was half of this, and every 16 features read the tokens again.
+// Against gemm_skinny_split, 8 tokens in a replayed graph, weights from memory: 0.5B gate-up (9,728 x 896) 8.1 to 6.7 us, down (896 x 4,864)
+// 5.3 in 8 slices to 4.3 in 4, 1.5B down 10.8 to 8.3, 2,048 x 2,048 5.1 to 4.3, 896 x 896 3.2 to 3.3.
+constexpr int line_buffers(int nb) { return nb % 2 == 0 ? 3 : 4; }
+constexpr int line_lds_bytes(int nb) { return 4 * line_buffers(nb) * (nb * 16 + 16) * 128; }  // 64, 72, 128 and 120 KB
+
+template <int NB, bool QKV>
+__global__ __launch_bounds__(256) void gemm_lines_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, GemmEpilogue ep,
+                                                        QkvTarget qkv, int M, int N, int K) {
+  constexpr int BUF = line_buffers(NB);
+  constexpr int kRowsInSlice = NB * 16 + 16;  // weights, then tokens
+  constexpr int kSlice = kRowsInSlice * 128;
+  constexpr int kLoads = kRowsInSlice / 8;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  __shared__ float scales[16];
+  RowScaleLoads<4, 4> owed;
+  if (ep.row_sumsq != nullptr) row_scales_issue(ep, owed, 0, M, M);
+  const int lane = threadIdx.x % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int r = lane % 16, q = lane / 16;
+  const int n0 = blockIdx.x * (NB * 16);
+  const int slices = gridDim.y;
+  const int chunks = K / 8;
+  const int k_slices = (K + 63) / 64;
+  const int per = (k_slices + slices - 1) / slices;
+  const int sb = blockIdx.y * per, se = min(k_slices, sb + per);
+  // The weight row behind row 8 * half of block `block` of 16.  Query/key/value: a block of a rotated head is 8 of its dims and the 8
+  // they are rotated with.
+  auto run_row = [&](int block, int half) {
+    const int at = blockIdx.x * NB + block;
+    int first = at * 16 + half * 8;
+    if (QKV) {
+      const int per_head = qkv.head_dim / 16, head = at / per_head;
+      if (qkv.cos != nullptr && head < qkv.heads + qkv.kv_heads)
+        first = head * qkv.head_dim + (at - head * per_head) * 8 + half * (qkv.head_dim / 2);
+    }
+    return first;
+  };
+  __amdgpu_buffer_rsrc_t w_buf[8];  // rows in one piece, or 8 at a time
+  if constexpr (QKV) {
+#pragma unroll
+    for (int p = 0; p < 8; ++p) {
+      if (p >= 2 * NB) break;
+      const bool there = n0 + p / 2 * 16 < N;  // N is a multiple of 16
+      w_buf[p] = make_buffer(w + (there ? static_cast<int64_t>(run_row(p / 2, p % 2)) * K : 0), there ? 16u * K : 0u);
+    }
+  } else {
+    w_buf[0] = make_buffer(w + static_cast<int64_t>(n0) * K, static_cast<unsigned>(min(NB * 16, N - n0)) * K * 2u);
+  }
+  const __amdgpu_buffer_rsrc_t x_buf = make_buffer(x, static_cast<unsigned>(M) * K * 2u);
+  const int piece0 = lane % 8, row = lane / 8;  // load p brings rows 8 p .. + 8; pieces in the order piece ^ (row / 2) % 8
+  auto fetch = [&](int it) {
+    const int s = sb + it * 4 + wave;
+#pragma unroll
+    for (int p = 0; p < 10; ++p) {
+      if (p >= kLoads) break;
+      const bool weights = p < NB * 2;
+      const int piece = piece0 ^ ((4 * (p % 2) + row / 2) % 8);
+      const unsigned at = static_cast<unsigned>((weights ? (QKV ? 0 : 8 * p) : 8 * (p - NB * 2)) + row) * K * 2u + s * 128u + piece * 16u;
+      const unsigned from = s < se && s * 8 + piece < chunks ? at : kOutOfBuffer;
+      auto* const to = (__attribute__((address_space(3))) void*)(smem + (wave * BUF + it % BUF) * kSlice + p * 1024);
+      if (weights)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(w_buf[QKV ? p % 8 : 0], to, 16, from, 0, 0, 2);  // non-temporal: read once a step
+      else
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(x_buf, to, 16, from, 0, 0, 0);
+    }
+  };
+  f32x4_t acc[NB];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) acc[b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < BUF; ++i) fetch(i);
+  const int iterations = (per + 3) / 4;
+  const int swz = (r / 2) % 8;
+  for (int it = 0; it < iterations; ++it) {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((BUF - 1) * kLoads) : "memory");  // the oldest slice has landed; only this wavefront reads it
+    const unsigned char* const base = smem + (wave * BUF + it % BUF) * kSlice;
+    bf16x8_t a[2][NB], b[2];
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      const int at = ((kk * 4 + q) ^ swz) * 16;
+#pragma unroll
+      for (int i = 0; i < NB; ++i) a[kk][i] = load_bf16x8(base + (i * 16 + r) * 128 + at);
+      b[kk] = load_bf16x8(base + (NB * 16 + r) * 128 + at);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    fetch(it + BUF);
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int i = 0; i < NB; ++i) acc[i] = mfma_16x16x32(a[kk][i], b[kk], acc[i]);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing may still be on its way into LDS
+  if (ep.row_sumsq != nullptr) row_scales_finish(ep, owed, 0, M, M, K, scales);
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < NB; ++i) *reinterpret_cast<f32x4_t*>(smem + ((wave * NB + i) * kWave + lane) * 16) = acc[i];
+  __syncthreads();
+  if (wave >= NB) return;
+  float v[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int ww = 0; ww < 4; ++ww) {
+    const f32x4_t part = *reinterpret_cast<const f32x4_t*>(smem + ((ww * NB + wave) * kWave + lane) * 16);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] += part[i];
+  }
+  if (ep.row_sumsq != nullptr && r < M) {
+    const float scale = scales[r];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] *= scale;
+  }
+  if constexpr (QKV) {
+    if (n0 + wave * 16 >= N) return;
+    const int per_head = qkv.head_dim / 16, block = blockIdx.x * NB + wave, head = block / per_head;
+    const bool rotated = qkv.cos != nullptr && head < qkv.heads + qkv.kv_heads;
+    // the lane holds rows 4q .. 4q + 3 of the block: four consecutive dims of one head
+    qkv_finish(ep, qkv, head, block - head * per_head, rotated, run_row(wave, q / 2) + q % 2 * 4 - head * qkv.head_dim, q, min(r, M - 1), r < M, v);
+  } else {
+    finish4(ep, blockIdx.y, slices, r, n0 + wave * 16 + q * 4, M, N, v);
+  }
+}
+template <int NB, bool QKV = false>
+static int launch_lines(const bf16* xb, const bf16* wb, const GemmEpilogue& ep, int m, int n, int k, int slices, hipStream_t stream,
+                        const QkvTarget& qkv = QkvTarget{}) {
+  constexpr int kLds = line_lds_bytes(NB);
+  static bool configured = false;
+  if (m > 16) {
+    set_error("mlr_gemm_bf16: kernels 71 to 74 take up to 16 tokens");
+    return -1;
+  }
+  if (!configured) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_lines_kernel<NB, QKV>), hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+    if (e != hipSuccess) {
+      set_error(std::string("mlr_gemm_bf16: cannot raise the LDS limit: ") + hipGetErrorString(e));
+      return -1;
+    }
+    configured = true;
+  }
+  gemm_lines_kernel<NB, QKV><<<dim3((n + NB * 16 - 1) / (NB * 16), slices), 256, kLds, stream>>>(xb, wb, ep, qkv, m, n, k);
+  return 0;
 }
 
 // ---- skinny fused query/key/value product, up to 8 tokens: 8 weight rows a workgroup ----------
@@ -1211,11 +1358,30 @@ static int tiles_64(int m, int n) { return ((n + 63) / 64) * ((m + 63) / 64); }
 // eighths of the compute units, the 16-feature streaming kernel below that.
 static bool few_tokens_tiled(int n, int slices) { return ((n + 63) / 64) * slices >= 224; }
 
-// Up to 8 tokens of the fused query/key/value product: workgroups of 8 weight rows instead of
-// 16 when that shortens the longest queue of workgroups on a compute unit (256 of them).
-static bool half_rows_fill_better(int blocks16) {
-  return (2 * blocks16 + 255) / 256 < 2 * ((blocks16 + 255) / 256);
+// Up to 16 tokens through gemm_lines: features a workgroup (16 x blocks) and, where the consumer adds up partial sums, slices of k.  A
+// product is done when the busiest compute unit has taken in its share, the tokens' rows of every workgroup included; a unit holds two
+// workgroups of 16 or 32 features or one of 48 or 64, and starts the next when one is done.  Estimates (us) that order 14 products of 8 and 16
+// tokens, 896 x 896 to 4,608 x 3,584, as they measured: 44 KB/us a unit (as for the few-token tiles below), 3 for the launch and the first
+// bytes, 1 or, with nobody beside it, 2.5 for every further round, 0.1 in the norm kernel for every slice that it adds.
+struct LinesPlan {
+  int blocks, slices;
+  float us;
+};
+static LinesPlan plan_lines(int m, int n, int k, int slices) {
+  LinesPlan best{0, slices, 0.f};
+  for (int blocks = 1; blocks <= 4; ++blocks) {
+    const int64_t groups = static_cast<int64_t>((n + blocks * 16 - 1) / (blocks * 16)) * slices;
+    const int resident = blocks <= 2 ? 2 : 1;
+    const float kb = (blocks * 16 + m) * (((k + 63) / 64 + slices - 1) / slices) * 0.128f;
+    const float us = 3.f + (groups + 255) / 256 * kb / 44.f + ((groups - 1) / (256 * resident)) * (resident == 2 ? 1.f : 2.5f) + 0.1f * slices;
+    if (best.blocks == 0 || us < best.us) best = {blocks, slices, us};
+  }
+  return best;
 }
+
+// Up to 8 tokens of the fused query/key/value product: workgroups of 8 weight rows instead of 16 while that makes one round of them; beyond,
+// gemm_lines makes one with more rows each.
+static bool half_rows_fill_better(int blocks16) { return 2 * blocks16 <= 256; }
 
 // Kernel and number of K slices for more than 64 tokens, when the consumer takes up to
 // `max_slices` partial sums: the pair with the smallest estimated time.  The estimate counts
@@ -1300,7 +1466,7 @@ static GemmPlan plan_many_tokens(int m, int n, int k, int max_slices) {
   return best;
 }
 
-// The kernel for a shape: 16 = gemm_skinny_split, 11 / 22 / 44 = gemm_tiled with 64 x 64,
+// The kernel for a shape: 16 = up to 16 tokens gemm_lines (71 to 74: 16 to 64 features), else gemm_skinny_split, 11 / 22 / 44 = gemm_tiled with 64 x 64,
 // 128 x 128 (four wavefronts each) and 256 x 256 (sixteen wavefronts) tiles, 23 = 128 x 128 by gemm_turns (24) or
 // gemm_direct (25) as takes_turns has it,
 // 45 = gemm_phased with 256 x 256 (eight wavefronts in two groups), 46 / 47 / 48 = gemm_direct with tiles of 256 tokens x 192 features (twelve
@@ -1365,7 +1531,8 @@ static int choose_few_token_tiles(int m, int n, int k, int slices) {
 }
 
 static int choose_kernel(int m, int n, int k, int slices) {
-  if (m <= 16 && !few_tokens_tiled(n, slices)) return 16;
+  // (2,048 x 4,096 in 8 slices at 8 tokens, 17 MB: 7.4 us in tiles, 6.5 here; 3,584 x 3,584, 26 MB: 8.7 and 10.4)
+  if (m <= 16 && (!few_tokens_tiled(n, slices) || static_cast<int64_t>(n) * k * 2 < (20ll << 20))) return 16;
   if (m <= 64 && small_matrix(n, k)) return 16;
   if (m <= 64) return choose_few_token_tiles(m, n, k, slices);
   const GemmPlan plan = plan_many_tokens(m, n, k, slices);
@@ -1387,11 +1554,15 @@ static int gemm_bf16(const bf16* xb, const bf16* wb, const GemmEpilogue& ep, int
         return -1;
       }
       dim3 grid((n + 15) / 16, slices);
-      if (m <= 16) gemm_skinny_split_kernel<4, false, 1><<<grid, 256, 0, stream>>>(xb, wb, ep, QkvTarget{}, m, n, k);
-      else if (m <= 32) gemm_skinny_split_kernel<4, false, 2><<<grid, 256, 0, stream>>>(xb, wb, ep, QkvTarget{}, m, n, k);
+      if (m <= 16) return gemm_bf16(xb, wb, ep, m, n, k, slices, 70 + plan_lines(m, n, k, slices).blocks, stream);
+      if (m <= 32) gemm_skinny_split_kernel<4, false, 2><<<grid, 256, 0, stream>>>(xb, wb, ep, QkvTarget{}, m, n, k);
       else gemm_skinny_split_kernel<4, false, 4><<<grid, 256, 0, stream>>>(xb, wb, ep, QkvTarget{}, m, n, k);
       return 0;
     }
+    case 71: return launch_lines<1>(xb, wb, ep, m, n, k, slices, stream);
+    case 72: return launch_lines<2>(xb, wb, ep, m, n, k, slices, stream);
+    case 73: return launch_lines<3>(xb, wb, ep, m, n, k, slices, stream);
+    case 74: return launch_lines<4>(xb, wb, ep, m, n, k, slices, stream);
     case 11: return launch_tiled<1, 1>(xb, wb, ep, m, n, k, slices, stream);
     case 14: return launch_tiled<1, 1, 1, 2>(xb, wb, ep, m, n, k, slices, stream);  // 32 tokens x 64 features, two wavefronts
     case 22: return launch_tiled<2, 2>(xb, wb, ep, m, n, k, slices, stream);
@@ -1466,7 +1637,7 @@ static int gemm_bf16(const bf16* xb, const bf16* wb, const GemmEpilogue& ep, int
       return launch_direct(gemm_direct_kernel<1, 2, 2, 2, 2>, 128, 128, 256, 2, direct_lds_bytes(128, 128, 4, 64, 2), configured,
                            xb, wb, ep, m, n, k, slices, stream);
     }
-    default: set_error("mlr_gemm_bf16: kernel must be 0 (chosen by shape), 16, 14, 11, 22 to 25, 44 to 48 or 62 to 68"); return -1;
+    default: set_error("mlr_gemm_bf16: kernel must be 0 (chosen by shape), 16, 14, 11, 22 to 25, 44 to 48, 62 to 68 or 71 to 74"); return -1;
   }
 }
 
@@ -1484,8 +1655,7 @@ int mlr_gemm_bf16_slices(int m, int n, int k, int max_slices) {
   if (m <= 16) {
     // Measured with the norm kernel that adds the slices up (its cost grows with their number):
     // a weight of 64 MB or more streams fastest through the LDS-tiled kernel cut into 8 slices;
-    // smaller ones through the 16-feature kernel, cut until the compute units are filled and at
-    // least once per 2,560 of k (up to 4 times).
+    // smaller ones through gemm_lines, as plan_lines has it.
     const int64_t bytes = static_cast<int64_t>(n) * k * 2;
     if (bytes >= (64ll << 20) && max_slices >= 8 && k >= 8 * 256 && few_tokens_tiled(n, 8)) return 8;
     // from 20 MB on, the LDS-tiled kernel cut into 4 once that fills the compute units, into 8 where
@@ -1493,10 +1663,13 @@ int mlr_gemm_bf16_slices(int m, int n, int k, int max_slices) {
     if (bytes >= (20ll << 20) && max_slices >= 8 && k >= 8 * 256 && few_tokens_tiled(n, 4) && !few_tokens_tiled(n, 2))
       return 8;
     if (bytes >= (20ll << 20) && max_slices >= 4 && k >= 4 * 256 && few_tokens_tiled(n, 4)) return 4;
-    // the 16-feature kernel: two workgroups per compute unit before the cutting stops (1.5B down at 8
-    // tokens: 384 workgroups 11.8 us, 768 workgroups 9.8 us), at most 8 slices for the norm to add up
-    const int by_fill = choose_slices((n + 15) / 16, (k / 8 + 3) / 4, min(max_slices, 8), 512);
-    return max(by_fill, min(min(4, max_slices), k / 2560));
+    // gemm_lines: at most 8 slices for the norm to add up, a step of k for each of a workgroup's wavefronts
+    LinesPlan best = plan_lines(m, n, k, 1);
+    for (int slices = 2; slices <= min(max_slices, 8) && k >= slices * 256; slices *= 2) {
+      const LinesPlan plan = plan_lines(m, n, k, slices);
+      if (plan.us < best.us) best = plan;
+    }
+    return best.slices;
   }
   // 17 to 64 tokens of a small matrix: the row-splitting kernel (see choose_kernel) cut into 4 where
   // every slice keeps a few steps of k
@@ -1601,9 +1774,17 @@ int mlr_qkv_rope_write_bf16(const void* x, const void* w, const void* bias, int 
     const dim3 grid(static_cast<unsigned>(n / 16));
     if (m <= 8 && half_rows_fill_better(static_cast<int>(n / 16)))
       gemm_skinny_qkv8_kernel<4><<<dim3(static_cast<unsigned>(n / 8)), 256, 0, stream>>>(xb, wb, ep, target, m, static_cast<int>(n), k);
-    else if (m <= 16)
-      gemm_skinny_split_kernel<4, true, 1><<<grid, 256, 0, stream>>>(xb, wb, ep, target, m, static_cast<int>(n), k);
-    else if (n * k * 2 <= (8ll << 20))
+    else if (m <= 16) {
+      const int rows = static_cast<int>(n);
+      int status = 0;
+      switch (plan_lines(m, rows, k, 1).blocks) {
+        case 1: status = launch_lines<1, true>(xb, wb, ep, m, rows, k, 1, stream, target); break;
+        case 2: status = launch_lines<2, true>(xb, wb, ep, m, rows, k, 1, stream, target); break;
+        case 3: status = launch_lines<3, true>(xb, wb, ep, m, rows, k, 1, stream, target); break;
+        default: status = launch_lines<4, true>(xb, wb, ep, m, rows, k, 1, stream, target); break;
+      }
+      if (status != 0) return -1;
+    } else if (n * k * 2 <= (8ll << 20))
       // a small matrix: a workgroup per slab of 16 tokens reads a quarter of the tokens and the weights
       // again from L2, where one workgroup for all slabs is held up by the tokens it takes in (0.5B at
       // 64 tokens 8.4 to 6.8 us, at 48 7.7 to 5.2; 1.5B at 64 12.0 to 10.1; a 10 MB matrix: 14.6 to 16.1).

@@ -590,7 +590,7 @@ class HipOps:
         of k (bias in slice 0).  Narrow products of a few tokens are cut that way so that
         all compute units stream the weight; the norm kernel adds the slices in order.
         out: a tensor of the result's shape and dtype to write it into (a stack [S, M, N] with `slices` = S > 1).
-        mfma_kernel, slices: force one of the matrix-core kernels (16, 14, 11, 22 to 25, 44 to 48, 62 to 68) and a number
+        mfma_kernel, slices: force one of the matrix-core kernels (16, 14, 11, 22 to 25, 44 to 48, 62 to 68, 71 to 74) and a number
         of k slices instead of letting the shape choose; for tests and tuning.
         """
         if kernel not in ("auto", "fma"):
