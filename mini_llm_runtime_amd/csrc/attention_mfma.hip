@@ -976,19 +976,20 @@ __global__ __launch_bounds__(256 * kKeyGroups) void attn_prefill_kernel(
 //  * Key rows in LDS: row r of 32 holds the key that makes a lane's accumulator elements 8 consecutive keys (see key_in_16),
 //    which is the operand of the second product; 16-byte pieces are stored in the order piece ^ key, as sixteen rows side by side
 //    would otherwise lie on the same banks.  Value rows need neither: 32 dims of 16 keys are 1 KB, read in one piece.
-//  * The running maximum only moves when a score exceeds it by 2^8: until then the weights are up to 2^8 instead of 1, which
-//    costs no precision (float32 sums, bfloat16's exponent), and the 64 (D = 128) accumulators are rarely rescaled.
+//  * The running maximum moves with every score that exceeds it, so the largest weight so far is 1, which bfloat16 holds as it is: a key
+//    that outweighs all others gives its value back unrounded.  (Moved only past a slack of 2^8 the loop is 1 to 5 % faster, 8,191 tokens
+//    at 28 heads of 128 499 us instead of 525, but the largest weight is rounded then: errors against 64 bits 1.03 to 1.23 times those of
+//    attn_prefill_kernel, here 0.98 to 1.02 times.)
 // KG: groups of wavefronts that take the key tiles in turn.  1: four wavefronts, 128 queries.  2: two and two, 64 queries, for
 // the head size whose few tiles are as many long chains on a part of the compute units.
 // CAP: capped scores.
 // Bound by the softmax's vector instructions beside the products (two wavefronts a SIMD overlap them in part).  Measured against
-// attn_prefill_kernel's best tiles, whole prompts, microseconds (TFLOP/s): 28 heads of 128: 1,024 tokens 35 to 28, 2,048 84 (358) to 52
-// (581), 8,191 902 (533; the wide tiles, which its rule chose, 1,098: 268 registers leave one wavefront a SIMD) to 547 (879), 16,384
-// 3,358 (573) to 2,029 (949); 14 heads of 64: 2,048 29 to 23, 8,191 263 (457) to 156 (770), 16,384 924 (521) to 556 (865).
+// attn_prefill_kernel's best tiles, whole prompts, microseconds (TFLOP/s): 28 heads of 128: 1,024 tokens 34 to 29, 2,048 83 (362) to 54
+// (557), 8,191 886 (543; the wide tiles, which its rule chose, 1,104: 268 registers leave one wavefront a SIMD) to 525 (916); 14 heads of
+// 64: 2,048 28 to 24, 4,096 76 to 58, 8,191 245 (491) to 156 (771).
 #if MLR_HEAD_DIM == 64 || MLR_HEAD_DIM == 128
 #define MLR_HAS_PROMPT 1
 constexpr int kPromptKeys = 64;
-constexpr float kPromptSlack = 8.0f;  // in base 2
 
 // The key, among 16, that LDS row w of 16 holds.
 __host__ __device__ constexpr int key_in_16(int w) { return (w / 4) % 2 * 8 + w / 8 * 4 + w % 4; }
@@ -1212,7 +1213,7 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(
 #pragma unroll
       for (int e = 0; e < 16; ++e) top = fmaxf(top, s[b][e]);
     top = max_of_halves(top) * scale2;
-    if (__any(top > m_run + kPromptSlack)) {  // always so with the first key that a query sees
+    if (__any(top > m_run)) {  // always so with the first key that a query sees
       const float m_new = fmaxf(m_run, top);
       const float alpha = m_new == -INFINITY ? 1.0f : fast_exp2(m_run - m_new);
       l_run *= alpha;

@@ -43,7 +43,7 @@ def test_edges(ops, heads, kv_heads, head_dim, block, mask, sink):
 
 @pytest.mark.parametrize("head_dim", [64, 128])
 def test_scores_that_keep_rising(ops, head_dim):
-    """Every tile of keys scores higher than all before it, by less and by more than the running maximum's slack."""
+    """Every tile of keys scores higher than all before it, by a little and by much."""
     for step in (0.5, 4.0, 40.0):
         n = 300
         q, kp, vp, table, ctx, *_ = _paged_case([(n, n)], 2, 1, head_dim, 16, torch.bfloat16, 53)
@@ -54,6 +54,25 @@ def test_scores_that_keep_rising(ops, head_dim):
         args = (q.cuda(), kp.cuda(), vp.cuda(), table.cuda(), ctx)
         got, plain = _attend(ops, *args, **kw).cpu(), _attend(ops, *args, kernel="fma", **kw).cpu()
         torch.testing.assert_close(got.double(), plain.double(), **_tol(torch.bfloat16))
+
+
+@pytest.mark.parametrize("head_dim", [64, 128])
+def test_a_key_that_outweighs_the_others(ops, head_dim):
+    """A late key outweighs the first one by 2^7 to 2^8 and all others by 2^30, and both have the same values.  The largest weight is 1,
+    which bfloat16 holds exactly, the first key's is at most 2^-7 and off by 2^-9 of that: the result is off by 2^-16, which rounds to the
+    values themselves."""
+    n, late = 192, 150
+    q, kp, vp, table, ctx, *_ = _paged_case([(n, n)], 2, 1, head_dim, 16, torch.bfloat16, 55)
+    values = _rand((head_dim,), torch.bfloat16, 56)
+    kp[table[0].long()] = -40.0 / head_dim
+    for p in (0, late):
+        kp[table[0, p // 16], :, p % 16] = 0.0 if p == 0 else 8.0 / head_dim
+        vp[table[0, p // 16], :, :, p % 16] = values
+    # scores in powers of two (scale ln 2): 8 times the query's factor, between 7 and 8
+    q[:, : 2 * head_dim] = (1.0 - torch.arange(n) % 32 / 256.0).bfloat16()[:, None]
+    kw = dict(num_heads=2, num_kv_heads=1, head_dim=head_dim, block_size=16, scale=0.6931471805599453, window=None)
+    got = _attend(ops, q.cuda(), kp.cuda(), vp.cuda(), table.cuda(), ctx, **kw).cpu()
+    assert torch.equal(got[late:].view(n - late, 2, head_dim), values.expand(n - late, 2, head_dim))
 
 
 def test_a_page_that_is_not_there(ops):
