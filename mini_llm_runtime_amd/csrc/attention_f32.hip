@@ -33,6 +33,64 @@ constexpr int kVLd = kTileK + 8;
 constexpr int kPieces = kTileK * D / 4 / 256;  // 16-byte pieces of a thread, of the key and of the value tile
 static_assert(kTileK * D / 4 % 256 == 0, "whole pieces for every thread");
 
+// One token's attention by a wavefront, as paged_attention_simple_kernel has it: a lane scores a key and then owns dims.  For the few workgroups
+// that meet values which are not finite (see sm_odd).
+__device__ void attend_alone(const float* __restrict__ q, int64_t q_stride, const float* __restrict__ key_pages,
+                             const float* __restrict__ value_pages, const int* __restrict__ table, int table_width, int t, int p, int head,
+                             int heads, int kvh, int kv_heads, int block_size, int num_pages, float scale, int window, int chunk,
+                             const float* __restrict__ sinks, float* __restrict__ out) {
+  constexpr int kOwn = (D + kWave - 1) / kWave;  // dims of a lane
+  const int lane = threadIdx.x % kWave;
+  const float* qrow = q + t * q_stride + static_cast<int64_t>(head) * D;
+  float m = -INFINITY, l = 0.f, acc[kOwn];
+#pragma unroll
+  for (int j = 0; j < kOwn; ++j) acc[j] = 0.f;
+  bool gone = false;
+  for (int k0 = first_visible_key(p, window, chunk); k0 <= p; k0 += kWave) {
+    const int key = k0 + lane;
+    int place = -1;  // the key's page
+    float s = -INFINITY;
+    if (key <= p) {
+      const int page = key / block_size < table_width ? table[key / block_size] : -1;
+      if (static_cast<unsigned>(page) < static_cast<unsigned>(num_pages)) {
+        place = page;
+        const float* row = key_pages + ((static_cast<int64_t>(page) * kv_heads + kvh) * block_size + key % block_size) * D;
+        s = 0.f;
+        for (int i = 0; i < D; ++i) s = fmaf(qrow[i] * scale, row[i], s);
+      } else {
+        gone = true;
+      }
+    }
+    const float m_new = fmaxf(m, wave_max(s));
+    const float weight = place >= 0 ? expf(s - m_new) : 0.f;
+    const float alpha = m == -INFINITY ? 0.f : expf(m - m_new);
+    l = l * alpha + wave_sum(weight);
+    m = m_new;
+#pragma unroll
+    for (int j = 0; j < kOwn; ++j) acc[j] *= alpha;
+    for (int i = 0; i < min(kWave, p - k0 + 1); ++i) {
+      const int page = __shfl(place, i, kWave);
+      const float w = __shfl(weight, i, kWave);
+      if (page < 0) continue;
+      const float* column = value_pages + (static_cast<int64_t>(page) * kv_heads + kvh) * D * block_size + (k0 + i) % block_size;
+#pragma unroll
+      for (int j = 0; j < kOwn; ++j)
+        if (lane + j * kWave < D) acc[j] = fmaf(w, column[static_cast<int64_t>(lane + j * kWave) * block_size], acc[j]);
+    }
+  }
+  float keep = 1.0f;
+  if (sinks != nullptr) {
+    const float m_new = fmaxf(m, sinks[head]);
+    keep = m == -INFINITY ? 0.f : expf(m - m_new);
+    l = l * keep + expf(sinks[head] - m_new);
+  }
+  const float inv = __any(gone) ? __builtin_nanf("") : keep / l;
+  float* orow = out + (static_cast<int64_t>(t) * heads + head) * D;
+#pragma unroll
+  for (int j = 0; j < kOwn; ++j)
+    if (lane + j * kWave < D) orow[lane + j * kWave] = acc[j] * inv;
+}
+
 __global__ __launch_bounds__(256) void attn_prefill_f32_kernel(
     const float* __restrict__ q, int64_t q_stride, const float* __restrict__ key_pages, const float* __restrict__ value_pages,
     const int* __restrict__ block_table, int table_width, const int* __restrict__ tiles, const int* __restrict__ cu_q,
@@ -41,6 +99,7 @@ __global__ __launch_bounds__(256) void attn_prefill_f32_kernel(
   __shared__ __attribute__((aligned(16))) float ks[kTileK * kKLd];
   __shared__ __attribute__((aligned(16))) float vs[D * kVLd];
   __shared__ int sm_bad;
+  __shared__ int sm_odd;  // a value that is not finite has come in a tile of keys that some query here does not see whole
   const int tile = blockIdx.x / heads;
   const int head = blockIdx.x - tile * heads;
   const int kvh = head / (heads / kv_heads);
@@ -54,7 +113,7 @@ __global__ __launch_bounds__(256) void attn_prefill_f32_kernel(
   const int q_len = cu_q[entry + 1] - t_first;
   const int pos0 = context_lens[entry] - q_len;
   const int* table = block_table + static_cast<int64_t>(entry) * table_width;
-  if (tid == 0) sm_bad = 0;
+  if (tid == 0) sm_bad = sm_odd = 0;
 
   const int qi = q0 + wave * 16 + col;
   const bool q_ok = qi < q_len;
@@ -121,12 +180,30 @@ __global__ __launch_bounds__(256) void attn_prefill_f32_kernel(
 #pragma unroll
   for (int dt = 0; dt < kDimTiles; ++dt) acc[dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
+  auto all_finite = [&]() {  // of the values that this thread brought
+    float zero = 0.f;
+#pragma unroll
+    for (int i = 0; i < kPieces; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) zero = fmaf(v_flight[i][e], 0.f, zero);
+    return zero == 0.f;
+  };
+
   const int k_begin = k_first / kTileK * kTileK;
+  const int k_all_first = first_visible_key(pos0 + q0 + kTileQ - 1, window, chunk);  // from here on no query here is past its window
+  bool odd = false;
   fetch(k_begin);
   for (int kt0 = k_begin; kt0 < k_end; kt0 += kTileK) {
     __syncthreads();  // everybody has done with the tile before
     stash();
+    // A hidden key's weight is 0, but 0 times an infinity or NaN is NaN, and the products would hand it to queries that do not see the key.
+    const bool all_seen = kt0 + kTileK - 1 <= pos0 + q0 && kt0 >= k_all_first;
+    if (!all_seen && !all_finite()) sm_odd = 1;
     __syncthreads();
+    if (!all_seen && sm_odd != 0) {
+      odd = true;
+      break;
+    }
     fetch(kt0 + kTileK);  // on its way while this tile is computed
     if (!(wave_has_queries && kt0 <= w_last && kt0 + kTileK > w_first)) continue;
     f32x4_t s[kSubTiles];
@@ -180,6 +257,12 @@ __global__ __launch_bounds__(256) void attn_prefill_f32_kernel(
         for (int i = 0; i < 4; ++i) acc[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[i], s[sub][i], acc[dt], 0, 0, 0);
       }
     }
+  }
+  if (odd) {  // the same for the whole workgroup: its queries one after the other, each over the keys it sees
+    for (int u = 0; u < 16 && q0 + wave * 16 + u < q_len; ++u)
+      attend_alone(q, q_stride, key_pages, value_pages, table, table_width, t_first + q0 + wave * 16 + u, pos0 + q0 + wave * 16 + u, head,
+                   heads, kvh, kv_heads, block_size, num_pages, scale, window, chunk, sinks, out);
+    return;
   }
   if (bad) atomicOr(&sm_bad, 1);
   __syncthreads();

@@ -86,6 +86,23 @@ def test_prompt_attention(ops, heads, kv_heads, head_dim, block, mask):
         torch.testing.assert_close(_attend(ops, *args, **kw).cpu().double(), ref, atol=5e-6, rtol=1e-5)
 
 
+@pytest.mark.parametrize("head_dim,block", [(64, 16), (128, 16), (80, 8), (16, 4)])
+@pytest.mark.parametrize("mask", [dict(window=None), dict(window=20), dict(window=None, chunk=24)])
+@pytest.mark.parametrize("odd", [float("nan"), float("inf")])
+def test_values_that_are_not_finite_stay_with_the_tokens_that_see_them(ops, head_dim, block, mask, odd):
+    """0 * inf is NaN: a value that a token does not see must not enter its sum at all, as in the plain kernel."""
+    entries = [(130, 130), (190, 61)]
+    q, kp, vp, table, ctx, *_ = _paged_case(entries, 2, 1, head_dim, block, torch.float32, 17)
+    for entry, p in ((0, 70), (0, 129), (1, 131), (1, 150)):
+        vp[table[entry, p // block], 0, 3, p % block] = odd
+    vp[table[0, 10 // block], 0, :, 10 % block] = -odd
+    args = (q.cuda(), kp.cuda(), vp.cuda(), table.cuda(), ctx)
+    kw = dict(num_heads=2, num_kv_heads=1, head_dim=head_dim, block_size=block, scale=head_dim**-0.5, **mask)
+    got, plain = _attend(ops, *args, **kw).cpu(), _attend(ops, *args, kernel="fma", **kw).cpu()
+    assert torch.isfinite(plain[:10]).all() and not torch.isfinite(plain[129]).all()
+    torch.testing.assert_close(got, plain, atol=5e-6, rtol=1e-5, equal_nan=True)
+
+
 def test_prompt_attention_refuses_a_page_that_is_not_there(ops):
     q, kp, vp, table, ctx, *_ = _paged_case([(100, 100), (70, 70)], 2, 1, 64, 16, torch.float32, 16)
     table = table.clone()
