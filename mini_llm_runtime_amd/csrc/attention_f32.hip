@@ -91,6 +91,8 @@ __device__ void attend_alone(const float* __restrict__ q, int64_t q_stride, cons
     if (lane + j * kWave < D) orow[lane + j * kWave] = acc[j] * inv;
 }
 
+__device__ __attribute__((aligned(16))) const float kGoneKeys[4] = {__builtin_nanf(""), __builtin_nanf(""), __builtin_nanf(""), __builtin_nanf("")};
+
 __global__ __launch_bounds__(256) void attn_prefill_f32_kernel(
     const float* __restrict__ q, int64_t q_stride, const float* __restrict__ key_pages, const float* __restrict__ value_pages,
     const int* __restrict__ block_table, int table_width, const int* __restrict__ tiles, const int* __restrict__ cu_q,
@@ -98,7 +100,6 @@ __global__ __launch_bounds__(256) void attn_prefill_f32_kernel(
     float scale, int window, int chunk, const float* __restrict__ sinks) {
   __shared__ __attribute__((aligned(16))) float ks[kTileK * kKLd];
   __shared__ __attribute__((aligned(16))) float vs[D * kVLd];
-  __shared__ int sm_bad;
   __shared__ int sm_odd;  // a value that is not finite has come in a tile of keys that some query here does not see whole
   const int tile = blockIdx.x / heads;
   const int head = blockIdx.x - tile * heads;
@@ -113,7 +114,7 @@ __global__ __launch_bounds__(256) void attn_prefill_f32_kernel(
   const int q_len = cu_q[entry + 1] - t_first;
   const int pos0 = context_lens[entry] - q_len;
   const int* table = block_table + static_cast<int64_t>(entry) * table_width;
-  if (tid == 0) sm_bad = sm_odd = 0;
+  if (tid == 0) sm_odd = 0;
 
   const int qi = q0 + wave * 16 + col;
   const bool q_ok = qi < q_len;
@@ -136,7 +137,7 @@ __global__ __launch_bounds__(256) void attn_prefill_f32_kernel(
   const bool wave_has_queries = q0 + wave * 16 < q_len;
 
   f32x4_t k_flight[kPieces], v_flight[kPieces];
-  bool bad = false;
+  // A page that is not there (or lies past the table) brings keys that are NaN: so is the sum of every query that sees one, and of no other
   auto fetch = [&](int kt0) {
     if (kt0 >= k_end) return;
 #pragma unroll
@@ -144,19 +145,19 @@ __global__ __launch_bounds__(256) void attn_prefill_f32_kernel(
       const int c = tid + i * 256;
       const int key = kt0 + c / (D / 4), dim = c % (D / 4) * 4;
       const int logical = min(key, k_end - 1) / block_size;
-      const int page = table[logical];
-      const bool in = static_cast<unsigned>(page) < static_cast<unsigned>(num_pages);
-      if (!in) bad = bad || (key < k_end && key >= k_first);
+      const int page = table[min(logical, table_width - 1)];
+      const bool in = logical < table_width && static_cast<unsigned>(page) < static_cast<unsigned>(num_pages);
       const int64_t base = static_cast<int64_t>(in ? page : 0) * kv_heads + kvh;
-      k_flight[i] = *reinterpret_cast<const f32x4_t*>(key_pages + (base * block_size + key % block_size) * D + dim);
+      const float* piece = key_pages + (base * block_size + key % block_size) * D + dim;
+      k_flight[i] = *reinterpret_cast<const f32x4_t*>(in ? piece : kGoneKeys);  // (a choice behind the load would wait for it here)
     }
 #pragma unroll
     for (int i = 0; i < kPieces; ++i) {
       const int c = tid + i * 256;
       const int key = kt0 + c % (kTileK / 4) * 4, dim = c / (kTileK / 4);  // 4 keys: they lie in one page, whose size is a multiple of 4
       const int logical = min(key, k_end - 1) / block_size;
-      const int page = table[logical];
-      const bool in = static_cast<unsigned>(page) < static_cast<unsigned>(num_pages);
+      const int page = table[min(logical, table_width - 1)];
+      const bool in = logical < table_width && static_cast<unsigned>(page) < static_cast<unsigned>(num_pages);
       const int64_t base = static_cast<int64_t>(in ? page : 0) * kv_heads + kvh;
       f32x4_t v = *reinterpret_cast<const f32x4_t*>(value_pages + (base * D + dim) * block_size + key % block_size);
       // values that no query here may see are cleared: what a page holds there may be anything, and 0 * NaN would come through
@@ -264,8 +265,6 @@ __global__ __launch_bounds__(256) void attn_prefill_f32_kernel(
                    heads, kvh, kv_heads, block_size, num_pages, scale, window, chunk, sinks, out);
     return;
   }
-  if (bad) atomicOr(&sm_bad, 1);
-  __syncthreads();
   float l = l_run;
   l += __shfl_xor(l, 16, kWave);
   l += __shfl_xor(l, 32, kWave);
@@ -277,7 +276,7 @@ __global__ __launch_bounds__(256) void attn_prefill_f32_kernel(
     l = l * keep + expf(sink - m_new);
   }
   if (!q_ok) return;
-  const float inv = sm_bad != 0 ? __builtin_nanf("") : keep / l;
+  const float inv = keep / l;
   float* orow = out + (static_cast<int64_t>(t_first + qi) * heads + head) * D;
 #pragma unroll
   for (int dt = 0; dt < kDimTiles; ++dt) {
@@ -294,7 +293,7 @@ __global__ __launch_bounds__(256) void attn_prefill_f32_kernel(
 using namespace mlr;
 
 // Attention of the query tiles in `tiles` ([num_tiles][2]: entry, first query; 64 queries per tile) in float32, with the arguments
-// of mlr_attention_prefill.  A page id out of range among the keys that a tile sees makes the tile's rows NaN.
+// of mlr_attention_prefill.  A page id out of range makes the rows of the tokens that see its keys NaN, as in the plain kernel.
 extern "C" int mlr_attention_prefill_f32(const float* q, int64_t q_stride, const float* key_pages, const float* value_pages,
                                          const int* block_table, int table_width, const int* tiles, int num_tiles, const int* cu_q,
                                          const int* context_lens, float* out, int heads, int kv_heads, int block_size, int num_pages,

@@ -110,3 +110,17 @@ def test_prompt_attention_refuses_a_page_that_is_not_there(ops):
     kw = dict(num_heads=2, num_kv_heads=1, head_dim=64, block_size=16, scale=0.125, window=None)
     got = _attend(ops, q.cuda(), kp.cuda(), vp.cuda(), table.cuda(), ctx, **kw).cpu()
     assert torch.isfinite(got[:100]).all() and torch.isnan(got[100 + 64 :]).all()
+
+
+@pytest.mark.parametrize("mask", [dict(window=None), dict(window=20), dict(window=None, chunk=24)])
+@pytest.mark.parametrize("page", [-1, 10**6])
+def test_a_page_that_is_not_there_concerns_the_tokens_that_see_it(ops, mask, page):
+    """Those rows and no others are NaN, as in the plain kernel."""
+    q, kp, vp, table, ctx, *_ = _paged_case([(100, 100), (190, 70)], 2, 1, 64, 16, torch.float32, 16)
+    table = table.clone()
+    table[0, 2] = table[1, 8] = page  # positions 32..47 of the first request, 128..143 of the second
+    args = (q.cuda(), kp.cuda(), vp.cuda(), table.cuda(), ctx)
+    kw = dict(num_heads=2, num_kv_heads=1, head_dim=64, block_size=16, scale=0.125, **mask)
+    got, plain = _attend(ops, *args, **kw).cpu(), _attend(ops, *args, kernel="fma", **kw).cpu()
+    assert torch.isfinite(plain[:32]).all() and torch.isnan(plain[40]).all() and torch.isfinite(plain[100:108]).all()
+    torch.testing.assert_close(got, plain, atol=5e-6, rtol=1e-5, equal_nan=True)
