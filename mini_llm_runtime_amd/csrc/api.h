@@ -90,7 +90,8 @@ int mlr_gemm_f32(const float* x, const float* w, const float* bias, float* y, in
 // The same product in bfloat16 on the matrix cores (float32 accumulation).  Needs
 // k % 8 == 0 and 16-byte aligned x and w; any m and n.  With slices > 1 (a value
 // mlr_gemm_bf16_slices returned for this shape) y is float32 [slices, m, n]: partial
-// sums over slices of k, the bias in slice 0, for the consumer to add up in order.
+// sums over slices of k, the bias in slice 0, for the consumer to add up in order.  (The number is that for float32
+// sums: a consumer of slices takes one slice in float32, too.)
 int mlr_gemm_bf16_slices(int m, int n, int k, int max_slices);
 // The kernel mlr_gemm_bf16 chooses for a shape cut into `slices` (its `kernel` argument's numbers).
 int mlr_gemm_bf16_kernel(int m, int n, int k, int slices);

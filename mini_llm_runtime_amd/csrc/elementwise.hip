@@ -37,7 +37,10 @@ __global__ __launch_bounds__(256) void embedding_kernel(const T* __restrict__ ta
 // between the statistics and the scaling (hidden must be a multiple of 4).  Few wide rows
 // (a decode step of a large model) take 1,024 threads each: a compute unit takes in what its
 // wavefronts keep in flight, and a row with eight slices of partial sums is 100 KB and more.
-template <typename T, typename TW, int VPT, int THREADS = 256>
+// BATCH: slices that are asked for together.  A product of many tokens comes in one to four: asking for eight all the same reads the last
+// of them again and holds registers of which other rows' wavefronts could make use (8,191 rows of 3,584, one slice: 94 to 64 us, two
+// 107 to 87; a delta in bfloat16 54).
+template <typename T, typename TW, int VPT, int THREADS = 256, int BATCH = 8>
 __global__ __launch_bounds__(THREADS) void rmsnorm_kernel(float* __restrict__ x, const T* __restrict__ delta,
                                                       const float* __restrict__ partial, int slices, int rows,
                                                       const TW* __restrict__ weight, T* __restrict__ out,
@@ -48,7 +51,6 @@ __global__ __launch_bounds__(THREADS) void rmsnorm_kernel(float* __restrict__ x,
   // Loads first, all of them unconditional (an index past the end is clamped and its value
   // dropped), so that they are in flight together: a wait per slice would cost more than the
   // whole kernel otherwise.
-  constexpr int kSliceBatch = 8;
   f32x4 v[VPT];
 #pragma unroll
   for (int j = 0; j < VPT; ++j) {
@@ -60,19 +62,19 @@ __global__ __launch_bounds__(THREADS) void rmsnorm_kernel(float* __restrict__ x,
       for (int e = 0; e < 4; ++e) v[j][e] += to_f32(delta[at + e]);
     }
   }
-  for (int s0 = 0; s0 < slices; s0 += kSliceBatch) {
-    f32x4 p[VPT][kSliceBatch];
+  for (int s0 = 0; s0 < slices; s0 += BATCH) {
+    f32x4 p[VPT][BATCH];
 #pragma unroll
     for (int j = 0; j < VPT; ++j) {
       const int i = min(threadIdx.x + j * THREADS, quads - 1);
 #pragma unroll
-      for (int u = 0; u < kSliceBatch; ++u) {
+      for (int u = 0; u < BATCH; ++u) {
         const int sl = min(s0 + u, slices - 1);
         p[j][u] = *reinterpret_cast<const f32x4*>(partial + (static_cast<int64_t>(sl) * rows + row) * hidden + 4 * i);
       }
     }
 #pragma unroll
-    for (int u = 0; u < kSliceBatch; ++u) {
+    for (int u = 0; u < BATCH; ++u) {
       const bool live = s0 + u < slices;
 #pragma unroll
       for (int j = 0; j < VPT; ++j)
@@ -130,6 +132,20 @@ __global__ __launch_bounds__(256) void rmsnorm_any_kernel(float* __restrict__ x,
     orow[i] = from_f32<T>(to_f32(weight[i]) * (xr[i] * inv));
 }
 
+template <typename T, typename TW, int BATCH>
+static void launch_rmsnorm_rows(float* x, const T* d, const float* partial, int slices, const TW* w, T* o, int rows, int hidden, float eps,
+                                hipStream_t stream) {
+  const int quads = hidden / 4;
+  if (quads <= 256)
+    rmsnorm_kernel<T, TW, 1, 256, BATCH><<<rows, 256, 0, stream>>>(x, d, partial, slices, rows, w, o, hidden, eps);
+  else if (quads <= 512)
+    rmsnorm_kernel<T, TW, 2, 256, BATCH><<<rows, 256, 0, stream>>>(x, d, partial, slices, rows, w, o, hidden, eps);
+  else if (quads <= 1024)
+    rmsnorm_kernel<T, TW, 4, 256, BATCH><<<rows, 256, 0, stream>>>(x, d, partial, slices, rows, w, o, hidden, eps);
+  else
+    rmsnorm_kernel<T, TW, 8, 256, BATCH><<<rows, 256, 0, stream>>>(x, d, partial, slices, rows, w, o, hidden, eps);
+}
+
 template <typename T, typename TW>
 static void launch_rmsnorm(float* x, const void* delta, const float* partial, int slices, const void* weight,
                            void* out, int rows, int hidden, float eps, hipStream_t stream) {
@@ -143,14 +159,14 @@ static void launch_rmsnorm(float* x, const void* delta, const float* partial, in
     rmsnorm_kernel<T, TW, 1, 1024><<<rows, 1024, 0, stream>>>(x, d, partial, slices, rows, w, o, hidden, eps);
   else if (rows <= 64 && quads > 1024)
     rmsnorm_kernel<T, TW, 2, 1024><<<rows, 1024, 0, stream>>>(x, d, partial, slices, rows, w, o, hidden, eps);
-  else if (quads <= 256)
-    rmsnorm_kernel<T, TW, 1><<<rows, 256, 0, stream>>>(x, d, partial, slices, rows, w, o, hidden, eps);
-  else if (quads <= 512)
-    rmsnorm_kernel<T, TW, 2><<<rows, 256, 0, stream>>>(x, d, partial, slices, rows, w, o, hidden, eps);
-  else if (quads <= 1024)
-    rmsnorm_kernel<T, TW, 4><<<rows, 256, 0, stream>>>(x, d, partial, slices, rows, w, o, hidden, eps);
+  else if (rows > 64 && slices == 1)
+    launch_rmsnorm_rows<T, TW, 1>(x, d, partial, slices, w, o, rows, hidden, eps, stream);
+  else if (rows > 64 && slices == 2)
+    launch_rmsnorm_rows<T, TW, 2>(x, d, partial, slices, w, o, rows, hidden, eps, stream);
+  else if (rows > 64 && slices > 2 && slices <= 4)
+    launch_rmsnorm_rows<T, TW, 4>(x, d, partial, slices, w, o, rows, hidden, eps, stream);
   else
-    rmsnorm_kernel<T, TW, 8><<<rows, 256, 0, stream>>>(x, d, partial, slices, rows, w, o, hidden, eps);
+    launch_rmsnorm_rows<T, TW, 8>(x, d, partial, slices, w, o, rows, hidden, eps, stream);
 }
 
 template <typename T>

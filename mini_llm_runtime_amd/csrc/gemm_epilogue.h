@@ -292,6 +292,60 @@ __device__ __forceinline__ void stage_tile(const GemmEpilogue& ep, const f32x16_
   }
 }
 
+// The same for float32 sums, whole or of a slice of k (the bias in slice 0), which leave ROWS tokens of the tile at a time: a row is twice as
+// wide.  Straight from the accumulators a store fills 32 bytes of 32 rows.
+__host__ __device__ inline bool stages_sums(const GemmEpilogue& ep, int N) {
+  return ep.out_is_f32 && ep.multiply == nullptr && ep.swiglu == kEpNone && N % 4 == 0 && reinterpret_cast<uintptr_t>(ep.y) % 16 == 0;
+}
+constexpr int staged_sums_bytes(int tokens, int features) { return tokens * (features * 4 + 16); }
+// The most tokens of a tile whose sums fit `lds` bytes, in whole wavefronts of `wave_tokens`; 0: not even one.
+constexpr int staged_sums_rows(int tokens, int features, int wave_tokens, int lds) {
+  for (int rows = tokens; rows >= wave_tokens; rows /= 2)
+    if (rows % wave_tokens == 0 && staged_sums_bytes(rows, features) <= lds) return rows;
+  return 0;
+}
+
+template <int THREADS, int BM, int BN, int ROWS, int NI, int NJ>
+__device__ __forceinline__ void stage_sums(const GemmEpilogue& ep, const f32x16_t (&acc)[NI][NJ], unsigned char* lds, const float* scales,
+                                           int feature0, int token0, int r32, int h, int slice, int m0, int n0, int M, int N) {
+  constexpr int kRow = BN * 4 + 16;
+  constexpr int kRowPieces = BN / 4;
+  float* const y = static_cast<float*>(ep.y) + static_cast<int64_t>(slice) * M * N;
+#pragma unroll
+  for (int first = 0; first < BM; first += ROWS) {
+    if (first > 0) __syncthreads();  // the rows before have left
+    if (token0 / ROWS * ROWS == first) {
+#pragma unroll
+      for (int i = 0; i < NI; ++i)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const int f = feature0 + i * 32 + g * 8 + h * 4;
+          float b[4] = {0.f, 0.f, 0.f, 0.f};
+          if (ep.bias != nullptr && slice == 0 && n0 + f < N) {  // n0 + f + 3 < N too: both are multiples of 4
+#pragma unroll
+            for (int e = 0; e < 4; ++e) b[e] = load_as_f32(ep.bias, n0 + f + e, ep.bias_is_f32);
+          }
+#pragma unroll
+          for (int j = 0; j < NJ; ++j) {
+            const int token = token0 + j * 32 + r32;
+            const float scale = ep.row_sumsq != nullptr ? scales[token] : 1.f;
+            f32x4_t v;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = acc[i][j][g * 4 + e] * scale + b[e];
+            *reinterpret_cast<f32x4_t*>(lds + (token - first) * kRow + f * 4) = v;
+          }
+        }
+    }
+    __syncthreads();
+#pragma unroll 4
+    for (int p = threadIdx.x; p < ROWS * kRowPieces; p += THREADS) {
+      const int row = p / kRowPieces, col = p - row * kRowPieces;
+      const int m = m0 + first + row, n = n0 + col * 4;
+      if (m < M && n < N) *reinterpret_cast<u32x4_t*>(y + static_cast<int64_t>(m) * N + n) = *reinterpret_cast<const u32x4_t*>(lds + row * kRow + col * 16);
+    }
+  }
+}
+
 // Store one accumulator tile (4 consecutive features of one token per lane): the
 // final result, or this K slice's partial sums.
 template <bool ACTIVATIONS = true>

@@ -878,6 +878,14 @@ __global__ __launch_bounds__(64 * GM * GN) void gemm_direct_kernel(const bf16* _
   constexpr int kLds = NBUF * kBufferBytes;
   constexpr bool kStagesPairs = BM >= 128 && staged_tile_bytes(BM, BN / 2) <= kLds;
   constexpr bool kStagesPlain = BM >= 128 && FIXED < 0 && staged_tile_bytes(BM, BN) <= kLds;
+  constexpr int kSumRows = BM >= 128 && FIXED < 0 && WM * WN < 10 ? staged_sums_rows(BM, BN, 32 * WM, kLds) : 0;
+  if constexpr (kSumRows > 0) {
+    if (stages_sums(ep, N)) {
+      __syncthreads();  // as below
+      stage_sums<64 * GM * GN, BM, BN, kSumRows>(ep, acc, smem, scales, wn * 32 * WN, wm * 32 * WM, r32, h, slice, m0, n0, M, N);
+      return;
+    }
+  }
   if constexpr (kStagesPairs) {
     if (stages_tile(ep, slices, N) && (kStagesPlain || ep.swiglu != kEpNone)) {
       __syncthreads();  // everybody's loads have landed and nobody reads the slices any more
@@ -1090,6 +1098,10 @@ __global__ __launch_bounds__(512, 2) void gemm_phased_kernel(const bf16* __restr
       stage_tile<kEpNone, 512, 256, 256>(ep, acc, smem, scales, wn * 64, wm * 128, r32, h, m0, n0, M, N);
     return;
   }
+  if (stages_sums(ep, N)) {
+    stage_sums<512, 256, 256, staged_sums_rows(256, 256, 128, kPhaseLds)>(ep, acc, smem, scales, wn * 64, wm * 128, r32, h, slice, m0, n0, M, N);
+    return;
+  }
 #pragma unroll
   for (int j = 0; j < 2; ++j)
 #pragma unroll
@@ -1236,6 +1248,10 @@ __global__ __launch_bounds__(512, 2) void gemm_turns_kernel(const bf16* __restri
       stage_tile<kEpGeglu, 512, 128, 128>(ep, sum, smem + 65536, scales, feature0, token0, r32, h, m0, n0, M, N);
     else
       stage_tile<kEpNone, 512, 128, 128>(ep, sum, smem + 65536, scales, feature0, token0, r32, h, m0, n0, M, N);
+    return;
+  }
+  if (stages_sums(ep, N)) {
+    stage_sums<512, 128, 128, staged_sums_rows(128, 128, 64, kTurnLds - 65536)>(ep, sum, smem + 65536, scales, feature0, token0, r32, h, slice, m0, n0, M, N);
     return;
   }
 #pragma unroll
@@ -1390,18 +1406,21 @@ static bool half_rows_fill_better(int blocks16) { return 2 * blocks16 <= 256; }
 // or `busy` us times the workgroups resident beside each other (operand fetch and matrix cores
 // do not overlap within a compute unit, so co-resident workgroups queue); steps are faster, by up to the share
 // `eased`, while only a part of the compute units has work (less traffic into L2, a higher clock).
-// Slices of k cost their kernel `cut` us more a tile (float32 sums, stored without staging) and their consumer, a norm that streams at
-// 5.7 TB/s, 4 bytes per slice and element instead of 2.  Constants fitted to 3,800 measured times of the
+// Sums in float32, of slices of k or whole, cost their kernel `wide` us more a tile (twice the bytes, which leave in turns) and their
+// consumer, a norm that streams at 5.7 TB/s, 4 bytes per slice and element instead of 2.  A consumer that takes several slices gets
+// float32 from one, too: how many there are is a matter of speed and must not decide what the sums are rounded to before they are
+// added to the residual stream.  Constants fitted to 3,800 measured times of the
 // four products of a layer at five model sizes (hidden 896 to 5120) and 96 to 8,191 tokens, with weights that
 // rotate through more memory than the caches hold: rms error of the estimate 7 to 11 %, the chosen pair within
 // 1.1 % of the best one on average (3.0 % with the constants of the kernels before, whose tiles were stored
-// straight from the accumulators and whose square tile had sixteen wavefronts in step).
+// straight from the accumulators and whose square tile had sixteen wavefronts in step).  For float32 sums with their norm, 158 products of
+// six model sizes: the chosen pair within 0.4 % of the best on average, 14 % at worst (5,120 x 5,120 at 1,048 tokens).
 struct GemmPlan {
   int kernel, slices;
 };
 struct TilingCost {
   int kernel, tile_tokens, tile_features, resident;
-  float alone, busy, fixed, eased, cut;
+  float alone, busy, fixed, eased, wide;
 };
 // The narrower tiles of 256 tokens (gemm_direct; a step of k costs 7.2 ns per feature of the tile at 256
 // features, 7.6 at 192, 8.4 at 160) are there for products whose 256 x 256 tiles leave compute units
@@ -1432,7 +1451,7 @@ static bool takes_turns(int m, int n, int k, int slices) {
   const int ksteps = (k + kBK - 1) / kBK;
   return groups <= kComputeUnits && (ksteps + slices - 1) / slices >= 8;
 }
-static float tiled_time_us(const TilingCost& c, int m, int n, int k, int slices) {
+static float tiled_time_us(const TilingCost& c, int m, int n, int k, int slices, bool sums) {
   const int64_t tiles = static_cast<int64_t>((m + c.tile_tokens - 1) / c.tile_tokens) * ((n + c.tile_features - 1) / c.tile_features);
   const int64_t groups = tiles * slices;
   const int ksteps = (k + kBK - 1) / kBK;
@@ -1442,7 +1461,7 @@ static float tiled_time_us(const TilingCost& c, int m, int n, int k, int slices)
   };
   const int64_t capacity = static_cast<int64_t>(kComputeUnits) * c.resident;
   const int64_t full = groups / capacity, rest = groups % capacity;
-  const float fixed = c.fixed + (slices > 1 ? c.cut : 0.f);
+  const float fixed = c.fixed + (sums ? c.wide : 0.f);
   float t = full * (fixed + per * step(c.resident, 1.f));
   if (rest > 0) {
     const int resident = static_cast<int>((rest + kComputeUnits - 1) / kComputeUnits);
@@ -1450,7 +1469,8 @@ static float tiled_time_us(const TilingCost& c, int m, int n, int k, int slices)
   }
   return t;
 }
-static GemmPlan plan_many_tokens(int m, int n, int k, int max_slices) {
+// sums: the results are float32.
+static GemmPlan plan_many_tokens(int m, int n, int k, int max_slices, bool sums) {
   GemmPlan best{11, 1};
   float best_time = 0.f;
   const int ksteps = (k + kBK - 1) / kBK;
@@ -1459,8 +1479,8 @@ static GemmPlan plan_many_tokens(int m, int n, int k, int max_slices) {
       if (slices > 1 && ksteps / slices < 3) break;  // every slice keeps a few steps (0.5B output
                                                      // projection at 128 tokens, 14 steps: whole 8.0 us, in 4 slices 5.4)
       if (c.kernel == 23 && (c.resident == 1) != takes_turns(m, n, k, slices)) continue;
-      float t = tiled_time_us(c, m, n, k, slices);
-      if (slices > 1) t += (4.f * slices - 2.f) * m * n / 5.7e6f;
+      float t = tiled_time_us(c, m, n, k, slices, sums);
+      if (sums) t += 4.f * slices * m * n / 5.7e6f;
       if (best_time == 0.f || t < best_time) best = {c.kernel, slices}, best_time = t;
     }
   return best;
@@ -1530,12 +1550,12 @@ static int choose_few_token_tiles(int m, int n, int k, int slices) {
   return best;
 }
 
-static int choose_kernel(int m, int n, int k, int slices) {
+static int choose_kernel(int m, int n, int k, int slices, bool sums) {
   // (2,048 x 4,096 in 8 slices at 8 tokens, 17 MB: 7.4 us in tiles, 6.5 here; 3,584 x 3,584, 26 MB: 8.7 and 10.4)
   if (m <= 16 && (!few_tokens_tiled(n, slices) || static_cast<int64_t>(n) * k * 2 < (20ll << 20))) return 16;
   if (m <= 64 && small_matrix(n, k)) return 16;
   if (m <= 64) return choose_few_token_tiles(m, n, k, slices);
-  const GemmPlan plan = plan_many_tokens(m, n, k, slices);
+  const GemmPlan plan = plan_many_tokens(m, n, k, slices, sums);
   const int kernel = plan.slices == slices ? plan.kernel : 11;
   // up to 256 tokens in tiles of 64: the same choice of widths as for one tile of tokens (7B down at 128
   // tokens in 4 slices: 50.6 us staged, 41.8 in tiles of 128 features; 32B down at 192 tokens 131 and
@@ -1651,7 +1671,7 @@ extern "C" {
 // partial sums (at most `max_slices`); 1 means it writes the finished product.
 int mlr_gemm_bf16_slices(int m, int n, int k, int max_slices) {
   if (k % 8 != 0) return 1;
-  if (m > 64) return plan_many_tokens(m, n, k, max_slices).slices;
+  if (m > 64) return plan_many_tokens(m, n, k, max_slices, true).slices;
   if (m <= 16) {
     // Measured with the norm kernel that adds the slices up (its cost grows with their number):
     // a weight of 64 MB or more streams fastest through the LDS-tiled kernel cut into 8 slices;
@@ -1679,7 +1699,7 @@ int mlr_gemm_bf16_slices(int m, int n, int k, int max_slices) {
   return choose_slices(tiles_64(m, n), (k / 8 + 3) / 4, min(max_slices, 8), 512);
 }
 
-int mlr_gemm_bf16_kernel(int m, int n, int k, int slices) { return choose_kernel(m, n, k, slices); }
+int mlr_gemm_bf16_kernel(int m, int n, int k, int slices) { return choose_kernel(m, n, k, slices, slices > 1); }
 
 // y = x w^T (+ bias) in bfloat16 on the matrix cores; see mlr_gemm_simple for the
 // argument meanings.  Requires k % 8 == 0 and 16-byte aligned x and w.  With
@@ -1716,7 +1736,7 @@ int mlr_gemm_bf16(const void* x, const void* w, const void* bias, int bias_is_f3
   MLR_REQUIRE(multiply_rows == nullptr || multiply != nullptr, "row indices come with a multiplier");
   GemmEpilogue ep{bias, bias_is_f32, y, out_is_f32, swiglu, row_sumsq, sumsq_parts, norm_eps, multiply, glu_limit, glu_alpha,
                   multiply_rows};
-  if (kernel == 0) kernel = choose_kernel(m, n, k, slices);
+  if (kernel == 0) kernel = choose_kernel(m, n, k, slices, out_is_f32 != 0);
   // the 256 x 320 tile has no room for a choice of activations and the multiplier in its epilogue (the GELU gating has an
   // instance of its own)
   if (kernel == 48 && ((swiglu >= kEpRelu2 && swiglu != kEpGeglu) || multiply != nullptr)) kernel = 45;

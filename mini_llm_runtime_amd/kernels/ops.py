@@ -588,7 +588,8 @@ class HipOps:
         partial_sums: the caller hands the result to a norm as a not-yet-added delta and
         accepts, instead of [M, N], a float32 stack [S, M, N] of partial sums over slices
         of k (bias in slice 0).  Narrow products of a few tokens are cut that way so that
-        all compute units stream the weight; the norm kernel adds the slices in order.
+        all compute units stream the weight; the norm kernel adds the slices in order.  Beyond 64 tokens, where the number of
+        slices changes from count to count, it is a stack for one slice too: float32 sums, however many slices there are.
         out: a tensor of the result's shape and dtype to write it into (a stack [S, M, N] with `slices` = S > 1).
         mfma_kernel, slices: force one of the matrix-core kernels (16, 14, 11, 22 to 25, 44 to 48, 62 to 68, 71 to 74) and a number
         of k slices instead of letting the shape choose; for tests and tuning.
@@ -659,13 +660,15 @@ class HipOps:
         elif multiply is not None:
             self._check(multiply, "multiplier", self.dtype, (m, n))
         if kernel == "auto" and self.dtype == torch.bfloat16 and k % 8 == 0:
+            stacked = False
             if slices is None:
                 slices = 1
-                if partial_sums and not swiglu:
+                if partial_sums and not swiglu and self.max_k_slices > 1:
                     slices = self.lib.mlr_gemm_bf16_slices(m, n, k, self.max_k_slices)
+                    stacked = m > 64 and out is None
             elif slices < 1 or (slices > 1 and not (partial_sums and not swiglu)):
                 raise KernelError("k slices need partial_sums and no SwiGLU")
-            if slices > 1:
+            if slices > 1 or stacked:
                 y = self._into(out, (slices, m, n), torch.float32)
                 out_f32 = 1
             else:

@@ -23,7 +23,7 @@ def ops():
 @pytest.mark.parametrize("m,n,k", [(1, 16, 8), (255, 256, 64), (257, 272, 136), (384, 528, 72), (385, 976, 200), (130, 1328, 424)])
 @pytest.mark.parametrize("epilogue", ["plain", "bias", "swiglu", "geglu"])
 def test_staged_results_are_the_stored_ones(ops, kernel, m, n, k, epilogue):
-    """The same sums in float32 take the way without staging: rounded, they are the staged bits."""
+    """The same sums in float32 leave their own way: rounded, they are the staged bits."""
     x, w = _rand((m, k), torch.bfloat16, 71).cuda(), _rand((n, k), torch.bfloat16, 72, 0.1).cuda()
     bias = _rand((n,), torch.float32, 73).cuda() if epilogue in ("bias", "geglu") else None
     kw = {"swiglu": dict(swiglu=True), "geglu": dict(geglu=True)}.get(epilogue, {})
@@ -59,3 +59,39 @@ def test_tiles_cut_along_k(ops, slices, kernel):
     ref = x.double() @ w.double().t()
     bound = k * 2.0**-24 * (x.double().abs() @ w.double().abs().t()) + 1e-6
     assert got.shape == (slices, m, n) and ((got.double().sum(0) - ref).abs() <= bound).all()
+
+
+# tokens in every part of a tile's rows that leave in turns, features that end inside a tile (a row of 4 n bytes is whole pieces of 16)
+@pytest.mark.parametrize("kernel", [24, 25, 45, 46, 47, 48])
+@pytest.mark.parametrize("m,n,k", [(1, 4, 8), (63, 132, 64), (65, 128, 200), (193, 260, 72), (257, 516, 136), (129, 324, 264)])
+@pytest.mark.parametrize("slices", [1, 2])
+@pytest.mark.parametrize("bias", [False, True])
+def test_staged_sums_are_the_stored_ones(ops, kernel, m, n, k, slices, bias):
+    """float32 sums leave through LDS where their rows start at 16 bytes; in a tensor that does not, they are stored directly."""
+    x, w = _rand((m, k), torch.bfloat16, 79).cuda(), _rand((n, k), torch.bfloat16, 80, 0.1).cuda()
+    b = _rand((n,), torch.float32, 81).cuda() if bias else None
+    kw = dict(partial_sums=True, slices=slices) if slices > 1 else dict(out_dtype=torch.float32)
+    staged = ops.linear(x, w, b, mfma_kernel=kernel, **kw)
+    flat = torch.empty(staged.numel() + 1, dtype=torch.float32, device="cuda")
+    stored = ops.linear(x, w, b, mfma_kernel=kernel, out=flat[1:].view(staged.shape), **kw)
+    assert torch.equal(staged, stored)
+    ref = x.double() @ w.double().t() + (0 if b is None else b.double())
+    bound = k * 2.0**-24 * (x.double().abs() @ w.double().abs().t()) + 2.0**-23 * ref.abs() + 1e-6
+    assert ((staged.double().reshape(-1, m, n).sum(0) - ref).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("m,n,k", [(65, 48, 64), (300, 300, 136), (1048, 3584, 3584), (2000, 2048, 2048), (2048, 3584, 7168)])
+def test_sums_for_the_stream_are_not_rounded(ops, m, n, k):
+    """What is added to the residual stream comes in float32 however many slices of k its product is cut into; rounded to bfloat16 the
+    sums would be off by up to 2^-9 of themselves."""
+    x, w = _rand((m, k), torch.bfloat16, 82).cuda(), _rand((n, k), torch.bfloat16, 83, 0.1).cuda()
+    for kw in (dict(partial_sums=True), dict(for_stream=True)):
+        got = ops.linear(x, w, **kw)
+        assert got.dtype == torch.float32 and got.shape[1:] == (m, n)
+        ref = x.double() @ w.double().t()
+        bound = k * 2.0**-24 * (x.double().abs() @ w.double().abs().t()) + 2.0**-23 * ref.abs() + 1e-6
+        assert ((got.double().sum(0) - ref).abs() <= bound).all()
+    stream, weight = _rand((m, n), torch.float32, 84).cuda(), torch.ones(n, device="cuda")
+    want = stream.double() + got.double().sum(0)
+    ops.rmsnorm(stream, weight, 1e-6, delta=got)
+    assert ((stream.double() - want).abs() <= 2.0**-22 * (want.abs() + got.double().abs().sum(0))).all()
