@@ -469,6 +469,10 @@ __global__ __launch_bounds__(256) void moe_gemm_simple_kernel(const T* __restric
 // expert weights it streams, read once (non-temporal).
 constexpr int kMoeDepth = 8;
 
+// The offset that stands for no row of the input, and for k past its end: at or past the end of any input below 4 GB whose rows are whole
+// pieces of 16 bytes.  (An expert's matrix stays below 2 GB, where kOutOfBuffer serves.)
+constexpr unsigned kNoRow = 0xfffffff0u;
+
 template <bool UP>
 __global__ __launch_bounds__(256) void moe_gemm_mfma_kernel(const bf16* __restrict__ a, const bf16* __restrict__ w,
                                                             const int* __restrict__ sorted,
@@ -497,7 +501,7 @@ __global__ __launch_bounds__(256) void moe_gemm_mfma_kernel(const bf16* __restri
   const __amdgpu_buffer_rsrc_t abuf = make_buffer(a, static_cast<unsigned>(a_rows) * row_bytes);
   const int wn = n_base + col;
   const unsigned w_off = wn < N ? static_cast<unsigned>(wn) * row_bytes : kOutOfBuffer;
-  const unsigned a_off = a_row >= 0 ? static_cast<unsigned>(a_row) * row_bytes : kOutOfBuffer;
+  const unsigned a_off = a_row >= 0 ? static_cast<unsigned>(a_row) * row_bytes : kNoRow;
   f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
   for (int kb = 0; kb < K; kb += 32 * kMoeDepth) {
     bf16x8_t wv[kMoeDepth], xv[kMoeDepth];
@@ -507,7 +511,7 @@ __global__ __launch_bounds__(256) void moe_gemm_mfma_kernel(const bf16* __restri
       const unsigned koff = static_cast<unsigned>(k) * 2u;
       const bool in = k < K;
       wv[u] = buffer_load_bf16x8_once(wbuf, in && w_off != kOutOfBuffer ? w_off + koff : kOutOfBuffer);
-      xv[u] = buffer_load_bf16x8(abuf, in && a_off != kOutOfBuffer ? a_off + koff : kOutOfBuffer);
+      xv[u] = buffer_load_bf16x8(abuf, in && a_off != kNoRow ? a_off + koff : kNoRow);
     }
 #pragma unroll
     for (int u = 0; u < kMoeDepth; ++u) acc = mfma_16x16x32(wv[u], xv[u], acc);
@@ -602,15 +606,15 @@ __global__ __launch_bounds__(256) void moe_gemm_stream_kernel(const bf16* __rest
                                                in && w_off[i] != kOutOfBuffer ? w_off[i] + koff : kOutOfBuffer, 0, 0, 2);
   };
   auto fetch_rows = [&](int slice, int buf) {
-    const bool in = slice < slices && slice * kStK + piece * 8 < K && x_off != kOutOfBuffer;
+    const bool in = slice < slices && slice * kStK + piece * 8 < K && x_off != kNoRow;
     __builtin_amdgcn_raw_ptr_buffer_load_lds(
         abuf, (__attribute__((address_space(3))) void*)(moe_lds + buf * kStBufferBytes + wave * 1024 + 16384), 16,
-        in ? x_off + static_cast<unsigned>(slice) * kStK * 2u : kOutOfBuffer, 0, 0, 0);
+        in ? x_off + static_cast<unsigned>(slice) * kStK * 2u : kNoRow, 0, 0, 0);
   };
   // the weights do not wait for the lookup of the rows
 #pragma unroll
   for (int s = 0; s < kStBuffers - 1; ++s) fetch_weights(s, s);
-  x_off = row0 + my_row < row_end ? static_cast<unsigned>(UP ? my_pair / top : row0 + my_row) * row_bytes + piece * 16u : kOutOfBuffer;
+  x_off = row0 + my_row < row_end ? static_cast<unsigned>(UP ? my_pair / top : row0 + my_row) * row_bytes + piece * 16u : kNoRow;
 #pragma unroll
   for (int s = 0; s < kStBuffers - 1; ++s) fetch_rows(s, s);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // they were sent together and arrive together; from here on slices are waited for one by one
@@ -745,7 +749,7 @@ __global__ __launch_bounds__(256) void moe_gemm_tiled_kernel(const bf16* __restr
     for (int p = 0; p < 8; ++p) {
       if (p >= kLoads) break;
       if ((p < 4) != weights) continue;
-      const unsigned at = p < 4 ? (off[p] + koff) | past : (past != 0u || off[p] == kOutOfBuffer ? kOutOfBuffer : off[p] + koff);
+      const unsigned at = p < 4 ? (off[p] + koff) | past : (past != 0u || off[p] == kNoRow ? kNoRow : off[p] + koff);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           p < 4 ? wbuf : abuf, (__attribute__((address_space(3))) void*)(moe_lds + buf * kBuffer + (4 * p + wave) * 1024), 16, at, 0, 0, 0);
     }
@@ -759,7 +763,7 @@ __global__ __launch_bounds__(256) void moe_gemm_tiled_kernel(const bf16* __restr
   for (int p = 0; p < 4; ++p) {
     if (p >= kRowLoads) break;
     const int at = 8 * (4 * p + wave) + lane / 8;
-    off[4 + p] = at < rows ? static_cast<unsigned>(UP ? pairs_of_lane[p] / top : row0 + at) * row_bytes + piece * 16u : kOutOfBuffer;
+    off[4 + p] = at < rows ? static_cast<unsigned>(UP ? pairs_of_lane[p] / top : row0 + at) * row_bytes + piece * 16u : kNoRow;
   }
   if (tid < kRows) pair_of[tid] = tid < rows ? pair_of_thread : -1;
   f32x16_t acc[RB][2];
@@ -882,7 +886,6 @@ constexpr int kSqBuffer = 4 * kSqQuarter;  // W0, W1, X0, X1: 64 k of 128 rows e
 constexpr int kSqRowF32 = kSqCols * 4 + 16, kSqRowBf16 = kSqCols * 2 + 16;
 constexpr int kSqLds = kSqRows * kSqRowBf16;
 static_assert(kSqLds >= 2 * kSqBuffer && kSqLds >= kSqRows / 2 * kSqRowF32, "two slices, and half a tile of 32-bit results, fit");
-constexpr unsigned kNoRow = 0xfffffff0u;  // at or past the end of any input below 4 GB whose rows are whole pieces of 16 bytes
 
 template <bool UP>
 __global__ __launch_bounds__(512, 2) void moe_gemm_phased_kernel(const bf16* __restrict__ a, const bf16* __restrict__ w,

@@ -128,3 +128,34 @@ def test_gated_products_of_woven_rows(inner, tiles):
     act = torch.full((1,), 2.0**-7, dtype=torch.double, device="cuda")
     bound = act * 8.0 * 7.0 * down.double().abs().sum(-1).max()
     assert ((got - want).abs() <= bound).all() and ((got - want).norm() <= 2.0**-7 * want.norm())
+
+
+# streaming from memory, streaming by whole lines (a matrix of a megabyte), tiles of 64, 128 and 256 rows
+@pytest.mark.parametrize("kind,wide", [("16 rows", 16), ("16 rows", 256), ("64", 16), ("128", 16), ("256", 16)])
+def test_inputs_beyond_two_gigabytes(kind, wide):
+    """Input rows lie at 32-bit offsets of up to 4 GB: those at and behind 2 GB, where the mark for weights out of range lies, are rows like
+    any other."""
+    from mini_llm_runtime_amd.kernels.ops import HipOps
+    from mini_llm_runtime_amd.kernels.tuning import KernelTuning
+
+    far = 1 << 30
+    ops = HipOps(torch.bfloat16, "cuda", tuning=KernelTuning(
+        moe_tiled_rows=far if kind == "16 rows" else 1, moe_wide_tiled_rows=1 if kind in ("128", "256") else far,
+        moe_square_groups=1 if kind == "256" else far))
+    hidden, first = 2048, (1 << 31) // (2048 * 2)
+    tokens = first + 40
+    g = torch.Generator(device="cuda")
+    g.manual_seed(85)
+    h = torch.empty((tokens, hidden), dtype=torch.bfloat16, device="cuda").normal_(generator=g)
+    up, down = _rand((2 * wide, hidden), torch.bfloat16, 86, 0.05).cuda(), _rand((2 * hidden, wide), torch.bfloat16, 87, 0.2).cuda()
+    ids = (torch.arange(tokens, dtype=torch.int32, device="cuda") % 2)[:, None].contiguous()
+    weights = torch.ones((tokens, 1), device="cuda")
+    out = ops.expert_products(h, up, down, ids, weights, experts=2, activation="relu2")[0]
+    for e in (0, 1):
+        rows = torch.arange(first - 2 + e, tokens, 2, device="cuda")
+        z = h[rows].double() @ up[e * wide : (e + 1) * wide].double().t()
+        act = z.clamp(min=0) ** 2
+        want = act @ down[e * hidden : (e + 1) * hidden].double().t()
+        # the activations are rounded to bfloat16 (2^-9 of themselves), everything else is float32
+        bound = 2.0**-8 * act.abs() @ down[e * hidden : (e + 1) * hidden].double().abs().t() + 1e-3
+        assert ((out[rows].double() - want).abs() <= bound).all()
