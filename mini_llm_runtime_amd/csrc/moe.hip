@@ -672,11 +672,22 @@ __global__ __launch_bounds__(256) void moe_gemm_stream_kernel(const bf16* __rest
 // piece ^ (row / 2) % 8).  Wavefront (wr, wc) of 2 x 2 owns rows wr * 32 RB .. + 32 RB and features wc * 64 .. + 64; the last
 // quarter of a slice's products is kept for behind the barrier, where the next slice's first operands are on their way.  Finished
 // tiles leave through LDS in whole lines: the down product's rows go to as many places as it has rows, 512 bytes each.
-// Workgroup -> (tile, features): workgroups go to the eight dies in turn; a die gets every eighth pair of neighbouring tiles (mostly one
-// expert's) and takes their features one after the other, both tiles at a time, so that the rows and the expert's weights come from its L2.
+// Workgroup -> (tile, features): workgroups go to the eight dies in turn; a pair of neighbouring tiles (mostly one expert's) belongs to one
+// die, or its features to `spread` of them where there are too few pairs for all (dies_of_a_pair); a die takes their features one after the
+// other, both tiles at a time, so that the rows and the expert's weights come from its L2.
 // Bound by the operands' way through L2 and LDS (each 64 x RB + 128 rows of a slice make 64 RB x 128 products of it) and by tiles
 // that are not full: 2,000 tokens, 64 experts with 6 choices (187 rows an expert in tiles of 128), 768 x 2,048: up 94.5 to 91.4 us,
 // down 128 to 93 (400 TFLOP/s of the asked-for products, 550 with the padding).  Four buffers of 32 k instead: up the same, down 102.
+struct TilePlace {
+  int tile, column;  // column -1: none
+};
+__device__ __forceinline__ TilePlace place_tile(int columns, int spread) {
+  const int each = (columns + spread - 1) / spread;  // of a die
+  const int local = blockIdx.x / 8, in_unit = local % (2 * each);
+  const int unit = local / (2 * each) * 8 + blockIdx.x % 8;
+  const int column = unit % spread * each + in_unit / 2;
+  return {unit / spread * 2 + in_unit % 2, column < columns ? column : -1};
+}
 constexpr int kBigCols = 128;
 constexpr int kBigK = 64;
 constexpr int big_rows(int rb) { return 64 * rb; }
@@ -703,7 +714,7 @@ template <bool UP, int RB>
 __global__ __launch_bounds__(256) void moe_gemm_tiled_kernel(const bf16* __restrict__ a, const bf16* __restrict__ w,
                                                              const int* __restrict__ sorted,
                                                              const int* __restrict__ offsets,
-                                                             const int* __restrict__ tiles, int max_tiles,
+                                                             const int* __restrict__ tiles, int max_tiles, int spread,
                                                              const float* __restrict__ pair_weights,
                                                              void* __restrict__ out, int tokens, int top, int N, int K,
                                                              int act, int a_rows, float glu_limit, float glu_alpha) {
@@ -712,13 +723,12 @@ __global__ __launch_bounds__(256) void moe_gemm_tiled_kernel(const bf16* __restr
   // runs of 8 rows, dealt out to four wavefronts: 4 of weights, then the input's (loops over them go to 8 and break: with a bound that
   // depends on the template's parameters the host pass left the kernel uninstantiated, without a message)
   constexpr int kLoads = (kBigCols + kRows) / 8 / 4;
-  const int columns = (N + kBigCols - 1) / kBigCols;
-  const int local = blockIdx.x / 8, in_pair = local % (2 * columns);
-  const int tile = (local / (2 * columns) * 8 + blockIdx.x % 8) * 2 + in_pair % 2;
-  if (tile >= max_tiles) return;
+  const TilePlace place = place_tile((N + kBigCols - 1) / kBigCols, spread);
+  const int tile = place.tile;
+  if (tile >= max_tiles || place.column < 0) return;
   const int expert = tiles[2 * tile];
   if (expert < 0) return;
-  const int n0 = in_pair / 2 * kBigCols;
+  const int n0 = place.column * kBigCols;
   const int row0 = tiles[2 * tile + 1];
   const int rows = min(kRows, offsets[expert + 1] - row0);
   extern __shared__ __attribute__((aligned(16))) unsigned char moe_lds[];
@@ -890,19 +900,18 @@ static_assert(kSqLds >= 2 * kSqBuffer && kSqLds >= kSqRows / 2 * kSqRowF32, "two
 template <bool UP>
 __global__ __launch_bounds__(512, 2) void moe_gemm_phased_kernel(const bf16* __restrict__ a, const bf16* __restrict__ w,
                                                                 const int* __restrict__ sorted, const int* __restrict__ offsets,
-                                                                const int* __restrict__ tiles, int max_tiles,
+                                                                const int* __restrict__ tiles, int max_tiles, int spread,
                                                                 const float* __restrict__ pair_weights, void* __restrict__ out,
                                                                 int tokens, int top, int N, int K, int act, int a_rows,
                                                                 float glu_limit, float glu_alpha) {
   extern __shared__ __attribute__((aligned(16))) unsigned char moe_lds[];
   __shared__ int pair_of[kSqRows];
-  const int columns = (N + kSqCols - 1) / kSqCols;
-  const int local = blockIdx.x / 8, in_pair = local % (2 * columns);
-  const int tile = (local / (2 * columns) * 8 + blockIdx.x % 8) * 2 + in_pair % 2;
-  if (tile >= max_tiles) return;
+  const TilePlace place = place_tile((N + kSqCols - 1) / kSqCols, spread);
+  const int tile = place.tile;
+  if (tile >= max_tiles || place.column < 0) return;
   const int expert = tiles[2 * tile];
   if (expert < 0) return;
-  const int n0 = in_pair / 2 * kSqCols;
+  const int n0 = place.column * kSqCols;
   const int row0 = tiles[2 * tile + 1];
   const int rows = min(kSqRows, offsets[expert + 1] - row0);
   const int tid = threadIdx.x;
@@ -1102,12 +1111,25 @@ __global__ __launch_bounds__(512, 2) void moe_gemm_phased_kernel(const bf16* __r
   }
 }
 
-using MoeTiledKernel = void (*)(const bf16*, const bf16*, const int*, const int*, const int*, int, const float*, void*, int, int, int, int,
+using MoeTiledKernel = void (*)(const bf16*, const bf16*, const int*, const int*, const int*, int, int, const float*, void*, int, int, int, int,
                                 int, int, float, float);
 struct MoeTiles {
   MoeTiledKernel kernel;
-  int threads, cols, lds;
+  int threads, rows, cols, lds;
 };
+// How many dies share a pair of tiles: as few as leave none without work and none with more than 1.15 times its share, by the number of tiles
+// that experts with equal shares of the pairs would have (the host does not know the routing).  Fewer dies read a pair's rows fewer times.
+// With one die for each pair / as chosen here, both products with their gating, microseconds: 8 experts of 14,336 x 4,096 (4 pairs on 8 dies): 48
+// rows an expert 786 / 617, 97 900 / 692; 12 of 8,192 x 5,120: 97 798 / 646, 320 1,521 / 1,296; 64 of 768 x 2,048 (32 pairs and more: one
+// die) the same, where eight dies take 1.1 to 1.4 times as long.
+static int dies_of_a_pair(int max_tiles, int64_t pairs, int rows) {
+  const int64_t experts = max_tiles - pairs / rows > 1 ? max_tiles - pairs / rows : 1;
+  const int64_t tiles = experts * ((pairs + experts * rows - 1) / (experts * rows));
+  const int64_t tile_pairs = (tiles + 1) / 2;
+  for (int spread = 1; spread < 8; spread *= 2)
+    if ((tile_pairs * spread + 7) / 8 * 8 * 100 <= tile_pairs * spread * 115) return spread;
+  return 8;
+}
 static int launch_moe_tiled(const MoeTiles& t, bool& configured, const bf16* a, const bf16* w, const int* sorted, const int* offsets,
                             const int* tiles, const float* pair_weights, void* out, int max_tiles, int tokens, int top, int n, int k,
                             int act, int a_rows, float glu_limit, float glu_alpha, hipStream_t stream) {
@@ -1119,13 +1141,16 @@ static int launch_moe_tiled(const MoeTiles& t, bool& configured, const bf16* a, 
     }
     configured = true;
   }
-  const int64_t groups = static_cast<int64_t>((max_tiles + 15) / 16 * 16) * ((n + t.cols - 1) / t.cols);
+  const int64_t columns = (n + t.cols - 1) / t.cols;
+  const int spread = dies_of_a_pair(max_tiles, static_cast<int64_t>(tokens) * top, t.rows);
+  const int64_t units = (static_cast<int64_t>((max_tiles + 1) / 2) * spread + 7) / 8 * 8;
+  const int64_t groups = units * 2 * ((columns + spread - 1) / spread);
   if (groups >= (1ll << 31)) {
     set_error("mlr_moe_gemm: too many tiles for one launch");
     return -1;
   }
   hipLaunchKernelGGL(t.kernel, dim3(static_cast<unsigned>(groups)), dim3(t.threads), t.lds, stream, a, w, sorted, offsets, tiles, max_tiles,
-                     pair_weights, out, tokens, top, n, k, act, a_rows, glu_limit, glu_alpha);
+                     spread, pair_weights, out, tokens, top, n, k, act, a_rows, glu_limit, glu_alpha);
   return 0;
 }
 
@@ -1231,9 +1256,9 @@ int mlr_moe_gemm(const void* a, const void* w, const int* sorted, const int* off
     const int rows = static_cast<int>(a_rows);
     if (mfma >= 2) {
       static const MoeTiles kinds[3][2] = {
-          {{moe_gemm_tiled_kernel<false, 1>, 256, kBigCols, big_lds_bytes(1)}, {moe_gemm_tiled_kernel<true, 1>, 256, kBigCols, big_lds_bytes(1)}},
-          {{moe_gemm_tiled_kernel<false, 2>, 256, kBigCols, big_lds_bytes(2)}, {moe_gemm_tiled_kernel<true, 2>, 256, kBigCols, big_lds_bytes(2)}},
-          {{moe_gemm_phased_kernel<false>, 512, kSqCols, kSqLds}, {moe_gemm_phased_kernel<true>, 512, kSqCols, kSqLds}}};
+          {{moe_gemm_tiled_kernel<false, 1>, 256, big_rows(1), kBigCols, big_lds_bytes(1)}, {moe_gemm_tiled_kernel<true, 1>, 256, big_rows(1), kBigCols, big_lds_bytes(1)}},
+          {{moe_gemm_tiled_kernel<false, 2>, 256, big_rows(2), kBigCols, big_lds_bytes(2)}, {moe_gemm_tiled_kernel<true, 2>, 256, big_rows(2), kBigCols, big_lds_bytes(2)}},
+          {{moe_gemm_phased_kernel<false>, 512, kSqRows, kSqCols, kSqLds}, {moe_gemm_phased_kernel<true>, 512, kSqRows, kSqCols, kSqLds}}};
       static bool configured[3][2] = {};
       const int status = launch_moe_tiled(kinds[mfma - 2][up != 0], configured[mfma - 2][up != 0], ab, wb, sorted, offsets, tiles, pair_weights,
                                           out, max_tiles, tokens, top, n, k, act, rows, glu_limit, glu_alpha, stream);

@@ -106,6 +106,12 @@ def test_grouped_products(rows, hidden, inner, tiles):
     assert torch.equal(got, same)
 
 
+@pytest.mark.parametrize("experts", [6, 8, 12, 16])  # 3, 4, 6 and 8 pairs of tiles: their features on eight, two, four dies and on one
+@pytest.mark.parametrize("tiles", [1, 2, 3])
+def test_few_tiles_on_all_dies(experts, tiles):
+    test_grouped_products((20,) * experts, 1160, 1032, tiles)  # 10 and 9 runs of 128 features, 5 of 256: not the same number for every die
+
+
 @pytest.mark.parametrize("inner", [4, 12, 72])  # 8, 24 and 144 woven rows: results of 8, 24 and 144 bytes (the second is stored directly)
 @pytest.mark.parametrize("tiles", [1, 2, 3])
 def test_gated_products_of_woven_rows(inner, tiles):
