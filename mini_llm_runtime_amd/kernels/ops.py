@@ -1199,15 +1199,20 @@ class HipOps:
             tiles, wide = plan.query_tiles, 0
             num_wide = int(getattr(plan, "num_wide_query_tiles", 0))
             enough = self.tuning.wide_attention_groups
-            if head_dim == 128 and block_size >= 16 and score_bias is None and not keep_first:
-                # the 32 x 32 kernel: at this head size its narrow tiles have a compute unit to themselves (128 KB of LDS), so the
-                # wide ones win from half as many on
+            # the 32 x 32 kernel: at this head size its narrow tiles have a compute unit to themselves (128 KB of LDS), so the
+            # wide ones win from half as many on
+            alone = head_dim == 128 and block_size >= 16 and score_bias is None and not keep_first
+            if alone:
                 enough //= 2
             behind = int(getattr(plan, "long_prefix", 0))  # 1: thousands of keys before every tile, 2: twice that
             if behind:
                 enough = enough * 3 // 4  # heavy tiles everywhere: fewer of them keep the compute units busy
             if (
                 num_wide * num_heads >= enough
+                # portions of up to 64 tokens fill half of a wide tile, whose keys cost as much as a full one's (64 tokens behind 4,096 for 16
+                # requests, 16 heads of 128: 114 us wide, 83 narrow), unless there are more narrow tiles than units that they have to
+                # themselves (16 behind 2,048 for 8, 40 heads: 66 and 74)
+                and not (behind and 4 * num_wide > 3 * num_tiles and (not alone or num_tiles * num_heads <= 256))
                 and getattr(plan, "wide_query_tiles", None) is not None
                 and lib.mlr_attention_wide_tile() == WIDE_QUERY_TILE
             ):
@@ -1217,8 +1222,17 @@ class HipOps:
             # are cut into runs with a workgroup each, merged by a second kernel
             groups = num_tiles * num_heads
             key_runs = 1
-            if behind == 2 and groups < self.tuning.key_run_groups:
+            # A tile reads no more keys than its mask reaches back: runs of those pay only where few tiles reach far.  In runs / whole, us: 2,048
+            # tokens behind 6,144, 16 heads of 128 (256 tiles of 128), a window of 512 73 / 26, of 3,000 114 / 78; 512 behind 8,192, 14 heads of 64
+            # (112 tiles), 3,000 41 / 32; 16 behind 16,384, 32 heads of 64, 512 13.3 / 11.9, 1,024 15.5 / 16.0, 2,040 19 / 24, 3,000 19 / 32.
+            reach = int(window or 0) or chunk
+            pays = not reach or (reach >= 1024 and groups <= 64)
+            if behind == 2 and pays and groups < self.tuning.key_run_groups:
                 key_runs = min(8, -(-self.tuning.key_run_groups // groups))
+                if alone and not wide and groups <= 256:
+                    # no more of them than compute units: a workgroup more would wait for a round of its own (16 tokens behind 16,384, 40 heads:
+                    # 8 runs 95 us, 6 71; 512 behind 8,192, 28 heads: 2 runs 141, 1 115; but 40 heads, 320 tiles: 1 run 214, 2 187)
+                    key_runs = min(key_runs, 256 // groups)
             partial = None
             if key_runs > 1 or share is not None:
                 partial = self._empty(

@@ -57,6 +57,19 @@ def test_scores_that_keep_rising(ops, head_dim):
 
 
 @pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("entries", [[(6300, 200)], [(6300, 64)] * 5, [(9000, 16), (5000, 70)]])
+@pytest.mark.parametrize("mask", [dict(window=None), dict(window=300), dict(window=1100), dict(window=None, chunk=700), dict(window=None, chunk=2000)])
+def test_portions_behind_long_prefixes(ops, head_dim, entries, mask):
+    """Keys in runs or whole, narrow tiles or wide ones, as what the mask lets a tile see and the tiles' number have it."""
+    q, kp, vp, table, ctx, *_ = _paged_case(entries, 8, 2, head_dim, 16, torch.bfloat16, 57, spike=True)
+    assert ctx.long_prefix == 2
+    args = (q.cuda(), kp.cuda(), vp.cuda(), table.cuda(), ctx)
+    kw = dict(num_heads=8, num_kv_heads=2, head_dim=head_dim, block_size=16, scale=head_dim**-0.5, **mask)
+    got, plain = _attend(ops, *args, **kw).cpu(), _attend(ops, *args, kernel="fma", **kw).cpu()
+    torch.testing.assert_close(got.double(), plain.double(), **_tol(torch.bfloat16))
+
+
+@pytest.mark.parametrize("head_dim", [64, 128])
 def test_a_key_that_outweighs_the_others(ops, head_dim):
     """A late key outweighs the first one by 2^7 to 2^8 and all others by 2^30, and both have the same values.  The largest weight is 1,
     which bfloat16 holds exactly, the first key's is at most 2^-7 and off by 2^-9 of that: the result is off by 2^-16, which rounds to the
