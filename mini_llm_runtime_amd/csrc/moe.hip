@@ -547,20 +547,21 @@ __global__ __launch_bounds__(256) void moe_gemm_mfma_kernel(const bf16* __restri
 }
 
 // Streaming through LDS (tiles of 16 rows, as above): the same work with loads that cover whole lines.
-// A workgroup owns 16 rows of a tile and 64 features; k in slices of 128, loaded straight into four LDS buffers, three of them
-// on their way (48 KB of weights a workgroup, two workgroups a compute unit: a step through registers had 16 to 32 KB on their way).  Sixteen
-// neighbouring lanes fetch the 256 contiguous bytes that a slice holds of one weight row (the kernel above reads 64 bytes of 16
-// different rows per instruction, which streams a large matrix at little more than half the rate); the 16-byte pieces of a row lie in the
-// order piece ^ row % 16, so that the operand reads of sixteen rows fall on different banks.  Wavefront w multiplies features w * 16 .. + 16.
-// Bound by HBM: 8 tokens, 64 experts with 6 choices, matrices of 768 x 2,048: up 25.5 to 22.3 us, down 23.7 to 23.3 (up to 48 experts'
-// 151 MB for each of the two: 6.5 TB/s).  Tiles start their features at different places, or neighbours would ask the same channels at once.
+// A workgroup owns 16 rows of a tile and 64 features; k in slices of STEP, loaded straight into four LDS buffers, three of them
+// on their way.  Neighbouring lanes fetch the contiguous bytes that a slice holds of one weight row, one or two lines (the kernel above
+// reads 64 bytes of 16 different rows per instruction, which streams a large matrix at little more than half the rate); the 16-byte pieces of a
+// row lie in another order from row to row, so that the operand reads of sixteen rows fall on different banks.  Wavefront w multiplies
+// features w * 16 .. + 16.
+// STEP 128: 80 KB, two workgroups a compute unit with 48 KB of weights each on their way; 64: 40 KB, four with 24.  The first has
+// the whole stream under way with few workgroups, the second loses less at the end of a round of many; see narrow_steps_pay.
+// Bound by HBM: 8 tokens, 64 experts with 6 choices, matrices of 768 x 2,048, up 22.3 us, down 23.3 (up to 48 experts' 151 MB for
+// each of the two: 6.5 TB/s).
 constexpr int kStCols = 64;
-constexpr int kStK = 128;
 constexpr int kStBuffers = 4;
-constexpr int kStBufferBytes = (kStCols + kMoeRows) * kStK * 2;
-constexpr int kStLds = kStBuffers * kStBufferBytes;
+constexpr int stream_buffer_bytes(int step) { return (kStCols + kMoeRows) * step * 2; }
+constexpr int stream_lds_bytes(int step) { return kStBuffers * stream_buffer_bytes(step); }
 
-template <bool UP>
+template <bool UP, int STEP>
 __global__ __launch_bounds__(256) void moe_gemm_stream_kernel(const bf16* __restrict__ a, const bf16* __restrict__ w,
                                                               const int* __restrict__ sorted,
                                                               const int* __restrict__ offsets,
@@ -568,9 +569,13 @@ __global__ __launch_bounds__(256) void moe_gemm_stream_kernel(const bf16* __rest
                                                               const float* __restrict__ pair_weights,
                                                               void* __restrict__ out, int tokens, int top, int N, int K,
                                                               int act, int a_rows, float glu_limit, float glu_alpha) {
-  // Workgroups go to the eight dies in turn and the unused tiles lie at the end of the list: each run of features starts at
-  // another tile, or the same dies would find them every time (35 of 48 tiles used: five on some dies, four on others).
-  const int tile = (blockIdx.x + blockIdx.y) % gridDim.x;
+  constexpr int kRowLanes = STEP / 8;             // lanes that bring a row's piece of a slice, 16 bytes each
+  constexpr int kRunRows = kWave / kRowLanes;     // rows of a load (1 KB)
+  constexpr int kWeightRuns = kStCols / kRunRows / 4, kInputRuns = kMoeRows / kRunRows;
+  constexpr int kBuffer = stream_buffer_bytes(STEP);
+  // Workgroups go to the eight dies in turn and the unused tiles lie at the end of the list: where a tile would be on the same die for every
+  // run of features, each run starts at another tile (35 of 48 tiles used: five on some dies, four on others).
+  const int tile = gridDim.x % 8 == 0 ? (blockIdx.x + blockIdx.y) % gridDim.x : blockIdx.x;
   const int expert = tiles[2 * tile];
   if (expert < 0) return;
   const int row0 = tiles[2 * tile + 1];
@@ -583,33 +588,37 @@ __global__ __launch_bounds__(256) void moe_gemm_stream_kernel(const bf16* __rest
   const __amdgpu_buffer_rsrc_t wbuf =
       make_buffer(w + static_cast<int64_t>(expert) * N * K, static_cast<unsigned>(N) * row_bytes);
   const __amdgpu_buffer_rsrc_t abuf = make_buffer(a, static_cast<unsigned>(a_rows) * row_bytes);
-  // A load fills 4 rows of a buffer (1 KB): rows 4 * (4 * i + wave) + lane / 16 of the weights for i = 0..3, then rows 4 * wave +
-  // lane / 16 of the input tile; the row modulo 16 is the same for all five, so is the piece that this lane brings
-  const int my_row = 4 * wave + lane / 16;
-  const int piece = (lane % 16) ^ my_row;
-  unsigned w_off[4];
+  // This wavefront brings runs `wave`, `wave` + 4, ... of the weights and, where there are as many, run `wave` of the input tile; what
+  // orders a row's pieces is the same for all of them, so is the piece that this lane brings
+  auto order_of = [](int row) { return STEP == 128 ? row % 16 : row / 2 % 8; };
+  const int my_row = kRunRows * wave + lane / kRowLanes;
+  const int piece = (lane % kRowLanes) ^ order_of(my_row);
+  unsigned w_off[4];  // loops over the runs go to 4 and break, see moe_gemm_tiled_kernel
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const int row = n0 + i * 16 + my_row;
+    const int row = n0 + i * 4 * kRunRows + my_row;
     w_off[i] = row < N ? static_cast<unsigned>(row) * row_bytes + piece * 16u : kOutOfBuffer;
   }
   const int my_pair = sorted[min(row0 + my_row, row_end - 1)];
-  const int slices = (K + kStK - 1) / kStK;
+  const int slices = (K + STEP - 1) / STEP;
   unsigned x_off = 0;
   auto fetch_weights = [&](int slice, int buf) {
-    const unsigned koff = static_cast<unsigned>(slice) * kStK * 2u;
-    const bool in = slice < slices && slice * kStK + piece * 8 < K;
-    unsigned char* const dst = moe_lds + buf * kStBufferBytes + wave * 1024;
+    const unsigned koff = static_cast<unsigned>(slice) * STEP * 2u;
+    const bool in = slice < slices && slice * STEP + piece * 8 < K;
+    unsigned char* const dst = moe_lds + buf * kBuffer + wave * 1024;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < 4; ++i) {
+      if (i >= kWeightRuns) break;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(wbuf, (__attribute__((address_space(3))) void*)(dst + i * 4096), 16,
                                                in && w_off[i] != kOutOfBuffer ? w_off[i] + koff : kOutOfBuffer, 0, 0, 2);
+    }
   };
   auto fetch_rows = [&](int slice, int buf) {
-    const bool in = slice < slices && slice * kStK + piece * 8 < K && x_off != kNoRow;
+    if (wave >= kInputRuns) return;
+    const bool in = slice < slices && slice * STEP + piece * 8 < K && x_off != kNoRow;
     __builtin_amdgcn_raw_ptr_buffer_load_lds(
-        abuf, (__attribute__((address_space(3))) void*)(moe_lds + buf * kStBufferBytes + wave * 1024 + 16384), 16,
-        in ? x_off + static_cast<unsigned>(slice) * kStK * 2u : kNoRow, 0, 0, 0);
+        abuf, (__attribute__((address_space(3))) void*)(moe_lds + buf * kBuffer + kStCols * STEP * 2 + wave * 1024), 16,
+        in ? x_off + static_cast<unsigned>(slice) * STEP * 2u : kNoRow, 0, 0, 0);
   };
   // the weights do not wait for the lookup of the rows
 #pragma unroll
@@ -623,16 +632,20 @@ __global__ __launch_bounds__(256) void moe_gemm_stream_kernel(const bf16* __rest
   f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
   for (int s = 0; s < slices; ++s) {
     // this slice has landed (this wavefront's share; the barrier answers for the others), and everybody has multiplied the one before
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((kStBuffers - 2) * 5) : "memory");
+    if (wave < kInputRuns)
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((kStBuffers - 2) * (kWeightRuns + 1)) : "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((kStBuffers - 2) * kWeightRuns) : "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     fetch_weights(s + kStBuffers - 1, (s + kStBuffers - 1) % kStBuffers);
     fetch_rows(s + kStBuffers - 1, (s + kStBuffers - 1) % kStBuffers);  // into the buffer of the slice before
-    const unsigned char* const base = moe_lds + s % kStBuffers * kStBufferBytes;
+    const unsigned char* const base = moe_lds + s % kStBuffers * kBuffer;
 #pragma unroll
-    for (int ks = 0; ks < kStK / 32; ++ks) {
-      const int slot = ((ks * 4 + quad) ^ col) * 16;
-      acc = mfma_16x16x32(load_bf16x8(base + (wave * 16 + col) * 256 + slot), load_bf16x8(base + 16384 + col * 256 + slot), acc);
+    for (int ks = 0; ks < 4; ++ks) {
+      if (ks >= STEP / 32) break;
+      const int slot = ((ks * 4 + quad) ^ order_of(col)) * 16;
+      acc = mfma_16x16x32(load_bf16x8(base + (wave * 16 + col) * STEP * 2 + slot), load_bf16x8(base + (kStCols + col) * STEP * 2 + slot), acc);
     }
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing may still be on its way into LDS when the workgroup ends
@@ -1130,6 +1143,15 @@ static int dies_of_a_pair(int max_tiles, int64_t pairs, int rows) {
     if ((tile_pairs * spread + 7) / 8 * 8 * 100 <= tile_pairs * spread * 115) return spread;
   return 8;
 }
+// Steps of 64 in moe_gemm_stream: where there are more pairs than experts, of matrices of 64 MB or more eight times as many.  Steps of 128 / 64, both
+// products, microseconds: 64 experts of 768 x 2,048 with 6 choices: 2 tokens 25 / 26, 8 51 / 55, 13 69 / 64, 32 79 / 77, 64 87 / 80; 128 of it
+// with 8: 2 26 / 28, 6 59 / 61, 16 98 / 93, 64 146 / 141; 32 of 2,880 x 2,880 with 4: 1 32 / 35, 8 130 / 125, 48 170 / 169; 16 of 6,400 x
+// 4,096 with 2: 4 112 / 116, 10 209 / 205, 24 250 / 245; 8 of 14,336 x 4,096 (117 MB) with 2: 8 233 / 272, 13 259 / 299, 32 320 / 292,
+// 48 377 / 360.  (A step through registers, three workgroups a unit: 64 experts at 13 tokens 64, at 64 82; 8 experts at 32 297.)
+static bool narrow_steps_pay(int max_tiles, int64_t pairs, int64_t matrix_bytes) {
+  if (max_tiles >= pairs) return false;  // mlr_moe_max_tiles: the pairs, or the full tiles and one for every expert
+  return matrix_bytes < (64ll << 20) || pairs >= 8 * (max_tiles - pairs / kMoeRows);
+}
 static int launch_moe_tiled(const MoeTiles& t, bool& configured, const bf16* a, const bf16* w, const int* sorted, const int* offsets,
                             const int* tiles, const float* pair_weights, void* out, int max_tiles, int tokens, int top, int n, int k,
                             int act, int a_rows, float glu_limit, float glu_alpha, hipStream_t stream) {
@@ -1265,19 +1287,21 @@ int mlr_moe_gemm(const void* a, const void* w, const int* sorted, const int* off
       if (status != 0) return -1;
     } else if (static_cast<int64_t>(n) * k * 2 >= (1ll << 20)) {
       // an expert's matrix of a megabyte or more: whole lines through LDS
-      static bool configured = false;
-      if (!configured) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(moe_gemm_stream_kernel<true>), hipFuncAttributeMaxDynamicSharedMemorySize, kStLds);
-        if (e == hipSuccess)
-          e = hipFuncSetAttribute(reinterpret_cast<const void*>(moe_gemm_stream_kernel<false>), hipFuncAttributeMaxDynamicSharedMemorySize, kStLds);
+      using StreamKernel = void (*)(const bf16*, const bf16*, const int*, const int*, const int*, const float*, void*, int, int, int, int, int,
+                                    int, float, float);
+      static const StreamKernel kinds[2][2] = {{moe_gemm_stream_kernel<false, 128>, moe_gemm_stream_kernel<true, 128>},
+                                               {moe_gemm_stream_kernel<false, 64>, moe_gemm_stream_kernel<true, 64>}};
+      static bool configured[2][2] = {};
+      const bool narrow = narrow_steps_pay(max_tiles, static_cast<int64_t>(tokens) * top, static_cast<int64_t>(n) * k * 2);
+      const int lds = stream_lds_bytes(narrow ? 64 : 128);
+      const StreamKernel kernel = kinds[narrow][up != 0];
+      if (!configured[narrow][up != 0]) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
         MLR_REQUIRE(e == hipSuccess, std::string("cannot raise the LDS limit: ") + hipGetErrorString(e));
-        configured = true;
+        configured[narrow][up != 0] = true;
       }
-      const dim3 stream_grid(max_tiles, (n + kStCols - 1) / kStCols);
-      if (up)
-        moe_gemm_stream_kernel<true><<<stream_grid, 256, kStLds, stream>>>(ab, wb, sorted, offsets, tiles, pair_weights, out, tokens, top, n, k, act, rows, glu_limit, glu_alpha);
-      else
-        moe_gemm_stream_kernel<false><<<stream_grid, 256, kStLds, stream>>>(ab, wb, sorted, offsets, tiles, pair_weights, out, tokens, top, n, k, act, rows, glu_limit, glu_alpha);
+      hipLaunchKernelGGL(kernel, dim3(max_tiles, (n + kStCols - 1) / kStCols), dim3(256), lds, stream, ab, wb, sorted, offsets, tiles,
+                         pair_weights, out, tokens, top, n, k, act, rows, glu_limit, glu_alpha);
     } else {
       // four wavefronts (64 features) a workgroup, or two where that leaves the compute units with too
       // few workgroups to keep their loads in flight

@@ -106,6 +106,13 @@ def test_grouped_products(rows, hidden, inner, tiles):
     assert torch.equal(got, same)
 
 
+# matrices of a megabyte and more: whole lines through LDS; fewer slices of k than buffers and more, tails of k, features that end inside a tile
+@pytest.mark.parametrize("rows", [(1, 0, 15), (16, 17, 0), (33, 1, 20)])
+@pytest.mark.parametrize("hidden,inner", [(72, 8008), (8008, 72), (1160, 1032), (264, 2040)])
+def test_products_that_stream_from_memory(rows, hidden, inner):
+    test_grouped_products(rows, hidden, inner, 0)
+
+
 @pytest.mark.parametrize("experts", [6, 8, 12, 16])  # 3, 4, 6 and 8 pairs of tiles: their features on eight, two, four dies and on one
 @pytest.mark.parametrize("tiles", [1, 2, 3])
 def test_few_tiles_on_all_dies(experts, tiles):
