@@ -1405,22 +1405,24 @@ static bool half_rows_fill_better(int blocks16) { return 2 * blocks16 <= 256; }
 // outside its K loop and, per 64-wide step of K, `alone` us when it has its compute unit to itself
 // or `busy` us times the workgroups resident beside each other (operand fetch and matrix cores
 // do not overlap within a compute unit, so co-resident workgroups queue); steps are faster, by up to the share
-// `eased`, while only a part of the compute units has work (less traffic into L2, a higher clock).
+// `eased`, while only a part of the compute units has work (less traffic into L2, a higher clock), and by the share `empty` of
+// what the last tile of tokens has no rows for (its wavefronts without tokens read and multiply nothing).
 // Sums in float32, of slices of k or whole, cost their kernel `wide` us more a tile (twice the bytes, which leave in turns) and their
 // consumer, a norm that streams at 5.7 TB/s, 4 bytes per slice and element instead of 2.  A consumer that takes several slices gets
 // float32 from one, too: how many there are is a matter of speed and must not decide what the sums are rounded to before they are
-// added to the residual stream.  Constants fitted to 3,800 measured times of the
-// four products of a layer at five model sizes (hidden 896 to 5120) and 96 to 8,191 tokens, with weights that
-// rotate through more memory than the caches hold: rms error of the estimate 7 to 11 %, the chosen pair within
-// 1.1 % of the best one on average (3.0 % with the constants of the kernels before, whose tiles were stored
-// straight from the accumulators and whose square tile had sixteen wavefronts in step).  For float32 sums with their norm, 158 products of
-// six model sizes: the chosen pair within 0.4 % of the best on average, 14 % at worst (5,120 x 5,120 at 1,048 tokens).
+// added to the residual stream.  Constants fitted to 5,700 measured times (weights that rotate through more memory than the caches
+// hold) of the products of a layer at six model sizes (hidden 896 to 5120), 65 to 8,191 tokens, around the edges of tiles too, those
+// for the residual stream with the norm behind them.  What is fitted is the choice: of 815 products the chosen pair is 0.4 % off the best
+// on average and 15 % at worst, 21 are off by more than 5 %.  (Without `empty`, and with the few-token tiles only where the 64 x 64 ones
+// were chosen, it was 1.1 %, 64 by more than 5 %: 7B gate-up at 257 to 384 tokens 136 to 140 us in tiles of 128 x 128, 108 to 113 in
+// one round of 256 x 320; 1.5B gate-up at 65 to 128 tokens 22 to 24, 20 to 22 in tiles of 64 x 160.  Fitted to three quarters of
+// the matrices, the choice for the others is 0.7 to 1.0 % off.)
 struct GemmPlan {
   int kernel, slices;
 };
 struct TilingCost {
   int kernel, tile_tokens, tile_features, resident;
-  float alone, busy, fixed, eased, wide;
+  float alone, busy, fixed, eased, wide, empty;
 };
 // The narrower tiles of 256 tokens (gemm_direct; a step of k costs 7.2 ns per feature of the tile at 256
 // features, 7.6 at 192, 8.4 at 160) are there for products whose 256 x 256 tiles leave compute units
@@ -1434,14 +1436,21 @@ struct TilingCost {
 // two: 0.5B gate-up (248 tiles) 53 to 49 us, 7B gate-up at 512 tokens 168 to 135, 7B query/key/value at
 // 4,096 tokens 159 to 134, 32B down at 4,096 tokens 1,084 to 938; level or behind where the square
 // tiles already go round (7B gate-up at 2,048 tokens 533 against 517 on weights from memory).
-constexpr TilingCost kTilingCosts[] = {{11, 64, 64, 8, 0.314f, 0.226f, 4.6f, 0.9f, 1.3f},
-                                       {23, 128, 128, 2, 0.634f, 0.535f, 3.3f, 0.9f, 3.7f},
-                                       {23, 128, 128, 1, 0.424f, 0.559f, 4.943f, 0.275f, 3.f},  // where takes_turns
-                                       {45, 256, 256, 1, 1.024f, 1.655f, 7.8f, 0.421f, 5.7f},
-                                       {46, 256, 192, 1, 0.803f, 1.428f, 5.4f, 0.37f, 4.5f},
-                                       {47, 256, 160, 1, 0.804f, 1.3f, 5.4f, 0.305f, 3.6f},
-                                       {48, 256, 320, 1, 1.38f, 2.115f, 12.f, 0.289f, 1.2f}};
+constexpr TilingCost kTilingCosts[] = {{11, 64, 64, 8, 0.277f, 0.243f, 6.08f, 0.64f, 1.63f, 0.1f},
+                                       {23, 128, 128, 2, 0.641f, 0.528f, 4.52f, 0.91f, 6.52f, 0.05f},
+                                       {23, 128, 128, 1, 0.332f, 0.566f, 5.65f, 0.f, 4.11f, 0.03f},  // where takes_turns
+                                       {45, 256, 256, 1, 1.225f, 1.576f, 9.07f, 0.59f, 9.34f, 0.12f},
+                                       {46, 256, 192, 1, 1.226f, 1.453f, 5.5f, 0.45f, 6.9f, 0.13f},
+                                       {47, 256, 160, 1, 0.85f, 1.327f, 5.45f, 0.34f, 8.51f, 0.01f},
+                                       {48, 256, 320, 1, 1.419f, 2.21f, 9.82f, 0.22f, 13.99f, 0.32f}};
 constexpr int kComputeUnits = 256;
+// Up to 256 tokens of a matrix of 16 MB or more, tiles of 64 x 64 give way to the widths of choose_few_token_tiles (7B down at 128
+// tokens in 4 slices: 50.6 us staged, 41.8 in tiles of 128 features; 32B down at 192 tokens 131 and 106).  Not for small matrices: the
+// staged tiles, four workgroups to a compute unit, share the weights of neighbouring token tiles (1.5B query/key/value, 6 MB, at 192
+// tokens: 7.4 us against 9.1).  On the scale of this estimate theirs is 0.87 of what it says, and 4.1 us with the norm behind.
+constexpr float kFewTokenScale = 0.87f, kFewTokenNorm = 4.1f;
+static int choose_few_token_tiles(int m, int n, int k, int slices, float* estimate = nullptr);
+static bool few_token_tiles_pay(int m, int n, int k) { return m <= 256 && static_cast<int64_t>(n) * k * 2 >= (16ll << 20); }
 // 128 x 128 tiles: gemm_turns where a tile has its compute unit to itself and eight steps of k or more, gemm_direct elsewhere.  650
 // products cut into up to 4 slices, gemm_turns' time over gemm_direct's: up to 256 tiles, 24 steps or more 0.81 (0.58 to 0.91), 12 to 23
 // steps 0.93, 8 to 11 0.95 to 0.98, 4 to 7 1.01; more tiles 1.13 to 1.41: two workgroups of gemm_direct on a unit fill each other's waits
@@ -1455,13 +1464,14 @@ static float tiled_time_us(const TilingCost& c, int m, int n, int k, int slices,
   const int64_t tiles = static_cast<int64_t>((m + c.tile_tokens - 1) / c.tile_tokens) * ((n + c.tile_features - 1) / c.tile_features);
   const int64_t groups = tiles * slices;
   const int ksteps = (k + kBK - 1) / kBK;
-  const float per = static_cast<float>((ksteps + slices - 1) / slices);
   auto step = [&](int resident, float fill) {
     return fmaxf(c.alone, resident * c.busy * (1.f - c.eased + c.eased * fill));
   };
   const int64_t capacity = static_cast<int64_t>(kComputeUnits) * c.resident;
   const int64_t full = groups / capacity, rest = groups % capacity;
   const float fixed = c.fixed + (sums ? c.wide : 0.f);
+  const float rows = static_cast<float>((m + c.tile_tokens - 1) / c.tile_tokens) * c.tile_tokens;
+  const float per = static_cast<float>((ksteps + slices - 1) / slices) * (1.f - c.empty * (1.f - m / rows));
   float t = full * (fixed + per * step(c.resident, 1.f));
   if (rest > 0) {
     const int resident = static_cast<int>((rest + kComputeUnits - 1) / kComputeUnits);
@@ -1479,9 +1489,16 @@ static GemmPlan plan_many_tokens(int m, int n, int k, int max_slices, bool sums)
       if (slices > 1 && ksteps / slices < 3) break;  // every slice keeps a few steps (0.5B output
                                                      // projection at 128 tokens, 14 steps: whole 8.0 us, in 4 slices 5.4)
       if (c.kernel == 23 && (c.resident == 1) != takes_turns(m, n, k, slices)) continue;
-      float t = tiled_time_us(c, m, n, k, slices, sums);
+      int kernel = c.kernel;
+      float t = 0.f;
+      if (kernel == 11 && few_token_tiles_pay(m, n, k)) {
+        kernel = choose_few_token_tiles(m, n, k, slices, &t);
+        t = kFewTokenScale * t + (sums ? kFewTokenNorm : 0.f);
+      } else {
+        t = tiled_time_us(c, m, n, k, slices, sums);
+      }
       if (sums) t += 4.f * slices * m * n / 5.7e6f;
-      if (best_time == 0.f || t < best_time) best = {c.kernel, slices}, best_time = t;
+      if (best_time == 0.f || t < best_time) best = {kernel, slices}, best_time = t;
     }
   return best;
 }
@@ -1537,7 +1554,7 @@ static float few_token_time_us(const FewTokenTiling& t, int m, int n, int k, int
   if (rest > 0) time += tile_kb / fminf(unit, share * kComputeUnits / rest) + t.round_us;
   return time;
 }
-static int choose_few_token_tiles(int m, int n, int k, int slices) {
+static int choose_few_token_tiles(int m, int n, int k, int slices, float* estimate) {
   int best = 0;
   float best_time = 0.f;
   // narrow tiles first (at a tie the one that fills more units), the staged ones last and only when
@@ -1547,6 +1564,7 @@ static int choose_few_token_tiles(int m, int n, int k, int slices) {
     const float time = few_token_time_us(t, m, n, k, slices);
     if (best == 0 || time < (t.direct ? 0.99f : 0.97f) * best_time) best = t.kernel, best_time = time;
   }
+  if (estimate != nullptr) *estimate = best_time;
   return best;
 }
 
@@ -1556,13 +1574,8 @@ static int choose_kernel(int m, int n, int k, int slices, bool sums) {
   if (m <= 64 && small_matrix(n, k)) return 16;
   if (m <= 64) return choose_few_token_tiles(m, n, k, slices);
   const GemmPlan plan = plan_many_tokens(m, n, k, slices, sums);
-  const int kernel = plan.slices == slices ? plan.kernel : 11;
-  // up to 256 tokens in tiles of 64: the same choice of widths as for one tile of tokens (7B down at 128
-  // tokens in 4 slices: 50.6 us staged, 41.8 in tiles of 128 features; 32B down at 192 tokens 131 and
-  // 106).  Not for small matrices: the staged tiles, four workgroups to a compute unit, share the weights
-  // of neighbouring token tiles (1.5B query/key/value, 6 MB, at 192 tokens: 7.4 us against 9.1).
-  if (kernel == 11 && m <= 256 && static_cast<int64_t>(n) * k * 2 >= (16ll << 20)) return choose_few_token_tiles(m, n, k, slices);
-  return kernel;
+  if (plan.slices == slices) return plan.kernel;
+  return few_token_tiles_pay(m, n, k) ? choose_few_token_tiles(m, n, k, slices) : 11;  // more slices than the plan would make of it
 }
 
 static int gemm_bf16(const bf16* xb, const bf16* wb, const GemmEpilogue& ep, int m, int n, int k, int slices,
