@@ -95,3 +95,41 @@ def test_sums_for_the_stream_are_not_rounded(ops, m, n, k):
     want = stream.double() + got.double().sum(0)
     ops.rmsnorm(stream, weight, 1e-6, delta=got)
     assert ((stream.double() - want).abs() <= 2.0**-22 * (want.abs() + got.double().abs().sum(0))).all()
+
+
+# a token's factor in every part of a tile's rows; the last tile of 256 has rows for its first group of wavefronts only
+@pytest.mark.parametrize("kernel", [23, 24, 25, 45, 46, 47, 48])
+@pytest.mark.parametrize("m,n,k", [(130, 144, 72), (300, 272, 520)])
+@pytest.mark.parametrize("way", ["rounded", "sums", "stored", "slices", "swiglu"])
+def test_owed_norms(ops, kernel, m, n, k, way):
+    """Rows that owe their normalisation: float32 sums times the factor, one rounding more than the sums themselves."""
+    from mini_llm_runtime_amd.kernels.pending import PendingScale
+
+    x, w = _rand((m, k), torch.bfloat16, 85, 2.0).cuda(), _rand((n, k), torch.bfloat16, 86, 0.1).cuda()
+    sumsq = (torch.rand(m, 70, generator=torch.Generator().manual_seed(87)) * k * 3 / 70).cuda()
+    eps = 1e-6
+    owed = PendingScale(x, sumsq, torch.ones(k, dtype=torch.bfloat16).cuda(), eps, torch.zeros(m, k).cuda())
+    factor = torch.rsqrt(sumsq.double().sum(1, keepdim=True) / k + eps)
+    ref = factor * (x.double() @ w.double().t())
+    # k roundings of the products' sum, 70 of the squares' (of which the root halves), the factor's and the last product's own
+    bound = factor * (k * 2.0**-24 * (x.double().abs() @ w.double().abs().t())) + 40 * 2.0**-23 * ref.abs() + 1e-6
+    if way == "swiglu":  # its 32-bit results leave from the accumulators
+        got, want = (ops.linear(owed, w, swiglu=True, mfma_kernel=kernel, **kw) for kw in ({}, dict(out_dtype=torch.float32)))
+        assert torch.equal(got, want.to(torch.bfloat16))
+        pairs = ref.view(m, n // 4, 4)
+        gate, up = pairs[..., :2].reshape(m, n // 2), pairs[..., 2:].reshape(m, n // 2)
+        off = bound.view(m, n // 4, 4)
+        off_gate, off_up = off[..., :2].reshape(m, n // 2), off[..., 2:].reshape(m, n // 2)
+        # silu's slope is at most 1.1; its exponential and quotient are good to 2^-20
+        exact = torch.nn.functional.silu(gate) * up
+        assert ((want.double() - exact).abs() <= 1.1 * off_gate * (up.abs() + off_up) + gate.abs() * off_up + 2.0**-20 * exact.abs() + 1e-6).all()
+        return
+    kw = {"rounded": {}, "sums": dict(out_dtype=torch.float32), "slices": dict(partial_sums=True, slices=2),
+          "stored": dict(out_dtype=torch.float32, out=torch.empty(m * n + 1, dtype=torch.float32, device="cuda")[1:].view(m, n))}[way]
+    got = ops.linear(owed, w, mfma_kernel=kernel, **kw).double()
+    if way == "slices":
+        assert got.shape[0] == 2
+        got = got.sum(0)
+    if way == "rounded":
+        bound = bound + 2.0**-8 * (ref.abs() + bound)
+    assert ((got - ref).abs() <= bound).all()
