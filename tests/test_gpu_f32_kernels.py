@@ -6,6 +6,7 @@ import pytest
 import torch
 
 from test_gpu_kernels import _attend, _attention_reference, _paged_case, _rand
+from test_gpu_prompt_attention import give_back
 
 pytestmark = pytest.mark.gpu
 
@@ -124,3 +125,15 @@ def test_a_page_that_is_not_there_concerns_the_tokens_that_see_it(ops, mask, pag
     got, plain = _attend(ops, *args, **kw).cpu(), _attend(ops, *args, kernel="fma", **kw).cpu()
     assert torch.isfinite(plain[:32]).all() and torch.isnan(plain[40]).all() and torch.isfinite(plain[100:108]).all()
     torch.testing.assert_close(got, plain, atol=5e-6, rtol=1e-5, equal_nan=True)
+
+
+@pytest.mark.parametrize("head_dim,block", [(64, 16), (128, 32), (16, 4), (48, 12)])
+@pytest.mark.parametrize("mask", [dict(window=1), dict(window=17), dict(window=65), dict(window=None, chunk=48), dict(window=None, chunk=160)])
+def test_pages_that_were_given_back(ops, head_dim, block, mask):
+    entries = [(200, 70), (331, 5), (192, 130), (448, 64), (403, 140), (300, 1)]
+    q, kp, vp, table, ctx, *_ = _paged_case(entries, 2, 1, head_dim, block, torch.float32, 18)
+    kw = dict(num_heads=2, num_kv_heads=1, head_dim=head_dim, block_size=block, scale=head_dim**-0.5, **mask)
+    whole = _attend(ops, q.cuda(), kp.cuda(), vp.cuda(), table.cuda(), ctx, **kw).cpu()
+    left = give_back(entries, kp, vp, table, block, **mask)
+    got = _attend(ops, q.cuda(), *(t.cuda() for t in left), ctx, **kw).cpu()
+    assert torch.isfinite(whole).all() and torch.equal(got, whole)

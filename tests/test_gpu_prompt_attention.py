@@ -95,3 +95,32 @@ def test_a_page_that_is_not_there(ops):
     kw = dict(num_heads=2, num_kv_heads=1, head_dim=64, block_size=16, scale=0.125, window=None)
     got = _attend(ops, q.cuda(), kp.cuda(), vp.cuda(), table.cuda(), ctx, **kw).cpu()
     assert torch.isfinite(got[:228]).all() and torch.isnan(got[100 + 256 :]).all()
+
+
+def give_back(entries, kp, vp, table, block, window=None, chunk=None):
+    """The table and pages once every page wholly before the first visible key of a request's next token has been given back: its entry
+    is -1, and somebody else has written what has no value there."""
+    table, kp, vp = table.clone(), kp.clone(), vp.clone()
+    gone = 0
+    for r, (context, new) in enumerate(entries):
+        p = context - new
+        first = p // chunk * chunk if chunk else max(0, p - window + 1)
+        for page in range(first // block):
+            kp[table[r, page]] = vp[table[r, page]] = float("nan")
+            table[r, page] = -1
+            gone += 1
+    assert gone
+    return kp, vp, table
+
+
+# first visible keys at the start of a tile of 64 keys, at its end and inside, of a page and of 16 keys of a larger page
+@pytest.mark.parametrize("heads,kv_heads,head_dim,block", [(4, 2, 64, 16), (2, 1, 128, 16), (2, 2, 64, 64), (2, 1, 128, 32)])
+@pytest.mark.parametrize("mask", [dict(window=1), dict(window=17), dict(window=50), dict(window=65), dict(window=None, chunk=48), dict(window=None, chunk=160)])
+def test_pages_that_were_given_back(ops, heads, kv_heads, head_dim, block, mask):
+    entries = [(200, 70), (331, 5), (192, 130), (385, 129), (448, 64), (403, 140)]
+    q, kp, vp, table, ctx, *_ = _paged_case(entries, heads, kv_heads, head_dim, block, torch.bfloat16, 58)
+    kw = dict(num_heads=heads, num_kv_heads=kv_heads, head_dim=head_dim, block_size=block, scale=head_dim**-0.5, **mask)
+    whole = _attend(ops, q.cuda(), kp.cuda(), vp.cuda(), table.cuda(), ctx, **kw).cpu()
+    left = give_back(entries, kp, vp, table, block, **mask)
+    got = _attend(ops, q.cuda(), *(t.cuda() for t in left), ctx, **kw).cpu()
+    assert torch.isfinite(whole).all() and torch.equal(got, whole)
