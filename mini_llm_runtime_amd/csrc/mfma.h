@@ -33,7 +33,7 @@ __device__ __forceinline__ bf16x8_t zero_bf16x8() {
 // Buffer resource over `bytes` bytes at p: loads through it return zero beyond the end, so
 // tiles at the edge of a matrix need no branches.  Offsets are unsigned 32-bit byte counts.
 typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
-constexpr unsigned kOutOfBuffer = 0x80000000u;  // larger than any resource made here
+constexpr unsigned kOutOfBuffer = 0x80000000u;  // past the end of any resource of up to 2 GB (moe.hip has a mark of its own for larger ones)
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_buffer(const void* p, unsigned bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, static_cast<int>(bytes), 0x00020000);
 }

@@ -1046,8 +1046,14 @@ class HipOps:
         batch (StepContext).  bfloat16 with a head size in steps of 16 and a block
         size that is a multiple of 4 runs on the matrix cores: single-token entries
         through the split-KV decode kernel, the others through the tiled prefill
-        kernel.  Everything else (float32, other sizes, kernel="fma") runs the plain
-        32-bit kernel.
+        kernel.  float32 at the default head sizes up to 128, where block size and row stride are multiples
+        of 4, operands start at 16 bytes and the mask is causal, a window or a chunked one (no cap, pooled
+        entries, score bias or kept first tokens): entries of several tokens run in tiles of 64 queries on
+        the matrix cores, in float32.  Everything else (other sizes and masks, single tokens in float32,
+        kernel="fma") runs the plain 32-bit kernel.
+
+        A visible page that is not there makes NaN: in float32 of the rows of the tokens that see it, in
+        bfloat16 of all rows of a tile of queries of which one sees it.
         """
         self._check(qkv, "queries", self.dtype, (None, None))
         tokens, stride = qkv.shape
