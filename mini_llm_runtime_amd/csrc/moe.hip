@@ -9,6 +9,8 @@
 // inside an expert's run is whatever the atomics made it; every output row is computed from its own
 // input row alone, with the sums over k in a fixed order, so no value depends on that order or on
 // what else is in the batch.
+#include <cmath>
+
 #include "api.h"
 #include "common.h"
 #include "mfma.h"
@@ -686,7 +688,7 @@ __global__ __launch_bounds__(256) void moe_gemm_stream_kernel(const bf16* __rest
 // quarter of a slice's products is kept for behind the barrier, where the next slice's first operands are on their way.  Finished
 // tiles leave through LDS in whole lines: the down product's rows go to as many places as it has rows, 512 bytes each.
 // Workgroup -> (tile, features): workgroups go to the eight dies in turn; a pair of neighbouring tiles (mostly one expert's) belongs to one
-// die, or its features to `spread` of them where there are too few pairs for all (dies_of_a_pair); a die takes their features one after the
+// die, or its features to `spread` of them where there are too few pairs for all (order_tiles); a die takes their features one after the
 // other, both tiles at a time, so that the rows and the expert's weights come from its L2.
 // Bound by the operands' way through L2 and LDS (each 64 x RB + 128 rows of a slice make 64 RB x 128 products of it) and by tiles
 // that are not full: 2,000 tokens, 64 experts with 6 choices (187 rows an expert in tiles of 128), 768 x 2,048: up 94.5 to 91.4 us,
@@ -694,12 +696,24 @@ __global__ __launch_bounds__(256) void moe_gemm_stream_kernel(const bf16* __rest
 struct TilePlace {
   int tile, column;  // column -1: none
 };
-__device__ __forceinline__ TilePlace place_tile(int columns, int spread) {
-  const int each = (columns + spread - 1) / spread;  // of a die
-  const int local = blockIdx.x / 8, in_unit = local % (2 * each);
-  const int unit = local / (2 * each) * 8 + blockIdx.x % 8;
+struct PairOrder {
+  int spread;  // dies that share one of the first pairs
+  int first;   // how many those are: their runs of features are dealt out to the dies in whole rounds; every later pair belongs to all dies
+};
+__host__ __device__ inline int features_of_a_die(int columns, int spread) { return (columns + spread - 1) / spread; }
+__device__ __forceinline__ TilePlace place_tile(int columns, PairOrder order) {
+  int block = blockIdx.x, spread = order.spread, each = features_of_a_die(columns, spread), pair0 = 0;
+  const int firsts = order.first * spread * 2 * each;
+  if (block >= firsts) {
+    block -= firsts;
+    pair0 = order.first;
+    spread = 8;
+    each = features_of_a_die(columns, spread);
+  }
+  const int local = block / 8, in_unit = local % (2 * each);
+  const int unit = local / (2 * each) * 8 + block % 8;
   const int column = unit % spread * each + in_unit / 2;
-  return {unit / spread * 2 + in_unit % 2, column < columns ? column : -1};
+  return {(pair0 + unit / spread) * 2 + in_unit % 2, column < columns ? column : -1};
 }
 constexpr int kBigCols = 128;
 constexpr int kBigK = 64;
@@ -727,7 +741,7 @@ template <bool UP, int RB>
 __global__ __launch_bounds__(256) void moe_gemm_tiled_kernel(const bf16* __restrict__ a, const bf16* __restrict__ w,
                                                              const int* __restrict__ sorted,
                                                              const int* __restrict__ offsets,
-                                                             const int* __restrict__ tiles, int max_tiles, int spread,
+                                                             const int* __restrict__ tiles, int max_tiles, PairOrder order,
                                                              const float* __restrict__ pair_weights,
                                                              void* __restrict__ out, int tokens, int top, int N, int K,
                                                              int act, int a_rows, float glu_limit, float glu_alpha) {
@@ -736,7 +750,7 @@ __global__ __launch_bounds__(256) void moe_gemm_tiled_kernel(const bf16* __restr
   // runs of 8 rows, dealt out to four wavefronts: 4 of weights, then the input's (loops over them go to 8 and break: with a bound that
   // depends on the template's parameters the host pass left the kernel uninstantiated, without a message)
   constexpr int kLoads = (kBigCols + kRows) / 8 / 4;
-  const TilePlace place = place_tile((N + kBigCols - 1) / kBigCols, spread);
+  const TilePlace place = place_tile((N + kBigCols - 1) / kBigCols, order);
   const int tile = place.tile;
   if (tile >= max_tiles || place.column < 0) return;
   const int expert = tiles[2 * tile];
@@ -913,13 +927,13 @@ static_assert(kSqLds >= 2 * kSqBuffer && kSqLds >= kSqRows / 2 * kSqRowF32, "two
 template <bool UP>
 __global__ __launch_bounds__(512, 2) void moe_gemm_phased_kernel(const bf16* __restrict__ a, const bf16* __restrict__ w,
                                                                 const int* __restrict__ sorted, const int* __restrict__ offsets,
-                                                                const int* __restrict__ tiles, int max_tiles, int spread,
+                                                                const int* __restrict__ tiles, int max_tiles, PairOrder order,
                                                                 const float* __restrict__ pair_weights, void* __restrict__ out,
                                                                 int tokens, int top, int N, int K, int act, int a_rows,
                                                                 float glu_limit, float glu_alpha) {
   extern __shared__ __attribute__((aligned(16))) unsigned char moe_lds[];
   __shared__ int pair_of[kSqRows];
-  const TilePlace place = place_tile((N + kSqCols - 1) / kSqCols, spread);
+  const TilePlace place = place_tile((N + kSqCols - 1) / kSqCols, order);
   const int tile = place.tile;
   if (tile >= max_tiles || place.column < 0) return;
   const int expert = tiles[2 * tile];
@@ -1124,24 +1138,30 @@ __global__ __launch_bounds__(512, 2) void moe_gemm_phased_kernel(const bf16* __r
   }
 }
 
-using MoeTiledKernel = void (*)(const bf16*, const bf16*, const int*, const int*, const int*, int, int, const float*, void*, int, int, int, int,
+using MoeTiledKernel = void (*)(const bf16*, const bf16*, const int*, const int*, const int*, int, PairOrder, const float*, void*, int, int, int, int,
                                 int, int, float, float);
 struct MoeTiles {
   MoeTiledKernel kernel;
   int threads, rows, cols, lds;
 };
 // How many dies share a pair of tiles: as few as leave none without work and none with more than 1.15 times its share, by the number of tiles
-// that experts with equal shares of the pairs would have (the host does not know the routing).  Fewer dies read a pair's rows fewer times.
+// that experts chosen at random would have (the host does not know the routing).  Fewer dies read a pair's rows fewer times.
 // With one die for each pair / as chosen here, both products with their gating, microseconds: 8 experts of 14,336 x 4,096 (4 pairs on 8 dies): 48
 // rows an expert 786 / 617, 97 900 / 692; 12 of 8,192 x 5,120: 97 798 / 646, 320 1,521 / 1,296; 64 of 768 x 2,048 (32 pairs and more: one
 // die) the same, where eight dies take 1.1 to 1.4 times as long.
-static int dies_of_a_pair(int max_tiles, int64_t pairs, int rows) {
+// The features of what lies beyond these whole rounds of dies go to all of them: with a pair of tiles more on one die, that die had a round of
+// its own (both products: 32 experts of 2,880 x 2,880 at 50 rows an expert, 33 tiles of 64, 280 us so and 250 as here; 16 of 6,400 x 4,096 at
+// 64 rows 503 and 401; 8 of 14,336 x 4,096 at 500 rows 1,278 and 1,136).
+static PairOrder order_tiles(int max_tiles, int64_t pairs, int rows) {
   const int64_t experts = max_tiles - pairs / rows > 1 ? max_tiles - pairs / rows : 1;
-  const int64_t tiles = experts * ((pairs + experts * rows - 1) / (experts * rows));
-  const int64_t tile_pairs = (tiles + 1) / 2;
-  for (int spread = 1; spread < 8; spread *= 2)
-    if ((tile_pairs * spread + 7) / 8 * 8 * 100 <= tile_pairs * spread * 115) return spread;
-  return 8;
+  const double mean = static_cast<double>(pairs) / static_cast<double>(experts);
+  double each = 1.0;  // and a tile more for every `rows` that an expert's share exceeds: a normal distribution of variance `mean`
+  for (double full = rows; full < mean + 4.0 * std::sqrt(mean); full += rows) each += 0.5 * std::erfc((full - mean) / std::sqrt(2.0 * mean));
+  const double tiles = std::fmin(each * static_cast<double>(experts), max_tiles);
+  const int tile_pairs = static_cast<int>((tiles + 1.0) / 2.0);
+  int spread = 1;
+  while (spread < 8 && static_cast<int64_t>(tile_pairs * spread + 7) / 8 * 8 * 100 > static_cast<int64_t>(tile_pairs) * spread * 115) spread *= 2;
+  return {spread, tile_pairs * spread / 8 * 8 / spread};
 }
 // Steps of 64 in moe_gemm_stream: where there are more pairs than experts, of matrices of 64 MB or more eight times as many.  Steps of 128 / 64, both
 // products, microseconds: 64 experts of 768 x 2,048 with 6 choices: 2 tokens 25 / 26, 8 51 / 55, 13 69 / 64, 32 79 / 77, 64 87 / 80; 128 of it
@@ -1163,16 +1183,16 @@ static int launch_moe_tiled(const MoeTiles& t, bool& configured, const bf16* a, 
     }
     configured = true;
   }
-  const int64_t columns = (n + t.cols - 1) / t.cols;
-  const int spread = dies_of_a_pair(max_tiles, static_cast<int64_t>(tokens) * top, t.rows);
-  const int64_t units = (static_cast<int64_t>((max_tiles + 1) / 2) * spread + 7) / 8 * 8;
-  const int64_t groups = units * 2 * ((columns + spread - 1) / spread);
+  const int columns = (n + t.cols - 1) / t.cols;
+  const PairOrder order = order_tiles(max_tiles, static_cast<int64_t>(tokens) * top, t.rows);
+  const int64_t groups = static_cast<int64_t>(order.first) * order.spread * 2 * features_of_a_die(columns, order.spread) +
+                         static_cast<int64_t>(max((max_tiles + 1) / 2 - order.first, 0)) * 8 * 2 * features_of_a_die(columns, 8);
   if (groups >= (1ll << 31)) {
     set_error("mlr_moe_gemm: too many tiles for one launch");
     return -1;
   }
   hipLaunchKernelGGL(t.kernel, dim3(static_cast<unsigned>(groups)), dim3(t.threads), t.lds, stream, a, w, sorted, offsets, tiles, max_tiles,
-                     spread, pair_weights, out, tokens, top, n, k, act, a_rows, glu_limit, glu_alpha);
+                     order, pair_weights, out, tokens, top, n, k, act, a_rows, glu_limit, glu_alpha);
   return 0;
 }
 

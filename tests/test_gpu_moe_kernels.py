@@ -119,6 +119,14 @@ def test_few_tiles_on_all_dies(experts, tiles):
     test_grouped_products((20,) * experts, 1160, 1032, tiles)  # 10 and 9 runs of 128 features, 5 of 256: not the same number for every die
 
 
+# experts of more rows than others make a tile or two more than whole rounds of dies hold: their features go to all dies
+@pytest.mark.parametrize("more", [1, 2])
+@pytest.mark.parametrize("tiles", [1, 2, 3])
+def test_more_tiles_than_equal_shares_make(more, tiles):
+    full = (0, 64, 128, 256)[tiles]
+    test_grouped_products((full + 9,) * more + (full // 2,) * (16 - more), 1160, 264, tiles)
+
+
 @pytest.mark.parametrize("inner", [4, 12, 72])  # 8, 24 and 144 woven rows: results of 8, 24 and 144 bytes (the second is stored directly)
 @pytest.mark.parametrize("tiles", [1, 2, 3])
 def test_gated_products_of_woven_rows(inner, tiles):
