@@ -1376,9 +1376,10 @@ static bool few_tokens_tiled(int n, int slices) { return ((n + 63) / 64) * slice
 
 // Up to 16 tokens through gemm_lines: features a workgroup (16 x blocks) and, where the consumer adds up partial sums, slices of k.  A
 // product is done when the busiest compute unit has taken in its share, the tokens' rows of every workgroup included; a unit holds two
-// workgroups of 16 or 32 features or one of 48 or 64, and starts the next when one is done.  Estimates (us) that order 14 products of 8 and 16
-// tokens, 896 x 896 to 4,608 x 3,584, as they measured: 44 KB/us a unit (as for the few-token tiles below), 3 for the launch and the first
-// bytes, 1 or, with nobody beside it, 2.5 for every further round, 0.1 in the norm kernel for every slice that it adds.
+// workgroups of 16 or 32 features or one of 48 or 64, and starts the next when one is done.  Estimates (us): 44 KB/us a unit (as for the
+// few-token tiles below), 3 for the launch and the first bytes, 1 or, with nobody beside it, 2.5 for every further round, 0.1 in the norm
+// kernel for every slice that it adds.  83 products of 1 to 16 tokens that run here (1.5 to 49 MB of weights, those cut along k with the norm
+// behind them): the choice is 0.6 % off the best on average, 14 % at worst (2,048 x 11,008 at one token, 2 slices 15.0 us, 4 13.2).
 struct LinesPlan {
   int blocks, slices;
   float us;
@@ -1569,7 +1570,9 @@ static int choose_few_token_tiles(int m, int n, int k, int slices, float* estima
 }
 
 static int choose_kernel(int m, int n, int k, int slices, bool sums) {
-  // (2,048 x 4,096 in 8 slices at 8 tokens, 17 MB: 7.4 us in tiles, 6.5 here; 3,584 x 3,584, 26 MB: 8.7 and 10.4)
+  // 16 tokens: gemm_lines below 20 MB (2,048 x 4,096 in 8 slices at 8 tokens, 17 MB: 7.4 us in tiles, 6.5 here).  Of 29 products beyond
+  // that line gemm_lines would be ahead of the tiles, too, at 8 tokens: 14,336 x 768 (21 MB) 9.8 us in tiles, 7.0 there; 3,584 x 3,584
+  // with its norm (25 MB) 12.4 and 10.7; 17,920 x 1,536 (53 MB) 14.5 and 13.6; 22,016 x 2,048 (86 MB) 22.7 and 19.9; 5,120 x 5,120 17.5 and 16.4.
   if (m <= 16 && (!few_tokens_tiled(n, slices) || static_cast<int64_t>(n) * k * 2 < (20ll << 20))) return 16;
   if (m <= 64 && small_matrix(n, k)) return 16;
   if (m <= 64) return choose_few_token_tiles(m, n, k, slices);
