@@ -359,7 +359,7 @@ int mlr_moe_identity(const void* h, const int* ids, const float* weights, float*
                      int hidden, int first, hipStream_t stream);
 // The (token, choice) pairs p = token * top + choice sorted by expert: sorted [pairs], offsets
 // [experts + 1], tiles [max_tiles, 2] = (expert, first row of `sorted`) with up to
-// mlr_moe_tile_rows(big) rows each (16, or with `big` 1 to 3 64, 128 or 256), unused tiles (-1, 0).  max_tiles >=
+// mlr_moe_tile_rows(big) rows each (16, or with `big` 1 to 3 64, 128 or 256), unused tiles (-1, the number of used ones).  max_tiles >=
 // mlr_moe_max_tiles(pairs, experts, big).
 int mlr_moe_tile_rows(int big);
 int mlr_moe_max_tiles(int pairs, int experts, int big);

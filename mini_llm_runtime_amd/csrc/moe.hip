@@ -9,8 +9,6 @@
 // inside an expert's run is whatever the atomics made it; every output row is computed from its own
 // input row alone, with the sums over k in a fixed order, so no value depends on that order or on
 // what else is in the batch.
-#include <cmath>
-
 #include "api.h"
 #include "common.h"
 #include "mfma.h"
@@ -345,7 +343,7 @@ __global__ __launch_bounds__(1024) void moe_align_kernel(const int* __restrict__
   __syncthreads();
   for (int i = used_tiles + tid; i < max_tiles; i += blockDim.x) {
     tiles[2 * i] = -1;  // a workgroup that finds this has nothing to do
-    tiles[2 * i + 1] = 0;
+    tiles[2 * i + 1] = used_tiles;
   }
   for (int e = tid; e < experts; e += blockDim.x) counts[e] = 0;
   __syncthreads();
@@ -688,7 +686,7 @@ __global__ __launch_bounds__(256) void moe_gemm_stream_kernel(const bf16* __rest
 // quarter of a slice's products is kept for behind the barrier, where the next slice's first operands are on their way.  Finished
 // tiles leave through LDS in whole lines: the down product's rows go to as many places as it has rows, 512 bytes each.
 // Workgroup -> (tile, features): workgroups go to the eight dies in turn; a pair of neighbouring tiles (mostly one expert's) belongs to one
-// die, or its features to `spread` of them where there are too few pairs for all (order_tiles); a die takes their features one after the
+// die, or its features to a few of them where that would leave dies without work (order_tiles); a die takes their features one after the
 // other, both tiles at a time, so that the rows and the expert's weights come from its L2.
 // Bound by the operands' way through L2 and LDS (each 64 x RB + 128 rows of a slice make 64 RB x 128 products of it) and by tiles
 // that are not full: 2,000 tokens, 64 experts with 6 choices (187 rows an expert in tiles of 128), 768 x 2,048: up 94.5 to 91.4 us,
@@ -696,24 +694,44 @@ __global__ __launch_bounds__(256) void moe_gemm_stream_kernel(const bf16* __rest
 struct TilePlace {
   int tile, column;  // column -1: none
 };
+// How the pairs of `used` tiles go to the dies: all of them one by one where that leaves no die with more than 1.15 times its share; else the
+// whole rounds of eight, and the features of each pair of the rest to as many dies as make whole rounds of them, too.
+// With one die for each pair / as here, both products with their gating, microseconds: 8 experts of 14,336 x 4,096 (4 pairs on 8 dies): 48 rows an
+// expert 786 / 617, 97 900 / 692; 12 of 8,192 x 5,120: 97 798 / 646, 320 1,521 / 1,296; 32 of 2,880 x 2,880: 50 (33 tiles of 64) 280 / 251; 16 of
+// 6,400 x 4,096: 64 503 / 409; 64 of 768 x 2,048, some four times as popular as others: 187 184 / 174.  Fewer dies read a pair's rows fewer
+// times: that last one takes 204 where every pair beyond those of equal shares goes to all dies.  To look up how many tiles are used costs 0.5 us.
 struct PairOrder {
-  int spread;  // dies that share one of the first pairs
-  int first;   // how many those are: their runs of features are dealt out to the dies in whole rounds; every later pair belongs to all dies
+  int first;   // pairs that have a die to themselves
+  int spread;  // dies that share each of the others
 };
+__host__ __device__ inline PairOrder order_tiles(int used) {
+  const int pairs = (used + 1) / 2, whole = (pairs + 7) / 8 * 8, rest = pairs % 8;
+  if (whole * 100 <= pairs * 115) return {whole, 8};
+  return {pairs / 8 * 8, 8 >> __builtin_ctz(rest)};
+}
 __host__ __device__ inline int features_of_a_die(int columns, int spread) { return (columns + spread - 1) / spread; }
-__device__ __forceinline__ TilePlace place_tile(int columns, PairOrder order) {
-  int block = blockIdx.x, spread = order.spread, each = features_of_a_die(columns, spread), pair0 = 0;
-  const int firsts = order.first * spread * 2 * each;
-  if (block >= firsts) {
-    block -= firsts;
-    pair0 = order.first;
-    spread = 8;
-    each = features_of_a_die(columns, spread);
-  }
+__device__ __forceinline__ TilePlace place_tile(const int* __restrict__ tiles, int max_tiles, int columns) {
+  // an unused tile names how many are used
+  const PairOrder order = order_tiles(tiles[2 * max_tiles - 2] < 0 ? tiles[2 * max_tiles - 1] : max_tiles);
+  const int firsts = order.first * 2 * columns;
+  const bool shared = static_cast<int>(blockIdx.x) >= firsts;
+  const int block = shared ? blockIdx.x - firsts : blockIdx.x, spread = shared ? order.spread : 1, pair0 = shared ? order.first : 0;
+  const int each = features_of_a_die(columns, spread);
   const int local = block / 8, in_unit = local % (2 * each);
   const int unit = local / (2 * each) * 8 + block % 8;
   const int column = unit % spread * each + in_unit / 2;
   return {(pair0 + unit / spread) * 2 + in_unit % 2, column < columns ? column : -1};
+}
+// Workgroups that cover every number of used tiles.
+static int64_t groups_of_tiles(int max_tiles, int columns) {
+  int64_t most = 0;
+  for (int used = max(1, max_tiles - 32); used <= max_tiles; ++used) {
+    const PairOrder order = order_tiles(used);
+    const int rest = max((used + 1) / 2 - order.first, 0);
+    const int64_t groups = static_cast<int64_t>(order.first) * 2 * columns + static_cast<int64_t>(rest) * order.spread * 2 * features_of_a_die(columns, order.spread);
+    most = groups > most ? groups : most;
+  }
+  return most;
 }
 constexpr int kBigCols = 128;
 constexpr int kBigK = 64;
@@ -741,7 +759,7 @@ template <bool UP, int RB>
 __global__ __launch_bounds__(256) void moe_gemm_tiled_kernel(const bf16* __restrict__ a, const bf16* __restrict__ w,
                                                              const int* __restrict__ sorted,
                                                              const int* __restrict__ offsets,
-                                                             const int* __restrict__ tiles, int max_tiles, PairOrder order,
+                                                             const int* __restrict__ tiles, int max_tiles,
                                                              const float* __restrict__ pair_weights,
                                                              void* __restrict__ out, int tokens, int top, int N, int K,
                                                              int act, int a_rows, float glu_limit, float glu_alpha) {
@@ -750,7 +768,7 @@ __global__ __launch_bounds__(256) void moe_gemm_tiled_kernel(const bf16* __restr
   // runs of 8 rows, dealt out to four wavefronts: 4 of weights, then the input's (loops over them go to 8 and break: with a bound that
   // depends on the template's parameters the host pass left the kernel uninstantiated, without a message)
   constexpr int kLoads = (kBigCols + kRows) / 8 / 4;
-  const TilePlace place = place_tile((N + kBigCols - 1) / kBigCols, order);
+  const TilePlace place = place_tile(tiles, max_tiles, (N + kBigCols - 1) / kBigCols);
   const int tile = place.tile;
   if (tile >= max_tiles || place.column < 0) return;
   const int expert = tiles[2 * tile];
@@ -927,13 +945,13 @@ static_assert(kSqLds >= 2 * kSqBuffer && kSqLds >= kSqRows / 2 * kSqRowF32, "two
 template <bool UP>
 __global__ __launch_bounds__(512, 2) void moe_gemm_phased_kernel(const bf16* __restrict__ a, const bf16* __restrict__ w,
                                                                 const int* __restrict__ sorted, const int* __restrict__ offsets,
-                                                                const int* __restrict__ tiles, int max_tiles, PairOrder order,
+                                                                const int* __restrict__ tiles, int max_tiles,
                                                                 const float* __restrict__ pair_weights, void* __restrict__ out,
                                                                 int tokens, int top, int N, int K, int act, int a_rows,
                                                                 float glu_limit, float glu_alpha) {
   extern __shared__ __attribute__((aligned(16))) unsigned char moe_lds[];
   __shared__ int pair_of[kSqRows];
-  const TilePlace place = place_tile((N + kSqCols - 1) / kSqCols, order);
+  const TilePlace place = place_tile(tiles, max_tiles, (N + kSqCols - 1) / kSqCols);
   const int tile = place.tile;
   if (tile >= max_tiles || place.column < 0) return;
   const int expert = tiles[2 * tile];
@@ -1138,31 +1156,12 @@ __global__ __launch_bounds__(512, 2) void moe_gemm_phased_kernel(const bf16* __r
   }
 }
 
-using MoeTiledKernel = void (*)(const bf16*, const bf16*, const int*, const int*, const int*, int, PairOrder, const float*, void*, int, int, int, int,
+using MoeTiledKernel = void (*)(const bf16*, const bf16*, const int*, const int*, const int*, int, const float*, void*, int, int, int, int,
                                 int, int, float, float);
 struct MoeTiles {
   MoeTiledKernel kernel;
-  int threads, rows, cols, lds;
+  int threads, cols, lds;
 };
-// How many dies share a pair of tiles: as few as leave none without work and none with more than 1.15 times its share, by the number of tiles
-// that experts chosen at random would have (the host does not know the routing).  Fewer dies read a pair's rows fewer times.
-// With one die for each pair / as chosen here, both products with their gating, microseconds: 8 experts of 14,336 x 4,096 (4 pairs on 8 dies): 48
-// rows an expert 786 / 617, 97 900 / 692; 12 of 8,192 x 5,120: 97 798 / 646, 320 1,521 / 1,296; 64 of 768 x 2,048 (32 pairs and more: one
-// die) the same, where eight dies take 1.1 to 1.4 times as long.
-// The features of what lies beyond these whole rounds of dies go to all of them: with a pair of tiles more on one die, that die had a round of
-// its own (both products: 32 experts of 2,880 x 2,880 at 50 rows an expert, 33 tiles of 64, 280 us so and 250 as here; 16 of 6,400 x 4,096 at
-// 64 rows 503 and 401; 8 of 14,336 x 4,096 at 500 rows 1,278 and 1,136).
-static PairOrder order_tiles(int max_tiles, int64_t pairs, int rows) {
-  const int64_t experts = max_tiles - pairs / rows > 1 ? max_tiles - pairs / rows : 1;
-  const double mean = static_cast<double>(pairs) / static_cast<double>(experts);
-  double each = 1.0;  // and a tile more for every `rows` that an expert's share exceeds: a normal distribution of variance `mean`
-  for (double full = rows; full < mean + 4.0 * std::sqrt(mean); full += rows) each += 0.5 * std::erfc((full - mean) / std::sqrt(2.0 * mean));
-  const double tiles = std::fmin(each * static_cast<double>(experts), max_tiles);
-  const int tile_pairs = static_cast<int>((tiles + 1.0) / 2.0);
-  int spread = 1;
-  while (spread < 8 && static_cast<int64_t>(tile_pairs * spread + 7) / 8 * 8 * 100 > static_cast<int64_t>(tile_pairs) * spread * 115) spread *= 2;
-  return {spread, tile_pairs * spread / 8 * 8 / spread};
-}
 // Steps of 64 in moe_gemm_stream: where there are more pairs than experts, of matrices of 64 MB or more eight times as many.  Steps of 128 / 64, both
 // products, microseconds: 64 experts of 768 x 2,048 with 6 choices: 2 tokens 25 / 26, 8 51 / 55, 13 69 / 64, 32 79 / 77, 64 87 / 80; 128 of it
 // with 8: 2 26 / 28, 6 59 / 61, 16 98 / 93, 64 146 / 141; 32 of 2,880 x 2,880 with 4: 1 32 / 35, 8 130 / 125, 48 170 / 169; 16 of 6,400 x
@@ -1183,16 +1182,13 @@ static int launch_moe_tiled(const MoeTiles& t, bool& configured, const bf16* a, 
     }
     configured = true;
   }
-  const int columns = (n + t.cols - 1) / t.cols;
-  const PairOrder order = order_tiles(max_tiles, static_cast<int64_t>(tokens) * top, t.rows);
-  const int64_t groups = static_cast<int64_t>(order.first) * order.spread * 2 * features_of_a_die(columns, order.spread) +
-                         static_cast<int64_t>(max((max_tiles + 1) / 2 - order.first, 0)) * 8 * 2 * features_of_a_die(columns, 8);
+  const int64_t groups = groups_of_tiles(max_tiles, (n + t.cols - 1) / t.cols);
   if (groups >= (1ll << 31)) {
     set_error("mlr_moe_gemm: too many tiles for one launch");
     return -1;
   }
   hipLaunchKernelGGL(t.kernel, dim3(static_cast<unsigned>(groups)), dim3(t.threads), t.lds, stream, a, w, sorted, offsets, tiles, max_tiles,
-                     order, pair_weights, out, tokens, top, n, k, act, a_rows, glu_limit, glu_alpha);
+                     pair_weights, out, tokens, top, n, k, act, a_rows, glu_limit, glu_alpha);
   return 0;
 }
 
@@ -1298,9 +1294,9 @@ int mlr_moe_gemm(const void* a, const void* w, const int* sorted, const int* off
     const int rows = static_cast<int>(a_rows);
     if (mfma >= 2) {
       static const MoeTiles kinds[3][2] = {
-          {{moe_gemm_tiled_kernel<false, 1>, 256, big_rows(1), kBigCols, big_lds_bytes(1)}, {moe_gemm_tiled_kernel<true, 1>, 256, big_rows(1), kBigCols, big_lds_bytes(1)}},
-          {{moe_gemm_tiled_kernel<false, 2>, 256, big_rows(2), kBigCols, big_lds_bytes(2)}, {moe_gemm_tiled_kernel<true, 2>, 256, big_rows(2), kBigCols, big_lds_bytes(2)}},
-          {{moe_gemm_phased_kernel<false>, 512, kSqRows, kSqCols, kSqLds}, {moe_gemm_phased_kernel<true>, 512, kSqRows, kSqCols, kSqLds}}};
+          {{moe_gemm_tiled_kernel<false, 1>, 256, kBigCols, big_lds_bytes(1)}, {moe_gemm_tiled_kernel<true, 1>, 256, kBigCols, big_lds_bytes(1)}},
+          {{moe_gemm_tiled_kernel<false, 2>, 256, kBigCols, big_lds_bytes(2)}, {moe_gemm_tiled_kernel<true, 2>, 256, kBigCols, big_lds_bytes(2)}},
+          {{moe_gemm_phased_kernel<false>, 512, kSqCols, kSqLds}, {moe_gemm_phased_kernel<true>, 512, kSqCols, kSqLds}}};
       static bool configured[3][2] = {};
       const int status = launch_moe_tiled(kinds[mfma - 2][up != 0], configured[mfma - 2][up != 0], ab, wb, sorted, offsets, tiles, pair_weights,
                                           out, max_tiles, tokens, top, n, k, act, rows, glu_limit, glu_alpha, stream);
