@@ -244,41 +244,40 @@ __host__ __device__ inline bool stages_tile(const GemmEpilogue& ep, int slices, 
 // LDS that staging a tile takes: rows of `features` results, padded by 16 bytes so that neighbouring rows fall on other banks.
 constexpr int staged_tile_bytes(int tokens, int features) { return tokens * (features * 2 + 16); }
 
-// KIND: kEpNone, kEpSwiglu or kEpGeglu.  acc[i][j]: block i of 32 features, block j of 32 tokens of this wavefront, which starts at feature
-// `feature0` and token `token0` of the tile; lane column r32, half h.  All THREADS of the workgroup, behind a barrier.
+// KIND: kEpNone, kEpSwiglu or kEpGeglu.  acc[i][j]: block i of 16 features, block j of 16 tokens of this wavefront, which starts at feature
+// `feature0` and token `token0` of the tile.  All THREADS of the workgroup, behind a barrier.
 template <int KIND, int THREADS, int BM, int BN, int NI, int NJ>
-__device__ __forceinline__ void stage_tile(const GemmEpilogue& ep, const f32x16_t (&acc)[NI][NJ], unsigned char* lds, const float* scales,
-                                           int feature0, int token0, int r32, int h, int m0, int n0, int M, int N) {
+__device__ __forceinline__ void stage_tile(const GemmEpilogue& ep, const f32x4_t (&acc)[NI][NJ], unsigned char* lds, const float* scales,
+                                           int feature0, int token0, int m0, int n0, int M, int N) {
   constexpr bool kPaired = KIND == kEpSwiglu || KIND == kEpGeglu;
   constexpr int kOut = kPaired ? BN / 2 : BN;
   constexpr int kRow = kOut * 2 + 16;
+  const int c16 = threadIdx.x % 16, quad = threadIdx.x % kWave / 16;
 #pragma unroll
-  for (int i = 0; i < NI; ++i)
+  for (int i = 0; i < NI; ++i) {
+    const int f = feature0 + i * 16 + quad * 4;
+    float b[4] = {0.f, 0.f, 0.f, 0.f};
+    if (KIND != kEpSwiglu && ep.bias != nullptr && n0 + f < N) {  // n0 + f + 3 < N too: both are multiples of 4
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int f = feature0 + i * 32 + g * 8 + h * 4;
-      float b[4] = {0.f, 0.f, 0.f, 0.f};
-      if (KIND != kEpSwiglu && ep.bias != nullptr && n0 + f < N) {  // n0 + f + 3 < N too: both are multiples of 4
+      for (int e = 0; e < 4; ++e) b[e] = load_as_f32(ep.bias, n0 + f + e, ep.bias_is_f32);
+    }
 #pragma unroll
-        for (int e = 0; e < 4; ++e) b[e] = load_as_f32(ep.bias, n0 + f + e, ep.bias_is_f32);
-      }
+    for (int j = 0; j < NJ; ++j) {
+      const int token = token0 + j * 16 + c16;
+      const float scale = ep.row_sumsq != nullptr ? scales[token] : 1.f;
+      float v[4];
 #pragma unroll
-      for (int j = 0; j < NJ; ++j) {
-        const int token = token0 + j * 32 + r32;
-        const float scale = ep.row_sumsq != nullptr ? scales[token] : 1.f;
-        float v[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = acc[i][j][g * 4 + e] * scale + b[e];
-        if constexpr (KIND == kEpSwiglu) {
-          *reinterpret_cast<uint32_t*>(lds + token * kRow + f) = pack_bf16x2(silu(v[0]) * v[2], silu(v[1]) * v[3]);
-        } else if constexpr (KIND == kEpGeglu) {
-          *reinterpret_cast<uint32_t*>(lds + token * kRow + f) = pack_bf16x2(gelu_tanh(v[0]) * v[2], gelu_tanh(v[1]) * v[3]);
-        } else {
-          typedef uint32_t words_t __attribute__((ext_vector_type(2)));
-          *reinterpret_cast<words_t*>(lds + token * kRow + f * 2) = words_t{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
-        }
+      for (int e = 0; e < 4; ++e) v[e] = acc[i][j][e] * scale + b[e];
+      if constexpr (KIND == kEpSwiglu) {
+        *reinterpret_cast<uint32_t*>(lds + token * kRow + f) = pack_bf16x2(silu(v[0]) * v[2], silu(v[1]) * v[3]);
+      } else if constexpr (KIND == kEpGeglu) {
+        *reinterpret_cast<uint32_t*>(lds + token * kRow + f) = pack_bf16x2(gelu_tanh(v[0]) * v[2], gelu_tanh(v[1]) * v[3]);
+      } else {
+        typedef uint32_t words_t __attribute__((ext_vector_type(2)));
+        *reinterpret_cast<words_t*>(lds + token * kRow + f * 2) = words_t{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
       }
     }
+  }
   __syncthreads();
   const int n_out = kPaired ? N / 2 : N, first = kPaired ? n0 / 2 : n0;
   constexpr int kRowPieces = kOut / 8;
@@ -306,8 +305,9 @@ constexpr int staged_sums_rows(int tokens, int features, int wave_tokens, int ld
 }
 
 template <int THREADS, int BM, int BN, int ROWS, int NI, int NJ>
-__device__ __forceinline__ void stage_sums(const GemmEpilogue& ep, const f32x16_t (&acc)[NI][NJ], unsigned char* lds, const float* scales,
-                                           int feature0, int token0, int r32, int h, int slice, int m0, int n0, int M, int N) {
+__device__ __forceinline__ void stage_sums(const GemmEpilogue& ep, const f32x4_t (&acc)[NI][NJ], unsigned char* lds, const float* scales,
+                                           int feature0, int token0, int slice, int m0, int n0, int M, int N) {
+  const int c16 = threadIdx.x % 16, quad = threadIdx.x % kWave / 16;
   constexpr int kRow = BN * 4 + 16;
   constexpr int kRowPieces = BN / 4;
   float* const y = static_cast<float*>(ep.y) + static_cast<int64_t>(slice) * M * N;
@@ -316,25 +316,23 @@ __device__ __forceinline__ void stage_sums(const GemmEpilogue& ep, const f32x16_
     if (first > 0) __syncthreads();  // the rows before have left
     if (token0 / ROWS * ROWS == first) {
 #pragma unroll
-      for (int i = 0; i < NI; ++i)
+      for (int i = 0; i < NI; ++i) {
+        const int f = feature0 + i * 16 + quad * 4;
+        float b[4] = {0.f, 0.f, 0.f, 0.f};
+        if (ep.bias != nullptr && slice == 0 && n0 + f < N) {  // n0 + f + 3 < N too: both are multiples of 4
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const int f = feature0 + i * 32 + g * 8 + h * 4;
-          float b[4] = {0.f, 0.f, 0.f, 0.f};
-          if (ep.bias != nullptr && slice == 0 && n0 + f < N) {  // n0 + f + 3 < N too: both are multiples of 4
-#pragma unroll
-            for (int e = 0; e < 4; ++e) b[e] = load_as_f32(ep.bias, n0 + f + e, ep.bias_is_f32);
-          }
-#pragma unroll
-          for (int j = 0; j < NJ; ++j) {
-            const int token = token0 + j * 32 + r32;
-            const float scale = ep.row_sumsq != nullptr ? scales[token] : 1.f;
-            f32x4_t v;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = acc[i][j][g * 4 + e] * scale + b[e];
-            *reinterpret_cast<f32x4_t*>(lds + (token - first) * kRow + f * 4) = v;
-          }
+          for (int e = 0; e < 4; ++e) b[e] = load_as_f32(ep.bias, n0 + f + e, ep.bias_is_f32);
         }
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+          const int token = token0 + j * 16 + c16;
+          const float scale = ep.row_sumsq != nullptr ? scales[token] : 1.f;
+          f32x4_t v;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = acc[i][j][e] * scale + b[e];
+          *reinterpret_cast<f32x4_t*>(lds + (token - first) * kRow + f * 4) = v;
+        }
+      }
     }
     __syncthreads();
 #pragma unroll 4

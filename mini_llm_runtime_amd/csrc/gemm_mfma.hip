@@ -19,7 +19,7 @@
 //    is the largest that still keeps the compute units busy), K in
 //    slices of 64 staged through double-buffered LDS by range-checked
 //    buffer loads (edge tiles and the tail of K read zeros, no branches),
-//    32x32x16 MFMA.  Beyond 64 tokens the larger tilings run gemm_direct: tiles
+//    32x32x16 MFMA.  Beyond 64 tokens the larger tilings run gemm_direct (16x16x32 MFMA, as the kernels below): tiles
 //    loaded straight into LDS (no registers, no LDS stores; rows swizzled instead of padded),
 //    with a step's barrier ahead of its last quarter of products; and the 256 x 256 tile gemm_phased, whose
 //    two groups of wavefronts read and multiply in turn.  Workgroups are placed so that those resident on
@@ -711,8 +711,10 @@ __global__ __launch_bounds__(64 * GM * GN) void gemm_tiled_kernel(const bf16* __
 // three slices 541 to 493, 0.5B gate-up 57 to 51 (the library: 53); on a model's weights, which come
 // from memory, 1 to 10 %.  (The 256 x 256 tile has since moved on to gemm_phased_kernel.)  Results of whole products
 // leave through LDS (stage_tile), which took 128 x 128 tiles of the 0.5B gate-up from 57 to 47 us, 256 x 320 from 48 to 41,
-// 256 x 192 tiles of 2,048 x 4,608 x 3,584 from 73 to 70.  Variants that lost: two quarters kept (KEEP 2: spills a register, no gain);
-// slices of 32 in four buffers or of 64 in three (BKT, NBUF; NBUF - 1 slices on their way: 5 to 25 %
+// 256 x 192 tiles of 2,048 x 4,608 x 3,584 from 73 to 70.  With products of 32 x 32 x 16 (see mfma.h), each quarter 16 of k of all blocks,
+// 8,191 x 4,608 x 3,584 took 251 us in tiles of 192 features (238 here), 7B gate-up at 512 tokens 135 in tiles of 320 (129), products of
+// up to 64 tokens the same within 2 %.  Variants that lost: two quarters kept (spills a register, no gain);
+// slices of 32 in four buffers or of 64 in three (NBUF - 1 slices on their way: 5 to 25 %
 // slower from 512 tokens on, up to 16 % faster at 128 to 256, where other tilings are chosen); a 64 x 64
 // tile (7 to 15 % slower than the staged kernel, which has two slices on their way, at up to 512 tokens
 // of weights that come from memory; equal beyond); eight wavefronts of 128 x 64 or 64 x 128 on the
@@ -721,18 +723,18 @@ __global__ __launch_bounds__(64 * GM * GN) void gemm_tiled_kernel(const bf16* __
 
 // LDS of a tile of `tokens` x `features` under `waves` wavefronts: a buffer holds the tile's 1 KB runs
 // and, where they do not go round the wavefronts, one more for the surplus loads (see kPieces).
-constexpr int direct_lds_bytes(int tokens, int features, int waves, int bk, int buffers) {
-  const int runs = (tokens + features) * bk * 2 / 1024;
+constexpr int direct_lds_bytes(int tokens, int features, int waves, int buffers) {
+  const int runs = (tokens + features) * kBK * 2 / 1024;
   return buffers * (runs + (runs % waves != 0 ? 1 : 0)) * 1024;
 }
 
 // FIXED: an epilogue fixed at compile time (kEpGeglu, for the tile that has no room for a choice), or -1.
-template <int KEEP, int WM, int WN, int GM, int GN, int BKT = kBK, int NBUF = 2, bool ONCE = false, int FIXED = -1>
+template <int WM, int WN, int GM, int GN, int NBUF = 2, bool ONCE = false, int FIXED = -1>
 __global__ __launch_bounds__(64 * GM * GN) void gemm_direct_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w,
                                                                   GemmEpilogue ep, TileOrder order, int M, int N, int K) {
   constexpr int BM = 32 * WM * GM, BN = 32 * WN * GN, WAVES = GM * GN;
-  constexpr int kRowBytes = BKT * 2;            // 128 or 64
-  constexpr int kRowPieces = BKT / 8;           // 16-byte pieces of a row
+  constexpr int kRowBytes = kBK * 2;
+  constexpr int kRowPieces = kBK / 8;           // 16-byte pieces of a row
   constexpr int kRunRows = 1024 / kRowBytes;    // rows of a 1 KB run, the unit a wavefront loads
   constexpr int kBankRows = 256 / kRowBytes;    // rows that LDS serves side by side in one cycle
   constexpr int kRuns = (BM + BN) / kRunRows;   // dealt out to the wavefronts in turn
@@ -744,9 +746,9 @@ __global__ __launch_bounds__(64 * GM * GN) void gemm_direct_kernel(const bf16* _
   // (loops over a wavefront's runs go to this fixed bound and break: with a bound that depends on the
   // template's parameters the host pass left the kernel uninstantiated, without a message)
   constexpr int kMostPieces = 16;               // at most this many per wavefront
-  constexpr int kSteps = BKT / 16;              // products of k = 16 per slice
+  constexpr bool kSplitFeatures = WN > WM;      // the side whose operands come in two halves (see below)
   static_assert(kPieces <= kMostPieces && BN % 32 == 0 && BM % 32 == 0, "whole runs of weight rows and of token rows");
-  static_assert(WAVES % 2 == 0 && KEEP >= 1 && KEEP < kSteps + 1 && NBUF >= 2, "see the swizzle key and the loop");
+  static_assert(WAVES % 2 == 0 && NBUF >= 2, "see the swizzle key and the loop");
   constexpr int kInFlight = (NBUF - 2) * kPieces;  // loads of this wavefront that may still be out when a slice is needed
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   constexpr int kBufferBytes = (kRuns + (kRuns % WAVES != 0 ? 1 : 0)) * 1024;
@@ -757,8 +759,8 @@ __global__ __launch_bounds__(64 * GM * GN) void gemm_direct_kernel(const bf16* _
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int wn = wave % GN;
   const int wm = wave / GN;
-  const int r32 = lane % 32;
-  const int h = lane / 32;
+  const int c16 = lane % 16;
+  const int quad = lane / 16;
   int slice, mt, nt;
   place_workgroup(order, blockIdx.x, slice, mt, nt);
   const int n0 = nt * BN;
@@ -767,7 +769,7 @@ __global__ __launch_bounds__(64 * GM * GN) void gemm_direct_kernel(const bf16* _
   if (ep.row_sumsq != nullptr) row_scales_issue(ep, owed, m0, BM, M);
   const int chunks = K / 8;
   const int slices = order.slices;
-  const int k_slices = (K + BKT - 1) / BKT;
+  const int k_slices = (K + kBK - 1) / kBK;
   const int per = (k_slices + slices - 1) / slices;
   const int s_begin = slice * per;
   const int s_end = min(k_slices, s_begin + per);
@@ -796,43 +798,57 @@ __global__ __launch_bounds__(64 * GM * GN) void gemm_direct_kernel(const bf16* _
       __attribute__((address_space(3))) void* dst =
           (__attribute__((address_space(3))) void*)(smem + buf * kBufferBytes + min(WAVES * p + wave, kRuns) * 1024);
       const bool weights = (p + 1) * WAVES <= kWeightRuns || (p * WAVES < kWeightRuns && WAVES * p + wave < kWeightRuns);
-      const unsigned off = (piece_off[p] + s * (BKT * 2u)) | off_ok;
+      const unsigned off = (piece_off[p] + s * (kBK * 2u)) | off_ok;
       if (ONCE && weights) __builtin_amdgcn_raw_ptr_buffer_load_lds(w_buf, dst, 16, off, 0, 0, 2);  // read once: non-temporal
       else __builtin_amdgcn_raw_ptr_buffer_load_lds(weights ? w_buf : x_buf, dst, 16, off, 0, 0, 0);
     }
   };
 
-  f32x16_t acc[WN][WM];
+  f32x4_t acc[2 * WN][2 * WM];  // blocks of 16 features, of 16 tokens
 #pragma unroll
-  for (int i = 0; i < WN; ++i)
+  for (int i = 0; i < 2 * WN; ++i)
 #pragma unroll
-    for (int j = 0; j < WM; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+    for (int j = 0; j < 2 * WM; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
   const bool idle = __builtin_amdgcn_readfirstlane(static_cast<int>(wm * 32 * WM >= x_rows)) != 0;
-  // operand rows of this lane: weight rows (wn WN + i) * 32 + r32, token rows BN + (wm WM + j) * 32 + r32;
-  // piece kk * 2 + h of a row sits in slot (kk * 2 + h) ^ key, and the key is (r32 / kBankRows) % kRowPieces for all of them
-  const int swz = (r32 / kBankRows) % kRowPieces;
-  const int a_base = (wn * 32 * WN + r32) * kRowBytes;
-  const int b_base = (BN + wm * 32 * WM + r32) * kRowBytes;
-  struct Fragments {
-    bf16x8_t a[WN], b[WM];
+  // operand rows of this lane: weight rows wn * 32 WN + i * 16 + c16, token rows BN + wm * 32 WM + j * 16 + c16; piece
+  // kk * 4 + quad of a row sits in slot (kk * 4 + quad) ^ key, and the key is (c16 / kBankRows) % kRowPieces for all of them.
+  // A slice's products come in quarters: 32 of k, all blocks of one side (`whole`) with half the blocks of the other (`part`), the
+  // one with more of them, so that the operands of two quarters fit the registers.
+  constexpr int kWhole = 2 * (kSplitFeatures ? WM : WN), kPart = kSplitFeatures ? WN : WM;
+  const int swz = (c16 / kBankRows) % kRowPieces;
+  const int a_base = (wn * 32 * WN + c16) * kRowBytes;
+  const int b_base = (BN + wm * 32 * WM + c16) * kRowBytes;
+  struct Whole {
+    bf16x8_t v[kWhole];
   };
-  auto read = [&](int buf, int kk) {
-    Fragments f;
-    const unsigned char* base = smem + buf * kBufferBytes + (((kk * 2 + h) ^ swz) * 16);
+  struct Part {
+    bf16x8_t v[kPart];
+  };
+  auto read_whole = [&](int buf, int kk) {
+    Whole f;
+    const unsigned char* base = smem + buf * kBufferBytes + (((kk * 4 + quad) ^ swz) * 16) + (kSplitFeatures ? b_base : a_base);
 #pragma unroll
-    for (int i = 0; i < WN; ++i) f.a[i] = load_bf16x8(base + a_base + i * 32 * kRowBytes);
-#pragma unroll
-    for (int j = 0; j < WM; ++j) f.b[j] = load_bf16x8(base + b_base + j * 32 * kRowBytes);
+    for (int i = 0; i < kWhole; ++i) f.v[i] = load_bf16x8(base + i * 16 * kRowBytes);
     return f;
   };
-  auto multiply = [&](const Fragments& f) {
+  auto read_part = [&](int buf, int kk, int half) {
+    Part f;
+    const unsigned char* base = smem + buf * kBufferBytes + (((kk * 4 + quad) ^ swz) * 16) + (kSplitFeatures ? a_base : b_base);
 #pragma unroll
-    for (int i = 0; i < WN; ++i)
+    for (int i = 0; i < kPart; ++i) f.v[i] = load_bf16x8(base + (half * kPart + i) * 16 * kRowBytes);
+    return f;
+  };
+  auto multiply = [&](const Whole& u, const Part& v, int half) {
+    constexpr int kTokens = kSplitFeatures ? kWhole : kPart, kFeatures = kSplitFeatures ? kPart : kWhole;
 #pragma unroll
-      for (int j = 0; j < WM; ++j) acc[i][j] = mfma_32x32x16(f.a[i], f.b[j], acc[i][j]);
+    for (int j = 0; j < kTokens; ++j)
+#pragma unroll
+      for (int f = 0; f < kFeatures; ++f) {
+        const int i = turn_at(f, j, kFeatures);
+        f32x4_t& sum = kSplitFeatures ? acc[half * kPart + i][j] : acc[i][half * kPart + j];
+        sum = kSplitFeatures ? mfma_16x16x32(v.v[i], u.v[j], sum) : mfma_16x16x32(u.v[i], v.v[j], sum);
+      }
   };
 
   // NBUF - 1 slices are on their way or in LDS ahead of the one that is multiplied
@@ -840,20 +856,19 @@ __global__ __launch_bounds__(64 * GM * GN) void gemm_direct_kernel(const bf16* _
   for (int b = 0; b < NBUF; ++b) fetch(s_begin + b, b);
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NBUF - 1) * kPieces) : "memory");
   __syncthreads();
-  Fragments cur = read(0, 0);
+  Whole whole = read_whole(0, 0);
+  Part part = read_part(0, 0, 0);
   int buf = 0;
   for (int s = s_begin; s < s_end; ++s) {
-    Fragments kept[KEEP];
     if (!idle) {
-#pragma unroll
-      for (int kk = 0; kk < kSteps - KEEP; ++kk) {
-        const Fragments next = read(buf, kk + 1);
-        multiply(cur);
-        cur = next;
-      }
-      kept[0] = cur;
-#pragma unroll
-      for (int e = 1; e < KEEP; ++e) kept[e] = read(buf, kSteps - KEEP + e);
+      const Part second = read_part(buf, 0, 1);
+      multiply(whole, part, 0);
+      const Whole whole1 = read_whole(buf, 1);
+      const Part third = read_part(buf, 1, 0);
+      multiply(whole, second, 1);
+      part = read_part(buf, 1, 1);
+      multiply(whole1, third, 0);
+      whole = whole1;
     }
     // the slice after this one has landed (this wavefront's share; the barrier answers for the others),
     // and nobody reads this slice's buffer any more
@@ -862,9 +877,11 @@ __global__ __launch_bounds__(64 * GM * GN) void gemm_direct_kernel(const bf16* _
     fetch(s + NBUF, buf);
     const int next_buf = buf + 1 == NBUF ? 0 : buf + 1;
     if (!idle) {
-      cur = read(next_buf, 0);
-#pragma unroll
-      for (int e = 0; e < KEEP; ++e) multiply(kept[e]);  // the part kept for behind the barrier
+      const Whole kept_whole = whole;
+      const Part kept = part;
+      whole = read_whole(next_buf, 0);
+      part = read_part(next_buf, 0, 0);
+      multiply(kept_whole, kept, 1);  // the quarter kept for behind the barrier
     }
     buf = next_buf;
   }
@@ -882,7 +899,7 @@ __global__ __launch_bounds__(64 * GM * GN) void gemm_direct_kernel(const bf16* _
   if constexpr (kSumRows > 0) {
     if (stages_sums(ep, N)) {
       __syncthreads();  // as below
-      stage_sums<64 * GM * GN, BM, BN, kSumRows>(ep, acc, smem, scales, wn * 32 * WN, wm * 32 * WM, r32, h, slice, m0, n0, M, N);
+      stage_sums<64 * GM * GN, BM, BN, kSumRows>(ep, acc, smem, scales, wn * 32 * WN, wm * 32 * WM, slice, m0, n0, M, N);
       return;
     }
   }
@@ -892,36 +909,32 @@ __global__ __launch_bounds__(64 * GM * GN) void gemm_direct_kernel(const bf16* _
       constexpr int kThreads = 64 * GM * GN;
       if constexpr (FIXED < 0) {
         if (ep.swiglu == kEpSwiglu) {
-          stage_tile<kEpSwiglu, kThreads, BM, BN>(ep, acc, smem, scales, wn * 32 * WN, wm * 32 * WM, r32, h, m0, n0, M, N);
+          stage_tile<kEpSwiglu, kThreads, BM, BN>(ep, acc, smem, scales, wn * 32 * WN, wm * 32 * WM, m0, n0, M, N);
           return;
         }
       }
       if constexpr (kStagesPlain) {
         if (ep.swiglu == kEpNone) {
-          stage_tile<kEpNone, kThreads, BM, BN>(ep, acc, smem, scales, wn * 32 * WN, wm * 32 * WM, r32, h, m0, n0, M, N);
+          stage_tile<kEpNone, kThreads, BM, BN>(ep, acc, smem, scales, wn * 32 * WN, wm * 32 * WM, m0, n0, M, N);
           return;
         }
       }
-      stage_tile<kEpGeglu, kThreads, BM, BN>(ep, acc, smem, scales, wn * 32 * WN, wm * 32 * WM, r32, h, m0, n0, M, N);
+      stage_tile<kEpGeglu, kThreads, BM, BN>(ep, acc, smem, scales, wn * 32 * WN, wm * 32 * WM, m0, n0, M, N);
       return;
     }
   }
 #pragma unroll
-  for (int i = 0; i < WN; ++i)
+  for (int i = 0; i < 2 * WN; ++i)
 #pragma unroll
-    for (int j = 0; j < WM; ++j) {
-      const int m = m0 + (wm * WM + j) * 32 + r32;
-      const float scale = ep.row_sumsq != nullptr ? scales[(wm * WM + j) * 32 + r32] : 1.f;
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int n = n0 + (wn * WN + i) * 32 + g * 8 + h * 4;
-        const float v[4] = {acc[i][j][g * 4 + 0] * scale, acc[i][j][g * 4 + 1] * scale, acc[i][j][g * 4 + 2] * scale,
-                            acc[i][j][g * 4 + 3] * scale};
-        if constexpr (FIXED == kEpGeglu) {
-          if (m < M && n < N) store_geglu4(ep, m, n, N, v);
-        } else {
-          finish4<(WM * WN < 10)>(ep, slice, slices, m, n, M, N, v);  // ten blocks a wavefront: the registers are full
-        }
+    for (int j = 0; j < 2 * WM; ++j) {
+      const int token = wm * 32 * WM + j * 16 + c16;
+      const int m = m0 + token, n = n0 + wn * 32 * WN + i * 16 + quad * 4;
+      const float scale = ep.row_sumsq != nullptr ? scales[token] : 1.f;
+      const float v[4] = {acc[i][j][0] * scale, acc[i][j][1] * scale, acc[i][j][2] * scale, acc[i][j][3] * scale};
+      if constexpr (FIXED == kEpGeglu) {
+        if (m < M && n < N) store_geglu4(ep, m, n, N, v);
+      } else {
+        finish4<(WM * WN < 10)>(ep, slice, slices, m, n, M, N, v);  // 256 x 320: the registers are full
       }
     }
 }
@@ -931,7 +944,7 @@ __global__ __launch_bounds__(64 * GM * GN) void gemm_direct_kernel(const bf16* _
 // wavefronts of 64 x 64), two on every SIMD.  What gemm_direct_kernel loses beside its products is that all wavefronts wait, read and
 // multiply at the same time; here the two groups take turns: while one multiplies, the other reads its next operands from
 // LDS and asks for tiles from memory, and a barrier between the phases keeps them apart.
-//  * A step (64 of k) is four phases of 8 products: the tokens' halves X0, X1 (64 of a wavefront's 128) against the features'
+//  * A step (64 of k) is four phases of 16 products of 16 x 16 x 32: the tokens' halves X0, X1 (64 of a wavefront's 128) against the features'
 //    halves W0, W1 (32 of 64) in the order X0 W0, X0 W1, X1 W1, X1 W0; before each, its group reads what that phase still lacks: X0, W1,
 //    X1 and, in the last, W0 of the next step (into the registers of W1, so steps alternate between two sets).
 //  * The four quarters of a slice lie in LDS apart (16 KB each, two slices: 128 KB).  As soon as both groups have read a quarter, the
@@ -944,6 +957,9 @@ __global__ __launch_bounds__(64 * GM * GN) void gemm_direct_kernel(const bf16* _
 // to 505 (1,102), at 8,191 1,942 to 1,799 (1,236), at 1,048 299 to 280; 8,191 x 3,584 x 3,584 194 to 174 (1,210); 7B down at 8,191 984 to
 // 927 (1,200), at 2,048 in two slices 265 to 238.  Without the staging, whole products were level with the old kernel
 // (3,584 x 3,584 at 2,048: 78 there, 88 without and 70 with it).
+// Bound by power: with products of 32 x 32 x 16 (see mfma.h) the same loop took, on one card in turn, 7B gate-up at 2,048 tokens 470 us (432
+// here, 1,287 TFLOP/s), at 8,191 1,785 (1,647, 1,351), 7B down at 8,191 905 (838), at 2,048 in two slices 235 (215).  What is left of
+// that: the tiles' way from memory into LDS is 15 % of the time, the operands' from LDS 7 % (each left out in a copy of the kernel).
 constexpr int kPhaseQuarter = 128 * 128;             // bytes
 constexpr int kPhaseBuffer = 4 * kPhaseQuarter;      // W0, W1, X0, X1
 constexpr int kPhaseLds = staged_tile_bytes(256, 256);  // a little more than the two slices
@@ -956,7 +972,7 @@ __global__ __launch_bounds__(512, 2) void gemm_phased_kernel(const bf16* __restr
   const int lane = threadIdx.x % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int wm = wave / 4, wn = wave % 4;  // wavefronts w and w + 4 share a SIMD: one of each group
-  const int r32 = lane % 32, h = lane / 32;
+  const int c16 = lane % 16, quad = lane / 16;
   int slice, mt, nt;
   place_workgroup(order, blockIdx.x, slice, mt, nt);
   const int n0 = nt * 256, m0 = mt * 256;
@@ -990,37 +1006,37 @@ __global__ __launch_bounds__(512, 2) void gemm_phased_kernel(const bf16* __restr
                                                (off + p * 256u * K) | past, 0, 0, 0);
   };
 
-  f32x16_t acc[2][4];  // feature half; token half * 2 + block of 32
+  f32x4_t acc[4][8];  // blocks of 16 features (half * 2 + block) and of 16 tokens (half * 4 + block)
 #pragma unroll
-  for (int j = 0; j < 2; ++j)
+  for (int j = 0; j < 4; ++j)
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[j][i][e] = 0.f;
+    for (int i = 0; i < 8; ++i) acc[j][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
   const bool idle = __builtin_amdgcn_readfirstlane(static_cast<int>(wm * 128 >= x_rows)) != 0;  // no tokens: keeps time only
-  const int swz = (r32 / 2) % 8;
-  const int w_base = (wn * 32 + r32) * 128;
-  const int x_base = 2 * kPhaseQuarter + (wm * 64 + r32) * 128;
+  const int swz = c16 / 2;
+  const int w_base = (wn * 32 + c16) * 128;
+  const int x_base = 2 * kPhaseQuarter + (wm * 64 + c16) * 128;
   struct Weights {
-    bf16x8_t v[4];
+    bf16x8_t v[2][2];  // 32 of k, block of 16 features
   };
   struct Tokens {
-    bf16x8_t v[4][2];
+    bf16x8_t v[2][4];
   };
   auto read_weights = [&](Weights& t, int buf, int j) {
     if (idle) return;
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk)
-      t.v[kk] = load_bf16x8(smem + buf * kPhaseBuffer + j * kPhaseQuarter + w_base + (((kk * 2 + h) ^ swz) * 16));
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+        t.v[kk][b] = load_bf16x8(smem + buf * kPhaseBuffer + j * kPhaseQuarter + w_base + b * 16 * 128 + (((kk * 4 + quad) ^ swz) * 16));
   };
   auto read_tokens = [&](Tokens& t, int buf, int i) {
     if (idle) return;
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk)
+    for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
-      for (int b = 0; b < 2; ++b)
-        t.v[kk][b] = load_bf16x8(smem + buf * kPhaseBuffer + i * kPhaseQuarter + x_base + b * 32 * 128 + (((kk * 2 + h) ^ swz) * 16));
+      for (int b = 0; b < 4; ++b)
+        t.v[kk][b] = load_bf16x8(smem + buf * kPhaseBuffer + i * kPhaseQuarter + x_base + b * 16 * 128 + (((kk * 4 + quad) ^ swz) * 16));
   };
   // the end of a reading phase: operands are in registers, the quarter read next has landed (all but `pending` loads)
 #define MLR_READ_DONE(pending)                                                                   \
@@ -1034,9 +1050,14 @@ __global__ __launch_bounds__(512, 2) void gemm_phased_kernel(const bf16* __restr
     if (!idle) {
       __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-      for (int kk = 0; kk < 4; ++kk)
+      for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
-        for (int c = 0; c < 2; ++c) acc[j][i * 2 + c] = mfma_32x32x16(a.v[kk], b.v[kk][c], acc[j][i * 2 + c]);
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+          for (int f = 0; f < 2; ++f) {
+            f32x4_t& sum = acc[j * 2 + turn_at(f, c, 2)][i * 4 + c];
+            sum = mfma_16x16x32(a.v[kk][turn_at(f, c, 2)], b.v[kk][c], sum);
+          }
       __builtin_amdgcn_s_setprio(0);
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -1091,30 +1112,25 @@ __global__ __launch_bounds__(512, 2) void gemm_phased_kernel(const bf16* __restr
   __syncthreads();
   if (stages_tile(ep, slices, N)) {
     if (ep.swiglu == kEpSwiglu)
-      stage_tile<kEpSwiglu, 512, 256, 256>(ep, acc, smem, scales, wn * 64, wm * 128, r32, h, m0, n0, M, N);
+      stage_tile<kEpSwiglu, 512, 256, 256>(ep, acc, smem, scales, wn * 64, wm * 128, m0, n0, M, N);
     else if (ep.swiglu == kEpGeglu)
-      stage_tile<kEpGeglu, 512, 256, 256>(ep, acc, smem, scales, wn * 64, wm * 128, r32, h, m0, n0, M, N);
+      stage_tile<kEpGeglu, 512, 256, 256>(ep, acc, smem, scales, wn * 64, wm * 128, m0, n0, M, N);
     else
-      stage_tile<kEpNone, 512, 256, 256>(ep, acc, smem, scales, wn * 64, wm * 128, r32, h, m0, n0, M, N);
+      stage_tile<kEpNone, 512, 256, 256>(ep, acc, smem, scales, wn * 64, wm * 128, m0, n0, M, N);
     return;
   }
   if (stages_sums(ep, N)) {
-    stage_sums<512, 256, 256, staged_sums_rows(256, 256, 128, kPhaseLds)>(ep, acc, smem, scales, wn * 64, wm * 128, r32, h, slice, m0, n0, M, N);
+    stage_sums<512, 256, 256, staged_sums_rows(256, 256, 128, kPhaseLds)>(ep, acc, smem, scales, wn * 64, wm * 128, slice, m0, n0, M, N);
     return;
   }
 #pragma unroll
-  for (int j = 0; j < 2; ++j)
+  for (int j = 0; j < 4; ++j)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int m = m0 + wm * 128 + i * 32 + r32;
-      const float scale = ep.row_sumsq != nullptr ? scales[wm * 128 + i * 32 + r32] : 1.f;
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int n = n0 + wn * 64 + j * 32 + g * 8 + h * 4;
-        const float v[4] = {acc[j][i][g * 4 + 0] * scale, acc[j][i][g * 4 + 1] * scale, acc[j][i][g * 4 + 2] * scale,
-                            acc[j][i][g * 4 + 3] * scale};
-        finish4(ep, slice, slices, m, n, M, N, v);
-      }
+    for (int i = 0; i < 8; ++i) {
+      const int token = wm * 128 + i * 16 + c16;
+      const float scale = ep.row_sumsq != nullptr ? scales[token] : 1.f;
+      const float v[4] = {acc[j][i][0] * scale, acc[j][i][1] * scale, acc[j][i][2] * scale, acc[j][i][3] * scale};
+      finish4(ep, slice, slices, m0 + token, n0 + wn * 64 + j * 16 + quad * 4, M, N, v);
     }
 }
 
@@ -1123,7 +1139,8 @@ __global__ __launch_bounds__(512, 2) void gemm_phased_kernel(const bf16* __restr
 // and one the odd, and they take turns as in gemm_phased_kernel: while one multiplies a slice from registers the other reads
 // its next one from LDS.  A group has two LDS buffers of its own; a slice is asked for as soon as its buffer has been
 // read, an iteration (two slices of the tile) ahead.  At the end each group hands the sums of half the features to the other.
-// Bound, like the larger tile, by the LDS reads beside the products (64 x 64 a wavefront: as many cycles of one as of the other).
+// Bound, like the larger tile, by the LDS reads beside the products (64 x 64 a wavefront: as many cycles of one as of the other).  With
+// products of 32 x 32 x 16 2,000 x 2,048 x 2,048 took 24.2 us (23.2 here), 1,048 x 3,584 x 3,584 36.1 (34.5).
 // Measured against gemm_direct's 128 x 128 tile (two workgroups of four wavefronts a unit where there are as many), weights from
 // memory, microseconds: 2,000 x 2,048 x 2,048 (256 tiles) 27.1 to 24.8, k = 4,096 49.7 to 41.8; 1,048 x 3,584 x 3,584 38.6 to 34.7;
 // 768 x 4,608 x 3,584 41 to 32; in slices 1,024 x 1,536 x 8,960 46 to 42, 160 x 5,120 x 27,648 130 to 86.  See takes_turns for where it is used.
@@ -1139,7 +1156,7 @@ __global__ __launch_bounds__(512, 2) void gemm_turns_kernel(const bf16* __restri
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int group = wave / 4, w4 = wave % 4;  // wavefronts w and w + 4 share a SIMD: one of each group
   const int wr = w4 / 2, wc = w4 % 2;
-  const int r32 = lane % 32, h = lane / 32;
+  const int c16 = lane % 16, quad = lane / 16;
   int slice, mt, nt;
   place_workgroup(order, blockIdx.x, slice, mt, nt);
   const int n0 = nt * 128, m0 = mt * 128;
@@ -1166,15 +1183,13 @@ __global__ __launch_bounds__(512, 2) void gemm_turns_kernel(const bf16* __restri
       __builtin_amdgcn_raw_ptr_buffer_load_lds(p < 4 ? w_buf : x_buf, (__attribute__((address_space(3))) void*)(dst + p * 4096), 16,
                                                (row_off + (p % 4) * 64u * K + s * 128u) | past, 0, 0, 0);
   };
-  f32x16_t acc[2][2];  // features, tokens
+  f32x4_t acc[4][4];  // blocks of 16 features, of 16 tokens
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   const bool idle = __builtin_amdgcn_readfirstlane(static_cast<int>(wr * 64 >= x_rows)) != 0;  // no tokens: keeps time only
-  const int swz = (r32 / 2) % 8;
+  const int swz = c16 / 2;
 #define MLR_TURN()                        \
   do {                                    \
     __builtin_amdgcn_sched_barrier(0);    \
@@ -1189,15 +1204,15 @@ __global__ __launch_bounds__(512, 2) void gemm_turns_kernel(const bf16* __restri
   __builtin_amdgcn_sched_barrier(0);
   const int iterations = (steps + 1) / 2;
   for (int it = 0; it < iterations; ++it) {
-    bf16x8_t wv[4][2], xv[4][2];
+    bf16x8_t wv[2][4], xv[2][4];
     if (!idle) {
       const unsigned char* const base = smem + (group * 2 + (it & 1)) * kTurnSlice;
 #pragma unroll
-      for (int kk = 0; kk < 4; ++kk)
+      for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
-        for (int b = 0; b < 2; ++b) {
-          wv[kk][b] = load_bf16x8(base + (wc * 64 + b * 32 + r32) * 128 + (((kk * 2 + h) ^ swz) * 16));
-          xv[kk][b] = load_bf16x8(base + (128 + wr * 64 + b * 32 + r32) * 128 + (((kk * 2 + h) ^ swz) * 16));
+        for (int b = 0; b < 4; ++b) {
+          wv[kk][b] = load_bf16x8(base + (wc * 64 + b * 16 + c16) * 128 + (((kk * 4 + quad) ^ swz) * 16));
+          xv[kk][b] = load_bf16x8(base + (128 + wr * 64 + b * 16 + c16) * 128 + (((kk * 4 + quad) ^ swz) * 16));
         }
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the group has read its buffer once all of it is past the barrier
@@ -1206,11 +1221,14 @@ __global__ __launch_bounds__(512, 2) void gemm_turns_kernel(const bf16* __restri
     if (!idle) {
       __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-      for (int kk = 0; kk < 4; ++kk)
+      for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int j = 0; j < 4; ++j)
 #pragma unroll
-          for (int j = 0; j < 2; ++j) acc[i][j] = mfma_32x32x16(wv[kk][i], xv[kk][j], acc[i][j]);
+          for (int i = 0; i < 4; ++i) {
+            f32x4_t& sum = acc[turn_at(i, j, 4)][j];
+            sum = mfma_16x16x32(wv[kk][turn_at(i, j, 4)], xv[kk][j], sum);
+          }
       __builtin_amdgcn_s_setprio(0);
     }
     asm volatile("s_waitcnt vmcnt(8)" ::: "memory");  // all but the slice just asked for: the next one has landed
@@ -1222,49 +1240,42 @@ __global__ __launch_bounds__(512, 2) void gemm_turns_kernel(const bf16* __restri
   if (ep.row_sumsq != nullptr) row_scales_finish(ep, owed, m0, 128, M, K, scales);
   __syncthreads();
   // group g finishes feature block g of its wavefronts
-  f32x16_t sum[1][2];
+  f32x4_t sum[2][4];
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const f32x16_t given = group == 0 ? acc[1][j] : acc[0][j];
-    sum[0][j] = group == 0 ? acc[0][j] : acc[1][j];
+  for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int g = 0; g < 4; ++g)
-      *reinterpret_cast<f32x4_t*>(smem + ((wave * 2 + j) * 4 + g) * 1024 + lane * 16) = f32x4_t{given[g * 4], given[g * 4 + 1], given[g * 4 + 2], given[g * 4 + 3]};
-  }
+    for (int j = 0; j < 4; ++j) {
+      *reinterpret_cast<f32x4_t*>(smem + ((wave * 2 + i) * 4 + j) * 1024 + lane * 16) = group == 0 ? acc[2 + i][j] : acc[i][j];
+      sum[i][j] = group == 0 ? acc[i][j] : acc[2 + i][j];
+    }
   __syncthreads();
 #pragma unroll
-  for (int j = 0; j < 2; ++j)
+  for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const f32x4_t other = *reinterpret_cast<const f32x4_t*>(smem + (((wave ^ 4) * 2 + j) * 4 + g) * 1024 + lane * 16);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) sum[0][j][g * 4 + e] += other[e];
-    }
+    for (int j = 0; j < 4; ++j) sum[i][j] += *reinterpret_cast<const f32x4_t*>(smem + (((wave ^ 4) * 2 + i) * 4 + j) * 1024 + lane * 16);
   const int feature0 = wc * 64 + group * 32, token0 = wr * 64;
   if (stages_tile(ep, slices, N)) {
     if (ep.swiglu == kEpSwiglu)
-      stage_tile<kEpSwiglu, 512, 128, 128>(ep, sum, smem + 65536, scales, feature0, token0, r32, h, m0, n0, M, N);
+      stage_tile<kEpSwiglu, 512, 128, 128>(ep, sum, smem + 65536, scales, feature0, token0, m0, n0, M, N);
     else if (ep.swiglu == kEpGeglu)
-      stage_tile<kEpGeglu, 512, 128, 128>(ep, sum, smem + 65536, scales, feature0, token0, r32, h, m0, n0, M, N);
+      stage_tile<kEpGeglu, 512, 128, 128>(ep, sum, smem + 65536, scales, feature0, token0, m0, n0, M, N);
     else
-      stage_tile<kEpNone, 512, 128, 128>(ep, sum, smem + 65536, scales, feature0, token0, r32, h, m0, n0, M, N);
+      stage_tile<kEpNone, 512, 128, 128>(ep, sum, smem + 65536, scales, feature0, token0, m0, n0, M, N);
     return;
   }
   if (stages_sums(ep, N)) {
-    stage_sums<512, 128, 128, staged_sums_rows(128, 128, 64, kTurnLds - 65536)>(ep, sum, smem + 65536, scales, feature0, token0, r32, h, slice, m0, n0, M, N);
+    stage_sums<512, 128, 128, staged_sums_rows(128, 128, 64, kTurnLds - 65536)>(ep, sum, smem + 65536, scales, feature0, token0, slice, m0, n0, M, N);
     return;
   }
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int m = m0 + token0 + j * 32 + r32;
-    const float scale = ep.row_sumsq != nullptr ? scales[token0 + j * 32 + r32] : 1.f;
+  for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const float v[4] = {sum[0][j][g * 4 + 0] * scale, sum[0][j][g * 4 + 1] * scale, sum[0][j][g * 4 + 2] * scale,
-                          sum[0][j][g * 4 + 3] * scale};
-      finish4(ep, slice, slices, m, n0 + feature0 + g * 8 + h * 4, M, N, v);
+    for (int j = 0; j < 4; ++j) {
+      const int token = token0 + j * 16 + c16;
+      const float scale = ep.row_sumsq != nullptr ? scales[token] : 1.f;
+      const float v[4] = {sum[i][j][0] * scale, sum[i][j][1] * scale, sum[i][j][2] * scale, sum[i][j][3] * scale};
+      finish4(ep, slice, slices, m0 + token, n0 + feature0 + i * 16 + quad * 4, M, N, v);
     }
-  }
 }
 
 using DirectKernel = void (*)(const bf16*, const bf16*, GemmEpilogue, TileOrder, int, int, int);
@@ -1610,57 +1621,57 @@ static int gemm_bf16(const bf16* xb, const bf16* wb, const GemmEpilogue& ep, int
     // 64 tokens x 64 to 256 features, a wavefront per 32 x 32 block, as many slices of k in LDS as fit
     case 62: {
       static bool configured = false;
-      return launch_direct(gemm_direct_kernel<1, 1, 1, 2, 2, 64, 4, true>, 64, 64, 256, 2, direct_lds_bytes(64, 64, 4, 64, 4),
+      return launch_direct(gemm_direct_kernel<1, 1, 2, 2, 4, true>, 64, 64, 256, 2, direct_lds_bytes(64, 64, 4, 4),
                            configured, xb, wb, ep, m, n, k, slices, stream);
     }
     case 63: {
       static bool configured = false;
-      return launch_direct(gemm_direct_kernel<1, 1, 1, 2, 3, 64, 6, true>, 64, 96, 384, 2, direct_lds_bytes(64, 96, 6, 64, 6),
+      return launch_direct(gemm_direct_kernel<1, 1, 2, 3, 6, true>, 64, 96, 384, 2, direct_lds_bytes(64, 96, 6, 6),
                            configured, xb, wb, ep, m, n, k, slices, stream);
     }
     case 64: {
       static bool configured = false;
-      return launch_direct(gemm_direct_kernel<1, 1, 1, 2, 4, 64, 6, true>, 64, 128, 512, 2, direct_lds_bytes(64, 128, 8, 64, 6),
+      return launch_direct(gemm_direct_kernel<1, 1, 2, 4, 6, true>, 64, 128, 512, 2, direct_lds_bytes(64, 128, 8, 6),
                            configured, xb, wb, ep, m, n, k, slices, stream);
     }
     case 65: {
       static bool configured = false;
-      return launch_direct(gemm_direct_kernel<1, 1, 1, 2, 5, 64, 5, true>, 64, 160, 640, 2, direct_lds_bytes(64, 160, 10, 64, 5),
+      return launch_direct(gemm_direct_kernel<1, 1, 2, 5, 5, true>, 64, 160, 640, 2, direct_lds_bytes(64, 160, 10, 5),
                            configured, xb, wb, ep, m, n, k, slices, stream);
     }
     case 66: {
       static bool configured = false;
-      return launch_direct(gemm_direct_kernel<1, 1, 1, 2, 6, 64, 4, true>, 64, 192, 768, 2, direct_lds_bytes(64, 192, 12, 64, 4),
+      return launch_direct(gemm_direct_kernel<1, 1, 2, 6, 4, true>, 64, 192, 768, 2, direct_lds_bytes(64, 192, 12, 4),
                            configured, xb, wb, ep, m, n, k, slices, stream);
     }
     case 67: {
       static bool configured = false;
-      return launch_direct(gemm_direct_kernel<1, 1, 1, 2, 7, 64, 3, true>, 64, 224, 896, 2, direct_lds_bytes(64, 224, 14, 64, 3),
+      return launch_direct(gemm_direct_kernel<1, 1, 2, 7, 3, true>, 64, 224, 896, 2, direct_lds_bytes(64, 224, 14, 3),
                            configured, xb, wb, ep, m, n, k, slices, stream);
     }
     case 68: {
       static bool configured = false;
-      return launch_direct(gemm_direct_kernel<1, 1, 1, 2, 8, 64, 3, true>, 64, 256, 1024, 2, direct_lds_bytes(64, 256, 16, 64, 3),
+      return launch_direct(gemm_direct_kernel<1, 1, 2, 8, 3, true>, 64, 256, 1024, 2, direct_lds_bytes(64, 256, 16, 3),
                            configured, xb, wb, ep, m, n, k, slices, stream);
     }
     case 48: {  // 256 tokens x 320 features, eight wavefronts of 64 x 160
       if (ep.swiglu == kEpGeglu) {
         static bool configured_geglu = false;
-        return launch_direct(gemm_direct_kernel<1, 2, 5, 4, 2, kBK, 2, false, kEpGeglu>, 256, 320, 512, 4,
-                             direct_lds_bytes(256, 320, 8, 64, 2), configured_geglu, xb, wb, ep, m, n, k, slices, stream);
+        return launch_direct(gemm_direct_kernel<2, 5, 4, 2, 2, false, kEpGeglu>, 256, 320, 512, 4,
+                             direct_lds_bytes(256, 320, 8, 2), configured_geglu, xb, wb, ep, m, n, k, slices, stream);
       }
       static bool configured = false;
-      return launch_direct(gemm_direct_kernel<1, 2, 5, 4, 2>, 256, 320, 512, 4, direct_lds_bytes(256, 320, 8, 64, 2), configured,
+      return launch_direct(gemm_direct_kernel<2, 5, 4, 2>, 256, 320, 512, 4, direct_lds_bytes(256, 320, 8, 2), configured,
                            xb, wb, ep, m, n, k, slices, stream);
     }
     case 46: {  // 256 tokens x 192 features, twelve wavefronts of 64 x 64
       static bool configured = false;
-      return launch_direct(gemm_direct_kernel<1, 2, 2, 4, 3>, 256, 192, 768, 4, direct_lds_bytes(256, 192, 12, 64, 2), configured,
+      return launch_direct(gemm_direct_kernel<2, 2, 4, 3>, 256, 192, 768, 4, direct_lds_bytes(256, 192, 12, 2), configured,
                            xb, wb, ep, m, n, k, slices, stream);
     }
     case 47: {  // 256 tokens x 160 features, ten wavefronts of 128 x 32
       static bool configured = false;
-      return launch_direct(gemm_direct_kernel<1, 4, 1, 2, 5>, 256, 160, 640, 2, direct_lds_bytes(256, 160, 10, 64, 2), configured,
+      return launch_direct(gemm_direct_kernel<4, 1, 2, 5>, 256, 160, 640, 2, direct_lds_bytes(256, 160, 10, 2), configured,
                            xb, wb, ep, m, n, k, slices, stream);
     }
     case 23: return gemm_bf16(xb, wb, ep, m, n, k, slices, takes_turns(m, n, k, slices) ? 24 : 25, stream);
@@ -1670,7 +1681,7 @@ static int gemm_bf16(const bf16* xb, const bf16* wb, const GemmEpilogue& ep, int
     }
     case 25: {
       static bool configured = false;
-      return launch_direct(gemm_direct_kernel<1, 2, 2, 2, 2>, 128, 128, 256, 2, direct_lds_bytes(128, 128, 4, 64, 2), configured,
+      return launch_direct(gemm_direct_kernel<2, 2, 2, 2>, 128, 128, 256, 2, direct_lds_bytes(128, 128, 4, 2), configured,
                            xb, wb, ep, m, n, k, slices, stream);
     }
     default: set_error("mlr_gemm_bf16: kernel must be 0 (chosen by shape), 16, 14, 11, 22 to 25, 44 to 48, 62 to 68 or 71 to 74"); return -1;

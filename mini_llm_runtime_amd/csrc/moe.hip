@@ -821,49 +821,62 @@ __global__ __launch_bounds__(256) void moe_gemm_tiled_kernel(const bf16* __restr
     off[4 + p] = at < rows ? static_cast<unsigned>(UP ? pairs_of_lane[p] / top : row0 + at) * row_bytes + piece * 16u : kNoRow;
   }
   if (tid < kRows) pair_of[tid] = tid < rows ? pair_of_thread : -1;
-  f32x16_t acc[RB][2];
+  f32x4_t acc[2 * RB][4];  // blocks of 16 rows, of 16 features
 #pragma unroll
-  for (int r = 0; r < RB; ++r)
+  for (int r = 0; r < 2 * RB; ++r)
 #pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[r][b][i] = 0.f;
-  const int r32 = lane % 32;
-  const int khalf = lane / 32;  // which 8 of a block's 16 k
+    for (int b = 0; b < 4; ++b) acc[r][b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const int c16 = lane % 16;
+  const int quad = lane / 16;  // which 8 of a block's 32 k
   const bool idle = __builtin_amdgcn_readfirstlane(static_cast<int>(wr * 32 * RB >= rows)) != 0;  // a tile with rows for the first wavefronts only
-  const int swz = (r32 / 2) % 8;
-  struct Operands {
-    bf16x8_t w[2], x[RB];
+  const int swz = c16 / 2;
+  // A slice's products come in quarters: 32 of k, all features, half the rows.
+  struct Weights {
+    bf16x8_t v[4];
   };
-  auto read = [&](int buf, int ks) {
-    Operands o;
-    const unsigned char* const base = moe_lds + buf * kBuffer + (((ks * 2 + khalf) ^ swz) * 16);
+  struct Rows {
+    bf16x8_t v[RB];
+  };
+  auto read_weights = [&](int buf, int kk) {
+    Weights o;
+    const unsigned char* const base = moe_lds + buf * kBuffer + (((kk * 4 + quad) ^ swz) * 16) + (wc * 64 + c16) * 128;
 #pragma unroll
-    for (int b = 0; b < 2; ++b) o.w[b] = load_bf16x8(base + (wc * 64 + b * 32 + r32) * 128);
-#pragma unroll
-    for (int r = 0; r < RB; ++r) o.x[r] = load_bf16x8(base + (kBigCols + (wr * RB + r) * 32 + r32) * 128);
+    for (int b = 0; b < 4; ++b) o.v[b] = load_bf16x8(base + b * 16 * 128);
     return o;
   };
-  auto multiply = [&](const Operands& o) {
+  auto read_rows = [&](int buf, int kk, int half) {
+    Rows o;
+    const unsigned char* const base = moe_lds + buf * kBuffer + (((kk * 4 + quad) ^ swz) * 16) + (kBigCols + wr * 32 * RB + c16) * 128;
+#pragma unroll
+    for (int r = 0; r < RB; ++r) o.v[r] = load_bf16x8(base + (half * RB + r) * 16 * 128);
+    return o;
+  };
+  auto multiply = [&](const Weights& u, const Rows& x, int half) {
 #pragma unroll
     for (int r = 0; r < RB; ++r)
 #pragma unroll
-      for (int b = 0; b < 2; ++b) acc[r][b] = mfma_32x32x16(o.w[b], o.x[r], acc[r][b]);
+      for (int f = 0; f < 4; ++f) {
+        const int b = turn_at(f, r, 4);
+        acc[half * RB + r][b] = mfma_16x16x32(u.v[b], x.v[r], acc[half * RB + r][b]);
+      }
   };
   fetch(0, 0, false);
   fetch(1, 1, false);
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kRowLoads) : "memory");
   __syncthreads();
-  Operands cur = read(0, 0);
+  Weights u = read_weights(0, 0);
+  Rows x = read_rows(0, 0, 0);
   int buf = 0;
   for (int s = 0; s < slices; ++s) {
     if (!idle) {
-#pragma unroll
-      for (int ks = 0; ks < kBigK / 16 - 1; ++ks) {
-        const Operands next = read(buf, ks + 1);
-        multiply(cur);
-        cur = next;
-      }
+      const Rows second = read_rows(buf, 0, 1);
+      multiply(u, x, 0);
+      const Weights u1 = read_weights(buf, 1);
+      const Rows third = read_rows(buf, 1, 0);
+      multiply(u, second, 1);
+      x = read_rows(buf, 1, 1);
+      multiply(u1, third, 0);
+      u = u1;
     }
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     __syncthreads();
@@ -871,41 +884,41 @@ __global__ __launch_bounds__(256) void moe_gemm_tiled_kernel(const bf16* __restr
     fetch(s + 2, buf, false);
     buf ^= 1;
     if (!idle) {
-      const Operands kept = cur;
-      cur = read(buf, 0);
-      multiply(kept);
+      const Weights kept_u = u;
+      const Rows kept = x;
+      u = read_weights(buf, 0);
+      x = read_rows(buf, 0, 0);
+      multiply(kept_u, kept, 1);
     }
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();  // the slices are done with
-  // acc[r][b][i]: feature n0 + wc * 64 + b * 32 + (i / 4) * 8 + khalf * 4 + i % 4 of tile row wr * 32 RB + r * 32 + r32.
+  // acc[r][b][i]: feature n0 + wc * 64 + b * 16 + quad * 4 + i of tile row wr * 32 RB + r * 16 + c16.
   // N is a multiple of 8: four features are all inside or all outside.
   const bool paired = UP && act == 5;
   const bool staged = !UP || N % (paired ? 16 : 8) == 0;  // rows of results are multiples of 16 bytes
 #pragma unroll
-  for (int r = 0; r < RB; ++r) {
-    const int row = (wr * RB + r) * 32 + r32;
+  for (int r = 0; r < 2 * RB; ++r) {
+    const int row = wr * 32 * RB + r * 16 + c16;
     const int pair = pair_of[row];
     if (pair < 0) continue;
     const float pw = UP ? 1.f : pair_weights[pair];
 #pragma unroll
-    for (int b = 0; b < 2; ++b)
+    for (int b = 0; b < 4; ++b) {
+      const int f = wc * 64 + b * 16 + quad * 4;
+      float v[4];
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int f = wc * 64 + b * 32 + g * 8 + khalf * 4;
-        float v[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = acc[r][b][g * 4 + i];
-        if constexpr (!UP) {
-          *reinterpret_cast<f32x4_t*>(moe_lds + row * kBigRowF32 + f * 4) = f32x4_t{pw * v[0], pw * v[1], pw * v[2], pw * v[3]};
-        } else if (paired) {
-          bf16* const to = staged ? reinterpret_cast<bf16*>(moe_lds + row * kBigRowBf16) + f / 2
-                                  : static_cast<bf16*>(out) + static_cast<int64_t>(row0 + row) * (N / 2) + (n0 + f) / 2;
-          if (staged || n0 + f < N) store_clamped_glu(to, v, glu_limit, glu_alpha);
-        } else {
-          *reinterpret_cast<u16x4_t*>(moe_lds + row * kBigRowBf16 + f * 2) = activated4(v, act);
-        }
+      for (int i = 0; i < 4; ++i) v[i] = acc[r][b][i];
+      if constexpr (!UP) {
+        *reinterpret_cast<f32x4_t*>(moe_lds + row * kBigRowF32 + f * 4) = f32x4_t{pw * v[0], pw * v[1], pw * v[2], pw * v[3]};
+      } else if (paired) {
+        bf16* const to = staged ? reinterpret_cast<bf16*>(moe_lds + row * kBigRowBf16) + f / 2
+                                : static_cast<bf16*>(out) + static_cast<int64_t>(row0 + row) * (N / 2) + (n0 + f) / 2;
+        if (staged || n0 + f < N) store_clamped_glu(to, v, glu_limit, glu_alpha);
+      } else {
+        *reinterpret_cast<u16x4_t*>(moe_lds + row * kBigRowBf16 + f * 2) = activated4(v, act);
       }
+    }
   }
   if (!staged) return;
   __syncthreads();
@@ -926,9 +939,9 @@ __global__ __launch_bounds__(256) void moe_gemm_tiled_kernel(const bf16* __restr
 }
 
 // Tiles of 256 rows and 256 features by eight wavefronts in two groups that take turns, one multiplying while the other reads its
-// operands: the loop of gemm_phased_kernel (its comment explains the phases and the wait counts) over gathered rows.  What differs:
+// operands: the loop of gemm_phased_kernel (its comment explains the phases, the wait counts and the products' shape) over gathered rows.  What differs:
 //  * quarter X0 holds the tile's rows 0 .. 127 and X1 the others, and a group takes 64 of each, so that the groups share the work of a
-//    tile that is not full; blocks of 32 rows without rows are not multiplied (187 rows: six of eight).
+//    tile that is not full; blocks of 64 rows without rows are not multiplied (187 rows: three of four).
 //  * the first slice's weights are asked for ahead of its rows, whose places have to be looked up first.
 //  * the down product's rows are twice as wide as LDS has room for: they leave in two halves.
 // An expert with up to 256 rows has its weights read once.  The workgroup -> (tile, features) map is the kernel's above.
@@ -963,7 +976,7 @@ __global__ __launch_bounds__(512, 2) void moe_gemm_phased_kernel(const bf16* __r
   const int lane = tid % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int wm = wave / 4, wn = wave % 4;  // wavefronts w and w + 4 share a SIMD: one of each group
-  const int r32 = lane % 32, h = lane / 32;
+  const int c16 = lane % 16, quad = lane / 16;
   const unsigned row_bytes = static_cast<unsigned>(K) * 2u;
   const __amdgpu_buffer_rsrc_t w_buf = make_buffer(w + (static_cast<int64_t>(expert) * N + n0) * K, static_cast<unsigned>(min(kSqCols, N - n0)) * row_bytes);
   const __amdgpu_buffer_rsrc_t x_buf = make_buffer(a, static_cast<unsigned>(a_rows) * row_bytes);
@@ -1007,39 +1020,39 @@ __global__ __launch_bounds__(512, 2) void moe_gemm_phased_kernel(const bf16* __r
                                                in && x_off[i][p] != kNoRow ? x_off[i][p] + step * 128u : kNoRow, 0, 0, 0);
   };
 
-  f32x16_t acc[2][4];  // feature half; row half * 2 + block of 32
+  f32x4_t acc[4][8];  // blocks of 16 features (half * 2 + block) and of 16 rows (half * 4 + block)
 #pragma unroll
-  for (int j = 0; j < 2; ++j)
+  for (int j = 0; j < 4; ++j)
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[j][i][e] = 0.f;
+    for (int i = 0; i < 8; ++i) acc[j][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   // whether this group has rows in each half
   bool any[2];
 #pragma unroll
   for (int i = 0; i < 2; ++i) any[i] = __builtin_amdgcn_readfirstlane(static_cast<int>(i * 128 + wm * 64 < rows)) != 0;
-  const int swz = (r32 / 2) % 8;
-  const int w_base = (wn * 32 + r32) * 128;
-  const int x_base = 2 * kSqQuarter + (wm * 64 + r32) * 128;
+  const int swz = c16 / 2;
+  const int w_base = (wn * 32 + c16) * 128;
+  const int x_base = 2 * kSqQuarter + (wm * 64 + c16) * 128;
   struct Weights {
-    bf16x8_t v[4];
+    bf16x8_t v[2][2];  // 32 of k, block of 16 features
   };
   struct Rows {
-    bf16x8_t v[4][2];
+    bf16x8_t v[2][4];
   };
   auto read_weights = [&](Weights& t, int buf, int j) {
     if (!any[0]) return;
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk)
-      t.v[kk] = load_bf16x8(moe_lds + buf * kSqBuffer + j * kSqQuarter + w_base + (((kk * 2 + h) ^ swz) * 16));
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+        t.v[kk][b] = load_bf16x8(moe_lds + buf * kSqBuffer + j * kSqQuarter + w_base + b * 16 * 128 + (((kk * 4 + quad) ^ swz) * 16));
   };
   auto read_rows = [&](Rows& t, int buf, int i) {
     if (!any[i]) return;
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk)
+    for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
-      for (int b = 0; b < 2; ++b)
-        t.v[kk][b] = load_bf16x8(moe_lds + buf * kSqBuffer + i * kSqQuarter + x_base + b * 32 * 128 + (((kk * 2 + h) ^ swz) * 16));
+      for (int b = 0; b < 4; ++b)
+        t.v[kk][b] = load_bf16x8(moe_lds + buf * kSqBuffer + i * kSqQuarter + x_base + b * 16 * 128 + (((kk * 4 + quad) ^ swz) * 16));
   };
 #define MLR_READ_DONE(pending)                                                                   \
   do {                                                                                           \
@@ -1052,9 +1065,14 @@ __global__ __launch_bounds__(512, 2) void moe_gemm_phased_kernel(const bf16* __r
     __builtin_amdgcn_s_setprio(1);
     if (any[i]) {
 #pragma unroll
-      for (int kk = 0; kk < 4; ++kk)
+      for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
-        for (int c = 0; c < 2; ++c) acc[j][i * 2 + c] = mfma_32x32x16(t.v[kk], b.v[kk][c], acc[j][i * 2 + c]);
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+          for (int f = 0; f < 2; ++f) {
+            f32x4_t& sum = acc[j * 2 + turn_at(f, c, 2)][i * 4 + c];
+            sum = mfma_16x16x32(t.v[kk][turn_at(f, c, 2)], b.v[kk][c], sum);
+          }
     }
     __builtin_amdgcn_s_setprio(0);
     __builtin_amdgcn_sched_barrier(0);
@@ -1103,7 +1121,7 @@ __global__ __launch_bounds__(512, 2) void moe_gemm_phased_kernel(const bf16* __r
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing may still be on its way into LDS
   __syncthreads();
 
-  // acc[j][i * 2 + c][e]: feature n0 + wn * 64 + j * 32 + (e / 4) * 8 + h * 4 + e % 4 of tile row i * 128 + wm * 64 + c * 32 + r32.
+  // acc[j][i * 4 + c][e]: feature n0 + wn * 64 + j * 16 + quad * 4 + e of tile row i * 128 + wm * 64 + c * 16 + c16.
   // N is a multiple of 8: four features are all inside or all outside.
   const bool paired = UP && act == 5;
   const bool staged = !UP || N % (paired ? 16 : 8) == 0;  // rows of results are multiples of 16 bytes
@@ -1114,29 +1132,27 @@ __global__ __launch_bounds__(512, 2) void moe_gemm_phased_kernel(const bf16* __r
   for (int i = 0; i < 2; ++i) {
     const int half0 = UP ? 0 : i * 128;  // the first tile row that is in LDS
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      const int at = i * 128 + wm * 64 + c * 32 + r32;
+    for (int c = 0; c < 4; ++c) {
+      const int at = i * 128 + wm * 64 + c * 16 + c16;
       const int pair = pair_of[at];
       if (pair < 0) continue;
       const float pw = UP ? 1.f : pair_weights[pair];
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < 4; ++j) {
+        const int f = wn * 64 + j * 16 + quad * 4;
+        float v[4];
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const int f = wn * 64 + j * 32 + g * 8 + h * 4;
-          float v[4];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) v[e] = acc[j][i * 2 + c][g * 4 + e];
-          if constexpr (!UP) {
-            *reinterpret_cast<f32x4_t*>(moe_lds + (at - half0) * kSqRowF32 + f * 4) = f32x4_t{pw * v[0], pw * v[1], pw * v[2], pw * v[3]};
-          } else if (paired) {
-            bf16* const to = staged ? reinterpret_cast<bf16*>(moe_lds + at * kSqRowBf16) + f / 2
-                                    : static_cast<bf16*>(out) + static_cast<int64_t>(row0 + at) * (N / 2) + (n0 + f) / 2;
-            if (staged || n0 + f < N) store_clamped_glu(to, v, glu_limit, glu_alpha);
-          } else {
-            *reinterpret_cast<u16x4_t*>(moe_lds + at * kSqRowBf16 + f * 2) = activated4(v, act);
-          }
+        for (int e = 0; e < 4; ++e) v[e] = acc[j][i * 4 + c][e];
+        if constexpr (!UP) {
+          *reinterpret_cast<f32x4_t*>(moe_lds + (at - half0) * kSqRowF32 + f * 4) = f32x4_t{pw * v[0], pw * v[1], pw * v[2], pw * v[3]};
+        } else if (paired) {
+          bf16* const to = staged ? reinterpret_cast<bf16*>(moe_lds + at * kSqRowBf16) + f / 2
+                                  : static_cast<bf16*>(out) + static_cast<int64_t>(row0 + at) * (N / 2) + (n0 + f) / 2;
+          if (staged || n0 + f < N) store_clamped_glu(to, v, glu_limit, glu_alpha);
+        } else {
+          *reinterpret_cast<u16x4_t*>(moe_lds + at * kSqRowBf16 + f * 2) = activated4(v, act);
         }
+      }
     }
     if (!staged || (UP && i == 0)) continue;
     __syncthreads();
