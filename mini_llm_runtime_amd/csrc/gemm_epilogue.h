@@ -416,6 +416,100 @@ __device__ __forceinline__ void qkv_store4(const QkvTarget& qkv, int row0, int t
   }
 }
 
+// The whole epilogue for a tile whose features are whole heads (the head size divides BN), staged in LDS as by stage_tile: queries and
+// keys leave 16 bytes a lane, a piece and its rotation partner at a time, and so do the values where eight tokens behind one another
+// have slots behind one another in a page (a prompt's have), 8 tokens of a dim a lane.  The product as bfloat16 first, then the
+// rotation, as by the kernels one after the other.  q_out and the pages are 16-byte aligned and pages hold a multiple of 8 tokens.
+template <int THREADS, int BM, int BN, int NI, int NJ>
+__device__ __forceinline__ void stage_qkv(const GemmEpilogue& ep, const QkvTarget& qkv, const f32x4_t (&acc)[NI][NJ], unsigned char* lds,
+                                          const float* scales, int feature0, int token0, int m0, int n0, int M, int N) {
+  constexpr int kRow = BN * 2 + 16;
+  const int c16 = threadIdx.x % 16, quad = threadIdx.x % kWave / 16;
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int f = feature0 + i * 16 + quad * 4;
+    float b[4] = {0.f, 0.f, 0.f, 0.f};
+    if (ep.bias != nullptr && n0 + f < N) {  // N is a multiple of 16
+#pragma unroll
+      for (int e = 0; e < 4; ++e) b[e] = load_as_f32(ep.bias, n0 + f + e, ep.bias_is_f32);
+    }
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const int token = token0 + j * 16 + c16;
+      const float scale = ep.row_sumsq != nullptr ? scales[token] : 1.f;
+      float v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = acc[i][j][e] * scale + b[e];
+      typedef uint32_t words_t __attribute__((ext_vector_type(2)));
+      *reinterpret_cast<words_t*>(lds + token * kRow + f * 2) = words_t{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+    }
+  }
+  __syncthreads();
+  const int D = qkv.head_dim, half = D / 2, per_head = half / 8;  // pairs of pieces of a head
+  const int head0 = n0 / D, turning = qkv.heads + qkv.kv_heads;
+  // queries and keys: pairs of pieces
+  const int pairs = max(0, min(BN / D, turning - head0)) * per_head;  // of a token
+  for (int p = threadIdx.x; p < BM * pairs; p += THREADS) {
+    const int row = p / pairs, at = p - row * pairs, local = at / per_head, d = (at - local * per_head) * 8;
+    const int m = m0 + row, head = head0 + local;
+    if (m >= M) break;
+    const unsigned char* const from = lds + row * kRow + (local * D + d) * 2;
+    u16x8_t lo = *reinterpret_cast<const u16x8_t*>(from), hi = *reinterpret_cast<const u16x8_t*>(from + half * 2);
+    if (qkv.cos != nullptr) {
+      const float* const cs = qkv.cos + static_cast<int64_t>(m) * half + d;
+      const float* const sn = qkv.sin + static_cast<int64_t>(m) * half + d;
+      const f32x4_t c[2] = {*reinterpret_cast<const f32x4_t*>(cs), *reinterpret_cast<const f32x4_t*>(cs + 4)};
+      const f32x4_t t[2] = {*reinterpret_cast<const f32x4_t*>(sn), *reinterpret_cast<const f32x4_t*>(sn + 4)};
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float a = to_f32(bf16{lo[e]}), b = to_f32(bf16{hi[e]});
+        lo[e] = f32_to_bf16(a * c[e / 4][e % 4] - b * t[e / 4][e % 4]).bits;
+        hi[e] = f32_to_bf16(b * c[e / 4][e % 4] + a * t[e / 4][e % 4]).bits;
+      }
+    }
+    bf16* to = qkv.q_out + (static_cast<int64_t>(m) * qkv.heads + head) * D;
+    if (head >= qkv.heads) {
+      const int slot = qkv.slots != nullptr ? qkv.slots[m] : -1, page = slot / qkv.block_size;
+      if (slot < 0 || page >= qkv.num_pages) continue;
+      to = qkv.key_pages + ((static_cast<int64_t>(page) * qkv.kv_heads + head - qkv.heads) * qkv.block_size + slot - page * qkv.block_size) * D;
+    }
+    *reinterpret_cast<u16x8_t*>(to + d) = lo;
+    *reinterpret_cast<u16x8_t*>(to + d + half) = hi;
+  }
+  // values: eight tokens of a dim, pairs of eights side by side (32 bytes of a page of 16)
+  if (qkv.slots == nullptr) return;
+  const int first = max(0, turning - head0) * D, columns = min(BN, N - n0) - first;  // the tile's value columns
+  if (columns <= 0) return;
+  for (int p = threadIdx.x; p < BM / 8 * columns; p += THREADS) {
+    const int pair = p / (2 * columns), at = p - pair * 2 * columns;
+    const int row = (pair * 2 + at % 2) * 8, column = first + at / 2;
+    if (m0 + row >= M) continue;
+    const int count = min(8, M - m0 - row);
+    const int head = head0 + column / D - turning, d = column % D;
+    int slots[8];
+    bool together = count == 8;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      slots[e] = qkv.slots[min(m0 + row + e, M - 1)];
+      together = together && slots[e] == slots[0] + e;
+    }
+    const auto value_at = [&](int slot) {
+      const int page = slot / qkv.block_size;
+      return ((static_cast<int64_t>(page) * qkv.kv_heads + head) * D + d) * qkv.block_size + slot - page * qkv.block_size;
+    };
+    u16x8_t v;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = *reinterpret_cast<const unsigned short*>(lds + (row + e) * kRow + column * 2);
+    if (together && slots[0] >= 0 && slots[0] % 8 == 0 && slots[0] / qkv.block_size < qkv.num_pages) {
+      *reinterpret_cast<u16x8_t*>(qkv.value_pages + value_at(slots[0])) = v;
+      continue;
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      if (e < count && slots[e] >= 0 && slots[e] / qkv.block_size < qkv.num_pages) qkv.value_pages[value_at(slots[e])].bits = v[e];
+  }
+}
+
 // Rotation and stores of the fused query/key/value product for one token: the lane holds the
 // sums of four consecutive dims d0..d0+3 of `head`, which are the low halves (`low`) or the high
 // halves of the rotation pairs j0..j0+3; the lane `partner_mask` away holds the other halves.

@@ -28,9 +28,9 @@
 //    With more than one K slice both kernels write float32 partial sums
 //    [slice, M, N]; the consumer (the residual-adding norm kernel) sums them in a
 //    fixed order, so results do not depend on which slice finishes first.
-//  * Both also run the query/key/value product with bias, rotation and the cache write as
+//  * They also run the query/key/value product with bias, rotation and the cache write as
 //    their epilogue (QkvTarget): the streaming kernels for up to 64 tokens (in slabs of 16 beyond 16),
-//    the tiled one beyond.
+//    the tiled one beyond, and the 128 x 128 tiles (staged_qkv_kernel).
 // K must be a multiple of 8 (16-byte rows); other shapes take the FMA kernel.
 //
 // SwiGLU epilogue: with gate and up rows interleaved in pairs
@@ -729,9 +729,11 @@ constexpr int direct_lds_bytes(int tokens, int features, int waves, int buffers)
 }
 
 // FIXED: an epilogue fixed at compile time (kEpGeglu, for the tile that has no room for a choice), or -1.
-template <int WM, int WN, int GM, int GN, int NBUF = 2, bool ONCE = false, int FIXED = -1>
+// QKV: the query/key/value product, with its epilogue (stage_qkv).
+template <int WM, int WN, int GM, int GN, int NBUF = 2, bool ONCE = false, int FIXED = -1, bool QKV = false>
 __global__ __launch_bounds__(64 * GM * GN) void gemm_direct_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w,
-                                                                  GemmEpilogue ep, TileOrder order, int M, int N, int K) {
+                                                                  GemmEpilogue ep, QkvTarget qkv, TileOrder order, int M, int N,
+                                                                  int K) {
   constexpr int BM = 32 * WM * GM, BN = 32 * WN * GN, WAVES = GM * GN;
   constexpr int kRowBytes = kBK * 2;
   constexpr int kRowPieces = kBK / 8;           // 16-byte pieces of a row
@@ -893,6 +895,12 @@ __global__ __launch_bounds__(64 * GM * GN) void gemm_direct_kernel(const bf16* _
   }
   // finished tiles of many tokens leave through LDS where they fit it (see stage_tile)
   constexpr int kLds = NBUF * kBufferBytes;
+  if constexpr (QKV) {
+    static_assert(staged_tile_bytes(BM, BN) <= kLds, "the staged tile fits");
+    __syncthreads();  // everybody's loads have landed and nobody reads the slices any more
+    stage_qkv<64 * GM * GN, BM, BN>(ep, qkv, acc, smem, scales, wn * 32 * WN, wm * 32 * WM, m0, n0, M, N);
+    return;
+  }
   constexpr bool kStagesPairs = BM >= 128 && staged_tile_bytes(BM, BN / 2) <= kLds;
   constexpr bool kStagesPlain = BM >= 128 && FIXED < 0 && staged_tile_bytes(BM, BN) <= kLds;
   constexpr int kSumRows = BM >= 128 && FIXED < 0 && WM * WN < 10 ? staged_sums_rows(BM, BN, 32 * WM, kLds) : 0;
@@ -966,7 +974,7 @@ constexpr int kPhaseLds = staged_tile_bytes(256, 256);  // a little more than th
 static_assert(kPhaseLds >= 2 * kPhaseBuffer, "the slices fit");
 
 __global__ __launch_bounds__(512, 2) void gemm_phased_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, GemmEpilogue ep,
-                                                            TileOrder order, int M, int N, int K) {
+                                                            QkvTarget, TileOrder order, int M, int N, int K) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   __shared__ float scales[256];
   const int lane = threadIdx.x % kWave;
@@ -1148,8 +1156,9 @@ constexpr int kTurnSlice = 256 * 128;  // bytes: 64 k of 128 features, then of 1
 constexpr int kTurnLds = 4 * kTurnSlice;
 static_assert(kTurnLds >= 65536 + staged_tile_bytes(128, 128), "the sums that change hands, and the staged tile behind them, fit");
 
+template <bool QKV>
 __global__ __launch_bounds__(512, 2) void gemm_turns_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, GemmEpilogue ep,
-                                                           TileOrder order, int M, int N, int K) {
+                                                           QkvTarget qkv, TileOrder order, int M, int N, int K) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   __shared__ float scales[128];
   const int lane = threadIdx.x % kWave;
@@ -1254,6 +1263,10 @@ __global__ __launch_bounds__(512, 2) void gemm_turns_kernel(const bf16* __restri
 #pragma unroll
     for (int j = 0; j < 4; ++j) sum[i][j] += *reinterpret_cast<const f32x4_t*>(smem + (((wave ^ 4) * 2 + i) * 4 + j) * 1024 + lane * 16);
   const int feature0 = wc * 64 + group * 32, token0 = wr * 64;
+  if constexpr (QKV) {
+    stage_qkv<512, 128, 128>(ep, qkv, sum, smem + 65536, scales, feature0, token0, m0, n0, M, N);
+    return;
+  }
   if (stages_tile(ep, slices, N)) {
     if (ep.swiglu == kEpSwiglu)
       stage_tile<kEpSwiglu, 512, 128, 128>(ep, sum, smem + 65536, scales, feature0, token0, m0, n0, M, N);
@@ -1278,11 +1291,11 @@ __global__ __launch_bounds__(512, 2) void gemm_turns_kernel(const bf16* __restri
     }
 }
 
-using DirectKernel = void (*)(const bf16*, const bf16*, GemmEpilogue, TileOrder, int, int, int);
+using DirectKernel = void (*)(const bf16*, const bf16*, GemmEpilogue, QkvTarget, TileOrder, int, int, int);
 // `wave_rows`: rows of wavefronts in the tile (a last token tile that fills only the first is light)
 static int launch_direct(DirectKernel kernel, int tile_tokens, int tile_features, int threads, int wave_rows, int lds_bytes,
                          bool& configured, const bf16* xb, const bf16* wb, const GemmEpilogue& ep, int m, int n, int k,
-                         int slices, hipStream_t stream) {
+                         int slices, hipStream_t stream, const QkvTarget& qkv = QkvTarget{}) {
   const TileOrder order = make_tile_order(m, (n + tile_features - 1) / tile_features, slices, tile_tokens, wave_rows);
   const int64_t groups = static_cast<int64_t>(order.m_tiles) * order.n_tiles * slices;
   if (groups >= (1ll << 31)) {
@@ -1297,7 +1310,7 @@ static int launch_direct(DirectKernel kernel, int tile_tokens, int tile_features
     }
     configured = true;
   }
-  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(groups)), dim3(threads), lds_bytes, stream, xb, wb, ep, order, m, n, k);
+  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(groups)), dim3(threads), lds_bytes, stream, xb, wb, ep, qkv, order, m, n, k);
   return 0;
 }
 
@@ -1677,7 +1690,7 @@ static int gemm_bf16(const bf16* xb, const bf16* wb, const GemmEpilogue& ep, int
     case 23: return gemm_bf16(xb, wb, ep, m, n, k, slices, takes_turns(m, n, k, slices) ? 24 : 25, stream);
     case 24: {  // 128 x 128, eight wavefronts in two groups that share the slices of k
       static bool configured = false;
-      return launch_direct(gemm_turns_kernel, 128, 128, 512, 2, kTurnLds, configured, xb, wb, ep, m, n, k, slices, stream);
+      return launch_direct(gemm_turns_kernel<false>, 128, 128, 512, 2, kTurnLds, configured, xb, wb, ep, m, n, k, slices, stream);
     }
     case 25: {
       static bool configured = false;
@@ -1686,6 +1699,24 @@ static int gemm_bf16(const bf16* xb, const bf16* wb, const GemmEpilogue& ep, int
     }
     default: set_error("mlr_gemm_bf16: kernel must be 0 (chosen by shape), 16, 14, 11, 22 to 25, 44 to 48, 62 to 68 or 71 to 74"); return -1;
   }
+}
+
+// Whether the query/key/value product may take tiles of 128 x 128 with the staged epilogue (stage_qkv).
+static bool staged_qkv_fits(const QkvTarget& t) {
+  return 128 % t.head_dim == 0 && (t.slots == nullptr || t.block_size % 8 == 0) && reinterpret_cast<uintptr_t>(t.q_out) % 16 == 0 &&
+         reinterpret_cast<uintptr_t>(t.key_pages) % 16 == 0 && reinterpret_cast<uintptr_t>(t.value_pages) % 16 == 0;
+}
+// And which, if any: gemm_turns (24) for a round of tiles that leaves few units without one (up to 79 tiles, or 127 of a long k, the 64 x 64
+// tiles with their epilogue from registers, or the plain product and the rotation kernel, are as fast or faster), gemm_direct (25),
+// two tiles a unit, up to 512.  Microseconds in a replayed graph, weights from memory, the best of the other two ways / this one: 896 x 1,152 at
+// 768 tokens (54 tiles) 12.7 / 14.4, at 1,024 (72) 15.0 / 14.5, at 2,048 18.3 / 15.2, at 3,072 21.8 / 15.7, at 4,096 (288) 27.2 / 23.7, at
+// 6,000 (423) 31.2 / 25.0, at 8,191 (576) 36.8 / 37.0; 2,048 x 3,072 at 512 (96) 25.3 / 25.2, at 1,048 28.4 / 23.8, at 2,000 (384) 46.9 / 42.0, at
+// 3,072 (576) 59.3 / 64.0; 3,584 x 4,608 at 256 (72) 33.1 / 41.4, at 512 (144) 43.2 / 39.8, at 1,048 (324) 62.3 / 59.0, at 1,536 (432) 68.5 /
+// 62.5, at 2,000 (576) 86 / 116; 5,120 x 7,168 at 256 (112) 51.1 / 59.6, at 512 (224) 63.8 / 58.2, at 1,048 (504) 98.8 / 90.3.
+static int staged_qkv_kernel(int m, int64_t n, int k) {
+  const int64_t tiles = ((m + 127) / 128) * ((n + 127) / 128);
+  if (m <= 64 || k < 8 * kBK || tiles < (k <= 2048 ? 80 : 128) || tiles > 2 * kComputeUnits) return 0;
+  return tiles <= kComputeUnits ? 24 : 25;
 }
 
 }  // namespace mlr
@@ -1773,11 +1804,17 @@ int mlr_gemm_bf16(const void* x, const void* w, const void* bias, int bias_is_f3
   return 0;
 }
 
+// Whether mlr_qkv_rope_write_bf16 has tiles of 128 x 128 for a product of these sizes (block_size 0: no cache write), which make it
+// the fastest way; beyond them the plain product with the rotation kernel behind it may be faster.
+int mlr_qkv_bf16_staged(int m, int n, int k, int head_dim, int block_size) {
+  return head_dim > 0 && 128 % head_dim == 0 && block_size % 8 == 0 && k % 8 == 0 && staged_qkv_kernel(m, n, k) != 0;
+}
+
 // The query/key/value product with everything that follows it before attention: bias, rotation of the query and key heads (cos, sin: [m, head_dim / 2] float32,
 // or null for none), queries to q_out [m, heads * head_dim], keys and values into the slots
 // of their pages (`write` 0: another layer owns the pages).  w is [(heads + 2 kv_heads) *
 // head_dim, k]; head_dim a multiple of 16, k of 8.  kernel: 0 chooses (the streaming kernel up
-// to 64 tokens unless it would read x too often, else a tiled one), or 16, 11, 22, 44.
+// to 64 tokens unless it would read x too often, else a tiled one), or 16, 11, 22, 44, or 24 and 25 (tiles of 128 x 128 with a staged epilogue).
 int mlr_qkv_rope_write_bf16(const void* x, const void* w, const void* bias, int bias_is_f32, const float* cos,
                             const float* sin, const int* slots, void* key_pages, void* value_pages, void* q_out,
                             int m, int k, int heads, int kv_heads, int head_dim, int block_size, int num_pages,
@@ -1803,12 +1840,28 @@ int mlr_qkv_rope_write_bf16(const void* x, const void* w, const void* bias, int 
                    static_cast<bf16*>(q_out), heads, kv_heads, head_dim, block_size, num_pages};
   const bf16* xb = static_cast<const bf16*>(x);
   const bf16* wb = static_cast<const bf16*>(w);
+  const bool stages = staged_qkv_fits(target);
   if (kernel == 0) {
-    // Beyond 64 tokens the 64 x 64 tiles: with this epilogue (rotation, scattered cache stores) the
-    // larger tiles are slower than they are for the plain product, and where those would pay the
-    // caller does better with the plain product and the rotation kernel behind it.
+    // Beyond 64 tokens tiles of 128 x 128 where staged_qkv_kernel has them, else the 64 x 64 tiles: with the epilogue from registers
+    // (rotation, scattered cache stores) the larger tiles are slower than they are for the plain product.
     kernel = m <= 64 ? 16 : 11;
     if (kernel == 16 && m > 16 && (n / 16) * m * k * 2 > (32ll << 20)) kernel = 11;  // too many passes over x
+    if (stages && staged_qkv_kernel(m, n, k) != 0) kernel = staged_qkv_kernel(m, n, k);
+  }
+  MLR_REQUIRE((kernel != 24 && kernel != 25) || stages, "the staged kernels take head sizes that divide 128, pages of a multiple of 8 tokens and 16-byte alignment");
+  if (kernel == 24) {
+    static bool configured = false;
+    if (launch_direct(gemm_turns_kernel<true>, 128, 128, 512, 2, kTurnLds, configured, xb, wb, ep, m, static_cast<int>(n), k, 1, stream, target) != 0) return -1;
+    MLR_LAUNCH_CHECK();
+    return 0;
+  }
+  if (kernel == 25) {
+    static bool configured = false;
+    if (launch_direct(gemm_direct_kernel<2, 2, 2, 2, 2, false, -1, true>, 128, 128, 256, 2, direct_lds_bytes(128, 128, 4, 2), configured, xb, wb, ep, m,
+                      static_cast<int>(n), k, 1, stream, target) != 0)
+      return -1;
+    MLR_LAUNCH_CHECK();
+    return 0;
   }
   if (kernel == 8) {
     MLR_REQUIRE(m <= 8, "the 8-row kernel takes 1..8 tokens");

@@ -108,6 +108,7 @@ _SIGNATURES = {
     "mlr_gemm_residual_bf16": ([_VP, _VP, _VP, _I, _VP, _VP, _I, _VP, _VP, _I, _I, _I, _VP], _I),
     "mlr_gemm_bf16_slices": ([_I, _I, _I, _I], _I),
     "mlr_gemm_bf16_kernel": ([_I, _I, _I, _I], _I),
+    "mlr_qkv_bf16_staged": ([_I, _I, _I, _I, _I], _I),
     "mlr_qkv_rope_write_bf16": (
         [_VP, _VP, _VP, _I, _VP, _VP, _VP, _VP, _VP, _VP, _I, _I, _I, _I, _I, _I, _I, _I, _I, _VP, _I, _F, _VP],
         _I,
@@ -933,12 +934,13 @@ class HipOps:
             )
             return q
         if fused is None:
-            # The fused kernel has 64 x 64 tiles only; beyond 2^33 multiply-adds the plain product in the planner's tiles with the
-            # rotation kernel behind it is the faster way.  Fused / plain, in a replayed graph, us: 0.5B sizes at 4,096 tokens (4.2e9)
-            # 27 / 29; 1.5B at 1,536 (4.8e9) 25 / 27, at 4,096 (1.3e10) 60 / 43; 7B at 512 (8.5e9) 42 / 44, at 768 (1.3e10) 54 / 46, at
+            # The fused kernel is the fastest way where it has 128 x 128 tiles for the shape (one or two rounds of them, whole heads).
+            # Its 64 x 64 tiles, beyond 2^33 multiply-adds or 512 such tiles, are not: there the plain product in the planner's tiles
+            # with the rotation kernel behind it.  In 64 x 64 tiles / plain, in a replayed graph, us: 0.5B sizes at 4,096 tokens (4.2e9)
+            # 27 / 29, at 8,191 (576 tiles) 46 / 37; 1.5B at 4,096 (1.3e10) 60 / 43; 7B at 384 (6.3e9) 39 / 41, at 768 (1.3e10) 54 / 46, at
             # 1,024 69 / 58, at 2,048 129 / 83; 14B at 400 (1.5e10) 75 / 76, at 512 88 / 78.
-            large = m > 64 and m * width * k >= 1 << 33
-            fused = can_fuse and not large
+            large = m > 64 and (m * width * k >= 1 << 33 or -(-m // 128) * -(-width // 128) > 512)
+            fused = can_fuse and (not large or self.lib.mlr_qkv_bf16_staged(m, width, k, head_dim, block_size if write else 0) != 0)
         elif fused and not can_fuse:
             raise KernelError("the fused query/key/value kernel takes bfloat16 tokens and a full rotation")
         if pending is not None and not (

@@ -475,6 +475,42 @@ def test_fused_qkv_rotation_cache_write_equals_the_three_kernels(ops_for, heads,
     assert torch.isnan(out[True][1]).all() == (not write)
 
 
+@pytest.mark.parametrize("kernel", [24, 25])
+@pytest.mark.parametrize("heads,kv_heads,head_dim,hidden,tokens,bs,start,rotate,write,bias", [
+    # one token more than a tile, one fewer, fewer than eight; slots from the middle of a page and of eight of them on; a tile with the last queries, the keys and
+    # the first values; values only, keys only; k of one step, not a multiple of a step, an odd number of steps
+    (14, 2, 64, 896, 129, 16, 0, True, True, True), (14, 2, 64, 896, 127, 16, 5, True, True, True), (3, 2, 64, 520, 5, 16, 8, True, True, False),
+    (6, 1, 16, 40, 200, 8, 3, True, True, True), (3, 3, 128, 264, 140, 24, 16, True, True, True), (5, 4, 32, 72, 133, 16, 8, False, True, True),
+    (3, 1, 128, 192, 150, 16, 0, True, False, True),
+])
+def test_staged_qkv_product_of_consecutive_slots(ops_for, kernel, heads, kv_heads, head_dim, hidden, tokens, bs, start, rotate, write, bias):
+    """Tokens behind one another in pages, as a prompt's are, with a gap, a token without a slot and one out of range: eight values at a time and one by one."""
+    ops = ops_for(torch.bfloat16)
+    width, pages = (heads + 2 * kv_heads) * head_dim, (start + tokens) // bs + 4
+    x = _rand((tokens, hidden), torch.bfloat16, 71).cuda()
+    w = _rand((width, hidden), torch.bfloat16, 72, 0.2).cuda()
+    b = _rand((width,), torch.bfloat16, 73).cuda() if bias else None
+    rotation = None
+    if rotate:
+        inv = (1.0 / (1e6 ** (torch.arange(0, head_dim, 2, dtype=torch.float64) / head_dim))).cuda()
+        rotation = (*ops.rope_table(torch.arange(7, 7 + tokens, dtype=torch.int32).cuda(), inv), head_dim)
+    slots = torch.arange(start, start + tokens, dtype=torch.int32)
+    slots[tokens // 2 :] += 2 * bs  # another page, the same place in it
+    slots[2], slots[tokens - 1] = -1, pages * bs + 3
+    kp = torch.full((pages, kv_heads, bs, head_dim), float("nan"), dtype=torch.bfloat16).cuda()
+    vp = torch.full((pages, kv_heads, head_dim, bs), float("nan"), dtype=torch.bfloat16).cuda()
+    q = ops.qkv_rope_write(x, w, b, rotation, slots.cuda(), kp, vp, num_heads=heads, num_kv_heads=kv_heads, head_dim=head_dim,
+                           block_size=bs, write=write, fused=True, mfma_kernel=kernel)
+    reference = qkv_reference(x, w, b, rotation[0] if rotate else None, rotation[1] if rotate else None, heads, kv_heads, head_dim)
+    slots[tokens - 1] = -1  # nothing is written for it
+    check_qkv("staged", q.float().cpu(), kp.float().cpu(), vp.float().cpu(), slots, bs, reference, heads, kv_heads, head_dim, write=write)
+    written = torch.zeros(pages * bs, dtype=torch.bool)
+    written[slots[slots >= 0].long()] = write
+    written = written.view(pages, bs)
+    assert torch.isnan(kp.float().cpu()[~written[:, None, :, None].expand(kp.shape)]).all()
+    assert torch.isnan(vp.float().cpu()[~written[:, None, None, :].expand(vp.shape)]).all()
+
+
 @pytest.mark.parametrize("heads,kv_heads,head_dim,hidden,tokens,rotate,write", [
     (14, 2, 64, 896, 64, True, True), (14, 2, 64, 896, 33, True, True), (3, 1, 16, 520, 1, True, True),
     (5, 1, 128, 1208, 8, True, True), (4, 4, 80, 640, 17, False, True), (6, 3, 48, 2056, 5, True, False),
