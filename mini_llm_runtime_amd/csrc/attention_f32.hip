@@ -8,9 +8,11 @@
 //
 // Bound by the matrix cores (256 operations a clock and compute unit in float32): a 64-key tile of 64 queries at head size 64 is
 // 4,096 clocks of them for 32 KB of keys and values, which one LDS buffer with the next tile on its way in registers keeps up
-// with; a workgroup takes 64 queries of one head, four wavefronts 16 each.
+// with; and for short prompts by the chain of tiles that the last queries see.  A workgroup takes 64 queries of one head; two groups of four
+// wavefronts, 16 queries each, take the key tiles in turn and add up at the end, which halves that chain.
 // Measured at 0.5B sizes (14 query and 2 key/value heads of 64), prompts of 391, 268, 145 and 22 tokens in one step: 479 us with the
-// plain kernel (a wavefront per token and head, attention_simple.hip), 44 us here.
+// plain kernel (a wavefront per token and head, attention_simple.hip), 42 with one group and pages looked up beside the loads, 32 with
+// two groups, 27 here.
 #include "common.h"
 #include "mfma.h"
 
@@ -25,12 +27,16 @@ namespace f32_attention {
 constexpr int D = MLR_HEAD_DIM;
 constexpr int kDimTiles = D / 16;
 constexpr int kTileQ = 64;                 // queries of a workgroup
-constexpr int kTileK = D > 80 ? 32 : 64;   // keys in LDS at a time
+constexpr int kTileK = D > 80 ? 32 : 64;   // keys of a group in LDS at a time
+constexpr int kGroups = 2;                 // groups of four wavefronts, which take the key tiles in turn
 constexpr int kSubTiles = kTileK / 16;
 // rows padded to 32 bytes modulo 64: 16 rows x 4 pieces of 16 bytes are then read without bank conflicts
 constexpr int kKLd = D + 8;
 constexpr int kVLd = kTileK + 8;
 constexpr int kPieces = kTileK * D / 4 / 256;  // 16-byte pieces of a thread, of the key and of the value tile
+constexpr int kGroupFloats = kTileK * kKLd + D * kVLd;  // LDS of a group: its keys, then its values
+constexpr int kLdsBytes = kGroups * kGroupFloats * 4;
+static_assert(kGroupFloats >= (2 + D / 4) * 256, "what the second group hands over fits its tiles");
 static_assert(kTileK * D / 4 % 256 == 0, "whole pieces for every thread");
 
 // One token's attention by a wavefront, as paged_attention_simple_kernel has it: a lane scores a key and then owns dims.  For the few workgroups
@@ -93,28 +99,30 @@ __device__ void attend_alone(const float* __restrict__ q, int64_t q_stride, cons
 
 __device__ __attribute__((aligned(16))) const float kGoneKeys[4] = {__builtin_nanf(""), __builtin_nanf(""), __builtin_nanf(""), __builtin_nanf("")};
 
-__global__ __launch_bounds__(256) void attn_prefill_f32_kernel(
+__global__ __launch_bounds__(256 * kGroups) void attn_prefill_f32_kernel(
     const float* __restrict__ q, int64_t q_stride, const float* __restrict__ key_pages, const float* __restrict__ value_pages,
     const int* __restrict__ block_table, int table_width, const int* __restrict__ tiles, const int* __restrict__ cu_q,
     const int* __restrict__ context_lens, float* __restrict__ out, int heads, int kv_heads, int block_size, int num_pages,
     float scale, int window, int chunk, const float* __restrict__ sinks) {
-  __shared__ __attribute__((aligned(16))) float ks[kTileK * kKLd];
-  __shared__ __attribute__((aligned(16))) float vs[D * kVLd];
+  extern __shared__ __attribute__((aligned(16))) float tile_lds[];
   __shared__ int sm_odd;  // a value that is not finite has come in a tile of keys that some query here does not see whole
   const int tile = blockIdx.x / heads;
   const int head = blockIdx.x - tile * heads;
   const int kvh = head / (heads / kv_heads);
   const int entry = tiles[2 * tile];
   const int q0 = tiles[2 * tile + 1];
-  const int tid = threadIdx.x;
+  const int group = __builtin_amdgcn_readfirstlane(threadIdx.x / 256);
+  const int tid = threadIdx.x % 256;  // of the group
   const int lane = tid % kWave;
-  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);  // of the group: 16 queries
+  float* const ks = tile_lds + group * kGroupFloats;
+  float* const vs = ks + kTileK * kKLd;
   const int col = lane % 16, quarter = lane / 16;
   const int t_first = cu_q[entry];
   const int q_len = cu_q[entry + 1] - t_first;
   const int pos0 = context_lens[entry] - q_len;
   const int* table = block_table + static_cast<int64_t>(entry) * table_width;
-  if (tid == 0) sm_odd = 0;
+  if (threadIdx.x == 0) sm_odd = 0;
 
   const int qi = q0 + wave * 16 + col;
   const bool q_ok = qi < q_len;
@@ -137,6 +145,22 @@ __global__ __launch_bounds__(256) void attn_prefill_f32_kernel(
   const bool wave_has_queries = q0 + wave * 16 < q_len;
 
   f32x4_t k_flight[kPieces], v_flight[kPieces];
+  // The pages of a tile's pieces are looked up a turn ahead of their loads (looked up beside them they would be a trip to memory that
+  // everything waits for).  4 keys of a value piece lie in one page, whose size is a multiple of 4, and are the same for all of a thread's.
+  int k_page[kPieces], v_page = -1;
+  bool v_hidden[4] = {true, true, true, true};
+  static_assert(256 % (kTileK / 4) == 0, "a thread's value pieces are of the same keys");
+  auto page_of = [&](int key) {  // -1: past the table
+    const int logical = min(key, k_end - 1) / block_size;
+    const int page = table[min(logical, table_width - 1)];
+    return logical < table_width ? page : -1;
+  };
+  auto lookup = [&](int kt0) {
+    if (kt0 >= k_end) return;
+#pragma unroll
+    for (int i = 0; i < kPieces; ++i) k_page[i] = page_of(kt0 + (tid + i * 256) / (D / 4));
+    v_page = page_of(kt0 + tid % (kTileK / 4) * 4);
+  };
   // A page that is not there (or lies past the table) brings keys that are NaN: so is the sum of every query that sees one, and of no other
   auto fetch = [&](int kt0) {
     if (kt0 >= k_end) return;
@@ -144,33 +168,31 @@ __global__ __launch_bounds__(256) void attn_prefill_f32_kernel(
     for (int i = 0; i < kPieces; ++i) {
       const int c = tid + i * 256;
       const int key = kt0 + c / (D / 4), dim = c % (D / 4) * 4;
-      const int logical = min(key, k_end - 1) / block_size;
-      const int page = table[min(logical, table_width - 1)];
-      const bool in = logical < table_width && static_cast<unsigned>(page) < static_cast<unsigned>(num_pages);
-      const int64_t base = static_cast<int64_t>(in ? page : 0) * kv_heads + kvh;
+      const bool in = static_cast<unsigned>(k_page[i]) < static_cast<unsigned>(num_pages);
+      const int64_t base = static_cast<int64_t>(in ? k_page[i] : 0) * kv_heads + kvh;
       const float* piece = key_pages + (base * block_size + key % block_size) * D + dim;
       k_flight[i] = *reinterpret_cast<const f32x4_t*>(in ? piece : kGoneKeys);  // (a choice behind the load would wait for it here)
     }
+    const int key = kt0 + tid % (kTileK / 4) * 4;
+    const bool in = static_cast<unsigned>(v_page) < static_cast<unsigned>(num_pages);
+    const int64_t base = static_cast<int64_t>(in ? v_page : 0) * kv_heads + kvh;
 #pragma unroll
     for (int i = 0; i < kPieces; ++i) {
-      const int c = tid + i * 256;
-      const int key = kt0 + c % (kTileK / 4) * 4, dim = c / (kTileK / 4);  // 4 keys: they lie in one page, whose size is a multiple of 4
-      const int logical = min(key, k_end - 1) / block_size;
-      const int page = table[min(logical, table_width - 1)];
-      const bool in = logical < table_width && static_cast<unsigned>(page) < static_cast<unsigned>(num_pages);
-      const int64_t base = static_cast<int64_t>(in ? page : 0) * kv_heads + kvh;
-      f32x4_t v = *reinterpret_cast<const f32x4_t*>(value_pages + (base * D + dim) * block_size + key % block_size);
-      // values that no query here may see are cleared: what a page holds there may be anything, and 0 * NaN would come through
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (!in || key + e >= k_end || key + e < k_first) v[e] = 0.f;
-      v_flight[i] = v;
+      const int dim = (tid + i * 256) / (kTileK / 4);
+      v_flight[i] = *reinterpret_cast<const f32x4_t*>(value_pages + (base * D + dim) * block_size + key % block_size);
     }
+    // values that no query here may see are cleared where they are put down: what a page holds there may be anything, and 0 * NaN would
+    // come through
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v_hidden[e] = !in || key + e >= k_end || key + e < k_first;
   };
   auto stash = [&]() {
 #pragma unroll
     for (int i = 0; i < kPieces; ++i) {
       const int c = tid + i * 256;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (v_hidden[e]) v_flight[i][e] = 0.f;
       *reinterpret_cast<f32x4_t*>(ks + c / (D / 4) * kKLd + c % (D / 4) * 4) = k_flight[i];
       *reinterpret_cast<f32x4_t*>(vs + c / (kTileK / 4) * kVLd + c % (kTileK / 4) * 4) = v_flight[i];
     }
@@ -193,20 +215,25 @@ __global__ __launch_bounds__(256) void attn_prefill_f32_kernel(
   const int k_begin = k_first / kTileK * kTileK;
   const int k_all_first = first_visible_key(pos0 + q0 + kTileQ - 1, window, chunk);  // from here on no query here is past its window
   bool odd = false;
-  fetch(k_begin);
-  for (int kt0 = k_begin; kt0 < k_end; kt0 += kTileK) {
+  constexpr int kTurn = kGroups * kTileK;
+  lookup(k_begin + group * kTileK);
+  fetch(k_begin + group * kTileK);
+  lookup(k_begin + group * kTileK + kTurn);
+  for (int kt0 = k_begin + group * kTileK; kt0 - group * kTileK < k_end; kt0 += kTurn) {
     __syncthreads();  // everybody has done with the tile before
-    stash();
+    const bool any = kt0 < k_end;  // the last turn may have no tile for the second group
+    if (any) stash();
     // A hidden key's weight is 0, but 0 times an infinity or NaN is NaN, and the products would hand it to queries that do not see the key.
     const bool all_seen = kt0 + kTileK - 1 <= pos0 + q0 && kt0 >= k_all_first;
-    if (!all_seen && !all_finite()) sm_odd = 1;
+    if (any && !all_seen && !all_finite()) sm_odd = 1;
     __syncthreads();
-    if (!all_seen && sm_odd != 0) {
+    if (sm_odd != 0) {
       odd = true;
       break;
     }
-    fetch(kt0 + kTileK);  // on its way while this tile is computed
-    if (!(wave_has_queries && kt0 <= w_last && kt0 + kTileK > w_first)) continue;
+    fetch(kt0 + kTurn);  // on its way while this tile is computed
+    lookup(kt0 + 2 * kTurn);
+    if (!(any && wave_has_queries && kt0 <= w_last && kt0 + kTileK > w_first)) continue;
     f32x4_t s[kSubTiles];
 #pragma unroll
     for (int sub = 0; sub < kSubTiles; ++sub) {
@@ -260,10 +287,34 @@ __global__ __launch_bounds__(256) void attn_prefill_f32_kernel(
     }
   }
   if (odd) {  // the same for the whole workgroup: its queries one after the other, each over the keys it sees
-    for (int u = 0; u < 16 && q0 + wave * 16 + u < q_len; ++u)
+    for (int u = group; u < 16 && q0 + wave * 16 + u < q_len; u += kGroups)
       attend_alone(q, q_stride, key_pages, value_pages, table, table_width, t_first + q0 + wave * 16 + u, pos0 + q0 + wave * 16 + u, head,
                    heads, kvh, kv_heads, block_size, num_pages, scale, window, chunk, sinks, out);
     return;
+  }
+  // the second group's share to the first: [component][thread]
+  __syncthreads();
+  float* const given = tile_lds + kGroupFloats;
+  if (group > 0) {
+    given[tid] = m_run;
+    given[256 + tid] = l_run;
+#pragma unroll
+    for (int dt = 0; dt < kDimTiles; ++dt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) given[(2 + dt * 4 + i) * 256 + tid] = acc[dt][i];
+  }
+  __syncthreads();
+  if (group > 0) return;
+  {
+    const float m_other = given[tid];
+    const float m_new = fmaxf(m_run, m_other);
+    const float mine = m_run == -INFINITY ? 0.f : expf(m_run - m_new), other = m_other == -INFINITY ? 0.f : expf(m_other - m_new);
+    l_run = l_run * mine + given[256 + tid] * other;
+#pragma unroll
+    for (int dt = 0; dt < kDimTiles; ++dt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[dt][i] = acc[dt][i] * mine + given[(2 + dt * 4 + i) * 256 + tid] * other;
+    m_run = m_new;
   }
   float l = l_run;
   l += __shfl_xor(l, 16, kWave);
@@ -308,7 +359,18 @@ extern "C" int mlr_attention_prefill_f32(const float* q, int64_t q_stride, const
               "operands must be 16-byte aligned");
   MLR_REQUIRE(scale > 0.f && scale < INFINITY && window >= 0 && chunk >= 0 && !(window > 0 && chunk > 0), "bad scale, window or chunk");
   MLR_REQUIRE(static_cast<int64_t>(num_tiles) * heads < (1ll << 31), "too many tiles for one launch");
-  f32_attention::attn_prefill_f32_kernel<<<dim3(static_cast<unsigned>(num_tiles) * heads), 256, 0, stream>>>(
+  static bool configured = false;
+  if (!configured) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(f32_attention::attn_prefill_f32_kernel),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, f32_attention::kLdsBytes);
+    if (e != hipSuccess) {
+      set_error(std::string("mlr_attention_prefill_f32: cannot raise the LDS limit: ") + hipGetErrorString(e));
+      return -1;
+    }
+    configured = true;
+  }
+  f32_attention::attn_prefill_f32_kernel<<<dim3(static_cast<unsigned>(num_tiles) * heads), 256 * f32_attention::kGroups, f32_attention::kLdsBytes,
+                                           stream>>>(
       q, q_stride, key_pages, value_pages, block_table, table_width, tiles, cu_q, context_lens, out, heads, kv_heads, block_size,
       num_pages, scale, window, chunk, sinks);
   MLR_LAUNCH_CHECK();

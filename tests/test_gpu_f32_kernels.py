@@ -87,6 +87,18 @@ def test_prompt_attention(ops, heads, kv_heads, head_dim, block, mask):
         torch.testing.assert_close(_attend(ops, *args, **kw).cpu().double(), ref, atol=5e-6, rtol=1e-5)
 
 
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("window", [None, 70, 300])
+def test_prompt_attention_over_several_turns(ops, head_dim, window):
+    """Key tiles for one group of wavefronts and for both, an odd and an even number of them, several turns of each; the first key visible in either's tile."""
+    entries = [(321, 321), (449, 60), (128, 128), (129, 129), (32, 32), (33, 33)]
+    q, kp, vp, table, ctx, dense, te, pos = _paged_case(entries, 3, 1, head_dim, 16, torch.float32, 14)
+    got = _attend(ops, q.cuda(), kp.cuda(), vp.cuda(), table.cuda(), ctx, num_heads=3, num_kv_heads=1, head_dim=head_dim, block_size=16,
+                  scale=head_dim**-0.5, window=window)
+    ref = _attention_reference(q, dense, te, pos, 3, 1, head_dim, head_dim**-0.5, window)
+    torch.testing.assert_close(got.cpu().double(), ref, atol=5e-6, rtol=1e-5)  # as above
+
+
 @pytest.mark.parametrize("head_dim,block", [(64, 16), (128, 16), (80, 8), (16, 4)])
 @pytest.mark.parametrize("mask", [dict(window=None), dict(window=20), dict(window=None, chunk=24)])
 @pytest.mark.parametrize("odd", [float("nan"), float("inf")])
