@@ -356,6 +356,12 @@ int mlr_gate_group_norm(const float* y, const float* projected, int width, int g
 // sum of a token's chosen s (+ 1e-20) first.
 int mlr_moe_route(const float* logits, int slices, const float* correction, int* ids, float* weights, int tokens, int experts,
                   int top, int groups, int keep, float scale, int score_kind, int normalise, hipStream_t stream);
+// mlr_moe_route and mlr_moe_align with tiles of 16 rows in one launch, where mlr_moe_route_align_fits says so (few tokens).  `routed`: the
+// router's outputs; `experts`: how many of them, the first, have matrices.
+int mlr_moe_route_align_fits(int tokens, int routed, int top, int groups);
+int mlr_moe_route_align(const float* logits, int slices, const float* correction, int* ids, float* weights, int tokens, int routed,
+                        int top, int groups, int keep, float scale, int score_kind, int normalise, int experts, int max_tiles,
+                        int* sorted, int* offsets, int* tiles, hipStream_t stream);
 // out[j, t, :] = weights[t, j] * h[t, :] where ids[t, j] >= first: experts without matrices that hand their input on.
 int mlr_moe_identity(const void* h, const int* ids, const float* weights, float* out, int dtype, int tokens, int top,
                      int hidden, int first, hipStream_t stream);

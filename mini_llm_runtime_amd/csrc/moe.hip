@@ -137,14 +137,13 @@ __global__ __launch_bounds__(kWave) void moe_route_kernel(const float* __restric
 // LDS.  The logits may come as `slices` partial sums [slices, tokens, experts], added up in order.
 // Bound by latency: the plain kernel's rounds go through LDS six times each.  64 experts in 8 groups, 6 choices: 8 tokens 10.5 to 4.7
 // us, 2,000 tokens 13.3 to 6.9.
+// Routes token t by one wavefront; returns what lane j < top wrote as the token's j-th expert.  lds: R * 64 floats of this wavefront's own.  Every
+// wavefront of the workgroup calls it (it has a barrier).
 template <int R>
-__global__ __launch_bounds__(kWave) void moe_route_lanes_kernel(const float* __restrict__ logits, int slices,
-                                                                const float* __restrict__ correction, int* __restrict__ ids,
-                                                                float* __restrict__ weights, int tokens, int experts, int top,
-                                                                int groups, int keep, float scale, int score_kind, int normalise) {
-  __shared__ float lds[R * kWave];
-  const int t = blockIdx.x;
-  const int lane = threadIdx.x;
+__device__ __forceinline__ int route_by_lanes(const float* __restrict__ logits, int slices, const float* __restrict__ correction,
+                                              int* __restrict__ ids, float* __restrict__ weights, int tokens, int experts, int top,
+                                              int groups, int keep, float scale, int score_kind, int normalise, int t, float* lds) {
+  const int lane = threadIdx.x % kWave;
   float z[R], s[R], c[R];
 #pragma unroll
   for (int r = 0; r < R; ++r) {
@@ -263,6 +262,17 @@ __global__ __launch_bounds__(kWave) void moe_route_lanes_kernel(const float* __r
     ids[static_cast<int64_t>(t) * top + lane] = my_id;
     weights[static_cast<int64_t>(t) * top + lane] = normalise ? my_weight * (1.0f / (chosen_sum + 1e-20f)) : my_weight;
   }
+  return my_id;
+}
+
+template <int R>
+__global__ __launch_bounds__(kWave) void moe_route_lanes_kernel(const float* __restrict__ logits, int slices,
+                                                                const float* __restrict__ correction, int* __restrict__ ids,
+                                                                float* __restrict__ weights, int tokens, int experts, int top,
+                                                                int groups, int keep, float scale, int score_kind, int normalise) {
+  __shared__ float lds[R * kWave];
+  route_by_lanes<R>(logits, slices, correction, ids, weights, tokens, experts, top, groups, keep, scale, score_kind, normalise,
+                    static_cast<int>(blockIdx.x), lds);
 }
 
 // Experts that hand their input on: where ids[t, j] >= first (such an expert has no matrices and the grouped
@@ -283,28 +293,13 @@ __global__ __launch_bounds__(256) void moe_identity_kernel(const T* __restrict__
 
 // ---- pairs sorted by expert ------------------------------------------------------------------
 
-// One workgroup.  counts -> offsets and tiles (the first wavefront) -> placement.
-__global__ __launch_bounds__(1024) void moe_align_kernel(const int* __restrict__ ids, int pairs, int experts,
-                                                         int tile_rows, int max_tiles, int* __restrict__ sorted,
-                                                         int* __restrict__ offsets, int* __restrict__ tiles) {
-  extern __shared__ int align_lds[];
-  int* counts = align_lds;            // [experts]
-  int* start = align_lds + experts;   // [experts]
-  __shared__ int used_tiles;
+// One workgroup.  counts -> offsets and tiles (the first wavefront) -> placement.  counts (cleared, behind a barrier) and start: LDS,
+// [experts]; for_each_pair calls what it is given with every pair that this thread has and the pair's expert (one with matrices).
+template <class EachPair>
+__device__ __forceinline__ void align_pairs(int experts, int tile_rows, int max_tiles, int* counts, int* start, int* used_tiles,
+                                            int* __restrict__ sorted, int* __restrict__ offsets, int* __restrict__ tiles,
+                                            const EachPair& for_each_pair) {
   const int tid = threadIdx.x;
-  for (int e = tid; e < experts; e += blockDim.x) counts[e] = 0;
-  __syncthreads();
-  // eight ids of a thread are asked for at once: one after the other each would be a trip to L2
-  auto for_each_pair = [&](auto&& use) {
-    for (int p0 = tid; p0 < pairs; p0 += 8 * 1024) {
-      int e[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) e[u] = ids[min(p0 + u * 1024, pairs - 1)];
-#pragma unroll
-      for (int u = 0; u < 8; ++u)
-        if (p0 + u * 1024 < pairs && e[u] >= 0 && e[u] < experts) use(p0 + u * 1024, e[u]);
-    }
-  };
   for_each_pair([&](int, int e) { atomicAdd(&counts[e], 1); });
   __syncthreads();
   if (tid < kWave) {  // the first wavefront: where every expert's run and tiles start, 64 experts at a time
@@ -337,17 +332,59 @@ __global__ __launch_bounds__(1024) void moe_align_kernel(const int* __restrict__
     }
     if (tid == 0) {
       offsets[experts] = at;
-      used_tiles = min(nt, max_tiles);
+      *used_tiles = min(nt, max_tiles);
     }
   }
   __syncthreads();
-  for (int i = used_tiles + tid; i < max_tiles; i += blockDim.x) {
+  for (int i = *used_tiles + tid; i < max_tiles; i += blockDim.x) {
     tiles[2 * i] = -1;  // a workgroup that finds this has nothing to do
-    tiles[2 * i + 1] = used_tiles;
+    tiles[2 * i + 1] = *used_tiles;
   }
   for (int e = tid; e < experts; e += blockDim.x) counts[e] = 0;
   __syncthreads();
   for_each_pair([&](int p, int e) { sorted[start[e] + atomicAdd(&counts[e], 1)] = p; });
+}
+
+__global__ __launch_bounds__(1024) void moe_align_kernel(const int* __restrict__ ids, int pairs, int experts,
+                                                         int tile_rows, int max_tiles, int* __restrict__ sorted,
+                                                         int* __restrict__ offsets, int* __restrict__ tiles) {
+  extern __shared__ int align_lds[];
+  int* counts = align_lds;            // [experts]
+  int* start = align_lds + experts;   // [experts]
+  __shared__ int used_tiles;
+  const int tid = threadIdx.x;
+  for (int e = tid; e < experts; e += blockDim.x) counts[e] = 0;
+  __syncthreads();
+  // eight ids of a thread are asked for at once: one after the other each would be a trip to L2
+  align_pairs(experts, tile_rows, max_tiles, counts, start, &used_tiles, sorted, offsets, tiles, [&](auto&& use) {
+    for (int p0 = tid; p0 < pairs; p0 += 8 * 1024) {
+      int e[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) e[u] = ids[min(p0 + u * 1024, pairs - 1)];
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (p0 + u * 1024 < pairs && e[u] >= 0 && e[u] < experts) use(p0 + u * 1024, e[u]);
+    }
+  });
+}
+
+// Both at once for up to 8 tokens: a workgroup with a wavefront for each.  A launch is most of what either costs: 64 experts in 8
+// groups, 6 choices, in a replayed graph the two / this one: 1 token 6.9 / 5.0 us, 8 tokens 7.3 / 5.9, 16 7.3 / 7.5.
+constexpr int kRouteAlignTokens = 8;
+template <int R>
+__global__ __launch_bounds__(kRouteAlignTokens* kWave) void moe_route_align_kernel(
+    const float* __restrict__ logits, int slices, const float* __restrict__ correction, int* __restrict__ ids, float* __restrict__ weights,
+    int tokens, int routed, int top, int groups, int keep, float scale, int score_kind, int normalise, int experts, int tile_rows, int max_tiles,
+    int* __restrict__ sorted, int* __restrict__ offsets, int* __restrict__ tiles) {
+  __shared__ float lds[kRouteAlignTokens][R * kWave];
+  __shared__ int counts[R * kWave], start[R * kWave], used_tiles;
+  const int t = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+  for (int e = threadIdx.x; e < R * kWave; e += blockDim.x) counts[e] = 0;
+  const int id = route_by_lanes<R>(logits, slices, correction, ids, weights, tokens, routed, top, groups, keep, scale, score_kind, normalise, t, lds[t]);
+  __syncthreads();
+  align_pairs(experts, tile_rows, max_tiles, counts, start, &used_tiles, sorted, offsets, tiles, [&](auto&& use) {
+    if (lane < top && id < experts) use(t * top + lane, id);
+  });
 }
 
 // ---- the clamped gating in a grouped product's epilogue ------------------------------------------------
@@ -1238,6 +1275,34 @@ int mlr_moe_route(const float* logits, int slices, const float* correction, int*
   const size_t lds = (2 * static_cast<size_t>(experts) + groups) * sizeof(float);
   moe_route_kernel<<<tokens, kWave, lds, stream>>>(logits, slices, correction, ids, weights, tokens, experts, top, groups, keep,
                                                    scale, score_kind, norm);
+  MLR_LAUNCH_CHECK();
+  return 0;
+}
+
+// mlr_moe_route and mlr_moe_align (16 rows a tile) in one launch: up to 8 tokens, 256 router outputs, 64 groups and choices.  experts: how
+// many of the `routed` router outputs have matrices (the first ones).
+int mlr_moe_route_align_fits(int tokens, int routed, int top, int groups) {
+  return tokens <= kRouteAlignTokens && routed <= 4 * kWave && groups <= kWave && top <= kWave;
+}
+int mlr_moe_route_align(const float* logits, int slices, const float* correction, int* ids, float* weights, int tokens, int routed, int top,
+                        int groups, int keep, float scale, int score_kind, int normalise, int experts, int max_tiles, int* sorted, int* offsets,
+                        int* tiles, hipStream_t stream) {
+  MLR_REQUIRE(logits && ids && weights && sorted && offsets && tiles, "null pointer");
+  MLR_REQUIRE(slices >= 1, "logits come whole or in slices");
+  MLR_REQUIRE(score_kind >= 0 && score_kind <= 2, "scores are sigmoids (0), a softmax (1) or the logits themselves (2)");
+  MLR_REQUIRE(score_kind != 2 || correction == nullptr, "a softmax over the chosen logits has no correction");
+  MLR_REQUIRE(tokens > 0 && routed > 0 && top > 0 && top <= routed && experts > 0 && experts <= routed, "sizes must be > 0 and top <= experts");
+  MLR_REQUIRE(groups > 0 && routed % groups == 0 && keep > 0 && keep <= groups, "bad groups");
+  MLR_REQUIRE(top <= keep * (routed / groups), "the kept groups hold fewer experts than a token uses");
+  MLR_REQUIRE(mlr_moe_route_align_fits(tokens, routed, top, groups), "too many tokens or experts for one launch");
+  MLR_REQUIRE(max_tiles >= mlr_moe_max_tiles(tokens * top, experts, 0), "too few tiles for these pairs");
+  const int norm = normalise || score_kind == 2;
+  if (routed <= kWave)
+    moe_route_align_kernel<1><<<1, tokens * kWave, 0, stream>>>(logits, slices, correction, ids, weights, tokens, routed, top, groups, keep, scale,
+                                                                score_kind, norm, experts, kMoeRows, max_tiles, sorted, offsets, tiles);
+  else
+    moe_route_align_kernel<4><<<1, tokens * kWave, 0, stream>>>(logits, slices, correction, ids, weights, tokens, routed, top, groups, keep, scale,
+                                                                score_kind, norm, experts, kMoeRows, max_tiles, sorted, offsets, tiles);
   MLR_LAUNCH_CHECK();
   return 0;
 }

@@ -102,6 +102,8 @@ _SIGNATURES = {
     "mlr_moe_route": ([_VP, _I, _VP, _VP, _VP, _I, _I, _I, _I, _I, _F, _I, _I, _VP], _I),
     "mlr_moe_tile_rows": ([_I], _I),
     "mlr_moe_max_tiles": ([_I, _I, _I], _I),
+    "mlr_moe_route_align_fits": ([_I, _I, _I, _I], _I),
+    "mlr_moe_route_align": ([_VP, _I, _VP, _VP, _VP, _I, _I, _I, _I, _I, _F, _I, _I, _I, _I, _VP, _VP, _VP, _VP], _I),
     "mlr_moe_align": ([_VP, _I, _I, _I, _I, _VP, _VP, _VP, _VP], _I),
     "mlr_moe_gemm": ([_VP, _VP, _VP, _VP, _VP, _VP, _VP, _I, _I, _I, _I, _I, _I, _I, _I, _I, _F, _F, _VP], _I),
     "mlr_gemm_residual_parts": ([_I, _I], _I),
@@ -227,6 +229,7 @@ class HipOps:
 
     # ---- plans --------------------------------------------------------------------------------
     ATTENTION_PLAN = PAGED_ATTENTION
+    ROUTING_SORTS = True  # `route_experts` takes `order`
 
     @staticmethod
     def attention_plan(shape):
@@ -2135,15 +2138,17 @@ class HipOps:
     # ---- routed experts --------------------------------------------------------------------------------
     def route_experts(
         self, logits: torch.Tensor, correction: Optional[torch.Tensor], *, top: int, groups: int, keep_groups: int,
-        scale: float, scores: str = "sigmoid", normalise: bool = False,
-    ) -> tuple[torch.Tensor, torch.Tensor]:
+        scale: float, scores: str = "sigmoid", normalise: bool = False, order: Optional[int] = None,
+    ) -> tuple[Any, ...]:
         """Which experts every token uses (int32 [T, top]) and with what weight (float32 [T, top]),
         from the router's float32 logits z [T, experts]: s = sigmoid(z), c = s + correction; the expert
         axis is cut into `groups` contiguous blocks, a block scores the top-2 sum of its c, and ids are
         the arg-top-`top` of c over the experts of the `keep_groups` highest blocks; weights = s[ids] *
         `scale` (c only decides).  scores="softmax": s = softmax(z) over all experts instead.  normalise: the
         chosen weights are divided by their sum (+ 1e-20) before the scale.  scores="chosen_softmax": the choice goes by z itself
-        (no correction) and the weights are the softmax over the chosen z."""
+        (no correction) and the weights are the softmax over the chosen z.
+        order: the number of experts with matrices (the first ones); a third value is returned then, the pairs sorted for
+        `expert_products` where few tokens have that done by the same kernel, or None."""
         kinds = ("sigmoid", "softmax", "chosen_softmax")
         if scores not in kinds:
             raise KernelError(f"router scores are one of {', '.join(kinds)}")
@@ -2157,12 +2162,26 @@ class HipOps:
             self._check(correction, "router correction", torch.float32, (experts,))
         ids = self._empty((tokens, top), torch.int32)
         weights = self._empty((tokens, top), torch.float32)
+        if order is not None and self.lib.mlr_moe_route_align_fits(tokens, experts, int(top), int(groups)):
+            index = self._pair_index(tokens * top, order, 0)
+            self._call(
+                "mlr_moe_route_align", self._ptr(logits), slices, self._ptr(correction), self._ptr(ids), self._ptr(weights), tokens,
+                experts, int(top), int(groups), int(keep_groups), float(scale), kinds.index(scores), int(bool(normalise)), int(order),
+                index[3], *(self._ptr(t) for t in index[:3]), self._stream(),
+            )
+            return ids, weights, index
         self._call(
             "mlr_moe_route", self._ptr(logits), slices, self._ptr(correction), self._ptr(ids), self._ptr(weights), tokens,
             experts, int(top), int(groups), int(keep_groups), float(scale), kinds.index(scores), int(bool(normalise)),
             self._stream(),
         )
-        return ids, weights
+        return (ids, weights) if order is None else (ids, weights, None)
+
+    def _pair_index(self, pairs: int, experts: int, big: int) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, int]:
+        """Room for the pairs sorted by expert: (order, offsets, tiles, the most tiles there may be)."""
+        most = self.lib.mlr_moe_max_tiles(pairs, experts, big)
+        index = self._empty((pairs + experts + 1 + 2 * most,), torch.int32)
+        return index[:pairs], index[pairs : pairs + experts + 1], index[pairs + experts + 1 :], most
 
     def expert_products(
         self,
@@ -2179,6 +2198,7 @@ class HipOps:
         glu: Optional[tuple[float, float]] = None,
         woven: bool = False,
         beside: Optional[tuple[torch.Tensor, torch.Tensor]] = None,
+        order: Any = None,
     ) -> torch.Tensor:
         """The chosen experts' outputs, weighted: float32 [top, T, hidden] with [j, t] = weights[t, j]
         * down_e(act(up_e(h[t]))), e = ids[t, j]; the sum over j is the mixture's output, which a norm
@@ -2193,7 +2213,8 @@ class HipOps:
         `woven`: its gate and up rows lie in pairs as for `linear`, and the gating is the first product's epilogue; else
         they lie as for "swiglu" and it is a kernel of its own.
         beside: (x [T, k], weight [hidden, k]) of a product whose sums join the mixture (a shared expert's second matrix):
-        one more slice of the stack, or a few of partial sums over k."""
+        one more slice of the stack, or a few of partial sums over k.
+        order: the third value of `route_experts` for these ids, or None: the pairs are sorted here."""
         if kernel not in ("auto", "fma"):
             raise KernelError("kernel must be 'auto' or 'fma'")
         if activation not in ("relu2", "sigmoid", "swiglu", "clamped_glu"):
@@ -2231,13 +2252,16 @@ class HipOps:
                 big = 3  # tiles of 256 rows and 256 features
         if big:
             mfma = 1 + big
-        max_tiles = self.lib.mlr_moe_max_tiles(pairs, experts, big)
-        index = self._empty((pairs + experts + 1 + 2 * max_tiles,), torch.int32)
-        order, offsets, tiles = index[:pairs], index[pairs : pairs + experts + 1], index[pairs + experts + 1 :]
-        self._call(
-            "mlr_moe_align", self._ptr(ids), pairs, experts, big, max_tiles, self._ptr(order), self._ptr(offsets),
-            self._ptr(tiles), self._stream(),
-        )
+        if order is not None and not big:
+            by_expert, offsets, tiles, max_tiles = order
+            if by_expert.shape[0] != pairs or offsets.shape[0] != experts + 1:
+                raise KernelError("the pairs were sorted for other experts")
+        else:
+            by_expert, offsets, tiles, max_tiles = self._pair_index(pairs, experts, big)
+            self._call(
+                "mlr_moe_align", self._ptr(ids), pairs, experts, big, max_tiles, self._ptr(by_expert), self._ptr(offsets),
+                self._ptr(tiles), self._stream(),
+            )
         act = self._empty((pairs, inner if woven else wide), self.dtype)
         more = 0
         if beside is not None:
@@ -2251,7 +2275,7 @@ class HipOps:
             self.linear(x, weight, None, out_dtype=torch.float32, kernel=kernel, slices=None, out=out[top])
         elif more:
             self.linear(x, weight, None, partial_sums=True, slices=more, out=out[top:])
-        common = (self._ptr(order), self._ptr(offsets), self._ptr(tiles))
+        common = (self._ptr(by_expert), self._ptr(offsets), self._ptr(tiles))
         self._call(
             "mlr_moe_gemm", self._ptr(h), self._ptr(up_weight), *common, _VP(None), self._ptr(act), 1, self.code, mfma,
             max_tiles, tokens, top, wide, hidden, 0 if gated and not woven else _EPILOGUES[activation], limit, alpha,

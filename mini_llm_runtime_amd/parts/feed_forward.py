@@ -311,14 +311,17 @@ class RoutedExperts(FeedForward):
         ops = ctx.ops
         # a narrow product (as many features as experts): the routing adds up partial sums over slices of k
         logits = ops.linear(h, self.router_weight, self.router_bias, out_dtype=torch.float32, partial_sums=True)
-        ids, weights = ops.route_experts(
+        sorts = getattr(ops, "ROUTING_SORTS", False)  # the routing of few tokens may sort the pairs by expert, too
+        ids, weights, *order = ops.route_experts(
             logits, self.correction, top=self.top, groups=self.groups, keep_groups=self.keep_groups,
             scale=self.router_scale,
             **({"scores": self.scores, "normalise": self.normalise} if (self.scores != "sigmoid" or self.normalise) else {}),
+            **({"order": self.experts} if sorts else {}),
         )
         return ops.expert_products(
             h, self.up_weight, self.down_weight, ids, weights, experts=self.experts, activation=self.activation,
             **({"pass_through": self.identity} if self.identity else {}),
             **({"glu": (self.limit, self.alpha), "woven": self.woven} if self.activation == "clamped_glu" else {}),
             **({"beside": (self.shared.inner(ctx, h), self.shared.down_weight)} if self.shared is not None else {}),
+            **({"order": order[0]} if sorts else {}),
         )

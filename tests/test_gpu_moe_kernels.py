@@ -59,6 +59,28 @@ def test_routing(ops, experts, top, groups, keep, scores, normalise, slices):
     assert ((w.cpu().double() - want).abs() <= (experts + 16) * 2.0**-24 * want + 1e-12).all()
 
 
+# one token, a full workgroup and one token more (two kernels); every expert with matrices, all but some, one; more choices than a tile's rows
+@pytest.mark.parametrize("tokens", [1, 3, 8, 9])
+@pytest.mark.parametrize("routed,experts,top,groups,keep", [(64, 64, 6, 8, 4), (65, 60, 4, 5, 2), (256, 256, 64, 16, 9), (5, 1, 5, 1, 1), (40, 33, 2, 1, 1)])
+def test_routing_that_sorts(ops, tokens, routed, experts, top, groups, keep):
+    z, correction = _rand((tokens, routed), torch.float32, routed).cuda(), _rand((routed,), torch.float32, 3, 0.1).cuda()
+    rule = dict(top=top, groups=groups, keep_groups=keep, scale=1.7)
+    want_ids, want = ops.route_experts(z, correction, **rule)
+    ids, w, order = ops.route_experts(z, correction, order=experts, **rule)
+    assert torch.equal(ids, want_ids) and torch.equal(w, want)
+    assert (order is None) == (tokens > 8)
+    if order is None:
+        return
+    by_expert, offsets, tiles, most = (t.cpu() if isinstance(t, torch.Tensor) else t for t in order)
+    pairs = want_ids.cpu().flatten()
+    used = []
+    for e in range(experts):
+        rows = by_expert[offsets[e] : offsets[e + 1]].tolist()
+        assert sorted(rows) == (pairs == e).nonzero().flatten().tolist()
+        used += [[e, int(offsets[e]) + i] for i in range(0, len(rows), 16)]
+    assert tiles.view(-1, 2).tolist() == used + [[-1, len(used)]] * (most - len(used))
+
+
 def test_routing_of_infinities_and_nan(ops):
     inf, nan = float("inf"), float("nan")
     z = torch.tensor([[nan, 1.0, 0.5, 2.0], [-inf, -inf, -inf, -inf], [nan] * 4, [inf, 1.0, nan, -inf]])
