@@ -475,7 +475,7 @@ def test_fused_qkv_rotation_cache_write_equals_the_three_kernels(ops_for, heads,
     assert torch.isnan(out[True][1]).all() == (not write)
 
 
-@pytest.mark.parametrize("kernel", [24, 25])
+@pytest.mark.parametrize("kernel", [24, 25, None])  # None: the plain product and the rotation kernel
 @pytest.mark.parametrize("heads,kv_heads,head_dim,hidden,tokens,bs,start,rotate,write,bias", [
     # one token more than a tile, one fewer, fewer than eight; slots from the middle of a page and of eight of them on; a tile with the last queries, the keys and
     # the first values; values only, keys only; k of one step, not a multiple of a step, an odd number of steps
@@ -500,7 +500,7 @@ def test_staged_qkv_product_of_consecutive_slots(ops_for, kernel, heads, kv_head
     kp = torch.full((pages, kv_heads, bs, head_dim), float("nan"), dtype=torch.bfloat16).cuda()
     vp = torch.full((pages, kv_heads, head_dim, bs), float("nan"), dtype=torch.bfloat16).cuda()
     q = ops.qkv_rope_write(x, w, b, rotation, slots.cuda(), kp, vp, num_heads=heads, num_kv_heads=kv_heads, head_dim=head_dim,
-                           block_size=bs, write=write, fused=True, mfma_kernel=kernel)
+                           block_size=bs, write=write, fused=kernel is not None, mfma_kernel=kernel or 0)
     reference = qkv_reference(x, w, b, rotation[0] if rotate else None, rotation[1] if rotate else None, heads, kv_heads, head_dim)
     slots[tokens - 1] = -1  # nothing is written for it
     check_qkv("staged", q.float().cpu(), kp.float().cpu(), vp.float().cpu(), slots, bs, reference, heads, kv_heads, head_dim, write=write)
