@@ -393,22 +393,26 @@ __global__ __launch_bounds__(kDecodeWaves* kWave) void attn_decode_kernel(
   }
 }
 
+constexpr int kMergeBatch = D <= 128 ? 16 : 8;  // partitions whose shares are on their way at once
+
 // Merge of the partitions of one (entry, query head): m = max m_j, w_j = exp(m_j - m),
 // O = sum w_j a_j / sum w_j l_j (csrc/paged_attention_split_cuda.cu:66-88 of the
 // reference).  Lane j holds partition j's max and sum, so the weights come from two
 // wavefront reductions; every lane then sums its output dims over the partitions
-// with independent loads.
-__global__ __launch_bounds__(kWave) void attn_decode_merge_kernel(const float* __restrict__ partial,
-                                                                  const int* __restrict__ cu_q,
-                                                                  const int* __restrict__ context_lens,
-                                                                  bf16* __restrict__ out, int heads, int window,
-                                                                  int chunk, int part, int all_splits,
-                                                                  const float* __restrict__ sinks,
-                                                                  const float* __restrict__ extra, int gated,
-                                                                  int keep_first) {
+// with independent loads.  WAVES wavefronts take the batches of partitions in turn and add up their sums in order at the end.
+template <int WAVES>
+__global__ __launch_bounds__(WAVES* kWave) void attn_decode_merge_kernel(const float* __restrict__ partial,
+                                                                         const int* __restrict__ cu_q,
+                                                                         const int* __restrict__ context_lens,
+                                                                         bf16* __restrict__ out, int heads, int window,
+                                                                         int chunk, int part, int all_splits,
+                                                                         const float* __restrict__ sinks,
+                                                                         const float* __restrict__ extra, int gated,
+                                                                         int keep_first) {
   const int entry = blockIdx.x;
   const int h = blockIdx.y;
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x % kWave;
+  const int wave = threadIdx.x / kWave;
   const int t = cu_q[entry];
   if (cu_q[entry + 1] - t != 1) return;
   const float* src = partial + (static_cast<int64_t>(entry) * heads + h) * all_splits * kPartialStride;
@@ -419,7 +423,6 @@ __global__ __launch_bounds__(kWave) void attn_decode_merge_kernel(const float* _
   // before the first is used, and the first batch before the reductions below: this kernel's
   // time is the latency of its loads, so they must not wait for one another.
   constexpr int kPerLane = (D + kWave - 1) / kWave;
-  constexpr int kMergeBatch = D <= 128 ? 16 : 8;
   float ms[kMergeBatch], piece[kMergeBatch][kPerLane];
   auto load_batch = [&](int s0) {
 #pragma unroll
@@ -433,7 +436,7 @@ __global__ __launch_bounds__(kWave) void attn_decode_merge_kernel(const float* _
       }
     }
   };
-  load_batch(0);
+  load_batch(wave * kMergeBatch);
 
   float mstar = -INFINITY;
   float den = 0.f;
@@ -452,16 +455,29 @@ __global__ __launch_bounds__(kWave) void attn_decode_merge_kernel(const float* _
   float num[kPerLane];
 #pragma unroll
   for (int j = 0; j < kPerLane; ++j) num[j] = 0.f;
-  for (int s0 = 0;;) {
+  for (int s0 = wave * kMergeBatch;;) {
 #pragma unroll
     for (int u = 0; u < kMergeBatch; ++u) {
       const float w = (s0 + u >= splits || ms[u] == -INFINITY) ? 0.f : fast_exp2(ms[u] - mstar);
 #pragma unroll
       for (int j = 0; j < kPerLane; ++j) num[j] += w * piece[u][j];
     }
-    s0 += kMergeBatch;
+    s0 += WAVES * kMergeBatch;
     if (s0 >= splits) break;
     load_batch(s0);
+  }
+  if constexpr (WAVES > 1) {
+    __shared__ float sums[WAVES - 1][kPerLane][kWave];
+    if (wave > 0) {
+#pragma unroll
+      for (int j = 0; j < kPerLane; ++j) sums[wave - 1][j][lane] = num[j];
+    }
+    __syncthreads();
+    if (wave > 0) return;
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w)
+#pragma unroll
+      for (int j = 0; j < kPerLane; ++j) num[j] += sums[w - 1][j][lane];
   }
   if (extra != nullptr) {  // one more share of the same softmax, made elsewhere: [token, head, head size + 2]
     const float* e = extra + (static_cast<int64_t>(t) * heads + h) * kPartialStride;
@@ -1366,6 +1382,19 @@ __global__ __launch_bounds__(256) void attn_prefill_merge_kernel(const float* __
   }
 }
 
+// Up to a batch of partitions one wavefront merges; beyond, four: one after the other every batch is a trip to memory.  In a replayed graph with
+// one / four, 8 entries x 14 heads of 64: 64 partitions 5.65 / 3.17 us, 32 3.91 / 3.23, 17 3.85 / 3.19 (16 with one: 2.72); 28 heads of 128: 64
+// 8.03 / 4.30, 17 4.48 / 3.41.  Not for the heads of many entries, which fill the units by themselves: 64 x 28 of 64, 17 partitions 5.71 / 6.53.
+static void launch_merge(dim3 grid, hipStream_t stream, const float* partial, const int* cu_q, const int* context_lens, bf16* out, int heads,
+                         int window, int chunk, int part, int splits, const float* sinks, const float* extra, int gated, int keep_first) {
+  if (splits > kMergeBatch && grid.x * grid.y <= 512)
+    attn_decode_merge_kernel<4><<<grid, 4 * kWave, 0, stream>>>(partial, cu_q, context_lens, out, heads, window, chunk, part, splits, sinks, extra,
+                                                                gated, keep_first);
+  else
+    attn_decode_merge_kernel<1><<<grid, kWave, 0, stream>>>(partial, cu_q, context_lens, out, heads, window, chunk, part, splits, sinks, extra, gated,
+                                                            keep_first);
+}
+
 }  // namespace mlr
 
 using namespace mlr;
@@ -1451,9 +1480,8 @@ int mlr_attention_decode(const void* q, int64_t q_stride, const void* key_pages,
   MLR_LAUNCH_CHECK();
   MLR_REQUIRE(sinks == nullptr || merge, "partitions left unmerged cannot carry sinks");
   if ((splits > 1 || keep_partial) && merge) {
-    attn_decode_merge_kernel<<<dim3(entries, heads), kWave, 0, stream>>>(
-        partial, cu_q, context_lens, static_cast<bf16*>(out), heads, window, chunk, part, splits, sinks, extra,
-        score_bias != nullptr, keep_first);
+    launch_merge(dim3(entries, heads), stream, partial, cu_q, context_lens, static_cast<bf16*>(out), heads, window, chunk, part, splits,
+                 sinks, extra, score_bias != nullptr, keep_first);
     MLR_LAUNCH_CHECK();
   }
   return 0;
@@ -1467,8 +1495,8 @@ int mlr_attention_decode_merge(const float* partial, const int* cu_q, const int*
   MLR_REQUIRE(partial && cu_q && context_lens && out, "null pointer");
   MLR_REQUIRE(entries > 0 && heads > 0 && heads <= 65535, "bad sizes");
   MLR_REQUIRE(part > 0 && part % 64 == 0 && splits > 1 && window >= 0 && chunk >= 0, "bad partitions");
-  attn_decode_merge_kernel<<<dim3(entries, heads), kWave, 0, stream>>>(partial, cu_q, context_lens,
-                                                                      static_cast<bf16*>(out), heads, window, chunk, part, splits, sinks, nullptr, 0, 0);
+  launch_merge(dim3(entries, heads), stream, partial, cu_q, context_lens, static_cast<bf16*>(out), heads, window, chunk, part, splits, sinks, nullptr,
+               0, 0);
   MLR_LAUNCH_CHECK();
   return 0;
 }

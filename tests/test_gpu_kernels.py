@@ -865,6 +865,26 @@ def test_decode_attention_partitions(ops_for, heads, kv_heads, head_dim, partiti
     torch.testing.assert_close(got.double(), fma.double(), **_tol(torch.bfloat16))
 
 
+@pytest.mark.parametrize("heads,kv_heads,head_dim", [(14, 2, 64), (4, 1, 128), (2, 1, 256), (3, 1, 16)])
+@pytest.mark.parametrize("longest", [1024, 1025, 3073, 4161])
+def test_decode_attention_merges_batches_of_partitions(ops_for, heads, kv_heads, head_dim, longest):
+    """16, 17, 49 and 66 partitions of 64 keys: one wavefront's batch, one more, a last batch that is not full, more than a wavefront has lanes; beside
+    the longest context some with partitions for the first wavefronts only."""
+    ops = ops_for(torch.bfloat16)
+    old = ops.decode_partition, ops.decode_max_groups
+    ops.decode_partition, ops.decode_max_groups = 64, 1 << 20
+    try:
+        entries = [(longest, 1), (3, 1), (900, 1), (1030, 1) if longest > 1030 else (64, 1)]
+        q, kp, vp, table, ctx, dense, te, pos = _paged_case(entries, heads, kv_heads, head_dim, 16, torch.bfloat16, 31)
+        scale = head_dim**-0.5
+        got = _attend(ops, q.cuda(), kp.cuda(), vp.cuda(), table.cuda(), ctx, num_heads=heads, num_kv_heads=kv_heads, head_dim=head_dim,
+                      block_size=16, scale=scale, window=None).cpu()
+    finally:
+        ops.decode_partition, ops.decode_max_groups = old
+    ref = _attention_reference(q, dense, te, pos, heads, kv_heads, head_dim, scale, None)
+    torch.testing.assert_close(got.double(), ref, **_tol(torch.bfloat16))
+
+
 @pytest.mark.parametrize("heads,kv_heads,head_dim,bs,long", [
     (14, 2, 64, 16, 2048), (8, 2, 128, 16, 1100), (3, 1, 96, 8, 700), (2, 1, 256, 32, 600), (5, 5, 16, 64, 900),
 ])
