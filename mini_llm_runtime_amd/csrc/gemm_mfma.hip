@@ -1410,7 +1410,10 @@ struct LinesPlan {
 };
 static LinesPlan plan_lines(int m, int n, int k, int slices) {
   LinesPlan best{0, slices, 0.f};
-  for (int blocks = 1; blocks <= 4; ++blocks) {
+  // From 20 MB on, once 32 features a workgroup make two of them a unit, these: the units share what memory gives, and two small workgroups
+  // leave less of a gap at their ends than one large (32,768 x 3,584 at 8 tokens 35.9 us, 37.6 with 64 features; 1.5 to 5 % over nine shapes).
+  const bool many = static_cast<int64_t>(n) * k * 2 >= (20ll << 20) && static_cast<int64_t>((n + 31) / 32) * slices >= 512;
+  for (int blocks = many ? 2 : 1; blocks <= (many ? 2 : 4); ++blocks) {
     const int64_t groups = static_cast<int64_t>((n + blocks * 16 - 1) / (blocks * 16)) * slices;
     const int resident = blocks <= 2 ? 2 : 1;
     const float kb = (blocks * 16 + m) * (((k + 63) / 64 + slices - 1) / slices) * 0.128f;
@@ -1418,6 +1421,21 @@ static LinesPlan plan_lines(int m, int n, int k, int slices) {
     if (best.blocks == 0 || us < best.us) best = {blocks, slices, us};
   }
   return best;
+}
+
+// Up to 16 tokens: whether gemm_lines takes the product also where the tiles would fill the compute units.  Below 20 MB always (2,048 x 4,096
+// in 8 slices at 8 tokens, 17 MB: 7.4 us in tiles, 6.5).  Beyond, over 46 matrices of 20 MB to 1.1 GB at 1 to 16 tokens, sums with their norm:
+// at 8 tokens 14,336 x 768 9.3 us in tiles, 6.6 here; 3,584 x 3,584 12.0 and 10.9; 2,048 x 11,008 at 12 tokens 18.1 and 13.6; 16,384 x 1,536
+// 15.4 and 10.5; 22,016 x 2,048 21.0 and 18.4; 3,584 x 18,944 29.0 and 26.4; 151,936 x 2,048 123 and 102; 152,064 x 3,584 167 and 158.  The
+// tiles keep what they do better: many rows that lie a multiple of 8 KB apart (28,672 x 4,096 43.9 and 51.6, 8,192 x 8,192 30.2 and 33.0: the
+// lines of a load's eight rows meet in the same channels), many rows with a short k, whose workgroups end before their loads are all on their
+// way (32,768 x 512 9.3 and 10.5, 65,536 x 1,024 24.0 and 25.6, 151,936 x 896 45.8 and 49.8), and from 200 MB on, where memory's rate is the
+// bound, more than 8 tokens, which every workgroup reads again (55,296 x 5,120 at 16 tokens 84 and 91).
+static bool lines_stream(int m, int n, int k) {
+  const int64_t bytes = static_cast<int64_t>(n) * k * 2;
+  if (bytes < (20ll << 20)) return true;
+  if ((n >= 8192 && k % 4096 == 0) || (n >= 16384 && k < 1536)) return false;
+  return bytes < (200ll << 20) || (m <= 8 && k >= 2048);
 }
 
 // Up to 8 tokens of the fused query/key/value product: workgroups of 8 weight rows instead of 16 while that makes one round of them; beyond,
@@ -1594,10 +1612,7 @@ static int choose_few_token_tiles(int m, int n, int k, int slices, float* estima
 }
 
 static int choose_kernel(int m, int n, int k, int slices, bool sums) {
-  // 16 tokens: gemm_lines below 20 MB (2,048 x 4,096 in 8 slices at 8 tokens, 17 MB: 7.4 us in tiles, 6.5 here).  Of 29 products beyond
-  // that line gemm_lines would be ahead of the tiles, too, at 8 tokens: 14,336 x 768 (21 MB) 9.8 us in tiles, 7.0 there; 3,584 x 3,584
-  // with its norm (25 MB) 12.4 and 10.7; 17,920 x 1,536 (53 MB) 14.5 and 13.6; 22,016 x 2,048 (86 MB) 22.7 and 19.9; 5,120 x 5,120 17.5 and 16.4.
-  if (m <= 16 && (!few_tokens_tiled(n, slices) || static_cast<int64_t>(n) * k * 2 < (20ll << 20))) return 16;
+  if (m <= 16 && (!few_tokens_tiled(n, slices) || lines_stream(m, n, k))) return 16;
   if (m <= 64 && small_matrix(n, k)) return 16;
   if (m <= 64) return choose_few_token_tiles(m, n, k, slices);
   const GemmPlan plan = plan_many_tokens(m, n, k, slices, sums);
@@ -1731,18 +1746,19 @@ int mlr_gemm_bf16_slices(int m, int n, int k, int max_slices) {
   if (k % 8 != 0) return 1;
   if (m > 64) return plan_many_tokens(m, n, k, max_slices, true).slices;
   if (m <= 16) {
-    // Measured with the norm kernel that adds the slices up (its cost grows with their number):
-    // a weight of 64 MB or more streams fastest through the LDS-tiled kernel cut into 8 slices;
-    // smaller ones through gemm_lines, as plan_lines has it.
+    // Measured with the norm kernel that adds the slices up (its cost grows with their number).  What gemm_lines leaves goes through the
+    // tiles, weights of 64 MB or more cut into 8 slices, others into 4 once that fills the compute units, into 8 where 4 would not fill
+    // them twice.
     const int64_t bytes = static_cast<int64_t>(n) * k * 2;
-    if (bytes >= (64ll << 20) && max_slices >= 8 && k >= 8 * 256 && few_tokens_tiled(n, 8)) return 8;
-    // from 20 MB on, the LDS-tiled kernel cut into 4 once that fills the compute units, into 8 where
-    // 4 would not fill them twice (7B output projection at 8 tokens: 10.1 us in 4 slices, 8.4 in 8)
-    if (bytes >= (20ll << 20) && max_slices >= 8 && k >= 8 * 256 && few_tokens_tiled(n, 4) && !few_tokens_tiled(n, 2))
-      return 8;
-    if (bytes >= (20ll << 20) && max_slices >= 4 && k >= 4 * 256 && few_tokens_tiled(n, 4)) return 4;
-    // gemm_lines: at most 8 slices for the norm to add up, a step of k for each of a workgroup's wavefronts
-    LinesPlan best = plan_lines(m, n, k, 1);
+    if (!lines_stream(m, n, k) && max_slices >= 4) {
+      const bool eight = max_slices >= 8 && k >= 8 * 256;
+      if (eight && bytes >= (64ll << 20) && few_tokens_tiled(n, 8)) return 8;
+      if (eight && few_tokens_tiled(n, 4) && !few_tokens_tiled(n, 2)) return 8;
+      if (k >= 4 * 256 && few_tokens_tiled(n, 4)) return 4;
+    }
+    // gemm_lines: at most 8 slices for the norm to add up, a step of k for each of a workgroup's wavefronts.  From 20 MB on never whole where
+    // the consumer takes slices, as in the tiles: one slice would be rounded to bfloat16 before it is added.
+    LinesPlan best = plan_lines(m, n, k, bytes >= (20ll << 20) && max_slices >= 4 && k >= 4 * 256 ? 4 : 1);
     for (int slices = 2; slices <= min(max_slices, 8) && k >= slices * 256; slices *= 2) {
       const LinesPlan plan = plan_lines(m, n, k, slices);
       if (plan.us < best.us) best = plan;

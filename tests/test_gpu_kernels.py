@@ -322,6 +322,31 @@ def test_tiles_for_up_to_64_tokens_chosen_by_rounds(ops_for, m, n, k, slices, ch
     torch.testing.assert_close(total, ref, atol=(2e-2 if swiglu else 2e-3) * max(1.0, scale), rtol=2e-2 if swiglu else 1e-4)
 
 
+@pytest.mark.parametrize("m,n,k,most,lines", [
+    (16, 14340, 808, 1, True), (1, 16390, 1544, 1, True), (8, 16390, 1528, 1, False),  # many rows: from 1,536 k on
+    (5, 8188, 4096, 8, True), (5, 8192, 4096, 8, False), (16, 5001, 3304, 8, True),  # rows 8 KB apart
+    (16, 29184, 3592, 1, True), (9, 29264, 3592, 1, False), (8, 29264, 3592, 1, True),  # either side of 200 MB
+    (8, 37889, 3584, 8, True), (12, 2047, 11000, 8, True), (3, 1536, 8960, 8, True),
+])
+def test_whole_lines_of_large_matrices(ops_for, m, n, k, most, lines):
+    """Up to 16 tokens of matrices of 20 MB and more: either side of each line between the kernel that streams whole lines and the tiles,
+    with and without partial sums, against 64 bits: a sum of k products in float32, in any order, is off by at most k times the unit
+    of rounding (2^-23 where products round towards zero) of the sum of their magnitudes."""
+    ops = ops_for(torch.bfloat16)
+    slices = ops.lib.mlr_gemm_bf16_slices(m, n, k, most)
+    assert slices <= most and (slices > 1) == (most > 1)
+    assert (ops.lib.mlr_gemm_bf16_kernel(m, n, k, slices) == 16) == lines
+    x = _rand((m, k), torch.bfloat16, 73)
+    w = (torch.randn((n, k), generator=torch.Generator(device="cuda").manual_seed(74), device="cuda") * 0.05).to(torch.bfloat16)
+    b = _rand((n,), torch.float32, 75)
+    got = ops.linear(x.cuda(), w, b.cuda(), out_dtype=torch.float32, partial_sums=most > 1)
+    assert got.shape == ((slices, m, n) if most > 1 else (m, n))
+    total = got.double().sum(0) if most > 1 else got.double()
+    ref = x.cuda().double() @ w.double().t() + b.cuda().double()
+    room = (k + 1) * 2.0**-23 * (x.cuda().double().abs() @ w.double().abs().t() + b.cuda().double().abs())
+    assert bool(((total - ref).abs() <= room).all())
+
+
 @pytest.mark.parametrize("m", [17, 31, 32, 33, 50, 64])
 @pytest.mark.parametrize("slices", [1, 4])
 @pytest.mark.parametrize("swiglu", [False, True])
