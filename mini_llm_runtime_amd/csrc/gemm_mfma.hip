@@ -1430,12 +1430,15 @@ static LinesPlan plan_lines(int m, int n, int k, int slices) {
 // tiles keep what they do better: many rows that lie a multiple of 8 KB apart (28,672 x 4,096 43.9 and 51.6, 8,192 x 8,192 30.2 and 33.0: the
 // lines of a load's eight rows meet in the same channels), many rows with a short k, whose workgroups end before their loads are all on their
 // way (32,768 x 512 9.3 and 10.5, 65,536 x 1,024 24.0 and 25.6, 151,936 x 896 45.8 and 49.8), and from 200 MB on, where memory's rate is the
-// bound, more than 8 tokens, which every workgroup reads again (55,296 x 5,120 at 16 tokens 84 and 91).
+// bound, more than 8 tokens, which every workgroup reads again (55,296 x 5,120 at 16 tokens 84 and 91), and more than 4 of up to 65,536 rows,
+// which tiles of up to 256 features stream in one round (at 8 tokens 55,296 x 5,120 83.8 both, 37,888 x 3,584 42.8 and 42.2; at one token,
+// where they cost as much as at 8, 43.4 and 41.5).
 static bool lines_stream(int m, int n, int k) {
   const int64_t bytes = static_cast<int64_t>(n) * k * 2;
   if (bytes < (20ll << 20)) return true;
   if ((n >= 8192 && k % 4096 == 0) || (n >= 16384 && k < 1536)) return false;
-  return bytes < (200ll << 20) || (m <= 8 && k >= 2048);
+  if (bytes < (200ll << 20)) return true;
+  return k >= 2048 && (m <= 4 || (m <= 8 && n > 65536));
 }
 
 // Up to 8 tokens of the fused query/key/value product: workgroups of 8 weight rows instead of 16 while that makes one round of them; beyond,

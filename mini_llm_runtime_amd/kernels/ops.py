@@ -1127,7 +1127,7 @@ class HipOps:
         if not use_mfma:
             # Prompt portions in float32 run in tiles on the matrix cores (in float32) where the mask is a plain one; the plain kernel
             # then takes the entries of one token only.  (0.5B sizes, prompts of 391, 268, 145 and 22 tokens: 479 us with the plain
-            # kernel, 44 us in tiles.)  Other masks, pages and head sizes keep the plain kernel, which takes them all.
+            # kernel, 27 in tiles.)  Other masks, pages and head sizes keep the plain kernel, which takes them all.
             singles = None
             if (
                 kernel == "auto" and self.dtype == torch.float32 and num_tiles and head_dim in F32_TILE_HEAD_DIMS

@@ -325,8 +325,8 @@ def test_tiles_for_up_to_64_tokens_chosen_by_rounds(ops_for, m, n, k, slices, ch
 @pytest.mark.parametrize("m,n,k,most,lines", [
     (16, 14340, 808, 1, True), (1, 16390, 1544, 1, True), (8, 16390, 1528, 1, False),  # many rows: from 1,536 k on
     (5, 8188, 4096, 8, True), (5, 8192, 4096, 8, False), (16, 5001, 3304, 8, True),  # rows 8 KB apart
-    (16, 29184, 3592, 1, True), (9, 29264, 3592, 1, False), (8, 29264, 3592, 1, True),  # either side of 200 MB
-    (8, 37889, 3584, 8, True), (12, 2047, 11000, 8, True), (3, 1536, 8960, 8, True),
+    (16, 29184, 3592, 1, True), (9, 29264, 3592, 1, False), (4, 29264, 3592, 1, True), (5, 29264, 3592, 1, False),  # either side of 200 MB
+    (8, 65544, 2056, 1, True), (4, 37889, 3584, 8, True), (12, 2047, 11000, 8, True), (3, 1536, 8960, 8, True),
 ])
 def test_whole_lines_of_large_matrices(ops_for, m, n, k, most, lines):
     """Up to 16 tokens of matrices of 20 MB and more: either side of each line between the kernel that streams whole lines and the tiles,
