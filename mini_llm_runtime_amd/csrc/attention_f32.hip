@@ -8,11 +8,12 @@
 //
 // Bound by the matrix cores (256 operations a clock and compute unit in float32): a 64-key tile of 64 queries at head size 64 is
 // 4,096 clocks of them for 32 KB of keys and values, which one LDS buffer with the next tile on its way in registers keeps up
-// with; and for short prompts by the chain of tiles that the last queries see.  A workgroup takes 64 queries of one head; two groups of four
-// wavefronts, 16 queries each, take the key tiles in turn and add up at the end, which halves that chain.
+// with; and for short prompts by the chain of tiles that the last queries see.  A workgroup takes 64 queries of one head; one group of four
+// wavefronts, 16 queries each, takes all key tiles, or two take them in turn and add up at the end, which halves that chain (groups_for).
 // Measured at 0.5B sizes (14 query and 2 key/value heads of 64), prompts of 391, 268, 145 and 22 tokens in one step: 479 us with the
-// plain kernel (a wavefront per token and head, attention_simple.hip), 42 with one group and pages looked up beside the loads, 32 with
-// two groups, 27 here.
+// plain kernel (a wavefront per token and head, attention_simple.hip), 36 with one group and pages looked up beside the loads, 31 with
+// pages looked up a turn ahead, 27 with two groups.  Error against 64 bits: with one group as with pages looked up beside the loads, bit for bit; with two the
+// same up to 64 tokens and 2 to 22 % less beyond (65 to 2,048 tokens, all head sizes here).
 #include "common.h"
 #include "mfma.h"
 
@@ -28,14 +29,12 @@ constexpr int D = MLR_HEAD_DIM;
 constexpr int kDimTiles = D / 16;
 constexpr int kTileQ = 64;                 // queries of a workgroup
 constexpr int kTileK = D > 80 ? 32 : 64;   // keys of a group in LDS at a time
-constexpr int kGroups = 2;                 // groups of four wavefronts, which take the key tiles in turn
 constexpr int kSubTiles = kTileK / 16;
 // rows padded to 32 bytes modulo 64: 16 rows x 4 pieces of 16 bytes are then read without bank conflicts
 constexpr int kKLd = D + 8;
 constexpr int kVLd = kTileK + 8;
 constexpr int kPieces = kTileK * D / 4 / 256;  // 16-byte pieces of a thread, of the key and of the value tile
 constexpr int kGroupFloats = kTileK * kKLd + D * kVLd;  // LDS of a group: its keys, then its values
-constexpr int kLdsBytes = kGroups * kGroupFloats * 4;
 static_assert(kGroupFloats >= (2 + D / 4) * 256, "what the second group hands over fits its tiles");
 static_assert(kTileK * D / 4 % 256 == 0, "whole pieces for every thread");
 
@@ -99,7 +98,9 @@ __device__ void attend_alone(const float* __restrict__ q, int64_t q_stride, cons
 
 __device__ __attribute__((aligned(16))) const float kGoneKeys[4] = {__builtin_nanf(""), __builtin_nanf(""), __builtin_nanf(""), __builtin_nanf("")};
 
-__global__ __launch_bounds__(256 * kGroups) void attn_prefill_f32_kernel(
+// GROUPS: of four wavefronts, which take the key tiles in turn (see groups_for)
+template <int GROUPS>
+__global__ __launch_bounds__(256 * GROUPS) void attn_prefill_f32_kernel(
     const float* __restrict__ q, int64_t q_stride, const float* __restrict__ key_pages, const float* __restrict__ value_pages,
     const int* __restrict__ block_table, int table_width, const int* __restrict__ tiles, const int* __restrict__ cu_q,
     const int* __restrict__ context_lens, float* __restrict__ out, int heads, int kv_heads, int block_size, int num_pages,
@@ -111,7 +112,7 @@ __global__ __launch_bounds__(256 * kGroups) void attn_prefill_f32_kernel(
   const int kvh = head / (heads / kv_heads);
   const int entry = tiles[2 * tile];
   const int q0 = tiles[2 * tile + 1];
-  const int group = __builtin_amdgcn_readfirstlane(threadIdx.x / 256);
+  const int group = GROUPS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / 256);
   const int tid = threadIdx.x % 256;  // of the group
   const int lane = tid % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);  // of the group: 16 queries
@@ -215,7 +216,7 @@ __global__ __launch_bounds__(256 * kGroups) void attn_prefill_f32_kernel(
   const int k_begin = k_first / kTileK * kTileK;
   const int k_all_first = first_visible_key(pos0 + q0 + kTileQ - 1, window, chunk);  // from here on no query here is past its window
   bool odd = false;
-  constexpr int kTurn = kGroups * kTileK;
+  constexpr int kTurn = GROUPS * kTileK;
   lookup(k_begin + group * kTileK);
   fetch(k_begin + group * kTileK);
   lookup(k_begin + group * kTileK + kTurn);
@@ -287,25 +288,25 @@ __global__ __launch_bounds__(256 * kGroups) void attn_prefill_f32_kernel(
     }
   }
   if (odd) {  // the same for the whole workgroup: its queries one after the other, each over the keys it sees
-    for (int u = group; u < 16 && q0 + wave * 16 + u < q_len; u += kGroups)
+    for (int u = group; u < 16 && q0 + wave * 16 + u < q_len; u += GROUPS)
       attend_alone(q, q_stride, key_pages, value_pages, table, table_width, t_first + q0 + wave * 16 + u, pos0 + q0 + wave * 16 + u, head,
                    heads, kvh, kv_heads, block_size, num_pages, scale, window, chunk, sinks, out);
     return;
   }
-  // the second group's share to the first: [component][thread]
-  __syncthreads();
-  float* const given = tile_lds + kGroupFloats;
-  if (group > 0) {
-    given[tid] = m_run;
-    given[256 + tid] = l_run;
+  if (GROUPS > 1 && k_begin + kTileK < k_end) {  // the second group's share to the first: [component][thread]
+    static_assert(GROUPS <= 2, "one group hands over");
+    __syncthreads();
+    float* const given = tile_lds + kGroupFloats;
+    if (group > 0) {
+      given[tid] = m_run;
+      given[256 + tid] = l_run;
 #pragma unroll
-    for (int dt = 0; dt < kDimTiles; ++dt)
+      for (int dt = 0; dt < kDimTiles; ++dt)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) given[(2 + dt * 4 + i) * 256 + tid] = acc[dt][i];
-  }
-  __syncthreads();
-  if (group > 0) return;
-  {
+        for (int i = 0; i < 4; ++i) given[(2 + dt * 4 + i) * 256 + tid] = acc[dt][i];
+    }
+    __syncthreads();
+    if (group > 0) return;
     const float m_other = given[tid];
     const float m_new = fmaxf(m_run, m_other);
     const float mine = m_run == -INFINITY ? 0.f : expf(m_run - m_new), other = m_other == -INFINITY ? 0.f : expf(m_other - m_new);
@@ -316,6 +317,7 @@ __global__ __launch_bounds__(256 * kGroups) void attn_prefill_f32_kernel(
       for (int i = 0; i < 4; ++i) acc[dt][i] = acc[dt][i] * mine + given[(2 + dt * 4 + i) * 256 + tid] * other;
     m_run = m_new;
   }
+  if (group > 0) return;
   float l = l_run;
   l += __shfl_xor(l, 16, kWave);
   l += __shfl_xor(l, 32, kWave);
@@ -338,17 +340,67 @@ __global__ __launch_bounds__(256 * kGroups) void attn_prefill_f32_kernel(
   }
 }
 
+template <int GROUPS>
+static int launch_groups(const float* q, int64_t q_stride, const float* key_pages, const float* value_pages, const int* block_table, int table_width,
+                         const int* tiles, int num_tiles, const int* cu_q, const int* context_lens, float* out, int heads, int kv_heads,
+                         int block_size, int num_pages, float scale, int window, int chunk, const float* sinks, hipStream_t stream) {
+  constexpr int kLdsBytes = GROUPS * kGroupFloats * 4;
+  static bool configured = false;
+  if (!configured) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(attn_prefill_f32_kernel<GROUPS>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes);
+    if (e != hipSuccess) {
+      set_error(std::string("mlr_attention_prefill_f32: cannot raise the LDS limit: ") + hipGetErrorString(e));
+      return -1;
+    }
+    configured = true;
+  }
+  attn_prefill_f32_kernel<GROUPS><<<dim3(static_cast<unsigned>(num_tiles) * heads), 256 * GROUPS, kLdsBytes, stream>>>(
+      q, q_stride, key_pages, value_pages, block_table, table_width, tiles, cu_q, context_lens, out, heads, kv_heads, block_size,
+      num_pages, scale, window, chunk, sinks);
+  return 0;
+}
+
+// One group of wavefronts or two.  A second halves a workgroup's chain of key tiles and takes the LDS of a second workgroup: 8 wavefronts a
+// workgroup and two of them on a unit up to head size 64, where four of one group are; one beyond, where three or four are.  So two while every
+// workgroup can have a unit to itself, and beyond that where the longest prompt (`longest` tiles of queries, 0: not known) makes chains that end
+// long after the others: its first tiles are short and leave early, its last ones are the step's end.  Microseconds, with one group and pages looked
+// up beside the loads (as it was) / one / two, 16 query heads unless stated: 64, 32 and so on in the first column are head sizes.
+//   64 (14 heads)  391, 268, 145 and 22 tokens 35.6 / 31.0 / 27.1, 2,048 tokens 185 / 165 / 146, 32 prompts of 64 12.1 / 11.5 / 12.2
+//   64 (28 heads)  2,048 tokens (896 workgroups) 255 / 238 / 224, 32 prompts of 64 21.5 / 20.4 / 24.5, 8 of 300 (1,120) 70.6 / 66.0 / 62.9
+//   80             391 tokens 40.8 / 35.9 / 32.3, 32 prompts of 64 (512) 16.2 / 14.9 / 21.4, 8 of 130 (384) 26.3 / 24.3 / 28.3, 2,048 behind a
+//                  window of 64 (512) 24.8 / 22.5 / 27.0
+//   96             1,024 tokens (256) 122 / 105 / 86, 4,096 (1,024) 792 / 774 / 815, 1,536 (384) 203 / 183 / 166
+//   128            64 tokens 12.7 / 11.5 / 12.1, 391 57.5 / 50.5 / 44.5, 2,048 (28 heads, 896) 484 / 445 / 475, 4,096 (1,792) 1,642 / 1,465 / 1,625,
+//                  32 prompts of 64 (28 heads, 896) 38.4 / 34.2 / 49.5, 1,024, 512, 256, 128 and 64 tokens (496) 166 / 123 / 105
+//   16             32 prompts of 64 6.1 / 6.3 / 6.6, 8 of 520 (1,152) 40.8 / 41.2 / 45.3, 391 tokens 16.0 / 15.8 / 13.4, 4 of 1,024 (1,024) 79.7 / 80.4 / 59.4
+static int groups_for(int num_tiles, int longest, int heads, int window, int chunk) {
+  constexpr int kUnits = 256;
+  constexpr bool kTwoFit = D <= 64;  // two workgroups of two groups on a unit
+  const int64_t workgroups = static_cast<int64_t>(num_tiles) * heads;
+  if (workgroups <= kUnits) return 2;
+  const int span = window > 0 ? window : chunk;
+  const int chain = span > 0 ? min(longest, span / kTileQ + 1) : longest;
+  if (workgroups <= 2 * kUnits) return chain >= (kTwoFit ? 3 : 6) ? 2 : 1;
+  return kTwoFit && chain >= (D > 16 ? 8 : 12) ? 2 : 1;
+}
+
 }  // namespace f32_attention
 }  // namespace mlr
 
 using namespace mlr;
 
+// How many groups of wavefronts mlr_attention_prefill_f32 has for these sizes.
+extern "C" int mlr_attention_prefill_f32_groups(int num_tiles, int longest, int heads, int window, int chunk) {
+  return f32_attention::groups_for(num_tiles, longest, heads, window, chunk);
+}
+
 // Attention of the query tiles in `tiles` ([num_tiles][2]: entry, first query; 64 queries per tile) in float32, with the arguments
-// of mlr_attention_prefill.  A page id out of range makes the rows of the tokens that see its keys NaN, as in the plain kernel.
+// of mlr_attention_prefill; longest: the most tiles of one entry, or 0.  A page id out of range makes the rows of the tokens that see its keys NaN, as in the plain kernel.
 extern "C" int mlr_attention_prefill_f32(const float* q, int64_t q_stride, const float* key_pages, const float* value_pages,
                                          const int* block_table, int table_width, const int* tiles, int num_tiles, const int* cu_q,
                                          const int* context_lens, float* out, int heads, int kv_heads, int block_size, int num_pages,
-                                         float scale, int window, int chunk, const float* sinks, hipStream_t stream) {
+                                         float scale, int window, int chunk, const float* sinks, int longest, hipStream_t stream) {
   MLR_REQUIRE(q && key_pages && value_pages && block_table && tiles && cu_q && context_lens && out, "null pointer");
   MLR_REQUIRE(num_tiles > 0 && heads > 0 && kv_heads > 0 && heads % kv_heads == 0, "bad sizes");
   MLR_REQUIRE(block_size > 0 && block_size % 4 == 0, "block_size must be a multiple of 4");
@@ -358,21 +410,12 @@ extern "C" int mlr_attention_prefill_f32(const float* q, int64_t q_stride, const
                   reinterpret_cast<uintptr_t>(value_pages) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0,
               "operands must be 16-byte aligned");
   MLR_REQUIRE(scale > 0.f && scale < INFINITY && window >= 0 && chunk >= 0 && !(window > 0 && chunk > 0), "bad scale, window or chunk");
+  MLR_REQUIRE(longest >= 0, "the longest prompt's tiles must be >= 0 (0: not known)");
   MLR_REQUIRE(static_cast<int64_t>(num_tiles) * heads < (1ll << 31), "too many tiles for one launch");
-  static bool configured = false;
-  if (!configured) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(f32_attention::attn_prefill_f32_kernel),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, f32_attention::kLdsBytes);
-    if (e != hipSuccess) {
-      set_error(std::string("mlr_attention_prefill_f32: cannot raise the LDS limit: ") + hipGetErrorString(e));
-      return -1;
-    }
-    configured = true;
-  }
-  f32_attention::attn_prefill_f32_kernel<<<dim3(static_cast<unsigned>(num_tiles) * heads), 256 * f32_attention::kGroups, f32_attention::kLdsBytes,
-                                           stream>>>(
-      q, q_stride, key_pages, value_pages, block_table, table_width, tiles, cu_q, context_lens, out, heads, kv_heads, block_size,
-      num_pages, scale, window, chunk, sinks);
+  const auto launch = f32_attention::groups_for(num_tiles, longest, heads, window, chunk) == 1 ? f32_attention::launch_groups<1> : f32_attention::launch_groups<2>;
+  if (launch(q, q_stride, key_pages, value_pages, block_table, table_width, tiles, num_tiles, cu_q, context_lens, out, heads, kv_heads, block_size,
+             num_pages, scale, window, chunk, sinks, stream) != 0)
+    return -1;
   MLR_LAUNCH_CHECK();
   return 0;
 }

@@ -130,8 +130,9 @@ _SIGNATURES = {
         _I,
     ),
     "mlr_attention_prefill_f32": (
-        [_VP, _I64, _VP, _VP, _VP, _I, _VP, _I, _VP, _VP, _VP, _I, _I, _I, _I, _F, _I, _I, _VP, _VP], _I,
+        [_VP, _I64, _VP, _VP, _VP, _I, _VP, _I, _VP, _VP, _VP, _I, _I, _I, _I, _F, _I, _I, _VP, _I, _VP], _I,
     ),
+    "mlr_attention_prefill_f32_groups": ([_I, _I, _I, _I, _I], _I),
     "mlr_sample": ([_VP, _VP, _VP, _VP, _VP, _I, _I, _VP], _I),
     "mlr_sample_scratch": ([_I, _I], _I64),
     "mlr_attention_head_dim": ([], _I),
@@ -1141,7 +1142,7 @@ class HipOps:
                     "mlr_attention_prefill_f32", self._ptr(qkv), stride, self._ptr(key_pages), self._ptr(value_pages),
                     self._ptr(block_table), width, self._ptr(tiles), num_tiles, self._ptr(ctx.cu_q), self._ptr(ctx.context_lens),
                     self._ptr(out), num_heads, num_kv_heads, block_size, num_pages, float(scale), int(window or 0), chunk,
-                    self._ptr(sinks), self._stream(), lib=self.attention_library(head_dim),
+                    self._ptr(sinks), int(getattr(plan, "longest_prompt_tiles", 0)), self._stream(), lib=self.attention_library(head_dim),
                 )
                 if not num_decode:
                     return out

@@ -12,6 +12,7 @@ from ..parts.context import MixerPlan, PlanInput
 QUERY_TILE = 64  # queries of one request that the prompt kernel takes together
 WIDE_QUERY_TILE = 128  # and in its variant for long prompts (two blocks of queries per wavefront)
 LONG_PREFIX_KEYS = 2048  # mean number of keys before a tile from which a step counts as behind long prefixes (twice: very long)
+LONG_PROMPT_TILES = 12  # from which a prompt counts as long (see attention_f32.hip, groups_for)
 PAGED_ATTENTION = "paged_attention"  # the plan's key: every mixer on these kernels shares one plan per step
 
 
@@ -29,7 +30,8 @@ def query_tiles(q_lens, q_starts=None, tile: int = QUERY_TILE) -> np.ndarray:
 
 def attention_plan(shape: PlanInput) -> MixerPlan:
     """Tiles of 64 and of 128 queries over the entries with several new tokens (for the prompt
-    kernel and its wide variant; the launch picks one by how many there are), and
+    kernel and its wide variant; the launch picks one by how many there are), how many of 64 the longest
+    portion has (up to where it counts as long), and
     how many entries have a single token and how long their contexts may be (for the split-KV
     decode kernel).  `shape.max_context` bounds the contexts; a recording is made with the
     capacity of its block tables there, so that it holds for every later step of its sizes."""
@@ -43,6 +45,7 @@ def attention_plan(shape: PlanInput) -> MixerPlan:
     keys_before = [int(shape.q_starts[e]) + int(q0) for e, q0 in wide]
     mean_before = sum(keys_before) / len(keys_before) if keys_before else 0
     long_prefix = int(mean_before >= LONG_PREFIX_KEYS) + int(mean_before >= 2 * LONG_PREFIX_KEYS)
+    most_new = max((int(n) for n in shape.q_lens if n > 1), default=0)
     return MixerPlan(
         key=PAGED_ATTENTION,
         arrays={"query_tiles": tiles, "wide_query_tiles": wide},
@@ -50,6 +53,7 @@ def attention_plan(shape: PlanInput) -> MixerPlan:
             "num_query_tiles": len(tiles),
             "num_wide_query_tiles": len(wide),
             "long_prefix": long_prefix,
+            "longest_prompt_tiles": min(-(-most_new // QUERY_TILE), LONG_PROMPT_TILES),
             "num_decode_entries": decodes,
             "max_decode_context": int(shape.max_context) if decodes else 0,
         },

@@ -107,3 +107,25 @@ def test_kernel_choice_where_tiles_of_tokens_are_not_full():
     for m in (96, 128):
         slices = lib.mlr_gemm_bf16_slices(m, 5120, 27648, 8)
         assert slices == 4 and lib.mlr_gemm_bf16_kernel(m, 5120, 27648, slices) == 65
+
+
+def test_second_group_of_wavefronts_where_it_has_room():
+    """32-bit prompt attention has one group of wavefronts a workgroup or two, which take the room of two workgroups up to head size 64 and of three or four
+    beyond: two while every workgroup can have a unit, and further only beside long prompts (host code, answers without a GPU)."""
+    import ctypes
+
+    import pytest
+
+    if not all(build.is_current(build.attention_module(d)) for d in (16, 64, 80, 128)):
+        pytest.skip("the attention libraries are not built from the present sources")
+    groups = {d: ctypes.CDLL(str(build.library_path(build.attention_module(d)))).mlr_attention_prefill_f32_groups for d in (16, 64, 80, 128)}
+    for d in groups:  # (tiles, the longest prompt's, heads, window, chunk)
+        assert groups[d](16, 1, 16, 0, 0) == 2 and groups[d](1, 1, 14, 0, 0) == 2  # 256 workgroups and fewer
+        assert groups[d](32, 1, 16, 0, 0) == 1, "32 prompts of one tile"
+        assert groups[d](32, 8, 16, 64, 0) == 1 and groups[d](32, 8, 16, 0, 64) == 1, "a window or chunk of a tile: chains of two"
+        assert groups[d](17, 0, 16, 0, 0) == 1, "not known how long"
+        assert groups[d](32, 8, 16, 0, 0) == 2, "one prompt of 2,048 tokens"
+    assert groups[64](24, 3, 16, 0, 0) == 2 and groups[128](24, 3, 16, 0, 0) == 1  # 8 prompts of 130 tokens
+    assert groups[64](128, 8, 16, 0, 0) == 2 and groups[80](128, 12, 16, 0, 0) == groups[16](128, 8, 16, 0, 0) == 1  # beyond two places a unit
+    assert groups[16](128, 12, 16, 0, 0) == 2
+    assert groups[64](40, 5, 16, 0, 0) == 1

@@ -333,3 +333,19 @@ def test_attention_plan_covers_every_query_once_in_both_tile_sizes():
     assert nearer.sizes["long_prefix"] == 1, "a portion behind 3,000 cached tokens"
     no_prompts = attention_plan(PlanInput(np.ones(3, dtype=np.int32), np.zeros(3, dtype=np.int32), 64))
     assert no_prompts.sizes["num_query_tiles"] == 0 and no_prompts.arrays["wide_query_tiles"].shape == (0, 2)
+
+
+def test_attention_plan_knows_the_longest_portion():
+    import numpy as np
+
+    from mini_llm_runtime_amd.kernels.plans import attention_plan
+    from mini_llm_runtime_amd.parts.context import PlanInput
+
+    def tiles(q_lens, q_starts):
+        return attention_plan(PlanInput(np.array(q_lens, dtype=np.int32), np.array(q_starts, dtype=np.int32), 16384)).sizes["longest_prompt_tiles"]
+
+    assert tiles([1, 300, 64, 1, 129, 2], [77, 0, 500, 9, 130, 4000]) == 5
+    assert tiles([1, 64], [900, 0]) == 1 and tiles([65], [700]) == 2
+    assert tiles([512], [6000]) == 8 and tiles([705], [0]) == 12 and tiles([704], [0]) == 11
+    assert tiles([5000], [0]) == 12, "long is long: one recording holds for all of them"
+    assert tiles([1, 1, 1], [0, 5, 9]) == 0

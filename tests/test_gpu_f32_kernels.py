@@ -99,6 +99,27 @@ def test_prompt_attention_over_several_turns(ops, head_dim, window):
     torch.testing.assert_close(got.cpu().double(), ref, atol=5e-6, rtol=1e-5)  # as above
 
 
+@pytest.mark.parametrize("head_dim", [16, 64, 80, 96, 128])
+@pytest.mark.parametrize("mask", [dict(window=None), dict(window=70), dict(window=None, chunk=96)])
+@pytest.mark.parametrize("odd", [False, True])
+def test_prompt_attention_by_one_group_of_wavefronts(ops, head_dim, mask, odd):
+    """More workgroups than places for two groups each: one group takes a tile's keys, one tile of them, several, and behind cached tokens; a value that is not
+    finite in one prompt.  A step whose longest prompt is known to be long keeps two groups up to head size 64: the same in another order."""
+    entries = [(64, 64), (65, 65), (3, 3), (150, 33), (130, 130), (200, 90), (128, 128)]
+    q, kp, vp, table, ctx, *_ = _paged_case(entries, 48, 8, head_dim, 16, torch.float32, 19)
+    if odd:
+        vp[table[4, 100 // 16], 1, 5, 100 % 16] = float("inf")
+    tiles, groups = ctx.num_query_tiles, ops.attention_library(head_dim).mlr_attention_prefill_f32_groups
+    assert tiles * 48 > 512 and groups(tiles, 0, 48, mask["window"] or 0, mask.get("chunk", 0)) == 1
+    args = (q.cuda(), kp.cuda(), vp.cuda(), table.cuda(), ctx)
+    kw = dict(num_heads=48, num_kv_heads=8, head_dim=head_dim, block_size=16, scale=head_dim**-0.5, sinks=_rand((48,), torch.float32, 15).cuda(), **mask)
+    got, plain = _attend(ops, *args, **kw).cpu(), _attend(ops, *args, kernel="fma", **kw).cpu()
+    assert torch.isfinite(plain).all() != odd
+    torch.testing.assert_close(got, plain, atol=5e-6, rtol=1e-5, equal_nan=True)
+    ctx.longest_prompt_tiles = 8
+    torch.testing.assert_close(_attend(ops, *args, **kw).cpu(), plain, atol=5e-6, rtol=1e-5, equal_nan=True)
+
+
 @pytest.mark.parametrize("head_dim,block", [(64, 16), (128, 16), (80, 8), (16, 4)])
 @pytest.mark.parametrize("mask", [dict(window=None), dict(window=20), dict(window=None, chunk=24)])
 @pytest.mark.parametrize("odd", [float("nan"), float("inf")])
