@@ -1402,8 +1402,9 @@ static bool few_tokens_tiled(int n, int slices) { return ((n + 63) / 64) * slice
 // product is done when the busiest compute unit has taken in its share, the tokens' rows of every workgroup included; a unit holds two
 // workgroups of 16 or 32 features or one of 48 or 64, and starts the next when one is done.  Estimates (us): 44 KB/us a unit (as for the
 // few-token tiles below), 3 for the launch and the first bytes, 1 or, with nobody beside it, 2.5 for every further round, 0.1 in the norm
-// kernel for every slice that it adds.  83 products of 1 to 16 tokens that run here (1.5 to 49 MB of weights, those cut along k with the norm
-// behind them): the choice is 0.6 % off the best on average, 14 % at worst (2,048 x 11,008 at one token, 2 slices 15.0 us, 4 13.2).
+// kernel for every slice that it adds.  83 products of 1 to 16 tokens that ran here below 20 MB or where the tiles would not fill the units (1.5 to 49 MB of weights, those
+// cut along k with the norm behind them): the choice was 0.6 % off the best on average, 14 % at worst (2,048 x 11,008 at one token, 2 slices 15.0 us,
+// 4 13.2).  Over 1,283 sums of the larger ones that lines_stream sends here it is 0.9 % off on average, 69 by more than 5 %, one by 37 % and no other by more than 18 %.
 struct LinesPlan {
   int blocks, slices;
   float us;
@@ -1424,19 +1425,36 @@ static LinesPlan plan_lines(int m, int n, int k, int slices) {
 }
 
 // Up to 16 tokens: whether gemm_lines takes the product also where the tiles would fill the compute units.  Below 20 MB always (2,048 x 4,096
-// in 8 slices at 8 tokens, 17 MB: 7.4 us in tiles, 6.5).  Beyond, over 46 matrices of 20 MB to 1.1 GB at 1 to 16 tokens, sums with their norm:
-// at 8 tokens 14,336 x 768 9.3 us in tiles, 6.6 here; 3,584 x 3,584 12.0 and 10.9; 2,048 x 11,008 at 12 tokens 18.1 and 13.6; 16,384 x 1,536
-// 15.4 and 10.5; 22,016 x 2,048 21.0 and 18.4; 3,584 x 18,944 29.0 and 26.4; 151,936 x 2,048 123 and 102; 152,064 x 3,584 167 and 158.  The
-// tiles keep what they do better: many rows that lie a multiple of 8 KB apart (28,672 x 4,096 43.9 and 51.6, 8,192 x 8,192 30.2 and 33.0: the
-// lines of a load's eight rows meet in the same channels), many rows with a short k, whose workgroups end before their loads are all on their
-// way (32,768 x 512 9.3 and 10.5, 65,536 x 1,024 24.0 and 25.6, 151,936 x 896 45.8 and 49.8), and from 200 MB on, where memory's rate is the
-// bound, more than 8 tokens, which every workgroup reads again (55,296 x 5,120 at 16 tokens 84 and 91), and more than 4 of up to 65,536 rows,
-// which tiles of up to 256 features stream in one round (at 8 tokens 55,296 x 5,120 83.8 both, 37,888 x 3,584 42.8 and 42.2; at one token,
-// where they cost as much as at 8, 43.4 and 41.5).
+// in 8 slices at 8 tokens, 17 MB: 7.4 us in tiles, 6.5).  Beyond, sums with their norm: at 8 tokens 14,336 x 768 9.3 us in tiles, 6.6 here;
+// 3,584 x 3,584 12.0 and 10.9; 2,048 x 11,008 at 12 tokens 18.1 and 13.6; 16,384 x 1,536 15.4 and 10.5; 22,016 x 2,048 21.0 and 18.4; 3,584 x
+// 18,944 29.0 and 26.4; 151,936 x 2,048 123 and 102; 152,064 x 3,584 167 and 158.  The tiles keep what they do better, by regions of some 7,000
+// timings of 1 to 16 tokens, in which gemm_lines' time over the tiles' is, on average:
+//  * rows that lie a multiple of 8 KB apart (and not of 32 KB, where both are slow: 0.9): from 4,096 rows on 1.01 to 1.09, up to 1.28 (8,064 x 8,192;
+//    at k = 4,096 from 7,168 rows on), 1.03 to 1.05 beyond 2,048 rows if it is a multiple of 16 KB; 0.74 to 0.97 else.  28,672 x 4,096 43.9 us in tiles and 51.6.
+//  * rows of which three make a multiple of 64 KB and up to 640 bytes: 1.07 to 1.1 for 4,096 to 8,192 rows (6,144 x 11,008 at 8 tokens 4.3 TB/s and
+//    5.0 in tiles; x 11,136 6.1 and 5.9), and up to 1 KB for 2,049 to 4,095 rows of 32 KB and more: 1.07.
+//  * many rows with a short k, whose workgroups end before their loads are all on their way (32,768 x 512 9.3 us in tiles and 10.5, 65,536 x
+//    1,024 24.0 and 25.6, 151,936 x 896 45.8 and 49.8).
+//  * more than 8 tokens, which every workgroup reads again, of more than 16,384 rows from k = 3,584 on: 1.03.
+//  * rows that do not begin on a line of 128 bytes, from 128 MB on: 1.03 to 1.09 for 14,336 to 16,384 rows, 1.03 to 1.1 for up to 32,768 at more than 8 tokens or
+//    beyond k = 8,192; 0.76 to 0.98 elsewhere.
+//  * more than 8 tokens of 4,097 to 4,608 rows from k = 10,240 on, which make one full round of tiles of 160 features in 8 slices: 1.01 to 1.08.
+//  * rows 4 KB apart from 196,608 of them on: 1.02 to 1.08.
+//  * from 200 MB on, where memory's rate is the bound, more than 8 tokens (55,296 x 5,120 at 16 tokens 84 us and 91), and more than 4 of up to 65,536
+//    rows, which tiles of up to 256 features stream in one round (at 8 tokens 55,296 x 5,120 83.8 both, 37,888 x 3,584 42.8 and 42.2; at one token,
+//    where they cost as much as at 8, 43.4 and 41.5).
+// What this makes of 3,503 drawn products (20 MB to 1.1 GB, k of 512 to 33,000, every alignment) whose route is gemm_lines or was: 2,862 times gemm_lines, 0.90 of the
+// tiles' time on average, 60 of them more than 3 % slower and 32 more than 5 %, the worst 31 % (4 tokens of 7,392 x 16,320).
 static bool lines_stream(int m, int n, int k) {
   const int64_t bytes = static_cast<int64_t>(n) * k * 2;
   if (bytes < (20ll << 20)) return true;
   if ((n >= 8192 && k % 4096 == 0) || (n >= 16384 && k < 1536)) return false;
+  if (k % 4096 == 0 && k % 16384 != 0 && (n >= 7168 || (n >= 4096 && k > 4096) || (n > 2048 && k % 8192 == 0))) return false;
+  const int three_rows = static_cast<int>(6ll * k % 65536);
+  if (three_rows > 0 && ((three_rows <= 640 && n >= 4096 && n <= 8192) || (three_rows <= 1024 && n > 2048 && n < 4096 && k >= 16384))) return false;
+  if (m > 8 && ((n > 16384 && k >= 3584) || (n > 4096 && n <= 4608 && k >= 10240))) return false;
+  if (k % 64 != 0 && bytes >= (128ll << 20) && n >= 14336 && n <= 32768 && (n <= 16384 || m > 8 || k > 8192)) return false;
+  if (k == 2048 && n >= 3 << 16) return false;
   if (bytes < (200ll << 20)) return true;
   return k >= 2048 && (m <= 4 || (m <= 8 && n > 65536));
 }
@@ -1462,7 +1480,9 @@ static bool half_rows_fill_better(int blocks16) { return 2 * blocks16 <= 256; }
 // on average and 15 % at worst, 21 are off by more than 5 %.  (Without `empty`, and with the few-token tiles only where the 64 x 64 ones
 // were chosen, it was 1.1 %, 64 by more than 5 %: 7B gate-up at 257 to 384 tokens 136 to 140 us in tiles of 128 x 128, 108 to 113 in
 // one round of 256 x 320; 1.5B gate-up at 65 to 128 tokens 22 to 24, 20 to 22 in tiles of 64 x 160.  Fitted to three quarters of
-// the matrices, the choice for the others is 0.7 to 1.0 % off.)
+// the matrices, the choice for the others is 0.7 to 1.0 % off.)  The kernels behind the tilings of 128 tokens and more have since moved on to products of 16 x 16 x 32,
+// by 0 to 8 %, without a new fit: timed again, over 635 products of the layers of six model sizes at 65 to 8,191 tokens, sums with their norm, the
+// choice is 0.7 % off the best on average, 31 are off by more than 5 %, and 21 % the worst (0.5B gate-up at 65 tokens: tiles of 64 x 96 11.6 us, of 64 x 64 9.6).
 struct GemmPlan {
   int kernel, slices;
 };
@@ -1759,10 +1779,14 @@ int mlr_gemm_bf16_slices(int m, int n, int k, int max_slices) {
       if (eight && few_tokens_tiled(n, 4) && !few_tokens_tiled(n, 2)) return 8;
       if (k >= 4 * 256 && few_tokens_tiled(n, 4)) return 4;
     }
-    // gemm_lines: at most 8 slices for the norm to add up, a step of k for each of a workgroup's wavefronts.  From 20 MB on never whole where
-    // the consumer takes slices, as in the tiles: one slice would be rounded to bfloat16 before it is added.
-    LinesPlan best = plan_lines(m, n, k, bytes >= (20ll << 20) && max_slices >= 4 && k >= 4 * 256 ? 4 : 1);
-    for (int slices = 2; slices <= min(max_slices, 8) && k >= slices * 256; slices *= 2) {
+    // gemm_lines: at most 8 slices for the norm to add up, a step of k for each of a workgroup's wavefronts; 2 from 20 MB on where its rows go through
+    // rmsnorm_any_kernel, one slice after the other (8 tokens of 10,240 x 2,816 in 4 slices 68 us with the norm, in 2 46).  From 20 MB on never whole if the
+    // consumer takes 4 slices or more and k >= 1,024, as in the tiles: one slice would be rounded to bfloat16 before it is added (one token of
+    // matrices of 20 to 40 MB pays for that with 1.1 us of 9).
+    const bool large = bytes >= (20ll << 20);
+    const int most = min(max_slices, large && n > 8192 ? 2 : 8);
+    LinesPlan best = plan_lines(m, n, k, large && max_slices >= 4 && k >= 4 * 256 ? min(most, 4) : 1);
+    for (int slices = 2; slices <= most && k >= slices * 256; slices *= 2) {
       const LinesPlan plan = plan_lines(m, n, k, slices);
       if (plan.us < best.us) best = plan;
     }

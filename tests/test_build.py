@@ -129,3 +129,28 @@ def test_second_group_of_wavefronts_where_it_has_room():
     assert groups[64](128, 8, 16, 0, 0) == 2 and groups[80](128, 12, 16, 0, 0) == groups[16](128, 8, 16, 0, 0) == 1  # beyond two places a unit
     assert groups[16](128, 12, 16, 0, 0) == 2
     assert groups[64](40, 5, 16, 0, 0) == 1
+
+
+def test_few_tokens_stream_whole_lines_where_that_is_faster():
+    """Up to 16 tokens of matrices of 20 MB and more: the kernel that streams whole lines or the tiles, by the regions that measured slower through it
+    (rows that meet modulo 64 KB, rows off a line, more than 8 tokens of many rows), and 2 slices where the norm adds them up one after the other."""
+    import ctypes
+
+    import pytest
+
+    if not build.is_current(build.CORE):
+        pytest.skip("the core library is not built from the present sources")
+    lib = ctypes.CDLL(str(build.library_path(build.CORE)))
+    for fn in (lib.mlr_gemm_bf16_kernel, lib.mlr_gemm_bf16_slices):
+        fn.argtypes, fn.restype = [ctypes.c_int] * 4, ctypes.c_int
+    lines = lambda m, n, k, most=8: lib.mlr_gemm_bf16_kernel(m, n, k, lib.mlr_gemm_bf16_slices(m, n, k, most)) == 16  # noqa: E731
+    for m in (1, 4, 8, 12, 16):
+        assert not any(lines(m, n, k) for n in (4096, 6144, 8064) for k in (8192, 12288, 20480, 11008)), m
+        assert not lines(m, 3584, 24576) and not lines(m, 3584, 8192) and not lines(m, 3000, 22016)
+        assert all(lines(m, n, k) for n in (3584, 6144) for k in (3584, 8320, 11136)), m
+        assert all(lines(m, n, k) for n, k in ((2048, 24576), (2048, 11008), (3584, 12288), (3584, 18944), (4096, 14336), (5120, 5120)))
+        assert not lines(m, 16384, 5848, 1) and lines(m, 16384, 3592, 1) and lines(m, 16384, 5632, 1)
+        assert not lines(m, 201088, 2048, 1)
+        assert lib.mlr_gemm_bf16_slices(m, 10240, 2816, 8) == 2 and 2 <= lib.mlr_gemm_bf16_slices(m, 8192, 2816, 8) <= 8
+    assert lines(8, 20480, 4096 + 512, 1) and not lines(9, 20480, 4096 + 512, 1)
+    assert lines(4, 152064, 2048, 1) and lines(4, 37888, 3584, 1) and not lines(5, 37888, 3584, 1)

@@ -322,19 +322,26 @@ def test_tiles_for_up_to_64_tokens_chosen_by_rounds(ops_for, m, n, k, slices, ch
     torch.testing.assert_close(total, ref, atol=(2e-2 if swiglu else 2e-3) * max(1.0, scale), rtol=2e-2 if swiglu else 1e-4)
 
 
-@pytest.mark.parametrize("m,n,k,most,lines", [
+LINE_SUMS = [  # m, n, k, slices at most, whether whole lines are streamed
     (16, 14340, 808, 1, True), (1, 16390, 1544, 1, True), (8, 16390, 1528, 1, False),  # many rows: from 1,536 k on
-    (5, 8188, 4096, 8, True), (5, 8192, 4096, 8, False), (16, 5001, 3304, 8, True),  # rows 8 KB apart
-    (16, 29184, 3592, 1, True), (9, 29264, 3592, 1, False), (4, 29264, 3592, 1, True), (5, 29264, 3592, 1, False),  # either side of 200 MB
-    (8, 65544, 2056, 1, True), (4, 37889, 3584, 8, True), (12, 2047, 11000, 8, True), (3, 1536, 8960, 8, True),
-])
+    (5, 7164, 4096, 8, True), (5, 7168, 4096, 8, False), (5, 8192, 4096, 8, False), (9, 4095, 12288, 8, True), (9, 4096, 12288, 8, False),  # rows 8 KB apart
+    (3, 3600, 12288, 8, True), (3, 3600, 8192, 8, False), (8, 4096, 16384, 8, True),  # 8 KB, 16 KB, 32 KB
+    (8, 6144, 11008, 8, False), (8, 6144, 11136, 8, True), (2, 3000, 22016, 8, False), (2, 2048, 22016, 8, True),  # three rows beside a multiple of 64 KB
+    (16, 29184, 3528, 1, False), (8, 29184, 3528, 1, True), (8, 16384, 4104, 1, False), (8, 16384, 4088, 1, True),  # rows off a line; more than 8 tokens of many rows
+    (16, 28740, 2688, 1, True), (16, 4608, 10240, 8, False), (8, 4608, 10240, 8, True),
+    (4, 28748, 3648, 1, True), (5, 28748, 3648, 1, False), (8, 65544, 2112, 1, True), (9, 65544, 2112, 1, False),  # from 200 MB on
+    (16, 5001, 3304, 8, True), (4, 37889, 3584, 8, True), (12, 2047, 11000, 8, True), (3, 1536, 8960, 8, True), (8, 8200, 2600, 8, True),
+]
+
+
+@pytest.mark.parametrize("m,n,k,most,lines", LINE_SUMS)
 def test_whole_lines_of_large_matrices(ops_for, m, n, k, most, lines):
     """Up to 16 tokens of matrices of 20 MB and more: either side of each line between the kernel that streams whole lines and the tiles,
     with and without partial sums, against 64 bits: a sum of k products in float32, in any order, is off by at most k times the unit
     of rounding (2^-23 where products round towards zero) of the sum of their magnitudes."""
     ops = ops_for(torch.bfloat16)
     slices = ops.lib.mlr_gemm_bf16_slices(m, n, k, most)
-    assert slices <= most and (slices > 1) == (most > 1)
+    assert slices <= (2 if lines and n > 8192 else most) and (slices > 1) == (most > 1)
     assert (ops.lib.mlr_gemm_bf16_kernel(m, n, k, slices) == 16) == lines
     x = _rand((m, k), torch.bfloat16, 73)
     w = (torch.randn((n, k), generator=torch.Generator(device="cuda").manual_seed(74), device="cuda") * 0.05).to(torch.bfloat16)
