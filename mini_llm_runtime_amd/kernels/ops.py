@@ -805,6 +805,12 @@ class HipOps:
         )
         return cos, sin
 
+    def _staged_qkv(self, m, width, k, head_dim, block_size, key_pages, value_pages, write) -> bool:
+        """Whether the fused query/key/value kernel takes this call in tiles of 128 x 128."""
+        return self.lib.mlr_qkv_bf16_staged(m, width, k, head_dim, block_size if write else 0) != 0 and (
+            not write or self._aligned(key_pages, value_pages)
+        )
+
     def _check_pages(self, key_pages, value_pages, num_kv_heads, head_dim, block_size) -> int:
         """Pages as the attention kernels read them: values as wide as keys."""
         self._check(key_pages, "key pages", self.dtype, (None, num_kv_heads, block_size, head_dim))
@@ -938,13 +944,15 @@ class HipOps:
             )
             return q
         if fused is None:
-            # The fused kernel is the fastest way where it has 128 x 128 tiles for the shape (one or two rounds of them, whole heads).
-            # Its 64 x 64 tiles, beyond 2^33 multiply-adds or 512 such tiles, are not: there the plain product in the planner's tiles
-            # with the rotation kernel behind it.  In 64 x 64 tiles / plain, in a replayed graph, us: 0.5B sizes at 4,096 tokens (4.2e9)
-            # 27 / 29, at 8,191 (576 tiles) 46 / 37; 1.5B at 4,096 (1.3e10) 60 / 43; 7B at 384 (6.3e9) 39 / 41, at 768 (1.3e10) 54 / 46, at
-            # 1,024 69 / 58, at 2,048 129 / 83; 14B at 400 (1.5e10) 75 / 76, at 512 88 / 78.
+            # The fused kernel is the fastest way where it has 128 x 128 tiles for the shape (one or two rounds of them, whole heads, pages
+            # that begin at 16 bytes).  Its 64 x 64 tiles, beyond 2^33 multiply-adds or 512 tiles of 128 x 128, are not: there the plain product in
+            # the planner's tiles with the rotation kernel behind it.  In 64 x 64 tiles / plain, in a replayed graph, us: 0.5B sizes at 4,096
+            # tokens (4.2e9) 27 / 29, at 8,191 (576 tiles of 128 x 128) 46 / 37; head sizes 48 and 80 with widths of 1,152 and 960 at 7,300 (522) 40.0 / 35.1
+            # and 10,000 tokens (632) 41.2 / 34.5, 96 with 2,304 at 4,096 (576) 42.1 / 41.4, k of 448 and 3,584 features at 3,000 (672) 40.4 / 36.2; 1.5B
+            # at 4,096 (1.3e10) 60 / 43; 7B at 384 (6.3e9) 39 / 41, at 768 (1.3e10) 54 / 46, at 1,024 69 / 58, at 2,048 129 / 83; 14B at 400 (1.5e10)
+            # 75 / 76, at 512 88 / 78.
             large = m > 64 and (m * width * k >= 1 << 33 or -(-m // 128) * -(-width // 128) > 512)
-            fused = can_fuse and (not large or self.lib.mlr_qkv_bf16_staged(m, width, k, head_dim, block_size if write else 0) != 0)
+            fused = can_fuse and (not large or self._staged_qkv(m, width, k, head_dim, block_size, key_pages, value_pages, write))
         elif fused and not can_fuse:
             raise KernelError("the fused query/key/value kernel takes bfloat16 tokens and a full rotation")
         if pending is not None and not (

@@ -543,6 +543,34 @@ def test_staged_qkv_product_of_consecutive_slots(ops_for, kernel, heads, kv_head
     assert torch.isnan(vp.float().cpu()[~written[:, None, None, :].expand(vp.shape)]).all()
 
 
+# either side of the fewest tiles of 128 x 128 (72 and 81), of one round of them (252 and 261) and of the most (504 and 513); a head size and pages that they
+# do not take; more than 2^33 multiply-adds with pages that begin at 8 bytes, which only the plain product and the rotation kernel take well
+@pytest.mark.parametrize("heads,kv_heads,head_dim,hidden,tokens,bs,offset,fused", [
+    (14, 2, 64, 896, 1024, 16, 0, True), (14, 2, 64, 896, 1025, 16, 0, True), (14, 2, 64, 896, 3584, 16, 0, True), (14, 2, 64, 896, 3700, 16, 0, True),
+    (14, 2, 64, 896, 7168, 16, 0, True), (14, 2, 64, 896, 7169, 16, 0, False), (14, 2, 64, 896, 1025, 4, 0, True), (16, 4, 48, 768, 7300, 16, 0, False),
+    (28, 4, 128, 3584, 512, 16, 0, True), (28, 4, 128, 3584, 521, 16, 4, False), (28, 4, 128, 3584, 512, 4, 0, True),
+])
+def test_query_key_value_product_of_a_prompt_as_chosen(ops_for, monkeypatch, heads, kv_heads, head_dim, hidden, tokens, bs, offset, fused):
+    ops = ops_for(torch.bfloat16)
+    width, pages = (heads + 2 * kv_heads) * head_dim, tokens // bs + 2
+    x = _rand((tokens, hidden), torch.bfloat16, 81).cuda()
+    w = _rand((width, hidden), torch.bfloat16, 82, 0.2).cuda()
+    b = _rand((width,), torch.float32, 83).cuda()
+    inv = (1.0 / (1e6 ** (torch.arange(0, head_dim, 2, dtype=torch.float64) / head_dim))).cuda()
+    rotation = (*ops.rope_table(torch.arange(tokens, dtype=torch.int32).cuda(), inv), head_dim)
+    room = pages * kv_heads * head_dim * bs
+    kp, vp = (torch.full((room + offset,), float("nan"), dtype=torch.bfloat16).cuda()[offset:] for _ in range(2))
+    kp, vp = kp.view(pages, kv_heads, bs, head_dim), vp.view(pages, kv_heads, head_dim, bs)
+    slots = torch.arange(3, tokens + 3, dtype=torch.int32)
+    slots[tokens // 2] = -1
+    launched, call = [], ops._call
+    monkeypatch.setattr(ops, "_call", lambda name, *a, **kw: (launched.append(name), call(name, *a, **kw))[1], raising=False)
+    q = ops.qkv_rope_write(x, w, b, rotation, slots.cuda(), kp, vp, num_heads=heads, num_kv_heads=kv_heads, head_dim=head_dim, block_size=bs)
+    assert ("mlr_qkv_rope_write_bf16" in launched) == fused, launched
+    reference = qkv_reference(x, w, b, rotation[0], rotation[1], heads, kv_heads, head_dim)
+    check_qkv("chosen", q.float().cpu(), kp.float().cpu(), vp.float().cpu(), slots, bs, reference, heads, kv_heads, head_dim)
+
+
 @pytest.mark.parametrize("heads,kv_heads,head_dim,hidden,tokens,rotate,write", [
     (14, 2, 64, 896, 64, True, True), (14, 2, 64, 896, 33, True, True), (3, 1, 16, 520, 1, True, True),
     (5, 1, 128, 1208, 8, True, True), (4, 4, 80, 640, 17, False, True), (6, 3, 48, 2056, 5, True, False),
