@@ -154,3 +154,19 @@ def test_few_tokens_stream_whole_lines_where_that_is_faster():
         assert lib.mlr_gemm_bf16_slices(m, 10240, 2816, 8) == 2 and 2 <= lib.mlr_gemm_bf16_slices(m, 8192, 2816, 8) <= 8
     assert lines(8, 20480, 4096 + 512, 1) and not lines(9, 20480, 4096 + 512, 1)
     assert lines(4, 152064, 2048, 1) and lines(4, 37888, 3584, 1) and not lines(5, 37888, 3584, 1)
+
+
+def test_query_key_value_tiles_of_whole_heads():
+    """The staged 128 x 128 tiles of the query/key/value product: from 80 tiles (128 of a long k) to two a unit, head sizes that divide 128, pages of eights, eight steps of k."""
+    import ctypes
+
+    import pytest
+
+    if not build.is_current(build.CORE):
+        pytest.skip("the core library is not built from the present sources")
+    staged = ctypes.CDLL(str(build.library_path(build.CORE))).mlr_qkv_bf16_staged
+    staged.argtypes, staged.restype = [ctypes.c_int] * 5, ctypes.c_int
+    assert [staged(m, 1152, 896, 64, 16) for m in (64, 1024, 1025, 7168, 7169)] == [0, 0, 1, 1, 0]  # 72, 81, 504 and 513 tiles
+    assert [staged(m, 4608, 3584, 128, 16) for m in (384, 385, 1792, 1793)] == [0, 1, 1, 0]  # 108, 144, 504 and 540
+    assert staged(2048, 1152, 896, 64, 0) == staged(2048, 1152, 896, 64, 8) == 1  # no cache write, pages of 8 tokens
+    assert staged(2048, 1152, 896, 64, 12) == staged(2048, 1152, 896, 48, 16) == staged(2048, 1152, 504, 64, 16) == staged(2048, 1152, 900, 64, 16) == 0

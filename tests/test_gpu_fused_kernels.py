@@ -362,6 +362,8 @@ def test_query_key_value_product_pays_the_owed_norm(gpu_device, heads, kv_heads,
     if tokens <= 64:
         ways["16 rows"] = dict(fused=True, mfma_kernel=16)
     ways["tiled"] = dict(fused=True, mfma_kernel=11)
+    if 128 % head_dim == 0:
+        ways["staged by turns"], ways["staged"] = dict(fused=True, mfma_kernel=24), dict(fused=True, mfma_kernel=25)
     if tokens <= 128 and hidden >= 512 and rotate:
         ways["cut along k"] = dict(sliced=True)
     for name, kw in ways.items():
