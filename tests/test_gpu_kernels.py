@@ -945,6 +945,57 @@ def test_decode_attention_merges_batches_of_partitions(ops_for, heads, kv_heads,
     torch.testing.assert_close(got.double(), ref, **_tol(torch.bfloat16))
 
 
+@pytest.mark.parametrize("heads,kv_heads,head_dim", [(14, 2, 64), (4, 1, 128), (2, 1, 256), (3, 1, 16)])
+@pytest.mark.parametrize("form", ["sinks", "window", "window that keeps first tokens", "chunk", "pooled entries", "weighed one by one", "capped", "left unmerged"])
+def test_decode_attention_merges_batches_of_every_form(ops_for, heads, kv_heads, head_dim, form):
+    """17 and more partitions of 64 keys through the merge by several wavefronts, in every form it has, against the plain 32-bit kernel."""
+    ops = ops_for(torch.bfloat16)
+    old = ops.decode_partition, ops.decode_max_groups
+    ops.decode_partition, ops.decode_max_groups = 64, 1 << 20
+    try:
+        # behind a window of 1,088 (17 partitions and what its alignment adds) and in runs of 1,500 (24): contexts at the run's first and last
+        entries = [(3073, 1), (1100, 1), (3000, 1), (3001, 1), (5, 1)]
+        q, kp, vp, table, ctx, dense, *_ = _paged_case(entries, heads, kv_heads, head_dim, 16, torch.bfloat16, 33)
+        args = (q.cuda(), kp.cuda(), vp.cuda(), table.cuda(), ctx)
+        kw = dict(num_heads=heads, num_kv_heads=kv_heads, head_dim=head_dim, block_size=16, scale=head_dim**-0.5, window=None)
+        per_head = _rand((heads,), torch.float32, 34, 2.0).cuda()
+        if form == "sinks":
+            kw["sinks"] = per_head
+        elif form == "window":
+            kw.update(window=1088, sinks=per_head)
+        elif form == "window that keeps first tokens":
+            kw.update(window=1088, keep_first=70)
+        elif form == "chunk":
+            kw["chunk"] = 1500
+        elif form == "pooled entries":
+            pooled_kp, pooled_vp, pooled_table = _paged_case([(3073 // 4, 1)] * 5, heads, kv_heads, head_dim, 16, torch.bfloat16, 35)[1:4]
+            kw.update(window=1088, sinks=per_head, pooled=(pooled_kp.cuda(), pooled_vp.cuda(), pooled_table.cuda(), 4))
+        elif form == "weighed one by one":
+            per_head = per_head - 6.0
+            kw["score_bias"] = per_head
+        elif form == "capped":
+            kw["softcap"] = 3.0
+        plain = _attend(ops, *args, kernel="fma", **kw).cpu()
+        got = _attend(ops, *args, defer_merge=form == "left unmerged", **kw)
+        if form == "left unmerged":
+            assert not isinstance(got, torch.Tensor)
+            got = ops.settle(got)
+            assert torch.equal(got, _attend(ops, *args, **kw))
+    finally:
+        ops.decode_partition, ops.decode_max_groups = old
+    assert torch.isfinite(plain).all()
+    if form != "weighed one by one":
+        torch.testing.assert_close(got.cpu().double(), plain.double(), **_tol(torch.bfloat16))
+        return
+    # a plain sum of thousands of weighed values: every weight goes to the matrix cores in bfloat16, whose spacing is up to 2^-7 of a value, so off by at most
+    # 2^-8 of it, and both results are rounded to bfloat16 likewise
+    for t, (k, v) in enumerate(dense):
+        kk, vv = (d.repeat_interleave(heads // kv_heads, dim=1) for d in (k, v))
+        weight = torch.sigmoid((kk * q[t, : heads * head_dim].double().view(heads, head_dim)).sum(-1) * kw["scale"] + per_head.cpu().double())
+        room = 2.0**-8 * (weight[:, :, None] * vv.abs()).sum(0).reshape(-1) + 2.0**-7 * plain[t].double().abs() + 1e-5
+        assert ((got[t].cpu().double() - plain[t].double()).abs() <= room).all()
+
+
 @pytest.mark.parametrize("heads,kv_heads,head_dim,bs,long", [
     (14, 2, 64, 16, 2048), (8, 2, 128, 16, 1100), (3, 1, 96, 8, 700), (2, 1, 256, 32, 600), (5, 5, 16, 64, 900),
 ])
