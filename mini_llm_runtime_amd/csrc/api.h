@@ -129,12 +129,14 @@ int mlr_gemm_residual_bf16(const void* a, const void* w, const void* bias, int b
 // kernel (up to 64 tokens); 8 its variant with 8 weight rows a workgroup (up to 8 tokens); 11,
 // 22, 44 the tiled kernels as in mlr_gemm_bf16, 24, 25 its 128 x 128 tiles (head sizes that divide 128, pages of a multiple of 8
 // tokens).  row_sumsq, sumsq_parts, norm_eps as there.
-int mlr_qkv_bf16_staged(int m, int n, int k, int head_dim, int block_size);
 int mlr_qkv_rope_write_bf16(const void* x, const void* w, const void* bias, int bias_is_f32, const float* cos,
                             const float* sin, const int* slots, void* key_pages, void* value_pages, void* q_out,
                             int m, int k, int heads, int kv_heads, int head_dim, int block_size, int num_pages,
                             int write, int kernel, const float* row_sumsq, int sumsq_parts, float norm_eps,
                             hipStream_t stream);
+// Whether it takes a product of these sizes in its 128 x 128 tiles by itself (block_size 0: no cache write), pages and q_out that begin at
+// 16 bytes provided.
+int mlr_qkv_bf16_staged(int m, int n, int k, int head_dim, int block_size);
 
 // Products of up to 16 tokens that make their own activations (gemm_fused.hip).
 // Norm prologue: h = RMSNorm(x_in + delta) * norm_weight with the delta a bfloat16 [m, k]

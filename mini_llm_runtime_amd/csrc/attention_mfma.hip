@@ -1382,8 +1382,8 @@ __global__ __launch_bounds__(256) void attn_prefill_merge_kernel(const float* __
   }
 }
 
-// Up to a batch of partitions one wavefront merges; beyond, four: one after the other every batch is a trip to memory.  In a replayed graph with
-// one / four, 8 entries x 14 heads of 64: 64 partitions 5.65 / 3.17 us, 32 3.91 / 3.23, 17 3.85 / 3.19 (16 with one: 2.72); 28 heads of 128: 64
+// Up to a batch of partitions one wavefront merges; beyond, four: one after the other every batch is a trip to memory.  Between the other kernels of
+// a step of 8 requests at 16,384 tokens (0.5B, 64 partitions) 5.8 us with one and 4.5 with four; by itself in a replayed graph with one / four, 8 entries x 14 heads of 64: 64 partitions 5.65 / 3.17 us, 32 3.91 / 3.23, 17 3.85 / 3.19 (16 with one: 2.72); 28 heads of 128: 64
 // 8.03 / 4.30, 17 4.48 / 3.41.  Not for the heads of many entries, which fill the units by themselves: 64 x 28 of 64, 17 partitions 5.71 / 6.53.
 static void launch_merge(dim3 grid, hipStream_t stream, const float* partial, const int* cu_q, const int* context_lens, bf16* out, int heads,
                          int window, int chunk, int part, int splits, const float* sinks, const float* extra, int gated, int keep_first) {

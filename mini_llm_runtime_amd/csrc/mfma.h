@@ -68,8 +68,8 @@ __device__ __forceinline__ f32x16_t mfma_32x32x16(bf16x8_t a, bf16x8_t b, f32x16
 
 // Which shape: both run at 2.45 PFLOP/s on zeros, but on data the matrix cores reach the power cap, and there a product of 16 x 16
 // blocks costs less: registers to registers, random bfloat16, 32 x 32 x 16 1.75 PFLOP/s, 16 x 16 x 32 2.02 (half the accumulator traffic per
-// operation: 32 of k are added up inside).  2.06 with the operand that two neighbouring instructions share held still and the other
-// walked to and fro:
+// operation: 32 of k are added up inside); 2.15 with two successive instructions on the same block, an order that made the kernels 0.5 to 2 %
+// slower.  2.06 with the operand that two neighbouring instructions share held still and the other walked to and fro:
 __host__ __device__ constexpr int turn_at(int i, int row, int count) { return row % 2 == 0 ? i : count - 1 - i; }
 
 }  // namespace mlr

@@ -137,8 +137,9 @@ __global__ __launch_bounds__(kWave) void moe_route_kernel(const float* __restric
 // LDS.  The logits may come as `slices` partial sums [slices, tokens, experts], added up in order.
 // Bound by latency: the plain kernel's rounds go through LDS six times each.  64 experts in 8 groups, 6 choices: 8 tokens 10.5 to 4.7
 // us, 2,000 tokens 13.3 to 6.9.
-// Routes token t by one wavefront; returns what lane j < top wrote as the token's j-th expert.  lds: R * 64 floats of this wavefront's own.  Every
-// wavefront of the workgroup calls it (it has a barrier).
+//
+// This is token t's part, by one wavefront: it returns what lane j < top wrote as the token's j-th expert.  lds: R * 64 floats of this
+// wavefront's own.  Every wavefront of the workgroup calls it (it has a barrier).
 template <int R>
 __device__ __forceinline__ int route_by_lanes(const float* __restrict__ logits, int slices, const float* __restrict__ correction,
                                               int* __restrict__ ids, float* __restrict__ weights, int tokens, int experts, int top,
