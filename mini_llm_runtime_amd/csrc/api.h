@@ -83,7 +83,9 @@ int mlr_gemm_simple(const void* x, const void* w, const void* bias, int bias_is_
 
 // The product of the 32-bit path on the matrix cores, in float32 throughout.  Needs k % 4 == 0 and 16-byte aligned
 // operands.  slices > 1 (a value mlr_gemm_f32_slices returned for this shape): as for mlr_gemm_bf16.
+// mlr_gemm_f32_tiling: the tiling of more than 64 tokens, 100 * (features / 32) + 10 * (tokens / 32) + groups of wavefronts.
 int mlr_gemm_f32_slices(int m, int n, int k, int max_slices);
+int mlr_gemm_f32_tiling(int m, int n, int k, int slices);
 int mlr_gemm_f32(const float* x, const float* w, const float* bias, float* y, int swiglu, int slices, int m, int n, int k,
                  const float* multiply, const int* multiply_rows, float glu_limit, float glu_alpha, hipStream_t stream);
 

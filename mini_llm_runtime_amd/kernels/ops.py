@@ -98,6 +98,7 @@ _SIGNATURES = {
     "mlr_gemm_simple": ([_VP, _VP, _VP, _I, _VP, _I, _I, _I, _I, _I, _I, _VP, _VP, _F, _F, _VP], _I),
     "mlr_gemm_f32": ([_VP, _VP, _VP, _VP, _I, _I, _I, _I, _I, _VP, _VP, _F, _F, _VP], _I),
     "mlr_gemm_f32_slices": ([_I, _I, _I, _I], _I),
+    "mlr_gemm_f32_tiling": ([_I, _I, _I, _I], _I),
     "mlr_gemm_bf16": ([_VP, _VP, _VP, _I, _VP, _I, _I, _I, _I, _I, _I, _I, _VP, _I, _F, _VP, _VP, _F, _F, _VP], _I),
     "mlr_moe_route": ([_VP, _I, _VP, _VP, _VP, _I, _I, _I, _I, _I, _F, _I, _I, _VP], _I),
     "mlr_moe_tile_rows": ([_I], _I),

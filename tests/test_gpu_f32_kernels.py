@@ -36,6 +36,26 @@ def test_product(ops, m, n, k):
     assert ((got - (ref + b.double())).abs() <= bound + 2.0**-23 * (ref.abs() + b.abs())).all()
 
 
+# every tiling where its last tiles hold one row or one feature (or three), k ends in a step of one piece, and the steps are odd in number (one group of
+# wavefronts has one less than the other), whole and in slices of which the last is short
+@pytest.mark.parametrize(
+    "tiling,m,n,k,slices",
+    [(221, 545, 2891, 36, 1), (221, 833, 4865, 36, 2), (211, 417, 3011, 36, 1), (211, 545, 2049, 420, 3), (212, 97, 3053, 36, 1),
+     (212, 161, 1030, 420, 2), (111, 97, 4097, 36, 1), (112, 129, 33, 100, 1), (112, 97, 130, 420, 5), (112, 65, 67, 4, 1)],
+)
+def test_every_tiling(ops, tiling, m, n, k, slices):
+    assert ops.lib.mlr_gemm_f32_tiling(m, n, k, slices) == tiling
+    x, w, b = _rand((m, k), torch.float32, 16), _rand((n, k), torch.float32, 17), _rand((n,), torch.float32, 18)
+    ref, bound = x.double() @ w.double().t() + b.double(), _sum_error(x, w)
+    got = torch.full((slices, m, n), float("nan"), device="cuda")
+    xd, wd, bd = x.cuda(), w.cuda(), b.cuda()
+    ops._call(
+        "mlr_gemm_f32", ops._ptr(xd), ops._ptr(wd), ops._ptr(bd), ops._ptr(got), 0, slices, m, n, k, None, None, 0.0, 0.0, ops._stream()
+    )
+    got = got.cpu().double().sum(0)
+    assert ((got - ref).abs() <= bound + 2.0**-23 * (ref.abs() + b.abs().double())).all()
+
+
 @pytest.mark.parametrize("m", [5, 40, 70])
 @pytest.mark.parametrize("epilogue", ["swiglu", "clamped", "geglu", "relu2", "sigmoid", "gelu_tanh", "multiply", "rows"])
 def test_epilogues_are_the_plain_kernels(ops, m, epilogue):
