@@ -295,13 +295,14 @@ __global__ __launch_bounds__(256) void moe_identity_kernel(const T* __restrict__
 // ---- pairs sorted by expert ------------------------------------------------------------------
 
 // One workgroup.  counts -> offsets and tiles (the first wavefront) -> placement.  counts (cleared, behind a barrier) and start: LDS,
-// [experts]; for_each_pair calls what it is given with every pair that this thread has and the pair's expert (one with matrices).
-template <class EachPair>
-__device__ __forceinline__ void align_pairs(int experts, int tile_rows, int max_tiles, int* counts, int* start, int* used_tiles,
+// [experts]; totals: LDS, the used tiles and the pairs with an expert here; count adds every pair of an expert with matrices to its expert's count, place writes where the pairs are once `start` is known.
+// What the count returned is the pair's place among its expert's: who keeps it needs neither the ids nor the atomics a second time.
+template <class Count, class Place>
+__device__ __forceinline__ void align_pairs(int experts, int tile_rows, int max_tiles, int* counts, int* start, int* totals,
                                             int* __restrict__ sorted, int* __restrict__ offsets, int* __restrict__ tiles,
-                                            const EachPair& for_each_pair) {
+                                            const Count& count, const Place& place) {
   const int tid = threadIdx.x;
-  for_each_pair([&](int, int e) { atomicAdd(&counts[e], 1); });
+  count();
   __syncthreads();
   if (tid < kWave) {  // the first wavefront: where every expert's run and tiles start, 64 experts at a time
     int at = 0, nt = 0;
@@ -333,40 +334,76 @@ __device__ __forceinline__ void align_pairs(int experts, int tile_rows, int max_
     }
     if (tid == 0) {
       offsets[experts] = at;
-      *used_tiles = min(nt, max_tiles);
+      totals[0] = min(nt, max_tiles);
+      totals[1] = at;
     }
   }
   __syncthreads();
-  for (int i = *used_tiles + tid; i < max_tiles; i += blockDim.x) {
+  for (int i = totals[0] + tid; i < max_tiles; i += blockDim.x) {
     tiles[2 * i] = -1;  // a workgroup that finds this has nothing to do
-    tiles[2 * i + 1] = *used_tiles;
+    tiles[2 * i + 1] = totals[0];
   }
-  for (int e = tid; e < experts; e += blockDim.x) counts[e] = 0;
-  __syncthreads();
-  for_each_pair([&](int p, int e) { sorted[start[e] + atomicAdd(&counts[e], 1)] = p; });
+  place();
 }
 
+// KEPT: pairs that a thread keeps, their experts and places, in registers; they are put in order in LDS and leave in whole lines (a wavefront's
+// 64 places are as many lines).  0: any number of pairs and experts, read and counted twice.
+// In a replayed graph, 64 experts, 0 / 4 or 16, microseconds: 192 pairs 2.9 / 2.5, 1,024 3.7 / 2.7, 3,072
+// 4.6 / 3.2, 6,144 5.9 / 4.8, 12,000 8.7 / 5.2, 16,384 10.7 / 6.1; 8 experts, 12,000 8.9 / 6.7; 256, 16,000 14.4 / 8.5.
+constexpr int kKeptExperts = 2048;  // 16 KB of counts and starts beside up to 32 KB of pairs
+template <int KEPT>
 __global__ __launch_bounds__(1024) void moe_align_kernel(const int* __restrict__ ids, int pairs, int experts,
                                                          int tile_rows, int max_tiles, int* __restrict__ sorted,
                                                          int* __restrict__ offsets, int* __restrict__ tiles) {
   extern __shared__ int align_lds[];
   int* counts = align_lds;            // [experts]
   int* start = align_lds + experts;   // [experts]
-  __shared__ int used_tiles;
+  __shared__ int totals[2];
   const int tid = threadIdx.x;
   for (int e = tid; e < experts; e += blockDim.x) counts[e] = 0;
   __syncthreads();
-  // eight ids of a thread are asked for at once: one after the other each would be a trip to L2
-  align_pairs(experts, tile_rows, max_tiles, counts, start, &used_tiles, sorted, offsets, tiles, [&](auto&& use) {
-    for (int p0 = tid; p0 < pairs; p0 += 8 * 1024) {
-      int e[8];
+  if constexpr (KEPT > 0) {
+    unsigned short* in_order = reinterpret_cast<unsigned short*>(start + experts);  // [pairs]
+    int held[KEPT > 0 ? KEPT : 1];  // place * 4,096 + expert, or -1
+    align_pairs(
+        experts, tile_rows, max_tiles, counts, start, totals, sorted, offsets, tiles,
+        [&] {
 #pragma unroll
-      for (int u = 0; u < 8; ++u) e[u] = ids[min(p0 + u * 1024, pairs - 1)];
+          for (int u = 0; u < KEPT; ++u) held[u] = u * 1024 + tid < pairs ? ids[u * 1024 + tid] : -1;
 #pragma unroll
-      for (int u = 0; u < 8; ++u)
-        if (p0 + u * 1024 < pairs && e[u] >= 0 && e[u] < experts) use(p0 + u * 1024, e[u]);
-    }
-  });
+          for (int u = 0; u < KEPT; ++u) {
+            const int e = held[u];
+            held[u] = e >= 0 && e < experts ? atomicAdd(&counts[e], 1) * 4096 + e : -1;
+          }
+        },
+        [&] {
+#pragma unroll
+          for (int u = 0; u < KEPT; ++u)
+            if (held[u] >= 0) in_order[start[held[u] % 4096] + held[u] / 4096] = static_cast<unsigned short>(u * 1024 + tid);
+          __syncthreads();
+          for (int i = tid; i < totals[1]; i += 1024) sorted[i] = in_order[i];
+        });
+  } else {
+    // eight ids of a thread are asked for at once: one after the other each would be a trip to L2
+    auto for_each_pair = [&](auto&& use) {
+      for (int p0 = tid; p0 < pairs; p0 += 8 * 1024) {
+        int e[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) e[u] = ids[min(p0 + u * 1024, pairs - 1)];
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+          if (p0 + u * 1024 < pairs && e[u] >= 0 && e[u] < experts) use(p0 + u * 1024, e[u]);
+      }
+    };
+    align_pairs(
+        experts, tile_rows, max_tiles, counts, start, totals, sorted, offsets, tiles,
+        [&] { for_each_pair([&](int, int e) { atomicAdd(&counts[e], 1); }); },
+        [&] {
+          for (int e = tid; e < experts; e += blockDim.x) counts[e] = 0;
+          __syncthreads();
+          for_each_pair([&](int p, int e) { sorted[start[e] + atomicAdd(&counts[e], 1)] = p; });
+        });
+  }
 }
 
 // Both at once for up to 8 tokens: a workgroup with a wavefront for each.  A launch is most of what either costs: 64 experts in 8
@@ -378,14 +415,21 @@ __global__ __launch_bounds__(kRouteAlignTokens* kWave) void moe_route_align_kern
     int tokens, int routed, int top, int groups, int keep, float scale, int score_kind, int normalise, int experts, int tile_rows, int max_tiles,
     int* __restrict__ sorted, int* __restrict__ offsets, int* __restrict__ tiles) {
   __shared__ float lds[kRouteAlignTokens][R * kWave];
-  __shared__ int counts[R * kWave], start[R * kWave], used_tiles;
+  __shared__ int counts[R * kWave], start[R * kWave], totals[2];
   const int t = threadIdx.x / kWave, lane = threadIdx.x % kWave;
   for (int e = threadIdx.x; e < R * kWave; e += blockDim.x) counts[e] = 0;
   const int id = route_by_lanes<R>(logits, slices, correction, ids, weights, tokens, routed, top, groups, keep, scale, score_kind, normalise, t, lds[t]);
   __syncthreads();
-  align_pairs(experts, tile_rows, max_tiles, counts, start, &used_tiles, sorted, offsets, tiles, [&](auto&& use) {
-    if (lane < top && id < experts) use(t * top + lane, id);
-  });
+  const bool counted = lane < top && id < experts;
+  int among = 0;
+  align_pairs(
+      experts, tile_rows, max_tiles, counts, start, totals, sorted, offsets, tiles,
+      [&] {
+        if (counted) among = atomicAdd(&counts[id], 1);
+      },
+      [&] {
+        if (counted) sorted[start[id] + among] = t * top + lane;
+      });
 }
 
 // ---- the clamped gating in a grouped product's epilogue ------------------------------------------------
@@ -1338,8 +1382,11 @@ int mlr_moe_align(const int* ids, int pairs, int experts, int big, int max_tiles
   MLR_REQUIRE(ids && sorted && offsets && tiles, "null pointer");
   MLR_REQUIRE(pairs > 0 && experts > 0 && experts <= 4096 && max_tiles > 0 && big >= 0 && big <= 3, "bad sizes");
   MLR_REQUIRE(max_tiles >= mlr_moe_max_tiles(pairs, experts, big), "too few tiles for these pairs");
-  moe_align_kernel<<<1, 1024, 2 * static_cast<size_t>(experts) * sizeof(int), stream>>>(
-      ids, pairs, experts, mlr_moe_tile_rows(big), max_tiles, sorted, offsets, tiles);
+  const int kept = experts > kKeptExperts || pairs > 16 * 1024 ? 0 : (pairs > 4 * 1024 ? 16 : 4);
+  const auto kernel = kept == 16 ? moe_align_kernel<16> : (kept == 4 ? moe_align_kernel<4> : moe_align_kernel<0>);
+  const size_t lds = 2 * static_cast<size_t>(experts) * sizeof(int) + (kept ? pairs * sizeof(unsigned short) : 0);
+  hipLaunchKernelGGL(kernel, dim3(1), dim3(1024), lds, stream, ids, pairs, experts, mlr_moe_tile_rows(big),
+                     max_tiles, sorted, offsets, tiles);
   MLR_LAUNCH_CHECK();
   return 0;
 }

@@ -81,6 +81,29 @@ def test_routing_that_sorts(ops, tokens, routed, experts, top, groups, keep):
     assert tiles.view(-1, 2).tolist() == used + [[-1, len(used)]] * (most - len(used))
 
 
+# pairs around a workgroup's threads and what its registers hold, experts around what its memory holds; ids without matrices among them
+@pytest.mark.parametrize("experts,pairs", [(1, 1), (64, 1023), (3, 1025), (64, 4096), (60, 4097), (2, 12000), (256, 16384), (64, 16385), (2048, 16384), (2049, 16384), (4096, 700)])
+@pytest.mark.parametrize("big", [0, 1, 3])
+def test_sorting(ops, experts, pairs, big):
+    ids = torch.randint(-1, experts + 1, (pairs,), generator=torch.Generator().manual_seed(pairs), dtype=torch.int32)
+    by_expert, offsets, tiles, most = ops._pair_index(pairs, experts, big)
+    by_expert.fill_(-7)
+    on_device = ids.cuda()
+    ops._call(
+        "mlr_moe_align", ops._ptr(on_device), pairs, experts, big, most, ops._ptr(by_expert), ops._ptr(offsets), ops._ptr(tiles), ops._stream()
+    )
+    by_expert, offsets, tiles = by_expert.tolist(), offsets.tolist(), tiles.view(-1, 2).tolist()
+    counts = torch.bincount(ids[(ids >= 0) & (ids < experts)].long(), minlength=experts)
+    assert offsets == [0] + counts.cumsum(0).tolist()
+    rows = ops.lib.mlr_moe_tile_rows(big)
+    used = [[e, offsets[e] + i] for e in range(experts) for i in range(0, offsets[e + 1] - offsets[e], rows)]
+    assert tiles == used + [[-1, len(used)]] * (most - len(used))
+    mine = by_expert[: offsets[-1]]
+    assert sorted(mine) == ((ids >= 0) & (ids < experts)).nonzero().flatten().tolist()
+    assert all(ids[p] == e for e in range(experts) for p in mine[offsets[e] : offsets[e + 1]])
+    assert by_expert[offsets[-1] :] == [-7] * (pairs - offsets[-1])
+
+
 def test_routing_of_infinities_and_nan(ops):
     inf, nan = float("inf"), float("nan")
     z = torch.tensor([[nan, 1.0, 0.5, 2.0], [-inf, -inf, -inf, -inf], [nan] * 4, [inf, 1.0, nan, -inf]])
