@@ -1000,9 +1000,9 @@ __global__ __launch_bounds__(256 * kKeyGroups) void attn_prefill_kernel(
 // the head size whose few tiles are as many long chains on a part of the compute units.
 // CAP: capped scores.
 // Bound by the softmax's vector instructions beside the products (two wavefronts a SIMD overlap them in part).  Measured against
-// attn_prefill_kernel's best tiles, whole prompts, microseconds (TFLOP/s): 28 heads of 128: 1,024 tokens 34 to 29, 2,048 83 (362) to 54
-// (557), 8,191 886 (543; the wide tiles, which its rule chose, 1,104: 268 registers leave one wavefront a SIMD) to 525 (916); 14 heads of
-// 64: 2,048 28 to 24, 4,096 76 to 58, 8,191 245 (491) to 156 (771).
+// attn_prefill_kernel's best tiles, whole prompts, microseconds (TFLOP/s): 28 heads of 128: 1,024 tokens 34 to 25, 2,048 83 (362) to 54
+// (557), 8,191 886 (543; the wide tiles, which its rule chose, 1,104: 268 registers leave one wavefront a SIMD) to 492 (977); 14 heads of
+// 64: 2,048 28 to 24, 4,096 76 to 52, 8,191 245 (491) to 151 (797).
 #if MLR_HEAD_DIM == 64 || MLR_HEAD_DIM == 128
 #define MLR_HAS_PROMPT 1
 constexpr int kPromptKeys = 64;
@@ -1046,10 +1046,15 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(
   constexpr int kHeadSteps = D / 16;                 // products over the head's dims
   constexpr int kDims = D / 32;                      // blocks of 32 dims
   const int block_size = 1 << bs_shift;
-  // workgroup -> (tile, head): as attn_prefill_kernel
+  // Workgroup -> (tile, head).  The tiles come heaviest first, and a compute unit takes its next workgroup when it has room.  One workgroup
+  // to a unit (128 KB of LDS): in that order, so that who is done first gets the heaviest that is left.  Two: those that all start together, the
+  // first 512, heavy ones beside light ones, then in order.  (Every second 256 from the light end, as where all are resident at once, leaves the
+  // middle for the end.)  Every second 256 from the light end / as here, microseconds: 64 queries, heads of 128: 16 heads, 1,500 tokens 30.2 /
+  // 25.2, 2,000 46.8 / 37.2; 8 heads, 4,096 79.5 / 62.9; 28 heads, 1,024 28.5 / 25.2.  128 queries: 28 heads, 2,048 53.8 / 53.8, 4,096 152 / 140,
+  // 8,191 523 / 492; 16 heads, 8,191 316 / 289.  Heads of 64, 14: 64 queries, 3,000 34.2 / 33.1, 4,096 57.4 / 52.1; 128, 8,191 155 / 151.
   const int total = num_tiles * heads;
-  const int round = blockIdx.x / 256, in_round = blockIdx.x % 256;
-  const int work = (round & 1) == 0 ? (round / 2) * 256 + in_round : total - 1 - ((round / 2) * 256 + in_round);
+  int work = blockIdx.x;
+  if (prompt_lds_bytes(KG) <= 80 * 1024 && work >= 256 && work < 512) work = min(total, 512) - 1 - (work - 256);
   const int tile = work / heads;
   const int head = work - tile * heads;
   const int entry = tiles[2 * tile];

@@ -160,7 +160,7 @@ _EPILOGUES = {None: 0, "swiglu": 1, "relu2": 2, "sigmoid": 3, "gelu_tanh": 4, "c
 # head sizes whose kernels every build has and whose tiles fit (attention_f32.hip)
 F32_TILE_HEAD_DIMS = tuple(d for d in build.DEFAULT_HEAD_DIMS if d <= 128)
 
-from .plans import PAGED_ATTENTION, QUERY_TILE, WIDE_QUERY_TILE, attention_plan, query_tiles  # noqa: F401
+from .plans import LONG_PROMPT_TILES, PAGED_ATTENTION, QUERY_TILE, WIDE_QUERY_TILE, attention_plan, query_tiles  # noqa: F401
 
 
 class KernelError(RuntimeError):
@@ -1226,10 +1226,23 @@ class HipOps:
             if alone:
                 enough //= 2
             behind = int(getattr(plan, "long_prefix", 0))  # 1: thousands of keys before every tile, 2: twice that
+            reach = int(window or 0) or chunk
+            # Two rounds of narrow tiles of long prompts, heavy ones first, add up alike on every unit; one round of wide ones lasts as long as
+            # its heaviest.  Narrow / wide, us: 16 heads, 2,000 tokens 37.2 / 47.5, twice 1,024 25.4 / 29.4; 8 heads, 4,096 62.9 / 89.7.  Not for
+            # short prompts (16 heads, 8 of 256 16.3 / 14.0, 4 of 500 19.3 / 18.9), a mask that reaches less far than most of a prompt (2,048, a
+            # window of 512 27.8 / 23.1), nor beyond two rounds (28 heads, 1,500 44.8 / 40.3).
+            in_two_rounds = (
+                alone
+                and not behind
+                and num_tiles * num_heads <= self.tuning.wide_attention_groups
+                and int(getattr(plan, "longest_prompt_tiles", 0)) >= LONG_PROMPT_TILES
+                and (not reach or 4 * reach >= 3 * QUERY_TILE * num_tiles)
+            )
             if behind:
                 enough = enough * 3 // 4  # heavy tiles everywhere: fewer of them keep the compute units busy
             if (
                 num_wide * num_heads >= enough
+                and not in_two_rounds
                 # portions of up to 64 tokens fill half of a wide tile, whose keys cost as much as a full one's (64 tokens behind 4,096 for 16
                 # requests, 16 heads of 128: 114 us wide, 83 narrow), unless there are more narrow tiles than units that they have to
                 # themselves (16 behind 2,048 for 8, 40 heads: 66 and 74)
@@ -1246,7 +1259,6 @@ class HipOps:
             # A tile reads no more keys than its mask reaches back: runs of those pay only where few tiles reach far.  In runs / whole, us: 2,048
             # tokens behind 6,144, 16 heads of 128 (256 tiles of 128), a window of 512 73 / 26, of 3,000 114 / 78; 512 behind 8,192, 14 heads of 64
             # (112 tiles), 3,000 41 / 32; 16 behind 16,384, 32 heads of 64, 512 13.3 / 11.9, 1,024 15.5 / 16.0, 2,040 19 / 24, 3,000 19 / 32.
-            reach = int(window or 0) or chunk
             pays = not reach or (reach >= 1024 and groups <= 64)
             if behind == 2 and pays and groups < self.tuning.key_run_groups:
                 key_runs = min(8, -(-self.tuning.key_run_groups // groups))

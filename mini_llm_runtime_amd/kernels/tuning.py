@@ -27,8 +27,9 @@ class KernelTuning:
     # workgroups (fewer leave compute units idle behind the heaviest tiles).
     # Behind thousands of cached keys every tile is heavy and three quarters of that are enough.
     # With the 32 x 32 kernel (head sizes 64 and 128), narrow / wide, microseconds: head size 64, 14 heads: 2,048 tokens (224 wide
-    # workgroups) 23 / 34, 4,096 (448) 60 / 65, 8,191 (896) 190 / 156; head size 128 (where half of this is the line), 28 heads:
-    # 1,024 (224) 29 / 29, 2,048 (448) 70 / 52, 4,096 203 / 148; 16 heads: 1,024 (128) 19 / 27, 2,048 (256) 46 / 47.
+    # workgroups) 24 / 35, 4,096 (448) 52 / 65, 6,000 (658) 102 / 101, 8,191 (896) 173 / 151; 32 heads, 2,048 (512) 34 / 38, 2,700 (704) 55 /
+    # 51; 64 heads, 1,100 (576) 28 / 25; head size 128 (where half of this is the line), 28 heads: 1,024 (224) 25 / 29, 1,200 (280) 34 / 32,
+    # 2,048 (448) 68 / 54, 4,096 214 / 140; 16 heads: 1,024 (128) 20 / 29, 4 of 500 (256) 19.3 / 18.9 (one of 2,000: see the launch).
     wide_attention_groups: int = 512
     # Behind twice as many keys, fewer workgroups than this have the keys of every tile cut into
     # runs (up to 8) with a workgroup each, until there are this many.

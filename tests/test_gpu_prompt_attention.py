@@ -88,6 +88,48 @@ def test_a_key_that_outweighs_the_others(ops, head_dim):
     assert torch.equal(got[late:].view(n - late, 2, head_dim), values.expand(n - late, 2, head_dim))
 
 
+# workgroups (entries x heads) around one and two to every compute unit, and many more; entries of unequal contexts
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("entries", [63, 64, 65, 127, 128, 129, 200])
+def test_every_workgroup_has_its_work(ops, head_dim, entries):
+    lens = [(2 + 3 * i % 50, 2) for i in range(entries)]
+    q, kp, vp, table, ctx, *_ = _paged_case(lens, 4, 2, head_dim, 16, torch.bfloat16, 59)
+    kw = dict(num_heads=4, num_kv_heads=2, head_dim=head_dim, block_size=16, scale=head_dim**-0.5, window=None)
+    args = (q.cuda(), kp.cuda(), vp.cuda(), table.cuda(), ctx)
+    got, plain = _attend(ops, *args, **kw).cpu(), _attend(ops, *args, kernel="fma", **kw).cpu()
+    torch.testing.assert_close(got.double(), plain.double(), **_tol(torch.bfloat16))
+
+
+# two rounds of narrow tiles or one of wide ones: long prompts up to 512 narrow tiles x heads, short ones, one tile more, masks that reach
+# three quarters of the prompts and less, cached tokens before them
+@pytest.mark.parametrize(
+    "heads,entries,mask,wide",
+    [
+        (8, [(4096, 4096)], {}, False), (8, [(4097, 4097)], {}, True), (16, [(1024, 1024)] * 2, {}, False), (16, [(704, 704)] * 2 + [(640, 640)], {}, True),
+        (8, [(4096, 4096)], dict(window=3072), False), (8, [(4096, 4096)], dict(chunk=3071), True), (16, [(4100, 2048)], {}, True),
+    ],
+)
+def test_two_rounds_of_narrow_tiles(heads, entries, mask, wide):
+    from mini_llm_runtime_amd.kernels.ops import HipOps
+
+    launches = []
+
+    class Spying(HipOps):
+        def _call(self, name, *args, lib=None):
+            if name == "mlr_attention_prefill":
+                launches.append(int(args[8]))
+            return super()._call(name, *args, lib=lib)
+
+    ops = Spying(torch.bfloat16, "cuda")
+    q, kp, vp, table, ctx, *_ = _paged_case(entries, heads, 1, 128, 16, torch.bfloat16, 60)
+    ctx.longest_prompt_tiles = min(12, max(-(-n // 64) for _, n in entries))
+    kw = dict(num_heads=heads, num_kv_heads=1, head_dim=128, block_size=16, scale=128**-0.5, **{"window": None, **mask})
+    args = (q.cuda(), kp.cuda(), vp.cuda(), table.cuda(), ctx)
+    got, plain = _attend(ops, *args, **kw).cpu(), _attend(ops, *args, kernel="fma", **kw).cpu()
+    assert launches == [int(wide)]
+    torch.testing.assert_close(got.double(), plain.double(), **_tol(torch.bfloat16))
+
+
 def test_a_page_that_is_not_there(ops):
     q, kp, vp, table, ctx, *_ = _paged_case([(100, 100), (300, 300)], 2, 1, 64, 16, torch.bfloat16, 54)
     table = table.clone()
