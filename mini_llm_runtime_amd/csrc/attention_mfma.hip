@@ -996,8 +996,12 @@ __global__ __launch_bounds__(256 * kKeyGroups) void attn_prefill_kernel(
 //    that outweighs all others gives its value back unrounded.  (Moved only past a slack of 2^8 the loop is 1 to 5 % faster, 8,191 tokens
 //    at 28 heads of 128 499 us instead of 525, but the largest weight is rounded then: errors against 64 bits 1.03 to 1.23 times those of
 //    attn_prefill_kernel, here 0.98 to 1.02 times.)
-// KG: groups of wavefronts that take the key tiles in turn.  1: four wavefronts, 128 queries.  2: two and two, 64 queries, for
-// the head size whose few tiles are as many long chains on a part of the compute units.
+// QW wavefronts of 32 queries, times KG groups that take the key tiles in turn.  4 x 1: 128 queries.  2 x 2: 64 queries, where few tiles are as
+// many long chains on a part of the compute units.  4 x 2, heads of 128: 128 queries and half the chain; like 2 x 2 it has the compute unit
+// to itself (128 KB), but with two wavefronts a SIMD, so that one's softmax runs beside the other's products where there is only one workgroup
+// to a unit.  4 x 1 / 4 x 2, microseconds: 28 heads, 1,300 tokens 36.6 / 29.0, 2,048 53.7 / 48.8, 1,024 behind 4,096 112 / 88, behind 16,384
+// (4 x 1 in two runs of keys) 317 / 284; 16 heads, 3,000 70.7 / 54.8; but 28 heads, 3,000 (672 workgroups) 83 / 94.  (2 x 4 for heads of 64:
+// 14 heads, 1,024 tokens 13.6 / 12.8, 2,048 23.2 / 24.3, 4,096 53 / 65.)
 // CAP: capped scores.
 // Bound by the softmax's vector instructions beside the products (two wavefronts a SIMD overlap them in part).  Measured against
 // attn_prefill_kernel's best tiles, whole prompts, microseconds (TFLOP/s): 28 heads of 128: 1,024 tokens 34 to 25, 2,048 83 (362) to 54
@@ -1027,10 +1031,11 @@ __device__ __forceinline__ void wait_and_meet() {
   asm volatile("" ::: "memory");
 }
 
+constexpr int kDoubleQW = D == 128 ? 4 : 2;  // the wide tiles' query wavefronts in two key groups, at the head size that has them
 constexpr int prompt_lds_bytes(int groups) { return 2 * groups * kPromptKeys * D * 4; }
 
-template <int KG, bool CAP>
-__global__ __launch_bounds__(256, 2) void attn_prompt_kernel(
+template <int QW, int KG, bool CAP>
+__global__ __launch_bounds__(QW * KG * kWave, QW * KG == 4 ? 2 : 1) void attn_prompt_kernel(
     const bf16* __restrict__ q, int64_t q_stride, const bf16* __restrict__ key_pages, const bf16* __restrict__ value_pages,
     const int* __restrict__ block_table, int table_width, const int* __restrict__ tiles, const int* __restrict__ cu_q,
     const int* __restrict__ context_lens, bf16* __restrict__ out, int num_tiles, int heads, int kv_heads, int bs_shift,
@@ -1038,8 +1043,8 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(
     int keep_partial, float softcap) {
   extern __shared__ __attribute__((aligned(16))) unsigned char prefill_lds[];
   __shared__ int sm_bad;
-  constexpr int kQueryWaves = 4 / KG;
-  constexpr int kWgQ = 32 * kQueryWaves;
+  constexpr int kWgQ = 32 * QW;
+  constexpr int kRuns = 4 / QW;                      // runs of 16 keys of a tile that a wavefront brings
   constexpr int kTileBytes = kPromptKeys * D * 2;    // of keys, and of values
   constexpr int kPieceRow = D / 8;                   // 16-byte pieces of a key row
   constexpr int kLoads = D / 32;                     // 1 KB loads of 16 keys, and of their values
@@ -1063,8 +1068,8 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(
   const int tid = threadIdx.x;
   const int lane = tid % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
-  const int group = wave / kQueryWaves;   // key group
-  const int qw = wave % kQueryWaves;      // which 32 queries
+  const int group = wave / QW;   // key group
+  const int qw = wave % QW;      // which 32 queries
   const int r32 = lane % 32, h = lane / 32;
 
   const int t_first = cu_q[entry];
@@ -1109,7 +1114,7 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(
     for (int e = 0; e < 16; ++e) acc[dt][e] = 0.f;
   bool bad = false;
 
-  // A wavefront brings KG times 16 keys of its group's tile.  Load i of them: LDS rows w = i * (64 / kPieceRow) + lane / kPieceRow,
+  // A wavefront brings kRuns times 16 keys of its group's tile.  Load i of them: LDS rows w = i * (64 / kPieceRow) + lane / kPieceRow,
   // slot lane % kPieceRow; of the values: dims i * 32 + lane / 2, 8 keys each.
   unsigned k_off[kLoads];
 #pragma unroll
@@ -1120,19 +1125,19 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(
   }
   const unsigned v_off = static_cast<unsigned>(lane / 2 * block_size + lane % 2 * 8) * 2u;
   const int last_page = (k_end - 1) >> bs_shift;
-  const int my_key = qw * KG * 16;  // first key of this wavefront's share of a tile
+  const int my_key = qw * kRuns * 16;  // first key of this wavefront's share of a tile
   // The page ids come as vector loads, which are counted with the tiles' own (a scalar load on its way would turn every wait for
   // LDS into a wait for everything); they are asked for a turn ahead of their use and waited for with that turn's tile.
   const __amdgpu_buffer_rsrc_t ids_buf = make_buffer(table, static_cast<unsigned>(table_width) * 4u);
-  int ids[KG];
+  int ids[kRuns];
   auto lookup = [&](int kt0) {
 #pragma unroll
-    for (int u = 0; u < KG; ++u)
+    for (int u = 0; u < kRuns; ++u)
       ids[u] = __builtin_amdgcn_raw_buffer_load_b32(ids_buf, static_cast<unsigned>(min((kt0 + my_key + u * 16) >> bs_shift, last_page)) * 4u, 0, 0);
   };
   auto fetch = [&](int kt0, int buf) {  // with the ids that lookup(kt0) left
 #pragma unroll
-    for (int u = 0; u < KG; ++u) {
+    for (int u = 0; u < kRuns; ++u) {
       const int key0 = kt0 + my_key + u * 16;
       const int page = __builtin_amdgcn_readfirstlane(ids[u]);
       const bool in = static_cast<unsigned>(page) < static_cast<unsigned>(num_pages);
@@ -1174,7 +1179,7 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(
     const int turn0 = kt0 - group * kPromptKeys;
     if (k_end % 8 != 0 && turn0 <= k_end && k_end < turn0 + kTurn) {
       // the 8 values that the last key is among: those past it are cleared, since 0 * NaN would come through
-      const int at = k_end - kt0, d = tid % (256 / KG);
+      const int at = k_end - kt0, d = tid % (QW * kWave);
       if (at >= 0 && at < kPromptKeys && d < D) {
         u16x8_t* const piece = reinterpret_cast<u16x8_t*>(vs + (at / 16 * D + d) * 32 + at % 16 / 8 * 16);
         u16x8_t bits = *piece;
@@ -1272,30 +1277,36 @@ __global__ __launch_bounds__(256, 2) void attn_prompt_kernel(
 
   __syncthreads();  // the tiles are done with
   if constexpr (KG > 1) {
-    float* const handover = reinterpret_cast<float*>(prefill_lds);  // [component][thread of the group]
-    static_assert(KG == 1 || (2 + kDims * 16) * 128 * 4 <= prompt_lds_bytes(KG), "the handover fits the tile buffers");
-    const int at = tid % 128;
+    float* const handover = reinterpret_cast<float*>(prefill_lds);  // [group - 1][component][thread of the group]
+    constexpr int kGroup = QW * kWave, kShare = (2 + kDims * 16) * kGroup;
+    static_assert(KG == 1 || (KG - 1) * kShare * 4 <= prompt_lds_bytes(KG), "the handover fits the tile buffers");
+    const int at = tid % kGroup;
     if (group > 0) {
-      handover[at] = m_run;
-      handover[128 + at] = l_run;
+      float* const to = handover + (group - 1) * kShare + at;
+      to[0] = m_run;
+      to[kGroup] = l_run;
 #pragma unroll
       for (int dt = 0; dt < kDims; ++dt)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) handover[(2 + dt * 16 + e) * 128 + at] = acc[dt][e];
+        for (int e = 0; e < 16; ++e) to[(2 + dt * 16 + e) * kGroup] = acc[dt][e];
     }
     if (bad) atomicOr(&sm_bad, 1);
     __syncthreads();
     if (group > 0) return;
-    const float m_other = handover[at];
-    const float m_new = fmaxf(m_run, m_other);
-    const float w_mine = m_run == -INFINITY ? 0.f : fast_exp2(m_run - m_new);
-    const float w_other = m_other == -INFINITY ? 0.f : fast_exp2(m_other - m_new);
-    l_run = l_run * w_mine + handover[128 + at] * w_other;
 #pragma unroll
-    for (int dt = 0; dt < kDims; ++dt)
+    for (int other = 0; other < KG - 1; ++other) {
+      const float* const from = handover + other * kShare + at;
+      const float m_other = from[0];
+      const float m_new = fmaxf(m_run, m_other);
+      const float w_mine = m_run == -INFINITY ? 0.f : fast_exp2(m_run - m_new);
+      const float w_other = m_other == -INFINITY ? 0.f : fast_exp2(m_other - m_new);
+      l_run = l_run * w_mine + from[kGroup] * w_other;
 #pragma unroll
-      for (int e = 0; e < 16; ++e) acc[dt][e] = acc[dt][e] * w_mine + handover[(2 + dt * 16 + e) * 128 + at] * w_other;
-    m_run = m_new;
+      for (int dt = 0; dt < kDims; ++dt)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[dt][e] = acc[dt][e] * w_mine + from[(2 + dt * 16 + e) * kGroup] * w_other;
+      m_run = m_new;
+    }
   } else {
     if (bad) atomicOr(&sm_bad, 1);
     __syncthreads();
@@ -1519,7 +1530,8 @@ int64_t mlr_attention_prefill_scratch(int num_tiles, int heads, int splits, int 
 
 // Attention of the query tiles listed in `tiles` ([num_tiles][2]: entry, first
 // query of the tile within the entry's new tokens; 64 queries per tile, or
-// mlr_attention_wide_tile() with `wide`).  splits > 1: the keys of every tile are cut into that
+// mlr_attention_wide_tile() with `wide`: 1, or 2 for eight wavefronts in two groups of keys, where there is such a kernel (head size 128,
+// pages of 16 or more, one range of keys; else as 1)).  splits > 1: the keys of every tile are cut into that
 // many runs, each a workgroup of its own, and merged by a second kernel; `partial` then holds
 // mlr_attention_prefill_scratch floats.  For few tiles behind long contexts.  `extra`: as for
 // mlr_attention_decode.
@@ -1564,13 +1576,15 @@ int mlr_attention_prefill(const void* q, int64_t q_stride, const void* key_pages
       if (e == hipSuccess) e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kPrefillLds);
 #ifdef MLR_HAS_PROMPT
     {
-      const void* wide_kernels[] = {reinterpret_cast<const void*>(attn_prompt_kernel<1, false>),
-                                    reinterpret_cast<const void*>(attn_prompt_kernel<1, true>)};
-      const void* narrow_kernels[] = {reinterpret_cast<const void*>(attn_prompt_kernel<2, false>),
-                                      reinterpret_cast<const void*>(attn_prompt_kernel<2, true>)};
+      const void* wide_kernels[] = {reinterpret_cast<const void*>(attn_prompt_kernel<4, 1, false>),
+                                    reinterpret_cast<const void*>(attn_prompt_kernel<4, 1, true>)};
+      const void* grouped_kernels[] = {reinterpret_cast<const void*>(attn_prompt_kernel<2, 2, false>),
+                                       reinterpret_cast<const void*>(attn_prompt_kernel<2, 2, true>),
+                                       reinterpret_cast<const void*>(attn_prompt_kernel<kDoubleQW, 2, false>),
+                                       reinterpret_cast<const void*>(attn_prompt_kernel<kDoubleQW, 2, true>)};
       for (const void* kernel : wide_kernels)
         if (e == hipSuccess) e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, prompt_lds_bytes(1));
-      for (const void* kernel : narrow_kernels)
+      for (const void* kernel : grouped_kernels)
         if (e == hipSuccess) e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, prompt_lds_bytes(2));
     }
 #endif
@@ -1586,15 +1600,17 @@ int mlr_attention_prefill(const void* q, int64_t q_stride, const void* key_pages
   bool launched = false;
 #ifdef MLR_HAS_PROMPT
   if (block_size >= 16 && score_bias == nullptr && keep_first == 0) {
-#define MLR_PROMPT(groups, cap)                                                                                       \
-  attn_prompt_kernel<groups, cap><<<grid, 256, prompt_lds_bytes(groups), stream>>>(                                   \
+#define MLR_PROMPT(queries, groups, cap)                                                                               \
+  attn_prompt_kernel<queries, groups, cap><<<grid, queries * groups * kWave, prompt_lds_bytes(groups), stream>>>(     \
       static_cast<const bf16*>(q), q_stride, static_cast<const bf16*>(key_pages), static_cast<const bf16*>(value_pages), \
       block_table, table_width, tiles, cu_q, context_lens, static_cast<bf16*>(out), num_tiles, heads, kv_heads, bs_shift, \
       num_pages, scale, window, chunk, partial, (splits > 1 || keep_partial) ? nullptr : sinks, keep_partial, softcap)
-      if (wide && softcap > 0.f) MLR_PROMPT(1, true);
-      else if (wide) MLR_PROMPT(1, false);
-      else if (softcap > 0.f) MLR_PROMPT(2, true);
-      else MLR_PROMPT(2, false);
+      if (wide == 2 && D == 128 && softcap > 0.f) MLR_PROMPT(kDoubleQW, 2, true);
+      else if (wide == 2 && D == 128) MLR_PROMPT(kDoubleQW, 2, false);
+      else if (wide && softcap > 0.f) MLR_PROMPT(4, 1, true);
+      else if (wide) MLR_PROMPT(4, 1, false);
+      else if (softcap > 0.f) MLR_PROMPT(2, 2, true);
+      else MLR_PROMPT(2, 2, false);
 #undef MLR_PROMPT
       launched = true;
   }

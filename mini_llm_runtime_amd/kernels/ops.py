@@ -1227,17 +1227,13 @@ class HipOps:
                 enough //= 2
             behind = int(getattr(plan, "long_prefix", 0))  # 1: thousands of keys before every tile, 2: twice that
             reach = int(window or 0) or chunk
+            # long chains of keys, not much shorter in the early tiles of a prompt only because of what the mask lets them see
+            long_chains = int(getattr(plan, "longest_prompt_tiles", 0)) >= LONG_PROMPT_TILES and (not reach or 4 * reach >= 3 * QUERY_TILE * num_tiles)
             # Two rounds of narrow tiles of long prompts, heavy ones first, add up alike on every unit; one round of wide ones lasts as long as
             # its heaviest.  Narrow / wide, us: 16 heads, 2,000 tokens 37.2 / 47.5, twice 1,024 25.4 / 29.4; 8 heads, 4,096 62.9 / 89.7.  Not for
             # short prompts (16 heads, 8 of 256 16.3 / 14.0, 4 of 500 19.3 / 18.9), a mask that reaches less far than most of a prompt (2,048, a
             # window of 512 27.8 / 23.1), nor beyond two rounds (28 heads, 1,500 44.8 / 40.3).
-            in_two_rounds = (
-                alone
-                and not behind
-                and num_tiles * num_heads <= self.tuning.wide_attention_groups
-                and int(getattr(plan, "longest_prompt_tiles", 0)) >= LONG_PROMPT_TILES
-                and (not reach or 4 * reach >= 3 * QUERY_TILE * num_tiles)
-            )
+            in_two_rounds = alone and not behind and num_tiles * num_heads <= self.tuning.wide_attention_groups and long_chains
             if behind:
                 enough = enough * 3 // 4  # heavy tiles everywhere: fewer of them keep the compute units busy
             if (
@@ -1251,6 +1247,11 @@ class HipOps:
                 and lib.mlr_attention_wide_tile() == WIDE_QUERY_TILE
             ):
                 tiles, num_tiles, wide = plan.wide_query_tiles, num_wide, 1
+                # In two groups of keys, a workgroup to a compute unit: where there is one for each (behind cached tokens a second round would
+                # be as long as the first: 28 heads, 1,500 behind 4,096, 336 tiles: 145 us, in groups 155), and up to 448 of long prompts, whose
+                # second round is short (28 heads, 2,048 53.7 / 48.8, twice 1,024 34.7 / 35.9; 64 heads, 900, 512 tiles: 29.9 / 33.5).
+                if alone and (num_wide * num_heads <= 256 or (not behind and long_chains and num_wide * num_heads <= 448)):
+                    wide = 2
             self._check(tiles, "query tiles", torch.int32, (num_tiles, 2))
             # few tiles behind long contexts: as many long chains on a few compute units; their keys
             # are cut into runs with a workgroup each, merged by a second kernel
@@ -1262,7 +1263,7 @@ class HipOps:
             pays = not reach or (reach >= 1024 and groups <= 64)
             if behind == 2 and pays and groups < self.tuning.key_run_groups:
                 key_runs = min(8, -(-self.tuning.key_run_groups // groups))
-                if alone and not wide and groups <= 256:
+                if alone and wide != 1 and groups <= 256:
                     # no more of them than compute units: a workgroup more would wait for a round of its own (16 tokens behind 16,384, 40 heads:
                     # 8 runs 95 us, 6 71; 512 behind 8,192, 28 heads: 2 runs 141, 1 115; but 40 heads, 320 tiles: 1 run 214, 2 187)
                     key_runs = min(key_runs, 256 // groups)

@@ -10,13 +10,23 @@ from test_gpu_kernels import _attend, _paged_case, _rand, _tol, _wide_ops
 pytestmark = pytest.mark.gpu
 
 
-@pytest.fixture(scope="module", params=["narrow", "wide"])
+# wide: four wavefronts; groups: the same tiles by eight in two groups of keys, which the launch takes for up to 256 of them at heads of 128
+@pytest.fixture(scope="module", params=["narrow", "wide", "groups"])
 def ops(request):
     from mini_llm_runtime_amd.kernels.ops import HipOps
     from mini_llm_runtime_amd.kernels.tuning import KernelTuning
 
-    if request.param == "wide":
+    if request.param == "groups":
         return _wide_ops()
+    if request.param == "wide":
+
+        class OneGroup(HipOps):
+            def _call(self, name, *args, lib=None):
+                if name == "mlr_attention_prefill":
+                    args = (*args[:8], min(args[8], 1), *args[9:])
+                return super()._call(name, *args, lib=lib)
+
+        return OneGroup(torch.bfloat16, "cuda", tuning=KernelTuning(wide_attention_groups=1))
     return HipOps(torch.bfloat16, "cuda", tuning=KernelTuning(wide_attention_groups=1 << 30))
 
 
@@ -101,12 +111,13 @@ def test_every_workgroup_has_its_work(ops, head_dim, entries):
 
 
 # two rounds of narrow tiles or one of wide ones: long prompts up to 512 narrow tiles x heads, short ones, one tile more, masks that reach
-# three quarters of the prompts and less, cached tokens before them
+# three quarters of the prompts and less, cached tokens before them; 2: wide tiles in two groups of keys, up to 256 of them or 448 of long prompts
 @pytest.mark.parametrize(
     "heads,entries,mask,wide",
     [
-        (8, [(4096, 4096)], {}, False), (8, [(4097, 4097)], {}, True), (16, [(1024, 1024)] * 2, {}, False), (16, [(704, 704)] * 2 + [(640, 640)], {}, True),
-        (8, [(4096, 4096)], dict(window=3072), False), (8, [(4096, 4096)], dict(chunk=3071), True), (16, [(4100, 2048)], {}, True),
+        (8, [(4096, 4096)], {}, 0), (16, [(2100, 2100)], {}, 2), (16, [(1024, 1024)] * 2, {}, 0), (16, [(704, 704)] * 2 + [(640, 640)], {}, 1),
+        (8, [(4096, 4096)], dict(window=3072), 0), (8, [(4096, 4096)], dict(chunk=3071), 2), (16, [(4100, 2048)], {}, 2),
+        (28, [(2048, 2048)], {}, 2), (28, [(2049, 2049)], {}, 1), (28, [(2048, 2048)], dict(window=1000), 1), (16, [(4200, 2049)], {}, 1),
     ],
 )
 def test_two_rounds_of_narrow_tiles(heads, entries, mask, wide):
@@ -126,7 +137,7 @@ def test_two_rounds_of_narrow_tiles(heads, entries, mask, wide):
     kw = dict(num_heads=heads, num_kv_heads=1, head_dim=128, block_size=16, scale=128**-0.5, **{"window": None, **mask})
     args = (q.cuda(), kp.cuda(), vp.cuda(), table.cuda(), ctx)
     got, plain = _attend(ops, *args, **kw).cpu(), _attend(ops, *args, kernel="fma", **kw).cpu()
-    assert launches == [int(wide)]
+    assert launches == [wide]
     torch.testing.assert_close(got.double(), plain.double(), **_tol(torch.bfloat16))
 
 
