@@ -636,8 +636,9 @@ __global__ __launch_bounds__(256) void moe_gemm_mfma_kernel(const bf16* __restri
 // features w * 16 .. + 16.
 // STEP 128: 80 KB, two workgroups a compute unit with 48 KB of weights each on their way; 64: 40 KB, four with 24.  The first has
 // the whole stream under way with few workgroups, the second loses less at the end of a round of many; see narrow_steps_pay.
-// Bound by HBM: 8 tokens, 64 experts with 6 choices, matrices of 768 x 2,048, up 22.3 us, down 23.3 (up to 48 experts' 151 MB for
-// each of the two: 6.5 TB/s).
+// Bound by HBM and by how long a launch takes to begin and end: 8 tokens, 64 experts with 6 choices, matrices of 768 x 2,048: 13 experts chosen up
+// 15.0 us, down 9.6, 34 (107 MB each) 21.9 and 23.2, 48 33 and 27; a plain product of 16 tokens takes 20 to 21 us for 100 MB.  (The input
+// rows by a wavefront of their own, so that the weights never wait for their lookup: 0.5 us less each, nothing in a step.)
 constexpr int kStCols = 64;
 constexpr int kStBuffers = 4;
 constexpr int stream_buffer_bytes(int step) { return (kStCols + kMoeRows) * step * 2; }

@@ -17,9 +17,9 @@ class KernelTuning:
     # only some 15 GB/s whatever the source: beyond this many bytes of prologue input per workgroup
     # the kernel of its own is the faster way.
     fuse_bytes: int = 1 << 30
-    # The fused kernels stream weights in blocks of 16 rows, half as fast as the LDS-tiled kernel once a
-    # matrix has tens of megabytes: beyond this many bytes of weight the norm and the merge keep kernels
-    # of their own.  Decode steps at batch 1 with everything fused / with this limit: 1.5B (gate-up
+    # The merge's fused kernel streams weights in blocks of 16 rows, half as fast as the LDS-tiled kernel once a
+    # matrix has tens of megabytes, and every workgroup of the norm's repeats the norm: beyond this many bytes of
+    # weight the norm and the merge keep kernels of their own.  Decode steps at batch 1 with everything fused / with this limit: 1.5B (gate-up
     # 55 MB) 1.66 / 1.50 ms, 3B (90 MB) 2.42 / 2.25 ms, 7B (query/key/value 33 MB, output 26 MB)
     # 3.29 / 3.21 ms; the 17 MB gate-up of 0.5B stays fused (0.75 ms against 0.79).
     fuse_weight_bytes: int = 20 << 20
