@@ -1001,7 +1001,8 @@ __global__ __launch_bounds__(256 * kKeyGroups) void attn_prefill_kernel(
 // to itself (128 KB), but with two wavefronts a SIMD, so that one's softmax runs beside the other's products where there is only one workgroup
 // to a unit.  4 x 1 / 4 x 2, microseconds: 28 heads, 1,300 tokens 36.6 / 29.0, 2,048 53.7 / 48.8, 1,024 behind 4,096 112 / 88, behind 16,384
 // (4 x 1 in two runs of keys) 317 / 284; 16 heads, 3,000 70.7 / 54.8; but 28 heads, 3,000 (672 workgroups) 83 / 94.  (2 x 4 for heads of 64:
-// 14 heads, 1,024 tokens 13.6 / 12.8, 2,048 23.2 / 24.3, 4,096 53 / 65.)
+// 14 heads, 1,024 tokens 13.6 / 12.8, 2,048 23.2 / 24.3, 4,096 53 / 65.)  Errors against 64 bits of 4 x 2 are those of 2 x 2, 0.98 to 1.00 times
+// those of 4 x 1 (700 to 3,000 tokens, queries of 0.3 to 8 times the usual size).
 // CAP: capped scores.
 // Bound by the softmax's vector instructions beside the products (two wavefronts a SIMD overlap them in part).  Measured against
 // attn_prefill_kernel's best tiles, whole prompts, microseconds (TFLOP/s): 28 heads of 128: 1,024 tokens 34 to 25, 2,048 83 (362) to 54
