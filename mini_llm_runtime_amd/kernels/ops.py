@@ -160,7 +160,9 @@ _EPILOGUES = {None: 0, "swiglu": 1, "relu2": 2, "sigmoid": 3, "gelu_tanh": 4, "c
 # head sizes whose kernels every build has and whose tiles fit (attention_f32.hip)
 F32_TILE_HEAD_DIMS = tuple(d for d in build.DEFAULT_HEAD_DIMS if d <= 128)
 
-from .plans import LONG_PROMPT_TILES, PAGED_ATTENTION, QUERY_TILE, WIDE_QUERY_TILE, attention_plan, query_tiles  # noqa: F401
+from .plans import (  # noqa: F401
+    PAGED_ATTENTION, QUERY_TILE, WIDE_QUERY_TILE, attention_plan, in_key_groups, long_chains, query_tiles, uneven_chains,
+)
 
 
 class KernelError(RuntimeError):
@@ -1227,13 +1229,15 @@ class HipOps:
                 enough //= 2
             behind = int(getattr(plan, "long_prefix", 0))  # 1: thousands of keys before every tile, 2: twice that
             reach = int(window or 0) or chunk
-            # long chains of keys, not much shorter in the early tiles of a prompt only because of what the mask lets them see
-            long_chains = int(getattr(plan, "longest_prompt_tiles", 0)) >= LONG_PROMPT_TILES and (not reach or 4 * reach >= 3 * QUERY_TILE * num_tiles)
             # Two rounds of narrow tiles of long prompts, heavy ones first, add up alike on every unit; one round of wide ones lasts as long as
             # its heaviest.  Narrow / wide, us: 16 heads, 2,000 tokens 37.2 / 47.5, twice 1,024 25.4 / 29.4; 8 heads, 4,096 62.9 / 89.7.  Not for
             # short prompts (16 heads, 8 of 256 16.3 / 14.0, 4 of 500 19.3 / 18.9), a mask that reaches less far than most of a prompt (2,048, a
-            # window of 512 27.8 / 23.1), nor beyond two rounds (28 heads, 1,500 44.8 / 40.3).
-            in_two_rounds = alone and not behind and num_tiles * num_heads <= self.tuning.wide_attention_groups and long_chains
+            # window of 512 27.8 / 23.1), cached tokens before it that make all chains long (32 heads, 1,000 behind 1,500 63.7 / 61.3), nor beyond
+            # two rounds (28 heads, 1,500 44.8 / 40.3).
+            in_two_rounds = (
+                alone and not behind and num_tiles * num_heads <= self.tuning.wide_attention_groups
+                and long_chains(plan, num_tiles, reach) and uneven_chains(plan, num_tiles)
+            )
             if behind:
                 enough = enough * 3 // 4  # heavy tiles everywhere: fewer of them keep the compute units busy
             if (
@@ -1246,12 +1250,8 @@ class HipOps:
                 and getattr(plan, "wide_query_tiles", None) is not None
                 and lib.mlr_attention_wide_tile() == WIDE_QUERY_TILE
             ):
-                tiles, num_tiles, wide = plan.wide_query_tiles, num_wide, 1
-                # In two groups of keys, a workgroup to a compute unit: where there is one for each (behind cached tokens a second round would
-                # be as long as the first: 28 heads, 1,500 behind 4,096, 336 tiles: 145 us, in groups 155), and up to 448 of long prompts, whose
-                # second round is short (28 heads, 2,048 53.7 / 48.8, twice 1,024 34.7 / 35.9; 64 heads, 900, 512 tiles: 29.9 / 33.5).
-                if alone and (num_wide * num_heads <= 256 or (not behind and long_chains and num_wide * num_heads <= 448)):
-                    wide = 2
+                wide = 2 if alone and in_key_groups(plan, num_tiles, num_wide * num_heads, behind, int(window or 0), chunk) else 1
+                tiles, num_tiles = plan.wide_query_tiles, num_wide
             self._check(tiles, "query tiles", torch.int32, (num_tiles, 2))
             # few tiles behind long contexts: as many long chains on a few compute units; their keys
             # are cut into runs with a workgroup each, merged by a second kernel

@@ -13,6 +13,7 @@ QUERY_TILE = 64  # queries of one request that the prompt kernel takes together
 WIDE_QUERY_TILE = 128  # and in its variant for long prompts (two blocks of queries per wavefront)
 LONG_PREFIX_KEYS = 2048  # mean number of keys before a tile from which a step counts as behind long prefixes (twice: very long)
 LONG_PROMPT_TILES = 12  # from which a prompt counts as long (see attention_f32.hip, groups_for)
+GROUPED_TILES = 448  # wide tiles x heads of long prompts up to which they come in two groups of keys (see in_key_groups)
 PAGED_ATTENTION = "paged_attention"  # the plan's key: every mixer on these kernels shares one plan per step
 
 
@@ -28,10 +29,17 @@ def query_tiles(q_lens, q_starts=None, tile: int = QUERY_TILE) -> np.ndarray:
     return np.asarray(tiles, dtype=np.int32).reshape(-1, 2)
 
 
+def _coarse(n: int) -> int:
+    """n rounded up to four binary digits: sizes of a plan are part of a recording's identity, and few recordings are kept."""
+    unit = 1 << max(0, n.bit_length() - 4)
+    return -(-n // unit) * unit
+
+
 def attention_plan(shape: PlanInput) -> MixerPlan:
     """Tiles of 64 and of 128 queries over the entries with several new tokens (for the prompt
     kernel and its wide variant; the launch picks one by how many there are), how many of 64 the longest
-    portion has (up to where it counts as long), and
+    portion has (up to where it counts as long), for long portions that are not behind long prefixes the most keys that a
+    wide tile of the step sees and the mean over its wide tiles, and
     how many entries have a single token and how long their contexts may be (for the split-KV
     decode kernel).  `shape.max_context` bounds the contexts; a recording is made with the
     capacity of its block tables there, so that it holds for every later step of its sizes."""
@@ -46,6 +54,10 @@ def attention_plan(shape: PlanInput) -> MixerPlan:
     mean_before = sum(keys_before) / len(keys_before) if keys_before else 0
     long_prefix = int(mean_before >= LONG_PREFIX_KEYS) + int(mean_before >= 2 * LONG_PREFIX_KEYS)
     most_new = max((int(n) for n in shape.q_lens if n > 1), default=0)
+    most_keys = mean_keys = 0
+    if -(-most_new // QUERY_TILE) >= LONG_PROMPT_TILES and not long_prefix:
+        keys = [int(shape.q_starts[e]) + min(int(q0) + WIDE_QUERY_TILE, int(shape.q_lens[e])) for e, q0 in wide]
+        most_keys, mean_keys = _coarse(max(keys)), _coarse(sum(keys) // len(keys))
     return MixerPlan(
         key=PAGED_ATTENTION,
         arrays={"query_tiles": tiles, "wide_query_tiles": wide},
@@ -54,7 +66,37 @@ def attention_plan(shape: PlanInput) -> MixerPlan:
             "num_wide_query_tiles": len(wide),
             "long_prefix": long_prefix,
             "longest_prompt_tiles": min(-(-most_new // QUERY_TILE), LONG_PROMPT_TILES),
+            "most_prompt_keys": most_keys,
+            "mean_prompt_keys": mean_keys,
             "num_decode_entries": decodes,
             "max_decode_context": int(shape.max_context) if decodes else 0,
         },
     )
+
+
+def _prompt_keys(plan, num_tiles: int) -> tuple[int, int]:
+    """The most keys that a wide tile sees and the mean; of a plan that does not say, as of one prompt."""
+    most = int(getattr(plan, "most_prompt_keys", 0)) or QUERY_TILE * num_tiles
+    return most, int(getattr(plan, "mean_prompt_keys", 0)) or (most + WIDE_QUERY_TILE) // 2
+
+
+def long_chains(plan, num_tiles: int, reach: int) -> bool:
+    """Whether a step's prompts make long chains of keys, the early tiles' shorter than the late ones': long prompts (the longest counts, however
+    many there are), and a mask that reaches most of the longest (0: all of it)."""
+    if int(getattr(plan, "longest_prompt_tiles", 0)) < LONG_PROMPT_TILES:
+        return False
+    return not reach or 4 * reach >= 3 * _prompt_keys(plan, num_tiles)[0]
+
+
+def uneven_chains(plan, num_tiles: int) -> bool:
+    """Whether the tiles' chains of keys run from short to long, as a whole prompt's do, instead of being long all alike behind cached tokens."""
+    most, mean = _prompt_keys(plan, num_tiles)
+    return 5 * mean <= 3 * most + 5 * QUERY_TILE
+
+
+def in_key_groups(plan, num_tiles: int, groups: int, behind: int, window: int, chunk: int) -> bool:
+    """Whether wide tiles of heads of 128 come with their keys in two groups (eight wavefronts, a workgroup to a compute unit) or in one (four,
+    two workgroups); groups: wide tiles x heads.  In two groups where there is a unit for each (behind cached tokens a second round would
+    be as long as the first: 28 heads, 1,500 behind 4,096, 336 tiles: 145 us, in groups 155), and up to 448 of long prompts, whose
+    second round is short (28 heads, 2,048 53.7 / 48.8, twice 1,024 34.7 / 35.9; 64 heads, 900, 512 tiles: 29.9 / 33.5)."""
+    return groups <= 256 or (not behind and groups <= GROUPED_TILES and long_chains(plan, num_tiles, window or chunk))

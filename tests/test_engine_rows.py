@@ -349,3 +349,32 @@ def test_attention_plan_knows_the_longest_portion():
     assert tiles([512], [6000]) == 8 and tiles([705], [0]) == 12 and tiles([704], [0]) == 11
     assert tiles([5000], [0]) == 12, "long is long: one recording holds for all of them"
     assert tiles([1, 1, 1], [0, 5, 9]) == 0
+
+
+def _prompt_plan(portions):
+    """(plan, its tiles of 64 queries) of prompt portions (cached tokens before it, tokens)."""
+    from types import SimpleNamespace
+
+    import numpy as np
+
+    from mini_llm_runtime_amd.kernels.plans import attention_plan
+    from mini_llm_runtime_amd.parts.context import PlanInput
+
+    starts, lens = (np.array(c, dtype=np.int32) for c in zip(*portions))
+    sizes = attention_plan(PlanInput(lens, starts, 16384)).sizes
+    return SimpleNamespace(**sizes), sizes["num_query_tiles"]
+
+
+def test_long_chains_of_keys_are_the_longest_prompts():
+    from mini_llm_runtime_amd.kernels.plans import long_chains, uneven_chains
+
+    two, tiles = _prompt_plan([(0, 1024), (0, 1024)])
+    assert two.most_prompt_keys == 1024 and two.mean_prompt_keys == 576  # (128 + ... + 1,024) / 8
+    assert long_chains(two, tiles, 0) and long_chains(two, tiles, 1024) and long_chains(two, tiles, 768) and not long_chains(two, tiles, 767)
+    many, tiles = _prompt_plan([(0, 900)] + [(0, 64)] * 20)
+    assert long_chains(many, tiles, 900) and many.most_prompt_keys == 960  # 900 in four binary digits, upwards
+    assert uneven_chains(*_prompt_plan([(0, 2048)])) and uneven_chains(*_prompt_plan([(100, 1000)])) and not uneven_chains(*_prompt_plan([(1500, 1000)]))
+    short, tiles = _prompt_plan([(0, 704), (0, 704)])
+    assert not long_chains(short, tiles, 0) and short.most_prompt_keys == 0, "one recording holds for all short ones"
+    behind, _ = _prompt_plan([(6000, 2048)])
+    assert behind.most_prompt_keys == behind.mean_prompt_keys == 0 and behind.long_prefix == 2

@@ -141,6 +141,44 @@ def test_two_rounds_of_narrow_tiles(heads, entries, mask, wide):
     torch.testing.assert_close(got.double(), plain.double(), **_tol(torch.bfloat16))
 
 
+# prompts in one step under a mask that reaches all of each, and long portions whose tiles all have cached tokens before them
+@pytest.mark.parametrize(
+    "heads,entries,mask,wide",
+    [(16, [(1792, 1792)] * 2, dict(window=1792), 2), (16, [(1792, 1792)] * 2, dict(window=1100), 1), (16, [(1024, 1024)] * 2, dict(chunk=1024), 0),
+     (32, [(2500, 1000)], {}, 2), (32, [(1100, 1000)], {}, 0)],
+)
+def test_forms_by_the_longest_prompt(heads, entries, mask, wide):
+    _check_form(heads, entries, mask, wide)
+
+
+def _check_form(heads, entries, mask, wide):
+    """The form that the launch takes for a step with this plan (as in the test above), and its result."""
+    import numpy as np
+
+    from mini_llm_runtime_amd.kernels.ops import HipOps
+    from mini_llm_runtime_amd.kernels.plans import attention_plan
+    from mini_llm_runtime_amd.parts.context import PlanInput
+
+    launches = []
+
+    class Spying(HipOps):
+        def _call(self, name, *args, lib=None):
+            if name == "mlr_attention_prefill":
+                launches.append(int(args[8]))
+            return super()._call(name, *args, lib=lib)
+
+    ops = Spying(torch.bfloat16, "cuda")
+    q, kp, vp, table, ctx, *_ = _paged_case(entries, heads, 1, 128, 16, torch.bfloat16, 61)
+    lens, starts = [np.array(n, dtype=np.int32) for n in ([n for _, n in entries], [c - n for c, n in entries])]
+    for name, value in attention_plan(PlanInput(lens, starts, max(c for c, _ in entries))).sizes.items():
+        setattr(ctx, name, value)
+    kw = dict(num_heads=heads, num_kv_heads=1, head_dim=128, block_size=16, scale=128**-0.5, **{"window": None, **mask})
+    args = (q.cuda(), kp.cuda(), vp.cuda(), table.cuda(), ctx)
+    got, plain = _attend(ops, *args, **kw).cpu(), _attend(ops, *args, kernel="fma", **kw).cpu()
+    assert launches == [wide]
+    torch.testing.assert_close(got.double(), plain.double(), **_tol(torch.bfloat16))
+
+
 def test_a_page_that_is_not_there(ops):
     q, kp, vp, table, ctx, *_ = _paged_case([(100, 100), (300, 300)], 2, 1, 64, 16, torch.bfloat16, 54)
     table = table.clone()
