@@ -96,7 +96,23 @@ def uneven_chains(plan, num_tiles: int) -> bool:
 
 def in_key_groups(plan, num_tiles: int, groups: int, behind: int, window: int, chunk: int) -> bool:
     """Whether wide tiles of heads of 128 come with their keys in two groups (eight wavefronts, a workgroup to a compute unit) or in one (four,
-    two workgroups); groups: wide tiles x heads.  In two groups where there is a unit for each (behind cached tokens a second round would
-    be as long as the first: 28 heads, 1,500 behind 4,096, 336 tiles: 145 us, in groups 155), and up to 448 of long prompts, whose
-    second round is short (28 heads, 2,048 53.7 / 48.8, twice 1,024 34.7 / 35.9; 64 heads, 900, 512 tiles: 29.9 / 33.5)."""
-    return groups <= 256 or (not behind and groups <= GROUPED_TILES and long_chains(plan, num_tiles, window or chunk))
+    two workgroups); groups: wide tiles x heads.  In microseconds, one / two groups:
+    Up to 256, one round: the chain is halved.  28 heads, 1,024 behind 4,096 112 / 90, 16 heads, 4 of 512 19.0 / 17.1, 8 of 256 13.8 / 13.4; not up
+    to three tiles of keys, which end before the groups have met: 8 of 192 10.5 / 10.9, 16 of 128 11.4 / 11.7 (behind 300 cached tokens 20.9 / 22.3), 2,048
+    in a window of 64 13.5 / 13.8 (of 80 15.5 / 14.6), in chunks of 128 11.6 / 11.9 (of 160 14.4 / 13.6).
+    Beyond, where the second round is short: a unit takes some groups / 256 chains of the mean length one after the other, and at least the 256th
+    and the 257th longest; in one group the longest decides.  1.4 most - 487 keys is where both took the same over 175 steps of whole prompts and
+    behind some cached tokens: 28 heads, 2,048 53.9 / 49.4, twice 1,024 32.6 / 34.0, 1,024, 512 and 256 together 31.7 / 28.0, twice 896 29.2 / 30.2,
+    twice 768 26.3 / 26.2; 32 heads, 1,596 42.0 / 38.1; 16 heads, 3,000 70 / 56; 64 heads, 760 behind 300 34.9 / 38.3; 40 heads, 1,000 behind 900 51.4 /
+    56.6; 28 heads, 1,300 behind 500 48.6 / 44.6, 1,500 behind 1,200 68.1 / 70.6.  From 449 to 512 it would hold as well (28 heads, 2,304 61.2 / 57.2,
+    twice 1,152 37.0 / 38.1), beyond there is a third round (28 heads, 2,432 65.9 / 67.3).  Behind long prefixes a second round is as long as the
+    first: 28 heads, 1,500 behind 4,096 145 / 155."""
+    if groups <= 256:
+        if behind or window:
+            return bool(behind) or window + WIDE_QUERY_TILE - 1 > 3 * QUERY_TILE
+        tiles = int(getattr(plan, "longest_prompt_tiles", 0))  # 0: not known
+        return chunk > 2 * QUERY_TILE if chunk else not 0 < tiles <= 3
+    most, mean = _prompt_keys(plan, num_tiles)
+    if behind or groups > GROUPED_TILES or not long_chains(plan, num_tiles, window or chunk):
+        return False
+    return max(mean * groups / 256, 2 * most - 1024 * (most - mean) / groups) < 1.4 * most - 487

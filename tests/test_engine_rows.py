@@ -378,3 +378,29 @@ def test_long_chains_of_keys_are_the_longest_prompts():
     assert not long_chains(short, tiles, 0) and short.most_prompt_keys == 0, "one recording holds for all short ones"
     behind, _ = _prompt_plan([(6000, 2048)])
     assert behind.most_prompt_keys == behind.mean_prompt_keys == 0 and behind.long_prefix == 2
+
+
+def test_key_groups_by_the_chains_of_a_round():
+    """The rule over its whole range: never for a step whose second round would outlast one group's longest chain, by the
+    tiles themselves."""
+    import random
+
+    from mini_llm_runtime_amd.kernels.plans import GROUPED_TILES, in_key_groups
+
+    rng = random.Random(3)
+    for _ in range(400):
+        heads = rng.choice([8, 12, 16, 28, 40, 64])
+        portions = [(rng.choice([0, 0, rng.randrange(1600)]), rng.randrange(2, 3000)) for _ in range(rng.randrange(1, 6))]
+        plan, tiles = _prompt_plan(portions)
+        groups = plan.num_wide_query_tiles * heads
+        chosen = in_key_groups(plan, tiles, groups, plan.long_prefix, 0, 0)
+        if groups > GROUPED_TILES or (groups > 256 and (plan.long_prefix or plan.longest_prompt_tiles < 12)):
+            assert not chosen
+        elif groups <= 256:
+            assert chosen == bool(plan.long_prefix or plan.longest_prompt_tiles > 3)
+        elif chosen:
+            keys = [before + min(q0 + 128, n) for before, n in portions for q0 in range(0, n, 128)]
+            # sizes are known to an eighth, upwards
+            assert sum(keys) * heads / 256 < 1.4 * 1.125 * max(keys) - 487
+    whole = lambda n, heads: in_key_groups(*_prompt_plan([(0, n)]), -(-n // 128) * heads, 0, 0, 0)  # noqa: E731
+    assert [whole(n, 32) for n in (1152, 1600, 1792, 1920)] == [True, True, True, False] and [whole(n, 64) for n in (768, 896)] == [False, False]

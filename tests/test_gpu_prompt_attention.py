@@ -151,6 +151,21 @@ def test_forms_by_the_longest_prompt(heads, entries, mask, wide):
     _check_form(heads, entries, mask, wide)
 
 
+# wide tiles in one group of keys or two: one round and chains of three key tiles or more, short ones behind masks; two rounds of long prompts whose
+# chains are long enough for their number, alike or not, of portions with few and with many cached tokens
+@pytest.mark.parametrize(
+    "heads,entries,mask,wide",
+    [
+        (16, [(192, 192)] * 8, {}, 1), (16, [(256, 256)] * 8, {}, 2), (8, [(600, 128)] * 32, {}, 1), (16, [(2048, 2048)], dict(window=65), 1),
+        (16, [(2048, 2048)], dict(window=66), 2), (16, [(2048, 2048)], dict(chunk=128), 1), (16, [(2048, 2048)], dict(chunk=160), 2),
+        (28, [(1024, 1024)] * 2, {}, 1), (28, [(1024, 1024), (512, 512), (256, 256)], {}, 2), (28, [(896, 896)] * 2, {}, 1), (28, [(1280, 1280)], {}, 2),
+        (40, [(1900, 1000)], {}, 1), (28, [(1800, 1300)], {}, 2), (28, [(2048, 2048)], {}, 2), (28, [(2049, 2049)], {}, 1),
+    ],
+)
+def test_one_group_of_keys_or_two(heads, entries, mask, wide):
+    _check_form(heads, entries, mask, wide)
+
+
 def _check_form(heads, entries, mask, wide):
     """The form that the launch takes for a step with this plan (as in the test above), and its result."""
     import numpy as np
