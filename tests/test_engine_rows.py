@@ -404,3 +404,13 @@ def test_key_groups_by_the_chains_of_a_round():
             assert sum(keys) * heads / 256 < 1.4 * 1.125 * max(keys) - 487
     whole = lambda n, heads: in_key_groups(*_prompt_plan([(0, n)]), -(-n // 128) * heads, 0, 0, 0)  # noqa: E731
     assert [whole(n, 32) for n in (1152, 1600, 1792, 1920)] == [True, True, True, False] and [whole(n, 64) for n in (768, 896)] == [False, False]
+
+
+def test_tiles_of_short_prompts_come_by_what_they_see():
+    from mini_llm_runtime_amd.kernels.plans import query_tiles
+
+    lens, starts = [43, 329, 93, 1, 303, 206], [0, 0, 0, 9, 0, 64]
+    for tile in (64, 128):
+        seen = [(starts[e] + q0, starts[e] + min(q0 + tile, lens[e])) for e, q0 in query_tiles(lens, starts, tile)]
+        assert seen == sorted(seen, reverse=True), "first the keys before a tile, then those that it sees"
+    assert query_tiles([43, 128, 93, 128], tile=128).tolist() == [[1, 0], [3, 0], [2, 0], [0, 0]], "equal ones in the order of their entries"
