@@ -146,11 +146,10 @@ int mlr_qkv_bf16_staged(int m, int n, int k, int head_dim, int block_size);
 // x_out (another buffer than x_in; null when nothing is added) receives x_in + delta.  Then
 // y = h w^T with the epilogues of mlr_gemm_bf16 (bias, float32 output, SwiGLU), or the
 // query/key/value epilogue of mlr_qkv_rope_write_bf16.  k a multiple of 8, at most 2048.
-// row_blocks: 0 chooses how many blocks of 16 features a workgroup owns, or 1, 2.
 int mlr_gemm_norm_fused_bf16(const float* x_in, float* x_out, const void* delta, const float* partial, int slices_in,
                              const void* norm_weight, int norm_weight_is_f32, float eps, const void* w,
-                             const void* bias, int bias_is_f32, void* y, int out_is_f32, int swiglu, int row_blocks,
-                             int m, int n, int k, hipStream_t stream);
+                             const void* bias, int bias_is_f32, void* y, int out_is_f32, int swiglu, int m, int n, int k,
+                             hipStream_t stream);
 int mlr_qkv_norm_fused_bf16(const float* x_in, float* x_out, const void* delta, const float* partial, int slices_in,
                             const void* norm_weight, int norm_weight_is_f32, float eps, const void* w,
                             const void* bias, int bias_is_f32, const float* cos, const float* sin, const int* slots,

@@ -117,7 +117,7 @@ _SIGNATURES = {
         _I,
     ),
     "mlr_gemm_norm_fused_bf16": (
-        [_VP, _VP, _VP, _VP, _I, _VP, _I, _F, _VP, _VP, _I, _VP, _I, _I, _I, _I, _I, _I, _VP],
+        [_VP, _VP, _VP, _VP, _I, _VP, _I, _F, _VP, _VP, _I, _VP, _I, _I, _I, _I, _I, _VP],
         _I,
     ),
     "mlr_qkv_norm_fused_bf16": (
@@ -739,7 +739,7 @@ class HipOps:
             y = self._empty((m, n // 2 if swiglu else n), out_dtype)
             self._call(
                 "mlr_gemm_norm_fused_bf16", *norm_args, self._ptr(weight), self._ptr(bias), bias_f32, self._ptr(y),
-                int(out_dtype == torch.float32), epilogue, 0, m, n, k, self._stream(),
+                int(out_dtype == torch.float32), epilogue, m, n, k, self._stream(),
             )
             x.residual = residual
             return y
