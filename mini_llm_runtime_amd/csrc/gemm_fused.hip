@@ -18,8 +18,14 @@
 // Behind the norm the weights stream as in gemm_lines (gemm_norm_lines): whole lines straight into LDS, asked for by four wavefronts before
 // the norm is there, which others make.  A workgroup has as many rows as make one round of the compute units, and one prologue.  Against 16 rows a
 // workgroup through registers, 64 bytes of a row a load, the norm by the same wavefronts (one token, 4 slices to add up, microseconds in a replayed graph, weights from
-// memory): 9,728 x 896 8.6 to 7.0 (4 tokens 10.6 to 7.6), 4,864 x 896 6.6 to 5.5, 5,120 x 2,048 10.6 to 7.7, 6,144 x 1,536 9.7 to 7.1, 2,048 x 2,048 7.4 to 5.9;
-// query/key/value 1,152 x 896 5.3 to 5.0, 2,560 x 2,048 7.7 to 7.0.  (One loss: rows off whole lines that need two rounds, 17,920 x 560 8.9 to 10.2.)
+// memory): 9,728 x 896 8.7 to 6.0 (4 tokens 10.7 to 6.5), 4,864 x 896 6.7 to 4.5, 5,120 x 2,048 11.0 to 6.7, 6,144 x 1,536 10.2 to 6.1, 2,048 x 2,048 7.5 to 5.3;
+// query/key/value 1,152 x 896 5.4 to 4.4, 2,560 x 2,048 7.9 to 6.1.  Over 972 products of all forms (1 to 4 tokens, up to 16 slices) 0.75 of the time,
+// two slower by more than 2 % (18,000 x 520, 4 tokens, 2 slices 11.0 to 11.5).
+// In one round the norm's loads go first: its rows come from L2, and behind some 30 KB of weights from memory they would wait for those
+// (9,728 x 896 7.3 instead of 6.0; query/key/value 3,072 x 1,024, 4 tokens, 8 slices 7.0 instead of 5.7, 6.2 through registers).
+// Beyond one round (MANY) other workgroups' loads fill that time, and what counts is how many fit a unit: no more LDS than the steps of k fill
+// (16 KB up to 256 columns) and one partial sum at a time (65 registers).  17,920 x 560 10.1 to 9.4 (10.5 with two workgroups a unit), 40,000 x
+// 256 13.5 to 7.6 (11.8).
 // Behind the merge they stream as in gemm_skinny_split: a workgroup owns 16 * NT output
 // features and one slice of K, its four wavefronts split K, range-checked buffer loads
 // keep two batches of eight 16-byte loads per lane in flight, the first of them issued
@@ -63,7 +69,7 @@ constexpr int fused_depth(int row_blocks) { return row_blocks == 1 ? 8 : 4; }
 // row (the stream, the delta, up to a batch of partial sums, the norm's weights), `finish` adds
 // up, takes the statistics and writes the normed row to LDS: one trip to L2.  Columns past the end are range-checked
 // away; what is absent (no delta, fewer partial sums than the batch holds) is not asked for: a load of an empty range
-// costs as much of the unit's way to memory as any (1,152 x 896, 4 tokens, nothing to add, microseconds: 4.8 so, 4.3 without).
+// costs as much of the unit's way to memory as any (query/key/value 1,152 x 896, 4 tokens, nothing to add, microseconds: 5.8 so, 5.4 without).
 //
 // Every workgroup reads the same few rows; were they all to read them in the same order, the
 // whole chip would ask the same few L2 channels for the same lines at the same moment.  So a
@@ -80,7 +86,7 @@ __device__ __forceinline__ u32x2 buffer_load_u32x2(__amdgpu_buffer_rsrc_t rsrc, 
 __device__ __forceinline__ float bf16_low(uint32_t pair) { return __builtin_bit_cast(float, pair << 16); }
 __device__ __forceinline__ float bf16_high(uint32_t pair) { return __builtin_bit_cast(float, pair & 0xffff0000u); }
 
-// SB: partial sums per trip: 8 of rows of up to 1,024 columns, 4 of longer ones (two wavefronts a SIMD have the registers for them).
+// SB: partial sums per trip: 8 of rows of up to 1,024 columns, 4 of longer ones (two wavefronts a SIMD have the registers for them), or 1.
 template <int VPT, int SB>
 struct NormRow {
   unsigned at[VPT];  // byte offset of this lane's columns within a float32 row, out of range past the end
@@ -388,23 +394,25 @@ __global__ __launch_bounds__(kFusedWaves* kWave) void gemm_few_fused_kernel(cons
 // The norm prologue with the weights streamed as by gemm_lines (gemm_mfma.hip): four wavefronts bring whole lines of 128 bytes of RUNS * 8
 // rows straight into LDS, each the lines of its own steps of 64 k through buffers of its own, and up to four others
 // norm a token's row each meanwhile.  (Wavefronts of their own: loads into registers and into LDS do not return in one order.)
+// BUF: slices of LDS a wavefront.  MANY: more workgroups than one round of the compute units.
 constexpr int norm_line_buffers(int runs) { return runs > 6 ? 3 : 4; }
-constexpr int norm_line_bytes(int runs) { return 4 * norm_line_buffers(runs) * runs * 1024; }
+constexpr int norm_line_bytes(int runs, int buffers) { return kFusedWaves * buffers * runs * 1024; }
+constexpr int norm_slice_batch(int vpt, bool many) { return many ? 1 : 32 / vpt; }
 
-template <int RUNS, int VPT, bool QKV>
+template <int RUNS, int VPT, bool QKV, int BUF, bool MANY>
 __device__ __forceinline__ void norm_lines(const bf16* __restrict__ w, const GemmEpilogue& ep, const QkvTarget& qkv, const NormPrologue& np, int ldk, int M, int N, int K) {
-  constexpr int NB = (RUNS + 1) / 2, BUF = norm_line_buffers(RUNS);
+  constexpr int NB = (RUNS + 1) / 2;
   static_assert(!QKV || RUNS % 2 == 0, "a block of 16 holds 8 dims and their partners");
   extern __shared__ __attribute__((aligned(16))) unsigned char fused_lds[];
-  bf16* const hb = reinterpret_cast<bf16*>(fused_lds + norm_line_bytes(RUNS));
+  bf16* const hb = reinterpret_cast<bf16*>(fused_lds + norm_line_bytes(RUNS, BUF));
   const int lane = threadIdx.x % kWave;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int steps = (K + 63) / 64;
   if (wave >= kFusedWaves) {
     const int row = wave - kFusedWaves;
-    NormRow<VPT, 32 / VPT> t;
+    NormRow<VPT, norm_slice_batch(VPT, MANY)> t;
     norm_issue(np, t, row, M, K);
-    __builtin_amdgcn_s_barrier();  // from here on the others send theirs
+    if (!MANY) __builtin_amdgcn_s_barrier();  // from here on the others send theirs
     norm_finish(np, t, hb, ldk, row, M, K, steps * 64);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
@@ -444,7 +452,7 @@ __device__ __forceinline__ void norm_lines(const bf16* __restrict__ w, const Gem
           w_buf, (__attribute__((address_space(3))) void*)(fused_lds + ((wave * BUF + it % BUF) * RUNS + p) * 1024), 16, at, 0, 0, 2);
     }
   };
-  __builtin_amdgcn_s_barrier();  // the norm's loads are on their way: behind these they would wait for memory
+  if (!MANY) __builtin_amdgcn_s_barrier();  // the norm's loads are on their way: behind these they would wait for memory
   asm volatile("" ::: "memory");
 #pragma unroll
   for (int i = 0; i < BUF; ++i) fetch(i);
@@ -499,21 +507,21 @@ __device__ __forceinline__ void norm_lines(const bf16* __restrict__ w, const Gem
   }
 }
 
-template <int RUNS, int VPT, bool QKV>
+template <int RUNS, int VPT, bool QKV, int BUF, bool MANY>
 __global__ __launch_bounds__(2 * kFusedWaves* kWave) void gemm_norm_lines_kernel(const bf16* __restrict__ w, GemmEpilogue ep, QkvTarget qkv, NormPrologue np,
                                                                                  int ldk, int M, int N, int K) {
-  norm_lines<RUNS, VPT, QKV>(w, ep, qkv, np, ldk, M, N, K);
+  norm_lines<RUNS, VPT, QKV, BUF, MANY>(w, ep, qkv, np, ldk, M, N, K);
 }
 
-template <int RUNS, int VPT, bool QKV>
+template <int RUNS, int VPT, bool QKV, int BUF = norm_line_buffers(RUNS), bool MANY = false>
 static int launch_norm_lines(const bf16* w, const GemmEpilogue& ep, const QkvTarget& qkv, const NormPrologue& np, int m, int n, int k,
                              hipStream_t stream, const char* who) {
   const int ldk = (k + 63) / 64 * 64 + 8;  // padded so that the rows of an operand load fall into different banks
-  const int lds = norm_line_bytes(RUNS) + m * ldk * 2;
-  constexpr int kMost = norm_line_bytes(RUNS) + kFusedWaves * (2048 + 8) * 2;
+  const int lds = norm_line_bytes(RUNS, BUF) + m * ldk * 2;
+  constexpr int kMost = norm_line_bytes(RUNS, BUF) + kFusedWaves * (2048 + 8) * 2;
   static bool configured = false;
   if (!configured) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_norm_lines_kernel<RUNS, VPT, QKV>),
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_norm_lines_kernel<RUNS, VPT, QKV, BUF, MANY>),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, kMost);
     if (e != hipSuccess) {
       set_error(std::string(who) + ": cannot raise the LDS limit: " + hipGetErrorString(e));
@@ -521,12 +529,13 @@ static int launch_norm_lines(const bf16* w, const GemmEpilogue& ep, const QkvTar
     }
     configured = true;
   }
-  gemm_norm_lines_kernel<RUNS, VPT, QKV><<<(n + RUNS * 8 - 1) / (RUNS * 8), (kFusedWaves + m) * kWave, lds, stream>>>(w, ep, qkv, np, ldk, m, n, k);
+  gemm_norm_lines_kernel<RUNS, VPT, QKV, BUF, MANY>
+      <<<(n + RUNS * 8 - 1) / (RUNS * 8), (kFusedWaves + m) * kWave, lds, stream>>>(w, ep, qkv, np, ldk, m, n, k);
   return 0;
 }
 
-// Runs of 8 rows a workgroup: the fewest that make one round of the compute units, 4 where none does (two workgroups a unit).  Microseconds in a replayed
-// graph, weights from memory, one token, with 1, 2, 3, 4, 5, 6 and 8 runs: 9,728 x 896 (1,216 runs) -, 9.7, 7.3, 7.8, 7.0, 7.1, 7.6; 4,864 x 896 -, 5.9, 5.5, 5.6, 6.1,
+// Runs of 8 rows a workgroup: the fewest that make one round of the compute units, 4 where none does.  Microseconds in a replayed
+// graph, weights from memory, one token (before the norm's loads went first, and with 64 KB of LDS beyond one round), with 1, 2, 3, 4, 5, 6 and 8 runs: 9,728 x 896 (1,216 runs) -, 9.7, 7.3, 7.8, 7.0, 7.1, 7.6; 4,864 x 896 -, 5.9, 5.5, 5.6, 6.1,
 // 6.4, 7.2; 2,048 x 2,048 5.9, 6.2, 6.7, 7.5, 8.2, 8.8, 10; 10,000 x 1,000 12.1, 10.4, 8.6, 9.3, 8.0, 8.5, 9.5; 14,336 x 512 11.7, 9.2, 8.2, 6.5, 9.3, 9.6, 6.5;
 // 20,000 x 512 15.9, 11.3, 10.4, 9.1, 10.1, 10.1, 10.8.
 static int norm_runs(int n, int multiple) {
@@ -538,6 +547,14 @@ static int norm_runs(int n, int multiple) {
 template <bool QKV>
 static int norm_lines_any(int runs, const bf16* w, const GemmEpilogue& ep, const QkvTarget& qkv, const NormPrologue& np, int m, int n, int k,
                           hipStream_t stream, const char* who) {
+  if (n > 256 * 64) {  // more than one round: four runs
+    const int iterations = ((k + 63) / 64 + kFusedWaves - 1) / kFusedWaves;
+    if (k > 1024) return launch_norm_lines<4, 8, QKV, 4, true>(w, ep, qkv, np, m, n, k, stream, who);
+    if (iterations == 1) return launch_norm_lines<4, 4, QKV, 1, true>(w, ep, qkv, np, m, n, k, stream, who);
+    if (iterations == 2) return launch_norm_lines<4, 4, QKV, 2, true>(w, ep, qkv, np, m, n, k, stream, who);
+    if (iterations == 3) return launch_norm_lines<4, 4, QKV, 3, true>(w, ep, qkv, np, m, n, k, stream, who);
+    return launch_norm_lines<4, 4, QKV, 4, true>(w, ep, qkv, np, m, n, k, stream, who);
+  }
 #define MLR_NORM_LINES(RUNS)                                                                              \
   case RUNS:                                                                                              \
     return k <= 1024 ? launch_norm_lines<RUNS, 4, QKV>(w, ep, qkv, np, m, n, k, stream, who)              \

@@ -73,29 +73,52 @@ def test_norm_as_the_prologue_of_a_product(ops, m, n, k, delta, weight_f32):
     assert torch.equal(again, got)
 
 
+@pytest.fixture(scope="module")
+def any_size(gpu_device):
+    """The norm in front of products of every size (the launch keeps matrices of more than 20 MB to kernels of their own), and what was launched."""
+    from mini_llm_runtime_amd.kernels.ops import HipOps
+
+    class Spying(HipOps):
+        def _call(self, name, *args, lib=None):
+            self.called.append(name)
+            return super()._call(name, *args, lib=lib)
+
+    ops = Spying(torch.bfloat16, gpu_device, tuning=KernelTuning(fuse_weight_bytes=1 << 30))
+    ops.called = []
+    return ops
+
+
 # 1, 2, 3, 4, 5, 6 and 8 runs of 8 rows a workgroup, and 4 where no number makes one round: the last workgroup has a run of three rows or one row, or
-# none of its second half; k ends inside a line, inside a step of 64 and inside the wavefronts' turns, and is longer than the buffers hold
+# none of its second half; k ends inside a line, inside a step of 64 and inside the wavefronts' turns (1,096: 18 steps, five turns of the first
+# two wavefronts), takes one to four turns, and more than the three or four that the buffers hold
 @pytest.mark.parametrize("n", [2043, 2051, 4099, 6145, 8195, 10244, 12291, 16387])
-@pytest.mark.parametrize("m,k", [(1, 200), (3, 1096), (4, 72)])
-def test_norm_prologue_with_every_number_of_rows_a_workgroup(ops, n, m, k):
+@pytest.mark.parametrize("m,k", [(1, 200), (3, 1096), (4, 72), (2, 456), (1, 712), (4, 1000), (2, 2048)])
+def test_norm_prologue_with_every_number_of_rows_a_workgroup(any_size, n, m, k):
+    ops = any_size
     x, d = _rand((m, k), torch.float32, 96, 2.0).cuda(), _rand((3, m, k), torch.float32, 97, 0.3).cuda()
     nw, w, b = (1 + _rand((k,), torch.float32, 98, 0.1)).cuda(), _rand((n, k), torch.bfloat16, 99, 0.05).cuda(), _rand((n,), torch.float32, 95).cuda()
     h = ops.rmsnorm(x.clone(), nw, 1e-5, delta=d)  # the same rows, rounded alike
     ref = h.double() @ w.double().t() + b.double()
+    ops.called.clear()
     got = ops.linear(ops.defer_norm(x, nw, 1e-5, d), w, b, out_dtype=torch.float32).double()
+    assert ops.called == ["mlr_gemm_norm_fused_bf16"]
     # k roundings of float32 sums, and where the norm's own sum falls to the other side of a rounding a bfloat16 step of one
     # activation in a few hundred
     bound = k * 2.0**-24 * (h.double().abs() @ w.double().abs().t()) + 2.0**-8 * h.abs().max() * w.abs().max().double() * 4
     assert ((got - ref).abs() <= bound).all()
 
 
-@pytest.mark.parametrize("heads,kv_heads,head_dim", [(64, 2, 64), (100, 4, 80), (192, 2, 64)])
-def test_norm_prologue_of_wide_query_key_value_products(ops, heads, kv_heads, head_dim):
-    """4, 6 and 8 runs of 8 rows a workgroup: the same queries and pages as by the norm kernel and the product."""
-    tokens, k, bs, pages = 3, 136, 8, 4
+# 2, 4, 6 and 8 runs of 8 rows a workgroup, and 4 beyond one round; one turn of the wavefronts, and more than the buffers hold
+@pytest.mark.parametrize("heads,kv_heads,head_dim", [(20, 2, 64), (64, 2, 64), (100, 4, 80), (192, 2, 64), (258, 1, 64)])
+@pytest.mark.parametrize("k", [136, 1096, 2048])
+def test_norm_prologue_of_wide_query_key_value_products(any_size, heads, kv_heads, head_dim, k):
+    """The same queries and pages as by the norm kernel and the product."""
+    ops = any_size
+    tokens, bs, pages = 3, 8, 4
     width = (heads + 2 * kv_heads) * head_dim
     x, d = _rand((tokens, k), torch.float32, 91, 2.0).cuda(), _rand((2, tokens, k), torch.float32, 92, 0.3).cuda()
-    nw, w, b = (1 + _rand((k,), torch.float32, 93, 0.1)).cuda(), _rand((width, k), torch.bfloat16, 94, 0.2).cuda(), _rand((width,), torch.float32, 95).cuda()
+    # products of a size that does not grow with k
+    nw, w, b = (1 + _rand((k,), torch.float32, 93, 0.1)).cuda(), _rand((width, k), torch.bfloat16, 94, 2.33 * k**-0.5).cuda(), _rand((width,), torch.float32, 95).cuda()
     cos, sin = ops.rope_table(torch.tensor([3, 911, 40000], dtype=torch.int32).cuda(), (1.0 / (1e6 ** (torch.arange(0, head_dim, 2, dtype=torch.float64) / head_dim))).cuda())
     slots = torch.tensor([5, -1, 30], dtype=torch.int32).cuda()
     outs = []
@@ -103,9 +126,11 @@ def test_norm_prologue_of_wide_query_key_value_products(ops, heads, kv_heads, he
         kp = torch.zeros(pages, kv_heads, bs, head_dim, dtype=torch.bfloat16, device="cuda")
         vp = torch.zeros(pages, kv_heads, head_dim, bs, dtype=torch.bfloat16, device="cuda")
         h = ops.defer_norm(x, nw, 1e-5, d) if fused else ops.rmsnorm(x.clone(), nw, 1e-5, delta=d)
+        ops.called.clear()
         q = ops.qkv_rope_write(
             h, w, b, (cos, sin, head_dim), slots, kp, vp, num_heads=heads, num_kv_heads=kv_heads, head_dim=head_dim, block_size=bs,
         )
+        assert (ops.called == ["mlr_qkv_norm_fused_bf16"]) == fused
         outs.append((q[:, : heads * head_dim].float(), kp.float(), vp.float()))
     for fused, plain_ones in zip(*outs):
         # sums of another order may round to the next bfloat16 before and behind the rotation
