@@ -8,6 +8,8 @@
 //    all units are busy: tiles of 64 x 64, 64 features x 32 tokens or 32 x 32, the smaller ones also with two groups of wavefronts that
 //    take the steps of k in turn (f32_time).  Tiles are loaded straight into LDS (rows of 32 floats are the 128 bytes of the bfloat16 kernels'
 //    rows of 64, swizzled the same way), one step on its way.  Products whose consumer adds up partial sums are cut along k.
+//    The order of a sum over k depends on the number of groups and of slices, and those on the number of tokens: the same token in
+//    a step of another size may differ in its last bits (1,152 x 896 has two groups at 391 and 826 tokens, one at 512 and 1,024).
 //  * gemm_f32_few: up to 64 tokens.  Bound by streaming w once: 16 weight rows a workgroup, whose eight wavefronts split k and
 //    add their sums through LDS.
 // Measured at 0.5B sizes and 826 tokens, against the plain kernel (gemm_simple.hip, 64 x 64 tiles of vector multiply-adds with
@@ -235,7 +237,8 @@ static void launch_f32(const float* x, const float* w, const F32Epilogue& ep, in
 // wavefronts half as often); and weights too large for the caches come from memory once for every row of tiles, with half the lines of a page
 // open where tiles have 32 rows of them.  Constants fitted to 621 products (65 to 2,100 tokens, 64 to 20,000 features, k of 80 to 9,000): what the
 // estimate chooses is 2.2 % over the best on average, 29 % at worst, 17 % of them by more than 5 %, and 22 % under 64 x 64 tiles everywhere; against the
-// kernel of 32 x 32 x 2 blocks over 573 other products 0.77 of the time on average, 5 of them slower by more than 3 %, one by 16 %.  64 x 64,
+// kernel of 32 x 32 x 2 blocks over 856 other products 0.76 of the time on average, 18 of them slower by more than 3 %: weights of 13 MB and more in 64 x 64 with a
+// k under 500 (1,164 x 4,071 x 488 52.8 to 56.0), and in 64 x 32 of two to five rounds (556 x 4,014 x 7,972, the worst, 1.31; 536 x 4,630 x 4,724 1.08).  64 x 64,
 // 64 x 32, 32 x 32 alone and with two groups, microseconds: 826 x 9,728 x 896 116, 121, 131, 138; 391 75, 65, 69, 75; 200 46, 41, 40, 42; 66 32, 22, 21,
 // 21; 826 x 1,152 x 896 21, 20, 20, 20 (64 x 32 with two groups 19); 391 21, 14, 13, 13 (12); 200 21, 14, 13, 8.8 (12); 1,794 x 5,692 x 3,916 (weights of
 // 89 MB) 657, 840, 845, 785.
@@ -265,6 +268,14 @@ static int f32_way(int m, int n, int k, int slices) {
     if (i > 0 && (m + 32 * t.tt - 1) / (32 * t.tt) >= 65536) continue;
     const double time = f32_time(t, m, n, k, slices) * (i == 0 ? 0.96 : 1.0);  // near the line the largest tile is the safer choice
     if (time < least) least = time, best = i;
+  }
+  // Six workgroups of 64 x 32 fit a compute unit (24 KB each): a seventh begins when one of them has ended, which the estimate, all beside one another, does
+  // not see.  With up to a round of those 64 x 64 (five to a unit, up to 1,280 at once) is faster.  32 x 32 x 2 blocks / 64 x 32 / 64 x 64, microseconds: 325 x
+  // 9,511 x 1,360 100 / 110 / 93, 1,450 x 2,194 x 3,464 232 / 254 / 219, 386 x 7,598 x 6,460 419 / 449 / 395, 854 x 3,651 x 7,532 1.07 and 0.94 of
+  // the first; one of 17 such products is slower so (804 x 3,789 x 3,512, 3 %).
+  if (best == 1 && slices == 1) {
+    const int64_t tiles = static_cast<int64_t>((m + 31) / 32) * ((n + 63) / 64);
+    if (tiles > 6 * 256 && tiles <= 7 * 256) best = 0;
   }
   return best;
 }

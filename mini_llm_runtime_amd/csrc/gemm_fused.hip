@@ -69,7 +69,7 @@ constexpr int fused_depth(int row_blocks) { return row_blocks == 1 ? 8 : 4; }
 // row (the stream, the delta, up to a batch of partial sums, the norm's weights), `finish` adds
 // up, takes the statistics and writes the normed row to LDS: one trip to L2.  Columns past the end are range-checked
 // away; what is absent (no delta, fewer partial sums than the batch holds) is not asked for: a load of an empty range
-// costs as much of the unit's way to memory as any (query/key/value 1,152 x 896, 4 tokens, nothing to add, microseconds: 5.8 so, 5.4 without).
+// costs as much of the unit's way to memory as any (query/key/value 1,152 x 896, 4 tokens, nothing to add, microseconds: 5.7 so, 5.3 without).
 //
 // Every workgroup reads the same few rows; were they all to read them in the same order, the
 // whole chip would ask the same few L2 channels for the same lines at the same moment.  So a

@@ -56,6 +56,14 @@ def test_every_tiling(ops, tiling, m, n, k, slices):
     assert ((got - ref).abs() <= bound + 2.0**-23 * (ref.abs() + b.abs().double())).all()
 
 
+# 64 x 32 tiles up to six to a compute unit and beyond seven, 64 x 64 between; in slices of k as before
+@pytest.mark.parametrize(
+    "m,n,k,slices,tiling", [(480, 6528, 800, 1, 211), (325, 9511, 1360, 1, 221), (1120, 3264, 1540, 1, 221), (218, 16503, 800, 1, 211), (545, 2049, 420, 3, 211)]
+)
+def test_tiling_of_a_round_that_begins_late(ops, m, n, k, slices, tiling):
+    assert ops.lib.mlr_gemm_f32_tiling(m, n, k, slices) == tiling
+
+
 @pytest.mark.parametrize("m", [5, 40, 70])
 @pytest.mark.parametrize("epilogue", ["swiglu", "clamped", "geglu", "relu2", "sigmoid", "gelu_tanh", "multiply", "rows"])
 def test_epilogues_are_the_plain_kernels(ops, m, epilogue):
