@@ -1532,7 +1532,7 @@ int64_t mlr_attention_prefill_scratch(int num_tiles, int heads, int splits, int 
 // Attention of the query tiles listed in `tiles` ([num_tiles][2]: entry, first
 // query of the tile within the entry's new tokens; 64 queries per tile, or
 // mlr_attention_wide_tile() with `wide`: 1, or 2 for eight wavefronts in two groups of keys, where there is such a kernel (head size 128,
-// pages of 16 or more, one range of keys; else as 1)).  splits > 1: the keys of every tile are cut into that
+// pages of 16 or more, softmax weights over one range of keys; else as 1)).  splits > 1: the keys of every tile are cut into that
 // many runs, each a workgroup of its own, and merged by a second kernel; `partial` then holds
 // mlr_attention_prefill_scratch floats.  For few tiles behind long contexts.  `extra`: as for
 // mlr_attention_decode.

@@ -5,28 +5,27 @@ from __future__ import annotations
 import pytest
 import torch
 
-from test_gpu_kernels import _attend, _paged_case, _rand, _tol, _wide_ops
+from test_gpu_kernels import _attend, _paged_case, _rand, _tol
 
 pytestmark = pytest.mark.gpu
 
 
-# wide: four wavefronts; groups: the same tiles by eight in two groups of keys, which the launch takes for up to 256 of them at heads of 128
+# wide: four wavefronts; groups: the same tiles by eight in two groups of keys at heads of 128, whichever the launch would take (plans.in_key_groups)
 @pytest.fixture(scope="module", params=["narrow", "wide", "groups"])
 def ops(request):
     from mini_llm_runtime_amd.kernels.ops import HipOps
     from mini_llm_runtime_amd.kernels.tuning import KernelTuning
 
-    if request.param == "groups":
-        return _wide_ops()
-    if request.param == "wide":
+    if request.param != "narrow":
+        form = 1 if request.param == "wide" else 2
 
-        class OneGroup(HipOps):
+        class OneForm(HipOps):
             def _call(self, name, *args, lib=None):
-                if name == "mlr_attention_prefill":
-                    args = (*args[:8], min(args[8], 1), *args[9:])
+                if name == "mlr_attention_prefill" and args[8]:
+                    args = (*args[:8], form, *args[9:])
                 return super()._call(name, *args, lib=lib)
 
-        return OneGroup(torch.bfloat16, "cuda", tuning=KernelTuning(wide_attention_groups=1))
+        return OneForm(torch.bfloat16, "cuda", tuning=KernelTuning(wide_attention_groups=1))
     return HipOps(torch.bfloat16, "cuda", tuning=KernelTuning(wide_attention_groups=1 << 30))
 
 
@@ -96,6 +95,25 @@ def test_a_key_that_outweighs_the_others(ops, head_dim):
     kw = dict(num_heads=2, num_kv_heads=1, head_dim=head_dim, block_size=16, scale=0.6931471805599453, window=None)
     got = _attend(ops, q.cuda(), kp.cuda(), vp.cuda(), table.cuda(), ctx, **kw).cpu()
     assert torch.equal(got[late:].view(n - late, 2, head_dim), values.expand(n - late, 2, head_dim))
+
+
+# long prompts and portions whose tiles leave their sums for the merge that takes the pooled entries' share in: tiles without any, with few, with
+# a part of a run past a page; one more query than a tile has
+@pytest.mark.parametrize("heads,kv_heads,head_dim,block", [(4, 1, 128, 16), (6, 2, 64, 16), (2, 2, 128, 32)])
+@pytest.mark.parametrize("window,pool", [(300, 4), (65, 7)])
+@pytest.mark.parametrize("sink", [False, True])
+def test_pooled_entries_beside_the_tiles(ops, heads, kv_heads, head_dim, block, window, pool, sink):
+    entries = [(1300, 1300), (900, 129), (331, 5), (64, 64), (700, 1)]
+    q, kp, vp, table, ctx, *_ = _paged_case(entries, heads, kv_heads, head_dim, block, torch.bfloat16, 62)
+    pooled_kp, pooled_vp, pooled_table = _paged_case([(-(-c // pool), 1) for c, _ in entries], heads, kv_heads, head_dim, block, torch.bfloat16, 63)[1:4]
+    kw = dict(num_heads=heads, num_kv_heads=kv_heads, head_dim=head_dim, block_size=block, scale=head_dim**-0.5, window=window)
+    kw["pooled"] = (pooled_kp.cuda(), pooled_vp.cuda(), pooled_table.cuda(), pool)
+    if sink:
+        kw["sinks"] = _rand((heads,), torch.float32, 64, 2.0).cuda()
+    args = (q.cuda(), kp.cuda(), vp.cuda(), table.cuda(), ctx)
+    got, plain = _attend(ops, *args, **kw).cpu(), _attend(ops, *args, kernel="fma", **kw).cpu()
+    assert torch.isfinite(plain).all()
+    torch.testing.assert_close(got.double(), plain.double(), **_tol(torch.bfloat16))
 
 
 # workgroups (entries x heads) around one and two to every compute unit, and many more; entries of unequal contexts
