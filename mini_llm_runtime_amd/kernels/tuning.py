@@ -19,9 +19,11 @@ class KernelTuning:
     fuse_bytes: int = 1 << 30
     # The merge's fused kernel streams weights in blocks of 16 rows, half as fast as the LDS-tiled kernel once a
     # matrix has tens of megabytes, and every workgroup of the norm's repeats the norm: beyond this many bytes of
-    # weight the norm and the merge keep kernels of their own.  Decode steps at batch 1 with everything fused / with this limit: 1.5B (gate-up
-    # 55 MB) 1.66 / 1.50 ms, 3B (90 MB) 2.42 / 2.25 ms, 7B (query/key/value 33 MB, output 26 MB)
-    # 3.29 / 3.21 ms; the 17 MB gate-up of 0.5B stays fused (0.75 ms against 0.79).
+    # weight the norm and the merge keep kernels of their own.  Decode steps at batch 1 with everything fused / with this limit, both prologues as the
+    # merge's is: 1.5B (gate-up 55 MB) 1.66 / 1.50 ms, 3B (90 MB) 2.42 / 2.25 ms, 7B (query/key/value 33 MB, output 26 MB) 3.29 / 3.21 ms.
+    # The norm's kernel by itself, fused / apart, one token, 4 slices to add up, microseconds: 16,384 x 512 (17 MB) 5.9 / 8.3, 10,240 x 1,024 (21 MB) 6.4 / 8.9,
+    # 8,192 x 2,048 (34 MB) 9.3 / 12.2, 16,384 x 1,280 (42 MB) 9.7 / 16.5, 13,000 x 2,048 (53 MB) 12.4 / 15.3, and beyond the 16,384 rows of one
+    # round of workgroups 40,000 x 512 (41 MB) 13.0 / 13.0, 20,480 x 1,024 (42 MB) 15.0 / 13.4, 22,016 x 2,048 (90 MB) 23.6 / 22.5.
     fuse_weight_bytes: int = 20 << 20
     # Prompt attention takes tiles of 128 queries instead of 64 once tiles x heads reach this many
     # workgroups (fewer leave compute units idle behind the heaviest tiles).
