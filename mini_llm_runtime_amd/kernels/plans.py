@@ -110,10 +110,12 @@ def in_key_groups(plan, num_tiles: int, groups: int, behind: int, window: int, c
     twice 1,152 37.0 / 38.1), beyond there is a third round (28 heads, 2,432 65.9 / 67.3).  Behind long prefixes a second round is as long as the
     first: 28 heads, 1,500 behind 4,096 145 / 155."""
     if groups <= 256:
-        if behind or window:
-            return bool(behind) or window + WIDE_QUERY_TILE - 1 > 3 * QUERY_TILE
         tiles = int(getattr(plan, "longest_prompt_tiles", 0))  # 0: not known
-        return chunk > 2 * QUERY_TILE if chunk else not 0 < tiles <= 3
+        if behind:
+            return True
+        if 0 < (window or chunk) < 8 * QUERY_TILE:  # what a tile sees, cached tokens before it or not
+            return window + WIDE_QUERY_TILE - 1 > 3 * QUERY_TILE if window else chunk > 2 * QUERY_TILE
+        return not 0 < tiles <= 3
     most, mean = _prompt_keys(plan, num_tiles)
     if behind or groups > GROUPED_TILES or not long_chains(plan, num_tiles, window or chunk):
         return False

@@ -174,7 +174,7 @@ def test_forms_by_the_longest_prompt(heads, entries, mask, wide):
 @pytest.mark.parametrize(
     "heads,entries,mask,wide",
     [
-        (16, [(192, 192)] * 8, {}, 1), (16, [(256, 256)] * 8, {}, 2), (8, [(600, 128)] * 32, {}, 1), (16, [(2048, 2048)], dict(window=65), 1),
+        (16, [(192, 192)] * 8, {}, 1), (16, [(256, 256)] * 8, {}, 2), (16, [(128, 128)] * 16, dict(window=4096), 1), (16, [(256, 256)] * 8, dict(chunk=512), 2), (8, [(600, 128)] * 32, {}, 1), (16, [(2048, 2048)], dict(window=65), 1),
         (16, [(2048, 2048)], dict(window=66), 2), (16, [(2048, 2048)], dict(chunk=128), 1), (16, [(2048, 2048)], dict(chunk=160), 2),
         (28, [(1024, 1024)] * 2, {}, 1), (28, [(1024, 1024), (512, 512), (256, 256)], {}, 2), (28, [(896, 896)] * 2, {}, 1), (28, [(1280, 1280)], {}, 2),
         (40, [(1900, 1000)], {}, 1), (28, [(1800, 1300)], {}, 2), (28, [(2048, 2048)], {}, 2), (28, [(2049, 2049)], {}, 1),
